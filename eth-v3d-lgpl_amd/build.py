@@ -24,9 +24,12 @@ HIP_FLAGS = [
     # packed FP32 instructions are kept out of every kernel
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
-# per-source additions: the sampled check's probe keeps its MFMA accumulators in ordinary
-# VGPRs (the default form moved every accumulator through AGPRs, 32 extra moves per tile)
-HIP_SOURCE_FLAGS = {"v3dm_check.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+# per-source additions: the sampled check's probe and the split score pass keep their MFMA
+# accumulators in ordinary VGPRs (the default form moved every accumulator through AGPRs, 32
+# extra moves per tile); the split pass takes finite sets only, and without NaN semantics its
+# maxima need no canonicalising instruction per operand
+HIP_SOURCE_FLAGS = {"v3dm_check.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                    "v3dm_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-fno-honor-nans"]}
 HIP_SOURCES = ["v3dm_fp32.hip", "v3dm_select.hip", "v3dm_short.hip", "v3dm_api.cpp", "v3dm_ext.cpp", "v3dm_batch.cpp",
                "v3dm_learned.cpp", "v3dm_features.cpp",
                "v3dm_voctree.cpp", "v3dm_ransac.cpp"]

@@ -19,6 +19,7 @@
 #include "v3dm_kernels.h"
 #include "v3dm_ext.h"
 #include "v3dm_context.h"
+#include "v3dm_split.h"
 
 using namespace v3dm;
 
@@ -66,6 +67,11 @@ void releaseBuffers(v3dm_context* h)
     freeDev(h->dR);
     freeDev(h->normL);
     freeDev(h->normR);
+    freeDev(h->splitL);
+    freeDev(h->splitR);
+    freeDev(h->splitInfo);
+    if (h->splitFitHost) (void)hipHostFree(h->splitFitHost);
+    h->splitFitHost = h->splitFitDev = nullptr;
     freeDev(h->maxNormBits);
     freeDev(h->colPart);
     freeDev(h->rowPart);
@@ -128,8 +134,6 @@ BatchState*& ctx_batch(v3dm_context* h) { return h->batch; }
 LearnedState*& ctx_learned(v3dm_context* h) { return h->learned; }
 int ctx_fail(v3dm_context* h, int code, const char* msg) { return fail(h, code, "%s", msg); }
 
-// Enqueue the plain FP32 exact path for the current features; leaves colMax/rowMax
-// decided and the compacted pairs + counters in h->results.
 int prof_begin(v3dm_context* h)
 {
     if (!h->profiling) return V3DM_OK;
@@ -149,6 +153,27 @@ int prof_end(v3dm_context* h)
     return V3DM_OK;
 }
 
+bool split_fits(v3dm_context const* h) { return h->splitFitHost[0] && h->splitFitHost[1]; }
+
+FusedPlan score_plan(v3dm_context const* h)
+{
+    return split_fits(h) ? plan_split(h->nL, h->nR) : plan_fused_fp32(h->nL, h->nR, 512);
+}
+
+void launch_score_pass(v3dm_context* h, FusedPlan const& p, unsigned const* bits, float minScore)
+{
+    hipStream_t const st = h->stream;
+    if (split_fits(h))
+        launch_split_pass(h->splitL, h->splitR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, bits,
+                          h->capL, minScore, st);
+    else if (bits)
+        launch_guided_fp32(h->dL, h->dR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, bits, h->capL, st);
+    else
+        launch_fused_fp32(h->dL, h->dR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, st);
+}
+
+// Enqueue the plain FP32 exact path for the current features; leaves colMax/rowMax
+// decided and the compacted pairs + counters in h->results.
 int enqueue_plain(v3dm_context* h, float minScore, float minRatio)
 {
     hipStream_t const st = h->stream;
@@ -156,9 +181,9 @@ int enqueue_plain(v3dm_context* h, float minScore, float minRatio)
     bool const work = nL > 0 && nR > 0;
     int rc;
     if (work) {
-        FusedPlan const p = plan_fused_fp32(nL, nR, 512);
+        FusedPlan const p = score_plan(h);
         if ((rc = prof_begin(h))) return rc;
-        launch_fused_fp32(h->dL, h->dR, nL, nR, p, h->colPart, h->capL, h->rowPart, h->capR, st);
+        launch_score_pass(h, p, nullptr, minScore);
         if ((rc = prof_end(h))) return rc;
         launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
                             h->normR, h->maxNormBits, h->epsRel, minScore, minRatio, h->colMax, h->rowMax,
@@ -243,6 +268,14 @@ int v3dm_allocate(v3dm_handle h, int nMaxLeft, int nMaxRight, int useGuidedMatch
     HIPCHECK(h, hipMemsetAsync(h->dR, 0, cr * kDim * sizeof(float), h->stream));
     HIPCHECK(h, hipMalloc(&h->normL, cl * sizeof(float)));
     HIPCHECK(h, hipMalloc(&h->normR, cr * sizeof(float)));
+    auto split_rows = [](int cap) { return (size_t)roundUp(cap, kSplitRowPad); };
+    HIPCHECK(h, hipMalloc(&h->splitL, split_rows(h->capL) * kSplitRowBytes));
+    HIPCHECK(h, hipMalloc(&h->splitR, split_rows(h->capR) * kSplitRowBytes));
+    HIPCHECK(h, hipMalloc(&h->splitInfo, kPrepInfo * sizeof(int)));
+    HIPCHECK(h, hipMemsetAsync(h->splitInfo, 0, kPrepInfo * sizeof(int), h->stream));
+    HIPCHECK(h, hipHostMalloc(&h->splitFitHost, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+    HIPCHECK(h, hipHostGetDevicePointer((void**)&h->splitFitDev, h->splitFitHost, 0));
+    h->splitFitHost[0] = h->splitFitHost[1] = 0;
     HIPCHECK(h, hipMalloc(&h->maxNormBits, 4 * sizeof(unsigned int)));
     HIPCHECK(h, hipMemsetAsync(h->maxNormBits, 0, 4 * sizeof(unsigned int), h->stream));
     HIPCHECK(h, hipMalloc(&h->colPart, (size_t)kMaxSplits * cl * sizeof(Top2)));
@@ -310,11 +343,23 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
     ext_quiesce(h);  // the sampled check's side stream reads the features
     float* dst = left ? h->dL : h->dR;
     size_t const bytes = (size_t)n * kDim * sizeof(float);
+    RowSource from = kRowsInPlace;
     if (n > 0) {
         if (kind == kHostF32) {
             HIPCHECK(h, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream));
         } else if (kind == kDeviceF32) {
-            HIPCHECK(h, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, h->stream));
+            // the row kernel reads this device's own memory, apart from the set's buffer and
+            // aligned for its loads; any other pointer the copy engine takes is copied first
+            char const *s0 = static_cast<char const*>(src), *d0 = reinterpret_cast<char const*>(dst);
+            bool const apart = s0 + bytes <= d0 || d0 + bytes <= s0;
+            hipPointerAttribute_t at{};
+            bool const known = hipPointerGetAttributes(&at, src) == hipSuccess;
+            if (!known) (void)hipGetLastError();
+            if (known && at.type == hipMemoryTypeDevice && at.device == h->device && apart &&
+                (reinterpret_cast<uintptr_t>(src) & 7) == 0)
+                from = kRowsF32;
+            else
+                HIPCHECK(h, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, h->stream));
         } else {
             size_t const qb = (size_t)(left ? h->capL : h->capR) * kDim;
             if (h->dQBytes < qb) {
@@ -323,12 +368,12 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
                 h->dQBytes = qb;
             }
             HIPCHECK(h, hipMemcpyAsync(h->dQ, src, (size_t)n * kDim, hipMemcpyHostToDevice, h->stream));
-            launch_dequant_u8(h->dQ, n, dst, h->stream);
+            from = kRowsU8;
         }
     }
-    unsigned int* mx = h->maxNormBits + (left ? 0 : 1);
-    HIPCHECK(h, hipMemsetAsync(mx, 0, sizeof(unsigned int), h->stream));
-    launch_norms(dst, n, left ? h->normL : h->normR, mx, h->stream);
+    launch_split_rows(from, from == kRowsU8 ? (void const*)h->dQ : src, dst, n, left ? h->normL : h->normR,
+                      h->maxNormBits + (left ? 0 : 1), left ? h->splitL : h->splitR, h->splitInfo,
+                      h->splitFitDev + (left ? 0 : 1), h->stream);
     HIPCHECK(h, hipGetLastError());
     HIPCHECK(h, hipStreamSynchronize(h->stream));
     if (left) h->nL = n;
@@ -415,10 +460,9 @@ int runGuided(v3dm_context* h, int kind, const double M[9], float distanceThresh
     h->masks.push_back(gm);
     int rc;
     if (work) {
-        FusedPlan const p = plan_fused_fp32(nL, nR, 512);
+        FusedPlan const p = score_plan(h);
         if ((rc = prof_begin(h))) return rc;
-        launch_guided_fp32(h->dL, h->dR, nL, nR, p, h->colPart, h->capL, h->rowPart, h->capR, h->guidedBits,
-                           h->capL, st);
+        launch_score_pass(h, p, h->guidedBits, minScore);
         if ((rc = prof_end(h))) return rc;
         launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
                             h->normR, h->maxNormBits, h->epsRel, minScore, minRatio, h->colMax, h->rowMax,
@@ -676,7 +720,10 @@ int v3dm_score_block(v3dm_handle h, int mode, int nRows, int nCols, float* score
     float* d = nullptr;
     size_t const bytes = (size_t)nRows * nCols * sizeof(float);
     HIPCHECK(h, hipMalloc(&d, bytes));
-    launch_score_block(mode, h->dL, h->dR, nRows, nCols, d, h->stream);
+    if (mode == V3DM_PREC_FP32 && split_fits(h))
+        launch_score_block_split(h->splitL, h->splitR, nRows, nCols, d, h->stream);
+    else
+        launch_score_block(mode, h->dL, h->dR, nRows, nCols, d, h->stream);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(scores, d, bytes, hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
@@ -702,10 +749,9 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
     int launches = 0, rc = V3DM_OK;
     if (h->precision == V3DM_PREC_FP32) {
         if (h->nL > 0 && h->nR > 0) {
-            FusedPlan const p = plan_fused_fp32(h->nL, h->nR, 512);
+            FusedPlan const p = score_plan(h);
             e = hipEventRecord(a, h->stream);
-            for (int r = 0; r < reps && e == hipSuccess; ++r)
-                launch_fused_fp32(h->dL, h->dR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, h->stream);
+            for (int r = 0; r < reps && e == hipSuccess; ++r) launch_score_pass(h, p, nullptr, h->lastMinScore);
             if (e == hipSuccess) e = hipEventRecord(b, h->stream);
             launches = reps;
         }

@@ -37,6 +37,11 @@ struct v3dm_context {
     float* dR = nullptr;
     float* normL = nullptr;
     float* normR = nullptr;
+    unsigned char* splitL = nullptr;  // rows in two FP16 parts (v3dm_split.h), written with the norms
+    unsigned char* splitR = nullptr;
+    int* splitInfo = nullptr;         // scratch of launch_split_rows
+    int* splitFitHost = nullptr;      // mapped: [0] left, [1] right set in the split pass's range
+    int* splitFitDev = nullptr;       // the same memory as the kernels address it
     unsigned int* maxNormBits = nullptr;  // [0] = left, [1] = right
     v3dm::Top2* colPart = nullptr;
     v3dm::Top2* rowPart = nullptr;

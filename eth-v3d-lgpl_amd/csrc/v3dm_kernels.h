@@ -78,9 +78,6 @@ struct MutualWait {
 void launch_mutual_compact(int const* colMax, int const* rowMax, int nL, int nR, unsigned long long* status,
                            unsigned epoch, int* stripes, int2* pairs, int* counters, hipStream_t st,
                            SampleOut const& so = {}, MutualWait const& mw = {});
-// uint8 SIFT descriptors -> floats, as SIFT_Feature::normalizeDescriptor
-// (V3D/Base/v3d_feature.h:30-38): var = sum q^2, d = q * (1/sqrtf(var)), IEEE rounding.
-void launch_dequant_u8(uint8_t const* q, int n, float* out, hipStream_t st);
 
 // plain FP32 fused score + top-2 kernel (v3dm_fp32.hip)
 FusedPlan plan_fused_fp32(int nL, int nR, int targetGroups, int maxSplits = kMaxSplits);

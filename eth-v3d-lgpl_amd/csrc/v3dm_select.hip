@@ -7,6 +7,7 @@
 // mutual check).
 #include "v3dm_device.h"
 #include "v3dm_kernels.h"
+#include "v3dm_split.h"
 
 namespace v3dm {
 
@@ -43,6 +44,137 @@ void launch_norms(float const* X, int n, float* norm, unsigned int* maxNormBits,
 {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_norms, dim3((n + 63) / 64), dim3(256), 0, st, X, n, norm, maxNormBits);
+}
+
+// ------------------------------------------------------------------------------ row preparation
+// Per row: the FP32 row (from a device array, from uint8 components, or in place), its norm
+// (summed as k_norms does) and its split parts, in one launch: the set is read once, where a
+// copy or a dequantisation, a fill of the maximum and k_norms took three launches.  A wave
+// takes 8 rows at a time, all loads in flight before the first reduction (k_norms waits for
+// each row's load in its turn: 14 us for any set up to 16384 rows).  Every work-group leaves
+// its largest norm and range flag in a slot and takes a ticket; the last one publishes the
+// set's (at most kPrepGroups work-groups, so one thread each reads a slot).  The slots are
+// device-coherent stores waited for before the ticket, not fenced: a fence would write back
+// the XCD's whole L2 (22 us for 512 work-groups).
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+constexpr int kPrepRows = 8;  // rows per wave and round
+
+__device__ __forceinline__ void split_pair(float2 v, unsigned& hi, unsigned& lo)
+{
+    float const x = v.x * kSplitScale, y = v.y * kSplitScale;
+    v2h const h = {(_Float16)x, (_Float16)y};
+    v2h const l = {(_Float16)(x - (float)h.x), (_Float16)(y - (float)h.y)};
+    hi = __builtin_bit_cast(unsigned, h);
+    lo = __builtin_bit_cast(unsigned, l);
+}
+
+template <int kFrom>
+__global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src, float* __restrict__ X, int n,
+                                                    float* __restrict__ norm, unsigned int* __restrict__ maxNormBits,
+                                                    unsigned char* __restrict__ split, int* __restrict__ info,
+                                                    int* __restrict__ hostFit)
+{
+    __shared__ unsigned int wmax[4];
+    __shared__ int wbad[4];
+    __shared__ int last;
+    int const lane = threadIdx.x & 63;
+    int const wave = threadIdx.x >> 6;
+    unsigned int mx = 0;
+    bool bad = false;
+    for (int row0 = (blockIdx.x * 4 + wave) * kPrepRows; row0 < n; row0 += gridDim.x * 4 * kPrepRows) {
+        float2 v[kPrepRows];
+        if constexpr (kFrom == kRowsU8) {
+            uchar2 q[kPrepRows];
+#pragma unroll
+            for (int k = 0; k < kPrepRows; ++k)
+                q[k] = (row0 + k < n) ? static_cast<uchar2 const*>(src)[(size_t)(row0 + k) * 64 + lane]
+                                      : make_uchar2(0, 0);
+#pragma unroll
+            for (int k = 0; k < kPrepRows; ++k)
+                v[k] = (row0 + k < n) ? dequant_u8_wave(q[k]) : make_float2(0.0f, 0.0f);
+        } else {
+            float2 const* const rows = kFrom == kRowsF32 ? static_cast<float2 const*>(src)
+                                                         : reinterpret_cast<float2 const*>(X);
+#pragma unroll
+            for (int k = 0; k < kPrepRows; ++k)
+                v[k] = (row0 + k < n) ? rows[(size_t)(row0 + k) * 64 + lane] : make_float2(0.0f, 0.0f);
+        }
+        float s[kPrepRows];
+#pragma unroll
+        for (int k = 0; k < kPrepRows; ++k) s[k] = v[k].x * v[k].x + v[k].y * v[k].y;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int k = 0; k < kPrepRows; ++k) s[k] += __shfl_xor(s[k], o);
+#pragma unroll
+        for (int k = 0; k < kPrepRows; ++k) {
+            float const nr = sqrtf(s[k]);
+            mx = max(mx, __float_as_uint(nr));  // norms are >= 0 or NaN: a NaN wins
+            bad = bad || !(nr == 0.0f || (nr >= kSplitNormMin && nr < kSplitNormMax));
+            if (row0 + k >= n) break;  // uniform over the wave; rows past n are zero above
+            if (lane == 0) norm[row0 + k] = nr;
+            if (kFrom != kRowsInPlace) reinterpret_cast<float2*>(X)[(size_t)(row0 + k) * 64 + lane] = v[k];
+            unsigned hi, lo;
+            split_pair(v[k], hi, lo);
+            unsigned* o = reinterpret_cast<unsigned*>(split + (size_t)(row0 + k) * kSplitRowBytes + (lane >> 5) * 256);
+            o[lane & 31] = hi;
+            o[32 + (lane & 31)] = lo;
+        }
+    }
+    if (lane == 0) {
+        wmax[wave] = mx;
+        wbad[wave] = bad;
+    }
+    __syncthreads();
+    int* const slot = info + kPrepSlot;  // two ints per work-group
+    if (threadIdx.x == 0) {
+        unsigned int const m = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+        int const f = wbad[0] | wbad[1] | wbad[2] | wbad[3];
+        __hip_atomic_store(slot + 2 * blockIdx.x, (int)m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(slot + 2 * blockIdx.x + 1, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        int const t = __hip_atomic_fetch_add(info, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = t == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    unsigned int m = 0;
+    int f = 0;
+    if (threadIdx.x < gridDim.x) {
+        m = (unsigned int)__hip_atomic_load(slot + 2 * threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        f = __hip_atomic_load(slot + 2 * threadIdx.x + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        m = max(m, __shfl_xor(m, o));
+        f |= __shfl_xor(f, o);
+    }
+    __syncthreads();
+    if (lane == 0) {
+        wmax[wave] = m;
+        wbad[wave] = f;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    *maxNormBits = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+    *hostFit = !(wbad[0] | wbad[1] | wbad[2] | wbad[3]);
+    __hip_atomic_store(info, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+void launch_split_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNormBits,
+                       unsigned char* split, int* info, int* hostFit, hipStream_t st)
+{
+    if (n <= 0) return;
+    int const per = 4 * kPrepRows;
+    dim3 const grid(min((n + per - 1) / per, kPrepGroups));
+    if (from == kRowsU8)
+        hipLaunchKernelGGL(k_split_rows<kRowsU8>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, info,
+                           hostFit);
+    else if (from == kRowsF32)
+        hipLaunchKernelGGL(k_split_rows<kRowsF32>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, info,
+                           hostFit);
+    else
+        hipLaunchKernelGGL(k_split_rows<kRowsInPlace>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split,
+                           info, hostFit);
 }
 
 // ------------------------------------------------------------------------------ merge + decide
@@ -420,23 +552,6 @@ void launch_mutual_compact(int const* colMax, int const* rowMax, int nL, int nR,
     int const nb = (nL + kMutualSlice - 1) / kMutualSlice;
     hipLaunchKernelGGL(k_mutual, dim3(nb > 0 ? nb : 1), dim3(256), 0, st, colMax, rowMax, nL, nR, status, epoch,
                        stripes, pairs, counters, so, mw);
-}
-
-// ------------------------------------------------------------------------------ uint8 dequantisation
-// One wave per descriptor, 2 components per lane (dequant_u8_wave).
-__global__ __launch_bounds__(256) void k_dequant_u8(uint8_t const* __restrict__ q, int n, float* __restrict__ out)
-{
-    int const lane = threadIdx.x & 63;
-    int const row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= n) return;
-    uchar2 const v = reinterpret_cast<uchar2 const*>(q + (size_t)row * kDim)[lane];
-    reinterpret_cast<float2*>(out + (size_t)row * kDim)[lane] = dequant_u8_wave(v);
-}
-
-void launch_dequant_u8(uint8_t const* q, int n, float* out, hipStream_t st)
-{
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_dequant_u8, dim3((n + 3) / 4), dim3(256), 0, st, q, n, out);
 }
 
 // ------------------------------------------------------------------------------ sampled check

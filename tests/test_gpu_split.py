@@ -1,0 +1,145 @@
+"""GPU tests of the plain form's score pass on FP16 parts (csrc/v3dm_split.hip) against the
+oracle at the edges of its tiles (32 right features, 32-feature column blocks, 256-feature
+work-groups, splits of the right features), at the edge of its range rule (row norms of 0 or
+in [2^-10, 2); any other set takes the FP32 instruction), for every source of the rows, and
+with thresholds that make it look for every position.
+
+The match set and the per-feature decisions must equal the oracle's.  The pass's scores must
+lie within 2^-18 |q| |c| of FP64: parts that keep 2^-22 of each component and a dropped
+product of 2^-22, 24 FP32 accumulations of at most 2^-23 each: 3 * 2^-22 + 24 * 2^-23 < 2^-18
+(v3dm_split.h), and 2^-39 sqrt(128) (|q| + |c|) from the smallest FP16 number.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import v3dmatch
+from oracle import oracle
+from v3dmatch import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def matcher():
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(2304, 2304)
+    yield m
+    m.close()
+
+
+def _pair(nL, nR, seed):
+    qL, qR, _ = synth.make_pair(nL, nR, 0.5, config=1, pair=seed)
+    return synth.dequantise(qL), synth.dequantise(qR)
+
+
+def _check(m, L, R, min_score=0.9, min_ratio=0.8):
+    got = m.find_putative_matches_array(min_score, min_ratio)
+    assert np.array_equal(got, oracle.find_putative_matches(L, R, min_score, min_ratio))
+    cm, rm = m.get_maxima()
+    S = oracle.scores(L, R)
+    assert np.array_equal(cm, oracle.column_maxima(S, min_score, min_ratio))
+    assert np.array_equal(rm, oracle.row_maxima(S, min_score, min_ratio))
+    return got
+
+
+def _set(m, L, R):
+    m.setLeftFeatures(L.shape[0], L)
+    m.setRightFeatures(R.shape[0], R)
+
+
+@pytest.mark.parametrize("nL,nR", [(32, 32), (64, 32), (32, 64), (96, 96), (224, 64), (256, 2304), (288, 32),
+                                   (320, 992), (2304, 32), (2272, 2080)])
+@pytest.mark.parametrize("min_score,min_ratio", [(0.9, 0.8), (-2.0, -1.0), (0.4, 0.99)])
+def test_tile_edges(matcher, nL, nR, min_score, min_ratio):
+    L, R = _pair(nL, nR, nL + nR)
+    _set(matcher, L, R)
+    _check(matcher, L, R, min_score, min_ratio)
+
+
+@pytest.mark.parametrize("factor", [2.0 ** -9, 2.0 ** -11, 1.875, 2.5, 2.0 ** -70, 2.0 ** 40])
+@pytest.mark.parametrize("both", [True, False])
+def test_range_rule(matcher, factor, both):
+    """Scaled sets on both sides of the range rule (2^-11, 2.5, 2^-70 and 2^40 are outside)."""
+    L, R = _pair(352, 416, 3)
+    L = (L * np.float32(factor)).astype(np.float32)
+    R = (R * np.float32(factor)).astype(np.float32) if both else R
+    _set(matcher, L, R)
+    scale = factor * factor if both else factor
+    _check(matcher, L, R, 0.9 * scale, -1.0)
+    _check(matcher, L, R, 0.9, 0.8)
+
+
+@pytest.mark.parametrize("row", ["nan", "inf", "zero", "tiny"])
+def test_special_rows(matcher, row):
+    L, R = _pair(96, 128, 4)
+    value = {"nan": np.nan, "inf": np.inf, "zero": 0.0, "tiny": 1e-20}[row]
+    L[17], R[40] = value, value
+    _set(matcher, L, R)
+    _check(matcher, L, R)
+
+
+def test_equal_rows(matcher):
+    """Exact duplicates: the first index of an ascending scan, and no match under a ratio."""
+    L, R = _pair(160, 192, 5)
+    L[33:64] = L[32]
+    R[64:192:32] = R[5]
+    R[100] = L[32]
+    _set(matcher, L, R)
+    _check(matcher, L, R, 0.5, -1.0)
+    _check(matcher, L, R)
+
+
+@pytest.mark.parametrize("source", ["device", "device_odd", "pinned", "u8"])
+@pytest.mark.parametrize("n", [32, 288, 2080])
+def test_row_sources(matcher, source, n):
+    """The rows read from device memory, from a device address aligned to 4 bytes only, from
+    pinned host memory handed over as a device pointer, and from uint8 components."""
+    qL, qR, _ = synth.make_pair(n, n, 0.5, config=1, pair=n)
+    L, R = synth.dequantise(qL), synth.dequantise(qR)
+    if source == "u8":
+        matcher.set_left_u8(qL)
+        matcher.set_right_u8(qR)
+        _check(matcher, L, R)
+        return
+    rt = C.CDLL("libamdhip64.so")
+    rt.hipMalloc.argtypes = rt.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    rt.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+    rt.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    rt.hipFree.argtypes = rt.hipHostFree.argtypes = [C.c_void_p]
+    held = []
+    for a, put in ((L, matcher.set_left_device), (R, matcher.set_right_device)):
+        p = C.c_void_p()
+        assert (rt.hipHostMalloc(C.byref(p), a.nbytes + 16, 0) if source == "pinned"
+                else rt.hipMalloc(C.byref(p), a.nbytes + 16)) == 0
+        at = p.value + (4 if source == "device_odd" else 0)
+        assert rt.hipMemcpy(at, a.ctypes.data, a.nbytes, 0 if source == "pinned" else 1) == 0
+        put(n, at)
+        held.append(p)
+    _check(matcher, L, R)
+    for p in held:
+        (rt.hipHostFree if source == "pinned" else rt.hipFree)(p)
+
+
+@pytest.mark.parametrize("kind", ["sift", "spread", "signed", "sparse"])
+def test_score_error(matcher, kind):
+    rng = np.random.default_rng(9)
+    L, R = _pair(1024, 1024, 6)
+    if kind == "spread":  # norms over the whole range
+        L = L * np.exp2(rng.uniform(-9.9, 0.9, (1024, 1))).astype(np.float32)
+        R = R * np.exp2(rng.uniform(-9.9, 0.9, (1024, 1))).astype(np.float32)
+    elif kind == "signed":
+        L, R = (rng.standard_cauchy((1024, 128)) for _ in range(2))
+    elif kind == "sparse":
+        L, R = L * (rng.random(L.shape) < 0.1) + 1e-5, R * (rng.random(R.shape) < 0.1) + 1e-5
+    if kind in ("signed", "sparse"):
+        L, R = (x / np.linalg.norm(x, axis=1, keepdims=True) for x in (L, R))
+    L, R = L.astype(np.float32), R.astype(np.float32)
+    _set(matcher, L, R)
+    got = matcher.score_block(v3dmatch.PREC_FP32, 1024, 1024).astype(np.float64)
+    nq = np.linalg.norm(L.astype(np.float64), axis=1)[:, None]
+    nc = np.linalg.norm(R.astype(np.float64), axis=1)[None, :]
+    err = np.abs(got - L.astype(np.float64) @ R.astype(np.float64).T)
+    assert (err <= 2.0 ** -18 * nq * nc + 2.0 ** -39 * np.sqrt(128) * (nq + nc)).all()
