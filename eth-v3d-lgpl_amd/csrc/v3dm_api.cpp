@@ -69,6 +69,11 @@ void releaseBuffers(v3dm_context* h)
     freeDev(h->normR);
     freeDev(h->splitL);
     freeDev(h->splitR);
+    freeDev(h->intL);
+    freeDev(h->intR);
+    freeDev(h->intScaleL);
+    freeDev(h->intScaleR);
+    h->haveIntL = h->haveIntR = false;
     freeDev(h->splitInfo);
     if (h->splitFitHost) (void)hipHostFree(h->splitFitHost);
     h->splitFitHost = h->splitFitDev = nullptr;
@@ -164,8 +169,9 @@ void launch_score_pass(v3dm_context* h, FusedPlan const& p, unsigned const* bits
 {
     hipStream_t const st = h->stream;
     if (split_fits(h))
-        launch_split_pass(h->splitL, h->splitR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, bits,
-                          h->capL, minScore, st);
+        launch_split_pass(SplitSet{h->splitL, h->haveIntL ? h->intL : nullptr, h->intScaleL, h->nL},
+                          SplitSet{h->splitR, h->haveIntR ? h->intR : nullptr, h->intScaleR, h->nR}, p, h->colPart,
+                          h->capL, h->rowPart, h->capR, bits, h->capL, minScore, st);
     else if (bits)
         launch_guided_fp32(h->dL, h->dR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, bits, h->capL, st);
     else
@@ -367,13 +373,19 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
                 HIPCHECK(h, hipMalloc(&h->dQ, qb));
                 h->dQBytes = qb;
             }
+            size_t const rows = (size_t)roundUp(left ? h->capL : h->capR, kSplitRowPad);
+            if (!(left ? h->intL : h->intR)) HIPCHECK(h, hipMalloc(left ? &h->intL : &h->intR, rows * kIntRowBytes));
+            if (!(left ? h->intScaleL : h->intScaleR))
+                HIPCHECK(h, hipMalloc(left ? &h->intScaleL : &h->intScaleR, rows * sizeof(float)));
             HIPCHECK(h, hipMemcpyAsync(h->dQ, src, (size_t)n * kDim, hipMemcpyHostToDevice, h->stream));
             from = kRowsU8;
         }
     }
     launch_split_rows(from, from == kRowsU8 ? (void const*)h->dQ : src, dst, n, left ? h->normL : h->normR,
-                      h->maxNormBits + (left ? 0 : 1), left ? h->splitL : h->splitR, h->splitInfo,
+                      h->maxNormBits + (left ? 0 : 1), left ? h->splitL : h->splitR,
+                      left ? h->intL : h->intR, left ? h->intScaleL : h->intScaleR, h->splitInfo,
                       h->splitFitDev + (left ? 0 : 1), h->stream);
+    (left ? h->haveIntL : h->haveIntR) = from == kRowsU8;
     HIPCHECK(h, hipGetLastError());
     HIPCHECK(h, hipStreamSynchronize(h->stream));
     if (left) h->nL = n;

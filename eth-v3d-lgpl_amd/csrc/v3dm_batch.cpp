@@ -18,6 +18,7 @@
 #include "v3dm_batch.h"
 #include "v3dm_context.h"
 #include "v3dm_learned.h"
+#include "v3dm_split.h"
 
 namespace v3dm {
 
@@ -69,6 +70,11 @@ struct BatchState {
     float* denom = nullptr;
     int2* rowCS = nullptr;          // sampled check of uint8 batches: row constants
     bool haveU8 = false;
+    unsigned char* split = nullptr;  // rows of the split pass (v3dm_split.h), made by the first plain run
+    size_t splitCap = 0;
+    int* notFit = nullptr;           // device: set by the norms of a row outside the range
+    bool splitValid = false;
+    bool splitFit = false;           // every row is in the split pass's range
     bool codesValid = false;
     float codesScale = 0.0f;
     int* imgBase = nullptr;
@@ -160,11 +166,12 @@ struct BatchState {
         float margin;
         int samples;
         float minRecall;
+        bool haveSplit;  // a learned run's fallback finds the split rows made
         bool operator<(GraphKey const& o) const
         {
-            return std::tie(mode, minScore, minRatio, epsRel, version, topK, margin, samples, minRecall) <
+            return std::tie(mode, minScore, minRatio, epsRel, version, topK, margin, samples, minRecall, haveSplit) <
                    std::tie(o.mode, o.minScore, o.minRatio, o.epsRel, o.version, o.topK, o.margin, o.samples,
-                            o.minRecall);
+                            o.minRecall, o.haveSplit);
         }
     };
     std::map<GraphKey, hipGraphExec_t> graphs;
@@ -223,6 +230,7 @@ BatchDev dev_view(BatchState* b, int form)
     d.codes = b->codes;
     d.u8 = b->haveU8 ? b->imgU8 : nullptr;
     d.denom = b->denom;
+    d.split = b->split;
     d.imgBase = b->imgBase;
     d.norm = b->norm;
     d.maxNorm = b->maxNorm;
@@ -588,11 +596,14 @@ int ensure_query_space(v3dm_context* h, BatchState* b)
 
 int form_of(int mode) { return mode == V3DM_PREC_FP32 ? 0 : (mode == V3DM_PREC_LEARNED ? 2 : 1); }
 
-// Derived copies of the images for a form: bf16 rows (BF16 form) or learned codes.
+// Derived copies of the images for a form: split rows (plain form), bf16 rows (BF16 form) or
+// learned codes.
 void enqueue_derived(v3dm_context* h, BatchState* b, int form)
 {
     hipStream_t const st = h->stream;
-    if (form == 1) {
+    if (form == 0) {
+        if (b->splitFit) launch_batch_split_rows(dev_view(b, 0), b->imgRows, b->split, st);
+    } else if (form == 1) {
         if (b->haveU8) launch_batch_u8_to_bf16(b->imgU8, b->denom, b->imgRows, b->imgB, st);
         else launch_to_bf16(b->img, b->imgRows, b->imgB, st);
     } else if (form == 2) {
@@ -601,6 +612,29 @@ void enqueue_derived(v3dm_context* h, BatchState* b, int form)
         if (b->haveU8) launch_mlp_codes_u8(b->imgU8, b->denom, b->imgRows, w, scale, b->codes, st);
         else launch_mlp_codes_f32(b->img, b->imgRows, w, scale, b->codes, st);
     }
+}
+
+int ensure_split(v3dm_context* h, BatchState* b)
+{
+    if (!b->splitFit) return V3DM_OK;
+    size_t const need = (size_t)b->imgRows * (b->haveU8 ? kIntRowBytes : kSplitRowBytes);
+    if (b->split && b->splitCap >= need) return V3DM_OK;
+    drop_graphs(b);  // captured runs hold the old buffer
+    b->splitValid = false;
+    return grow(h, b->split, b->splitCap, need);
+}
+
+// The plain pass of plan `form` (0, or 3: the pairs a learned run hands over) on the images'
+// split rows, or on the FP32 rows where a row is outside the split range.
+void launch_plain_pass(BatchState* b, int form, int4 const* items, int nItems, int* queue, float minScore,
+                       hipStream_t st, int const* nItemsDev = nullptr)
+{
+    Plan const& pl = b->plan[form];
+    BatchDev const d = dev_view(b, form);
+    if (b->splitFit)
+        launch_batch_split(d, b->haveU8, items, nItems, queue, b->partF, pl.grid, pl.qRows, minScore, st, nItemsDev);
+    else
+        launch_batch_fused_fp32(d, items, nItems, queue, b->partF, pl.grid, pl.qRows, st, nItemsDev);
 }
 
 // Enqueue one batch run of `mode` with the current plan of its form.
@@ -613,8 +647,7 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
     launch_batch_reset(b->counters, b->pairCount, b->nPairs, st);
     if (!h->cacheDerived) enqueue_derived(h, b, form);
     if (form == 0) {
-        launch_batch_fused_fp32(d, b->items[0], (int)pl.items.size(), b->counters + 0, b->partF, pl.grid, pl.qRows,
-                                st);
+        launch_plain_pass(b, 0, b->items[0], (int)pl.items.size(), b->counters + 0, minScore, st);
         launch_batch_merge_decide(d, b->partF, h->epsRel, minScore, minRatio, b->sel, b->flagList, b->counters, st);
         launch_batch_recheck(d, b->flagList, b->counters, minScore, minRatio, b->sel, 1024, st);
     } else if (form == 1) {
@@ -658,8 +691,10 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
             BatchDev const d0 = dev_view(b, 3);
             launch_batch_fb_filter(b->items[3], np, b->pairFlag, b->nPairs, b->fbItems, b->counters + kBCntFbItems,
                                    b->segMask, st);
-            launch_batch_fused_fp32(d0, b->fbItems, np, b->counters + 0, b->partF, pp.grid, pp.qRows, st,
-                                    b->counters + kBCntFbItems);
+            // (the split rows of a plain run may be there already, of the same images)
+            if (b->splitFit && !(h->cacheDerived && b->splitValid))
+                launch_batch_split_masked(d0, b->segMask, b->split, 2 * cus, st);
+            launch_plain_pass(b, 3, b->fbItems, np, b->counters + 0, minScore, st, b->counters + kBCntFbItems);
             launch_batch_merge_masked(d0, b->partF, h->epsRel, minScore, minRatio, b->sel, b->flagList, b->counters,
                                       b->segMask, 2 * cus, st);
             launch_batch_recheck(d0, b->flagList, b->counters, minScore, minRatio, b->sel, 1024, st);
@@ -684,8 +719,7 @@ int time_pass(v3dm_context* h, BatchState* b, int form, Plan const& pl, float& m
         launch_batch_reset(b->counters, b->pairCount, b->nPairs, st);
         BCHECK(h, hipEventRecord(b->evA, st));
         if (form == 0)
-            launch_batch_fused_fp32(d, b->items[0], (int)pl.items.size(), b->counters + 0, b->partF, pl.grid,
-                                    pl.qRows, st);
+            launch_plain_pass(b, 0, b->items[0], (int)pl.items.size(), b->counters + 0, b->lastMinScore, st);
         else if (form == 1)
             launch_batch_pass_bf16(d, b->items[1], (int)pl.items.size(), b->counters + 1, b->partB, pl.grid,
                                    pl.qRows, st);
@@ -776,7 +810,8 @@ int ensure_fallback_plan(v3dm_context* h, BatchState* b)
         (void)hipGetDevice(&dev);
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         drop_graphs(b);
-        Plan pl = plan_plain(b, kFallbackTiles, 2 * cus);
+        // 256 left features an item on split rows (109 -> see k_batch_split), 128 on FP32 rows
+        Plan pl = plan_plain(b, kFallbackTiles, 2 * cus, b->splitFit ? 256 : 128);
         if ((rc = upload_plan(h, b, 3, pl))) return rc;
         b->plan[3] = std::move(pl);
         b->planValid[3] = true;
@@ -875,6 +910,7 @@ int set_images(v3dm_context* h, int nImages, int32_t const* counts, void const* 
     if (b->blkImg) (void)hipFree(b->blkImg);
     b->nImgD = b->srcRow = b->blkImg = nullptr;
     b->maxNorm = nullptr;
+    if (!b->notFit) BCHECK(h, hipMalloc(&b->notFit, sizeof(int)));
     BCHECK(h, hipMalloc(&b->nImgD, nImages * sizeof(int)));
     BCHECK(h, hipMalloc(&b->srcRow, nImages * sizeof(int)));
     BCHECK(h, hipMalloc(&b->maxNorm, nImages * sizeof(unsigned int)));
@@ -922,11 +958,16 @@ int set_images(v3dm_context* h, int nImages, int32_t const* counts, void const* 
     else
         launch_batch_load_f32(static_cast<float const*>(b->upload), b->srcRow, b->nImgD, b->blkImg, b->imgBase, rows,
                               b->img, st);
-    launch_batch_norms(b->img, b->blkImg, rows, b->norm, b->maxNorm, st);
+    BCHECK(h, hipMemsetAsync(b->notFit, 0, sizeof(int), st));
+    launch_batch_norms(b->img, b->blkImg, rows, b->norm, b->maxNorm, b->notFit, st);
     b->bfValid = false;
     b->codesValid = false;
+    b->splitValid = false;
     BCHECK(h, hipGetLastError());
+    int notFit = 1;
+    BCHECK(h, hipMemcpyAsync(&notFit, b->notFit, sizeof(int), hipMemcpyDeviceToHost, st));
     BCHECK(h, hipStreamSynchronize(st));  // host vectors above go out of scope
+    b->splitFit = notFit == 0;
     return V3DM_OK;
 }
 
@@ -936,7 +977,7 @@ void batch_destroy(BatchState*& b)
 {
     if (!b) return;
     drop_graphs(b);
-    for (void* p : {(void*)b->img, (void*)b->imgB, (void*)b->codes, (void*)b->imgU8, (void*)b->denom, (void*)b->imgBase, (void*)b->blkImg, (void*)b->nImgD,
+    for (void* p : {(void*)b->split, (void*)b->notFit, (void*)b->img, (void*)b->imgB, (void*)b->codes, (void*)b->imgU8, (void*)b->denom, (void*)b->imgBase, (void*)b->blkImg, (void*)b->nImgD,
                     (void*)b->srcRow, (void*)b->norm, (void*)b->maxNorm, b->upload, (void*)b->segOfBlock,
                     (void*)b->items[0], (void*)b->items[1], (void*)b->items[2], (void*)b->items[3],
                     (void*)b->segD[0], (void*)b->segD[1], (void*)b->segD[2], (void*)b->segD[3], (void*)b->blkInfo[0],
@@ -1080,7 +1121,12 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
         if (b->codesScale != learned_code_scale(L)) b->codesValid = false;
         b->codesScale = learned_code_scale(L);
     }
+    if ((form == 0 || (form == 2 && h->fallbackSamples > 0)) && (rc = ensure_split(h, b))) return rc;
     // derived copies outside the run when they are cached (else every run derives them)
+    if (h->cacheDerived && form == 0 && !b->splitValid) {
+        enqueue_derived(h, b, 0);
+        b->splitValid = true;
+    }
     if (h->cacheDerived && form == 1 && !b->bfValid) {
         enqueue_derived(h, b, 1);
         b->bfValid = true;
@@ -1089,14 +1135,16 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
         enqueue_derived(h, b, 2);
         b->codesValid = true;
     }
-    if (!h->cacheDerived && form != 0 && !b->planValid[form]) enqueue_derived(h, b, form);  // for the tuner
+    if (!h->cacheDerived && !b->planValid[form]) enqueue_derived(h, b, form);  // for the tuner
+    if (!h->cacheDerived) b->splitValid = false;  // a learned run rewrites the rows of its failing pairs
     if ((rc = ensure_plan(h, b, form))) return rc;
     if (form == 2 && h->fallbackSamples > 0 && (rc = ensure_fallback_plan(h, b))) return rc;
     BCHECK(h, hipEventRecord(b->evA, st));
     if (b->useGraph) {
         BatchState::GraphKey const key{mode, minScore, minRatio, h->epsRel, b->version * 2 + (h->cacheDerived ? 1 : 0),
                                        h->learnedTopK, form == 2 ? learned_margin(h) : 0.0f,
-                                       form == 2 ? h->fallbackSamples : 0, form == 2 ? h->fallbackRecall : 0.0f};
+                                       form == 2 ? h->fallbackSamples : 0, form == 2 ? h->fallbackRecall : 0.0f,
+                                       form == 2 && b->splitValid};
         auto it = b->graphs.find(key);
         if (it == b->graphs.end()) {
             hipGraph_t g = nullptr;
@@ -1202,7 +1250,7 @@ int v3dm_batch_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
     if (e == hipSuccess) e = hipEventRecord(b->evA, st);
     for (int r = 0; r < reps && e == hipSuccess; ++r) {
         int const n = (int)pl.items.size();
-        if (form == 0) launch_batch_fused_fp32(d, b->items[0], n, q + r, b->partF, pl.grid, pl.qRows, st);
+        if (form == 0) launch_plain_pass(b, 0, b->items[0], n, q + r, b->lastMinScore, st);
         else if (form == 1) launch_batch_pass_bf16(d, b->items[1], n, q + r, b->partB, pl.grid, pl.qRows, st);
         else launch_batch_pass_code(d, b->items[2], n, q + r, b->partB, pl.grid, pl.qRows, st);
     }

@@ -74,6 +74,7 @@ struct BatchDev {
     signed char const* codes;     // learned codes, 32 bytes per image row
     uint8_t const* u8;            // uint8 rows (images uploaded as uint8) or null
     float const* denom;           // their scales: element k = (float)u8[k] * denom
+    unsigned char const* split;   // split rows of the images, or the uint8 components in FP16 (v3dm_split.h)
     int const* imgBase;
     float const* norm;            // per image row
     unsigned int const* maxNorm;  // per image (float bits)
@@ -119,6 +120,12 @@ void launch_batch_u8_to_bf16(uint8_t const* u8, float const* denom, int rows, __
 // count in device memory, at most nItems
 void launch_batch_fused_fp32(BatchDev const& b, int4 const* items, int nItems, int* queue, Top2* part, int grid,
                              int leftRows, hipStream_t st, int const* nItemsDev = nullptr);
+// the same on the images' split rows (ints: on their integer rows and scales; v3dm_split.hip)
+void launch_batch_split(BatchDev const& b, bool ints, int4 const* items, int nItems, int* queue, Top2* part, int grid,
+                        int leftRows, float minScore, hipStream_t st, int const* nItemsDev = nullptr);
+// the rows that pass reads, from the FP32 images or from the uint8 rows (v3dm_batch.hip)
+void launch_batch_split_rows(BatchDev const& b, int rows, unsigned char* out, hipStream_t st);
+void launch_batch_split_masked(BatchDev const& b, int const* segMask, unsigned char* out, int grid, hipStream_t st);
 // shortlist pass (v3dm_short.hip); queryRows: queries per work-group, 128 (2 waves) or 256
 // (4 waves), the plan's query blocks
 void launch_batch_pass_bf16(BatchDev const& b, int4 const* items, int nItems, int* queue, Cand2* part, int grid,
@@ -135,7 +142,7 @@ void launch_batch_pass_code(BatchDev const& b, int4 const* items, int nItems, in
 // selection and bookkeeping (v3dm_batch.hip)
 void launch_batch_reset(int* counters, int* pairCount, int nPairs, hipStream_t st);
 void launch_batch_norms(float const* img, int const* rowImg, int rows, float* norm, unsigned int* maxNorm,
-                        hipStream_t st);
+                        int* notFit, hipStream_t st);
 void launch_batch_merge_decide(BatchDev const& b, Top2 const* part, float epsRel, float minScore, float minRatio,
                                int* sel, int* flagList, int* counters, hipStream_t st);
 // the segments with segMask set only (the others keep their decisions); persistent grid

@@ -7,6 +7,7 @@
 // do one pair at a time (V3D/Apps/SfM/match_sequence.cpp:165-382).
 #include "v3dm_batch.h"
 #include "v3dm_kernels.h"
+#include "v3dm_split.h"
 
 namespace v3dm {
 
@@ -47,12 +48,13 @@ void launch_batch_reset(int* counters, int* pairCount, int nPairs, hipStream_t s
     hipLaunchKernelGGL(k_batch_reset, dim3((n + 255) / 256), dim3(256), 0, st, counters, pairCount, nPairs);
 }
 
-// Row norms of the image buffer and per-image maximum.  blkImg[row / kBatchRowAlign] =
+// Row norms of the image buffer and per-image maximum; *notFit = 1 when a row is outside the
+// split pass's range (v3dm_split.h).  blkImg[row / kBatchRowAlign] =
 // image of the row; a work-group's 64 rows lie in one image (images are aligned to 256
 // rows), so one atomicMax per work-group suffices.
 __global__ __launch_bounds__(256) void k_batch_norms(float const* __restrict__ X, int const* __restrict__ blkImg,
                                                      int rows, float* __restrict__ norm,
-                                                     unsigned int* __restrict__ maxNorm)
+                                                     unsigned int* __restrict__ maxNorm, int* __restrict__ notFit)
 {
     __shared__ unsigned int wmax[4];
     int const lane = threadIdx.x & 63;
@@ -67,6 +69,7 @@ __global__ __launch_bounds__(256) void k_batch_norms(float const* __restrict__ X
         float const nr = sqrtf(s);
         if (lane == 0) norm[row] = nr;
         mx = max(mx, __float_as_uint(nr));
+        if (lane == 0 && !(nr == 0.0f || (nr >= kSplitNormMin && nr < kSplitNormMax))) *notFit = 1;
     }
     if (lane == 0) wmax[wave] = mx;
     __syncthreads();
@@ -77,10 +80,11 @@ __global__ __launch_bounds__(256) void k_batch_norms(float const* __restrict__ X
 }
 
 void launch_batch_norms(float const* img, int const* blkImg, int rows, float* norm, unsigned int* maxNorm,
-                        hipStream_t st)
+                        int* notFit, hipStream_t st)
 {
     if (rows <= 0) return;
-    hipLaunchKernelGGL(k_batch_norms, dim3((rows + 63) / 64), dim3(256), 0, st, img, blkImg, rows, norm, maxNorm);
+    hipLaunchKernelGGL(k_batch_norms, dim3((rows + 63) / 64), dim3(256), 0, st, img, blkImg, rows, norm, maxNorm,
+                       notFit);
 }
 
 // 8 lanes (sub = lane & 7) per query row g of segment si: merge the segment's partials,
@@ -466,6 +470,87 @@ void launch_batch_u8_to_bf16(uint8_t const* u8, float const* denom, int rows, __
 {
     if (rows <= 0) return;
     hipLaunchKernelGGL(k_batch_u8_to_bf16, dim3((rows * 16 + 255) / 256), dim3(256), 0, st, u8, denom, rows, Y);
+}
+
+// The rows of the split pass (v3dm_split.h): of FP32 images the two FP16 parts, of uint8 images
+// the components as FP16 integers.  Eight elements per thread, chunk c of row `row`.  With a
+// segment mask only the rows of the flagged segments' images (a learned run's fallback; images
+// that several flagged pairs share are written more than once, with the same values).
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+template <bool kInt>
+__device__ __forceinline__ void batch_split_chunk(BatchDev const& b, size_t row, int c, unsigned char* __restrict__ out)
+{
+    if (kInt) {
+        uint2 const q = reinterpret_cast<uint2 const*>(b.u8)[row * 16 + c];
+        v8h v;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = (_Float16)(float)((q.x >> (8 * k)) & 0xffu);
+            v[4 + k] = (_Float16)(float)((q.y >> (8 * k)) & 0xffu);
+        }
+        reinterpret_cast<v8h*>(out)[row * 16 + c] = v;
+    } else {
+        float4 const* x = reinterpret_cast<float4 const*>(b.img) + row * 32 + 2 * c;
+        float4 const p = x[0], q = x[1];
+        float const f[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+        v8h hi, lo;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            float const s = f[k] * kSplitScale;
+            hi[k] = (_Float16)s;
+            lo[k] = (_Float16)(s - (float)hi[k]);
+        }
+        unsigned char* o = out + row * kSplitRowBytes + (c >> 3) * 256 + (c & 7) * 16;
+        *reinterpret_cast<v8h*>(o) = hi;
+        *reinterpret_cast<v8h*>(o + 128) = lo;
+    }
+}
+
+template <bool kInt>
+__global__ __launch_bounds__(256) void k_batch_split_rows(BatchDev b, int rows, unsigned char* __restrict__ out)
+{
+    size_t const t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if ((int)(t >> 4) < rows) batch_split_chunk<kInt>(b, t >> 4, (int)(t & 15), out);
+}
+
+template <bool kInt>
+__global__ __launch_bounds__(256) void k_batch_split_masked(BatchDev b, int const* __restrict__ segMask,
+                                                            unsigned char* __restrict__ out)
+{
+    __shared__ int list[1024];
+    __shared__ int nList;
+    int const nSeg = 2 * b.nPairs;
+    for (int base = 0; base < nSeg; base += 1024) {
+        __syncthreads();  // the previous chunk's list is consumed
+        if (threadIdx.x == 0) nList = 0;
+        __syncthreads();
+        for (int u = threadIdx.x; u < 1024 && base + u < nSeg; u += 256)
+            if (segMask[base + u]) list[atomicAdd(&nList, 1)] = base + u;
+        __syncthreads();
+        int const n = nList;
+        for (int e = 0; e < n; ++e) {
+            BatchSeg const sg = b.seg[list[e]];
+            size_t const row0 = b.imgBase[sg.img];
+            for (int r = blockIdx.x * 16 + (threadIdx.x >> 4); r < sg.n; r += gridDim.x * 16)
+                batch_split_chunk<kInt>(b, row0 + r, threadIdx.x & 15, out);
+        }
+    }
+}
+
+void launch_batch_split_rows(BatchDev const& b, int rows, unsigned char* out, hipStream_t st)
+{
+    if (rows <= 0) return;
+    dim3 const g(rows / 16);  // images are padded to 256 rows
+    if (b.u8) hipLaunchKernelGGL(k_batch_split_rows<true>, g, dim3(256), 0, st, b, rows, out);
+    else hipLaunchKernelGGL(k_batch_split_rows<false>, g, dim3(256), 0, st, b, rows, out);
+}
+
+void launch_batch_split_masked(BatchDev const& b, int const* segMask, unsigned char* out, int grid, hipStream_t st)
+{
+    if (b.nPairs <= 0) return;
+    if (b.u8) hipLaunchKernelGGL(k_batch_split_masked<true>, dim3(grid), dim3(256), 0, st, b, segMask, out);
+    else hipLaunchKernelGGL(k_batch_split_masked<false>, dim3(grid), dim3(256), 0, st, b, segMask, out);
 }
 
 void launch_batch_load_f32(float const* src, int const* srcRow, int const* nImg, int const* blkImg,

@@ -39,6 +39,11 @@ struct v3dm_context {
     float* normR = nullptr;
     unsigned char* splitL = nullptr;  // rows in two FP16 parts (v3dm_split.h), written with the norms
     unsigned char* splitR = nullptr;
+    unsigned char* intL = nullptr;    // uint8 sets: the components as FP16 integers ...
+    unsigned char* intR = nullptr;
+    float* intScaleL = nullptr;       // ... and the rows' scales (allocated by the first uint8 upload)
+    float* intScaleR = nullptr;
+    bool haveIntL = false, haveIntR = false;  // the current set has them
     int* splitInfo = nullptr;         // scratch of launch_split_rows
     int* splitFitHost = nullptr;      // mapped: [0] left, [1] right set in the split pass's range
     int* splitFitDev = nullptr;       // the same memory as the kernels address it

@@ -71,8 +71,9 @@ __device__ __forceinline__ void split_pair(float2 v, unsigned& hi, unsigned& lo)
 template <int kFrom>
 __global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src, float* __restrict__ X, int n,
                                                     float* __restrict__ norm, unsigned int* __restrict__ maxNormBits,
-                                                    unsigned char* __restrict__ split, int* __restrict__ info,
-                                                    int* __restrict__ hostFit)
+                                                    unsigned char* __restrict__ split,
+                                                    unsigned char* __restrict__ ints, float* __restrict__ scale,
+                                                    int* __restrict__ info, int* __restrict__ hostFit)
 {
     __shared__ unsigned int wmax[4];
     __shared__ int wbad[4];
@@ -90,8 +91,16 @@ __global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src
                 q[k] = (row0 + k < n) ? static_cast<uchar2 const*>(src)[(size_t)(row0 + k) * 64 + lane]
                                       : make_uchar2(0, 0);
 #pragma unroll
-            for (int k = 0; k < kPrepRows; ++k)
-                v[k] = (row0 + k < n) ? dequant_u8_wave(q[k]) : make_float2(0.0f, 0.0f);
+            for (int k = 0; k < kPrepRows; ++k) {
+                float const d = dequant_u8_denom(q[k]);
+                v[k] = (row0 + k < n) ? make_float2(dequant_u8_value(q[k].x, d), dequant_u8_value(q[k].y, d))
+                                      : make_float2(0.0f, 0.0f);
+                if (row0 + k < n) {
+                    v2h const i = {(_Float16)(float)q[k].x, (_Float16)(float)q[k].y};
+                    reinterpret_cast<v2h*>(ints + (size_t)(row0 + k) * kIntRowBytes)[lane] = i;
+                    if (lane == 0) scale[row0 + k] = d;
+                }
+            }
         } else {
             float2 const* const rows = kFrom == kRowsF32 ? static_cast<float2 const*>(src)
                                                          : reinterpret_cast<float2 const*>(X);
@@ -161,20 +170,21 @@ __global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src
 }
 
 void launch_split_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNormBits,
-                       unsigned char* split, int* info, int* hostFit, hipStream_t st)
+                       unsigned char* split, unsigned char* ints, float* scale, int* info, int* hostFit,
+                       hipStream_t st)
 {
     if (n <= 0) return;
     int const per = 4 * kPrepRows;
     dim3 const grid(min((n + per - 1) / per, kPrepGroups));
     if (from == kRowsU8)
-        hipLaunchKernelGGL(k_split_rows<kRowsU8>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, info,
-                           hostFit);
+        hipLaunchKernelGGL(k_split_rows<kRowsU8>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, ints,
+                           scale, info, hostFit);
     else if (from == kRowsF32)
-        hipLaunchKernelGGL(k_split_rows<kRowsF32>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, info,
-                           hostFit);
+        hipLaunchKernelGGL(k_split_rows<kRowsF32>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, ints,
+                           scale, info, hostFit);
     else
         hipLaunchKernelGGL(k_split_rows<kRowsInPlace>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split,
-                           info, hostFit);
+                           ints, scale, info, hostFit);
 }
 
 // ------------------------------------------------------------------------------ merge + decide

@@ -25,13 +25,15 @@ constexpr float kSplitScale = 16384.0f;
 constexpr float kSplitBack = 3.7252902984619140625e-09f;  // 2^-28
 constexpr float kSplitNormMin = 0.0009765625f;            // 2^-10
 constexpr float kSplitNormMax = 2.0f;
+constexpr int kIntRowBytes = 256;    // integer components in FP16
 constexpr int kSplitRowBytes = 512;  // per half (64 components): 128 B of hi, 128 B of lo
 constexpr int kSplitRowPad = 256;    // split buffers hold a multiple of 256 rows
 constexpr int kSplitTile = 32;       // right features per tile
 
 // One feature set in one launch: its FP32 rows X (copied from the device array src, or
 // dequantised from the uint8 rows src as SIFT_Feature::normalizeDescriptor, or in place), the
-// norms and the set's largest norm (as launch_norms) and the split rows.  info (device,
+// norms and the set's largest norm (as launch_norms), the split rows, and (uint8 rows) the
+// integer rows and their scales.  info (device,
 // kPrepInfo ints, zero before the first call, left ready for the next): scratch; *hostFit
 // (mapped host memory): 1 when the set is in the range of the split pass.
 enum RowSource { kRowsInPlace, kRowsF32, kRowsU8 };
@@ -39,16 +41,25 @@ constexpr int kPrepGroups = 256;
 constexpr int kPrepSlot = 32;
 constexpr int kPrepInfo = kPrepSlot + 2 * kPrepGroups;
 void launch_split_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNormBits,
-                       unsigned char* split, int* info, int* hostFit, hipStream_t st);
-
-// Score pass of two split sets: colPart[split][i], rowPart[leftBlock][j] as
-// launch_fused_fp32, with left blocks of 256 features and tiles of 32 right features.  bits:
-// guided-matching bitmap (pairs scored -1e20), or null.  A partial's index is -1 where its
-// best does not exceed minScore.
-FusedPlan plan_split(int nL, int nR);
-void launch_split_pass(unsigned char const* L, unsigned char const* R, int nL, int nR, FusedPlan const& p,
-                       Top2* colPart, int ldc, Top2* rowPart, int ldr, unsigned const* bits, int ldi, float minScore,
+                       unsigned char* split, unsigned char* ints, float* scale, int* info, int* hostFit,
                        hipStream_t st);
+
+// One side of a score pass: n split rows, and for sets uploaded as uint8 their components as
+// FP16 integers with the rows' scales (else null).  All padded to kSplitRowPad rows.
+struct SplitSet {
+    unsigned char const* split;
+    unsigned char const* ints;
+    float const* scale;
+    int n;
+};
+
+// Score pass of two sets in range: colPart[split][i], rowPart[leftBlock][j] as
+// launch_fused_fp32, with left blocks of 256 features and tiles of 32 right features; on the
+// integers where both sides have them.  bits: guided-matching bitmap (pairs scored -1e20), or
+// null.  A partial's index is -1 where its best does not exceed minScore.
+FusedPlan plan_split(int nL, int nR);
+void launch_split_pass(SplitSet const& L, SplitSet const& R, FusedPlan const& p, Top2* colPart, int ldc,
+                       Top2* rowPart, int ldr, unsigned const* bits, int ldi, float minScore, hipStream_t st);
 
 // Measurement: the scores of the split pass, out[i * nCols + j] (as launch_score_block).
 void launch_score_block_split(unsigned char const* L, unsigned char const* R, int nRows, int nCols, float* out,

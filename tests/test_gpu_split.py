@@ -143,3 +143,83 @@ def test_score_error(matcher, kind):
     nc = np.linalg.norm(R.astype(np.float64), axis=1)[None, :]
     err = np.abs(got - L.astype(np.float64) @ R.astype(np.float64).T)
     assert (err <= 2.0 ** -18 * nq * nc + 2.0 ** -39 * np.sqrt(128) * (nq + nc)).all()
+
+
+def _batch(sizes, seed):
+    images = []
+    for p, (nL, nR) in enumerate(sizes):
+        qL, qR, _ = synth.make_pair(nL, nR, 0.5, config=3, pair=100 * seed + p)
+        images += [qL, qR]
+    left = np.arange(0, 2 * len(sizes), 2, dtype=np.int32)
+    return images, left, left + 1
+
+
+def _want(images, left, right, min_score, min_ratio):
+    out = []
+    for a, b in zip(left, right):
+        L, R = images[a][:len(images[a]) // 32 * 32], images[b][:len(images[b]) // 32 * 32]
+        out.append(oracle.find_putative_matches(L, R, min_score, min_ratio) if len(L) and len(R)
+                   else np.zeros((0, 2), np.int32))
+    return out
+
+
+SIZES = [(33, 70), (512, 31), (256, 256), (300, 1700), (1056, 96), (32, 32), (640, 513)]
+
+
+@pytest.mark.parametrize("dtype", ["u8", "f32", "f32_wide", "f32_nan"])
+@pytest.mark.parametrize("rows", [128, 256])
+def test_batch_split(dtype, rows):
+    """Batches of uint8 images (integer rows), of FP32 images (split rows), and of images with
+    rows outside the range (the FP32 instruction), in both work-group shapes, with the rows made
+    by every run and kept."""
+    qs, left, right = _batch(SIZES, 1)
+    images = [synth.dequantise(q) for q in qs]
+    if dtype == "f32_wide":
+        images[3] = images[3] * np.float32(2.0 ** 30)
+    elif dtype == "f32_nan":
+        images[4][7] = np.nan
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([len(q) for q in qs], np.concatenate(qs if dtype == "u8" else images))
+    m.batch_set_pairs(left, right)
+    m.batch_set_tile_shape(v3dmatch.PREC_FP32, rows)
+    for cache in (False, True):
+        m.set_derived_cache(cache)
+        for tiles, score, ratio in ((1, 0.9, 0.8), (3, 0.9, 0.8), (3, -2.0, -1.0)):
+            m.batch_set_tuning(False, v3dmatch.PREC_FP32, tiles, 64)
+            for got, want in zip(m.batch_match(score, ratio), _want(images, left, right, score, ratio)):
+                assert np.array_equal(got, want)
+    m.close()
+
+
+@pytest.mark.parametrize("dtype", ["u8", "f32"])
+@pytest.mark.parametrize("cache", [False, True])
+@pytest.mark.parametrize("plain_first", [False, True])
+def test_batch_fallback_split(dtype, cache, plain_first):
+    """The pairs that a learned run hands to the plain form (a constant code with one
+    candidate per query) get the exact matches, with the split rows made for them alone or left
+    by a plain run of the same images."""
+    from v3dmatch import learned
+    qs, left, right = _batch(SIZES, 2)
+    images = [synth.dequantise(q) for q in qs]
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([len(q) for q in qs], np.concatenate(qs if dtype == "u8" else images))
+    m.batch_set_pairs(left, right)
+    m.set_derived_cache(cache)
+    net = learned.Network(m)
+    params = learned.init_params(3)
+    params["W2"][:] = 0.0  # the same code for every descriptor: its candidates are arbitrary
+    params["b2"][:] = 1.0
+    net.set_params(params)
+    net.set_code_scale(60.0)
+    m.set_learned_topk(1)
+    m.set_fallback(128, 1.0)
+    want = _want(images, left, right, 0.9, 0.8)
+    for mode in ([v3dmatch.PREC_FP32] if plain_first else []) + [v3dmatch.PREC_LEARNED] * 2:
+        m.set_precision(mode)
+        res = m.batch_match(0.9, 0.8)
+        flags = m.batch_get_fallback() if mode == v3dmatch.PREC_LEARNED else np.ones(len(want), int)
+        for p, w in enumerate(want):
+            if flags[p]:
+                assert np.array_equal(res[p], w)
+    assert flags.sum() >= 1
+    m.close()
