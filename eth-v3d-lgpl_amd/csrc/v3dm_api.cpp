@@ -84,6 +84,7 @@ void releaseBuffers(v3dm_context* h)
     freeDev(h->rowMax);
     freeDev(h->flagList);
     freeDev(h->rpart);
+    freeDev(h->rtickets);
     freeDev(h->mstatus);
     freeDev(h->stripes);
     freeDev(h->results);
@@ -160,6 +161,13 @@ int prof_end(v3dm_context* h)
 
 bool split_fits(v3dm_context const* h) { return h->splitFitHost[0] && h->splitFitHost[1]; }
 
+// The certified decisions' error bound for the scores of launch_score_pass.
+float score_eps(v3dm_context const* h, unsigned const* bits)
+{
+    if (!split_fits(h)) return h->epsRel;
+    return h->epsRel * (h->haveIntL && h->haveIntR && !bits ? kIntEps : kSplitEps);
+}
+
 FusedPlan score_plan(v3dm_context const* h)
 {
     return split_fits(h) ? plan_split(h->nL, h->nR) : plan_fused_fp32(h->nL, h->nR, 512);
@@ -192,10 +200,10 @@ int enqueue_plain(v3dm_context* h, float minScore, float minRatio)
         launch_score_pass(h, p, nullptr, minScore);
         if ((rc = prof_end(h))) return rc;
         launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
-                            h->normR, h->maxNormBits, h->epsRel, minScore, minRatio, h->colMax, h->rowMax,
+                            h->normR, h->maxNormBits, score_eps(h, nullptr), minScore, minRatio, h->colMax, h->rowMax,
                             h->flagList, h->capL, h->results, st);
-        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->results, minScore, minRatio,
-                             h->colMax, h->rowMax, h->rpart, kRecheckGrid, st);
+        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore,
+                             minRatio, h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st);
     }
     launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
                           reinterpret_cast<int2*>(h->results + kNumCounters), h->results, st, {}, h->mutualWait);
@@ -290,6 +298,8 @@ int v3dm_allocate(v3dm_handle h, int nMaxLeft, int nMaxRight, int useGuidedMatch
     HIPCHECK(h, hipMalloc(&h->rowMax, cr * sizeof(int)));
     HIPCHECK(h, hipMalloc(&h->flagList, (cl + cr) * sizeof(int)));
     HIPCHECK(h, hipMalloc(&h->rpart, (cl + cr) * kRecheckMaxChunks * sizeof(Top2)));
+    HIPCHECK(h, hipMalloc(&h->rtickets, (cl + cr) * sizeof(int)));
+    HIPCHECK(h, hipMemsetAsync(h->rtickets, 0, (cl + cr) * sizeof(int), h->stream));
     size_t const statusBytes = (cl / kMutualSlice + 1) * sizeof(unsigned long long);
     HIPCHECK(h, hipMalloc(&h->mstatus, statusBytes));
     HIPCHECK(h, hipMemsetAsync(h->mstatus, 0, statusBytes, h->stream));
@@ -477,10 +487,10 @@ int runGuided(v3dm_context* h, int kind, const double M[9], float distanceThresh
         launch_score_pass(h, p, h->guidedBits, minScore);
         if ((rc = prof_end(h))) return rc;
         launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
-                            h->normR, h->maxNormBits, h->epsRel, minScore, minRatio, h->colMax, h->rowMax,
+                            h->normR, h->maxNormBits, score_eps(h, h->guidedBits), minScore, minRatio, h->colMax, h->rowMax,
                             h->flagList, h->capL, h->results, st);
-        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->results, minScore, minRatio, h->colMax,
-                             h->rowMax, h->rpart, kRecheckGrid, st, h->guidedBits, h->capL);
+        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore, minRatio,
+                             h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st, h->guidedBits, h->capL);
     }
     launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
                           reinterpret_cast<int2*>(h->results + kNumCounters), h->results, st, {}, h->mutualWait);

@@ -116,6 +116,7 @@ struct BatchState {
     // selection / results
     int* sel = nullptr;
     int* flagList = nullptr;
+    int* tickets = nullptr;   // of the exact re-check, one per query row
     int* openList = nullptr;  // open decisions of the shortlist rescoring
     int selCap = 0;
     int* counters = nullptr;  // kBatchCounters ints
@@ -406,7 +407,8 @@ int upload_plan(v3dm_context* h, BatchState* b, int form, Plan const& pl)
     if ((rc = growi(h, b->segD[form], b->segCap[form], pl.seg.size()))) return rc;
     if ((rc = growi(h, b->blkInfo[form], b->blkInfoCap[form], pl.blocks.size()))) return rc;
     if (form == 0 || form == 3) {
-        if ((rc = grow(h, b->partF, b->partFCap, pl.partSlots))) return rc;
+        // at least one slot per query row: the re-check's partials go there after the merge
+        if ((rc = grow(h, b->partF, b->partFCap, std::max(pl.partSlots, (size_t)b->qRows)))) return rc;
     } else {
         if ((rc = grow(h, b->partB, b->partBCap, pl.partSlots * 2))) return rc;
     }
@@ -559,7 +561,10 @@ int ensure_query_space(v3dm_context* h, BatchState* b)
     if ((rc = growi(h, b->sel, b->selCap, b->qRows))) return rc;
     if (b->flagList) (void)hipFree(b->flagList);
     if (b->openList) (void)hipFree(b->openList);
-    b->flagList = b->openList = nullptr;
+    if (b->tickets) (void)hipFree(b->tickets);
+    b->flagList = b->openList = b->tickets = nullptr;
+    BCHECK(h, hipMalloc(&b->tickets, (size_t)std::max(b->qRows, 1) * sizeof(int)));
+    BCHECK(h, hipMemsetAsync(b->tickets, 0, (size_t)std::max(b->qRows, 1) * sizeof(int), h->stream));
     BCHECK(h, hipMalloc(&b->flagList, (size_t)std::max(b->qRows, 1) * sizeof(int)));
     BCHECK(h, hipMalloc(&b->openList, (size_t)std::max(b->qRows, 1) * sizeof(int)));
     int const nbMutual = (b->leftRows + 1023) / 1024;
@@ -624,6 +629,12 @@ int ensure_split(v3dm_context* h, BatchState* b)
     return grow(h, b->split, b->splitCap, need);
 }
 
+// The certified decisions' error bound for the scores of launch_plain_pass.
+float plain_eps(v3dm_context const* h, BatchState const* b)
+{
+    return b->splitFit ? h->epsRel * (b->haveU8 ? kIntEps : kSplitEps) : h->epsRel;
+}
+
 // The plain pass of plan `form` (0, or 3: the pairs a learned run hands over) on the images'
 // split rows, or on the FP32 rows where a row is outside the split range.
 void launch_plain_pass(BatchState* b, int form, int4 const* items, int nItems, int* queue, float minScore,
@@ -648,8 +659,9 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
     if (!h->cacheDerived) enqueue_derived(h, b, form);
     if (form == 0) {
         launch_plain_pass(b, 0, b->items[0], (int)pl.items.size(), b->counters + 0, minScore, st);
-        launch_batch_merge_decide(d, b->partF, h->epsRel, minScore, minRatio, b->sel, b->flagList, b->counters, st);
-        launch_batch_recheck(d, b->flagList, b->counters, minScore, minRatio, b->sel, 1024, st);
+        launch_batch_merge_decide(d, b->partF, plain_eps(h, b), minScore, minRatio, b->sel, b->flagList, b->counters, st);
+        launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio,
+                             b->sel, 1024, st);
     } else if (form == 1) {
         launch_batch_pass_bf16(d, b->items[1], (int)pl.items.size(), b->counters + 1, b->partB, pl.grid, pl.qRows,
                                st);
@@ -695,9 +707,10 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
             if (b->splitFit && !(h->cacheDerived && b->splitValid))
                 launch_batch_split_masked(d0, b->segMask, b->split, 2 * cus, st);
             launch_plain_pass(b, 3, b->fbItems, np, b->counters + 0, minScore, st, b->counters + kBCntFbItems);
-            launch_batch_merge_masked(d0, b->partF, h->epsRel, minScore, minRatio, b->sel, b->flagList, b->counters,
+            launch_batch_merge_masked(d0, b->partF, plain_eps(h, b), minScore, minRatio, b->sel, b->flagList, b->counters,
                                       b->segMask, 2 * cus, st);
-            launch_batch_recheck(d0, b->flagList, b->counters, minScore, minRatio, b->sel, 1024, st);
+            launch_batch_recheck(d0, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore,
+                                 minRatio, b->sel, 1024, st);
         }
     }
     launch_batch_mutual(d, b->sel, b->leftRows, b->tmp, b->blockCount, b->out, b->pairCount, b->stripes,
@@ -982,7 +995,7 @@ void batch_destroy(BatchState*& b)
                     (void*)b->items[0], (void*)b->items[1], (void*)b->items[2], (void*)b->items[3],
                     (void*)b->segD[0], (void*)b->segD[1], (void*)b->segD[2], (void*)b->segD[3], (void*)b->blkInfo[0],
                     (void*)b->blkInfo[1], (void*)b->blkInfo[2], (void*)b->blkInfo[3], (void*)b->partF,
-                    (void*)b->partB, (void*)b->sel, (void*)b->flagList, (void*)b->openList, (void*)b->sRows, (void*)b->sNorm, (void*)b->sIdx, (void*)b->sCount,
+                    (void*)b->partB, (void*)b->sel, (void*)b->flagList, (void*)b->openList, (void*)b->tickets, (void*)b->sRows, (void*)b->sNorm, (void*)b->sIdx, (void*)b->sCount,
                     (void*)b->sNSplits, (void*)b->sPart, (void*)b->sItems, (void*)b->pairFlag, (void*)b->fbItems,
                     (void*)b->segMask, (void*)b->rowCS, (void*)b->cItems[0],
                     (void*)b->cItems[1], (void*)b->cNSplits, (void*)b->cPart, (void*)b->cQB, (void*)b->cSlotB,

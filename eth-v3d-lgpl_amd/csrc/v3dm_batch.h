@@ -164,8 +164,10 @@ void launch_batch_check_probe(BatchDev const& b, CheckDev const& c, int phase, i
                               int cus, hipStream_t st);
 void launch_batch_check_decide(BatchDev const& b, CheckDev const& c, int phase, float minScore, float minRatio,
                                MissLimits const& lim, int const* sel, int* pairFlag, int* counts, hipStream_t st);
-void launch_batch_recheck(BatchDev const& b, int const* flagList, int* counters, float minScore, float minRatio,
-                          int* sel, int grid, hipStream_t st);
+// part: scratch for at least qRows partials (room of them); tickets: qRows ints, zero before the
+// first call and left zero
+void launch_batch_recheck(BatchDev const& b, int const* flagList, int* counters, Top2* part, size_t room,
+                          int* tickets, float minScore, float minRatio, int* sel, int grid, hipStream_t st);
 // the plain items of the pairs with pairFlag set -> fbItems (count in *fbCount, which must
 // be zero), segMask[s] = flag of segment s's pair (2 * nPairs segments)
 void launch_batch_fb_filter(int4 const* items, int nItems, int const* pairFlag, int nPairs, int4* fbItems,

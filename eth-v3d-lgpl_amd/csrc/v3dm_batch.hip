@@ -179,81 +179,58 @@ void launch_batch_merge_masked(BatchDev const& b, Top2 const* part, float epsRel
                        flagList, counters, segMask);
 }
 
-// Exact decision of one open query per work-group (grid-stride over the flag list).
-// Thread t scores candidates t, t + 256, ... as fl32(sum_k double(q_k) * double(c_k)) in
-// ascending k: the candidates pass through LDS 256 rows at a time, in two halves of 64
-// components, and each thread carries its FP64 sum across the halves, so the order of the
-// sum is the oracle's.  The per-thread top-2 states (ascending candidates) are merged by
-// an order-independent merge.
-constexpr int kBRecheckRows = 256;
-constexpr int kBRecheckStride = 68;  // floats per staged half row (64 + 4 pad)
-
+// Exact decisions of the open queries (listed rows of the query space), as the single-pair
+// re-check: a wave per unit of one query and a chunk of its candidates, the last wave of a
+// query merging the partials.  `room` partials (the pass's buffer, merged by now) bound the
+// chunks per query; the fewer queries are open, the shorter the chunks.  A query per
+// work-group through LDS, 256 candidates at a time: 570 us on the 256-pair uint8 batch, 23 us
+// so, most of the difference from the tighter bound of integer scores (fewer queries open).
 __global__ __launch_bounds__(256) void k_batch_recheck(BatchDev b, int const* __restrict__ flagList,
-                                                       int const* __restrict__ counters, float minScore,
+                                                       int const* __restrict__ counters, Top2* __restrict__ part,
+                                                       long long room, int* __restrict__ tickets, float minScore,
                                                        float minRatio, int* __restrict__ sel)
 {
-    __shared__ __attribute__((aligned(16))) float cand[kBRecheckRows * kBRecheckStride];
-    __shared__ double qd[kDim];
-    __shared__ Top2 wtop[4];
-    int const tid = threadIdx.x;
-    int const lane = tid & 63;
-    int const wave = tid >> 6;
-    int const nFlag = counters[kBCntFlag];
-    for (int w = blockIdx.x; w < nFlag; w += gridDim.x) {
-        int const g = flagList[w];
+    __shared__ __attribute__((aligned(16))) float stage[4][kExactLds];
+    __shared__ __attribute__((aligned(16))) double qd[4][kDim];
+    int const lane = threadIdx.x & 63;
+    int const wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * 256 + threadIdx.x) >> 6));
+    int const nFlag = __builtin_amdgcn_readfirstlane(counters[kBCntFlag]);
+    if (nFlag == 0) return;
+    int const most = (int)max(1ll, min(room / nFlag, 256ll));  // chunks per query
+    long long const units = (long long)nFlag * most;
+    for (long long w = wave; w < units; w += (long long)gridDim.x * 4) {
+        int const e = (int)(w / most), c = (int)(w - (long long)e * most);
+        int const g = __builtin_amdgcn_readfirstlane(flagList[e]);
         BatchSeg const sg = b.seg[b.segOfBlock[g / kBatchRowAlign]];
-        int const q = g - sg.qOff;
-        float const* Qd = b.img + (size_t)(b.imgBase[sg.img] + q) * kDim;
-        float const* Cd = b.img + (size_t)b.imgBase[sg.oImg] * kDim;
-        __syncthreads();  // the previous query's LDS contents are consumed
-        if (tid < kDim) qd[tid] = (double)Qd[tid];
+        int const nSub = (sg.nO + 63) / 64;
+        int const subs = (nSub + most - 1) / most;
+        int const nCh = (nSub + subs - 1) / subs;
+        if (c >= nCh) continue;  // uniform over the wave
+        float const* const q[1] = {b.img + (size_t)(b.imgBase[sg.img] + g - sg.qOff) * kDim};
+        exact_queries<1>(q, qd[threadIdx.x >> 6], lane);
+        float const* const C = b.img + (size_t)b.imgBase[sg.oImg] * kDim;
+        int const c1 = min((c + 1) * subs * 64, sg.nO);
         Top2 s = top2_init();
-        for (int c0 = 0; c0 < sg.nO; c0 += kBRecheckRows) {
-            double acc = 0.0;
-            for (int half = 0; half < 2; ++half) {
-                __syncthreads();  // every thread is done with the staged half
-                // 256 rows x 64 floats = 4096 float4: 16 per thread, row-contiguous
-#pragma unroll 4
-                for (int u = 0; u < 16; ++u) {
-                    int const f = u * 256 + tid;
-                    int const r = f >> 4, c4 = f & 15;
-                    // rows past nO are the image's zero padding (images are padded to
-                    // multiples of 256 rows): in bounds, and masked below
-                    float4 const v =
-                        reinterpret_cast<float4 const*>(Cd + (size_t)(c0 + r) * kDim + half * 64)[c4];
-                    *reinterpret_cast<float4*>(&cand[r * kBRecheckStride + 4 * c4]) = v;
-                }
-                __syncthreads();
-                float const* cr = &cand[tid * kBRecheckStride];
-                double const* qh = qd + half * 64;
-#pragma unroll 8
-                for (int k4 = 0; k4 < 16; ++k4) {
-                    float4 const y = *reinterpret_cast<float4 const*>(cr + 4 * k4);
-                    acc += qh[4 * k4 + 0] * (double)y.x;
-                    acc += qh[4 * k4 + 1] * (double)y.y;
-                    acc += qh[4 * k4 + 2] * (double)y.z;
-                    acc += qh[4 * k4 + 3] * (double)y.w;
-                }
-            }
-            int const j = c0 + tid;
-            float const sc = (float)acc;
-            if (j < sg.nO && sc == sc) top2_push(s, sc, j);
+        for (int c0 = c * subs * 64; c0 < c1; c0 += 64) {
+            int const j = c0 + lane;
+            float v[1];
+            exact_scores<1>(qd[threadIdx.x >> 6], C + (size_t)c0 * kDim, sg.nO - c0, stage[threadIdx.x >> 6], lane, v);
+            if (j < c1) top2_push(s, v[0], j);
         }
-#pragma unroll
         for (int o = 32; o > 0; o >>= 1) s = top2_merge(s, top2_shfl_xor(s, o));
-        if (lane == 0) wtop[wave] = s;
-        __syncthreads();
-        if (tid == 0) {
-            Top2 t = top2_merge(top2_merge(wtop[0], wtop[1]), top2_merge(wtop[2], wtop[3]));
-            sel[g] = decide_exact(t, minScore, minRatio);
+        Top2* const p = part + (size_t)e * most;
+        if (publish_partial(s, p, c, nCh, tickets + e, lane)) {
+            Top2 const t = merge_partials(p, nCh, lane);
+            if (lane == 0) sel[g] = decide_exact(t, minScore, minRatio);
         }
     }
 }
 
-void launch_batch_recheck(BatchDev const& b, int const* flagList, int* counters, float minScore, float minRatio,
-                          int* sel, int grid, hipStream_t st)
+void launch_batch_recheck(BatchDev const& b, int const* flagList, int* counters, Top2* part, size_t room,
+                          int* tickets, float minScore, float minRatio, int* sel, int grid, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_batch_recheck, dim3(grid), dim3(256), 0, st, b, flagList, counters, minScore, minRatio, sel);
+    hipLaunchKernelGGL(k_batch_recheck, dim3(grid), dim3(256), 0, st, b, flagList, counters, part, (long long)room,
+                       tickets, minScore, minRatio, sel);
 }
 
 // Mutual check over the left-query rows [0, leftRows) of the query space (segments 0 ..

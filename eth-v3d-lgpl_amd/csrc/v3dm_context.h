@@ -54,6 +54,7 @@ struct v3dm_context {
     int* rowMax = nullptr;
     int* flagList = nullptr;
     v3dm::Top2* rpart = nullptr;       // re-check chunk partials: (capL + capR) x kRecheckMaxChunks
+    int* rtickets = nullptr;           // re-check tickets: capL + capR
     unsigned long long* mstatus = nullptr;  // mutual-check status words: capL / kMutualSlice + 1
     unsigned mutualEpoch = 0;               // epoch of the last mutual check (never 0 once run)
     v3dm::MutualWait mutualWait;            // the look-back's wait (v3dm_debug_mutual_wait)

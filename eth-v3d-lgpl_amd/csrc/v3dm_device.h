@@ -205,4 +205,109 @@ __device__ __forceinline__ float group_best(v16f const& a0, v16f const& a1, int 
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
+// Exact re-check of open queries (single pair and batch).  A wave scores kQ queries (their
+// rows as doubles in the wave's own LDS, read by broadcast) against the 64 candidates from row c on (nRows of them exist; the rest
+// repeat the last), one per lane: fl32(sum_k double(q_k) * double(c_k)) in ascending k
+// (products of floats are exact in FP64, so fused multiply-adds give the same sum).  The
+// candidates' rows are loaded whole lines at a time (8 lanes a row) and pass through the wave's
+// own LDS a quarter (32 components) at a time, the next quarter in flight; no barrier.  Few
+// queries are open (tens of 32768), so what counts is the time of one unit: 38 us with the
+// units of a query in one work-group's loop through LDS, 62 us with every lane loading its own
+// row (each line fetched eight times); with the query rows as scalar loads their latency is
+// exposed every few components (20 us).
+constexpr int kExactRow = 36;  // floats per staged quarter row (32 + 4 pad)
+constexpr int kExactLds = 64 * kExactRow;
+
+// 16 bytes of a row: a quarter of 8 rows is one load of the wave, 8 lanes a row.
+__device__ __forceinline__ v4f exact_chunk(float const* __restrict__ c, int row, int chunk)
+{
+    return reinterpret_cast<v4f const*>(c + (size_t)row * kDim)[chunk];
+}
+
+// The wave's query rows into its LDS.
+template <int kQ>
+__device__ __forceinline__ void exact_queries(float const* const (&q)[kQ], double* __restrict__ qd, int lane)
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the previous unit's reads come first
+#pragma unroll
+    for (int j = 0; j < kQ; ++j) {
+        float2 const v = reinterpret_cast<float2 const*>(q[j])[lane];
+        qd[j * kDim + 2 * lane] = (double)v.x;
+        qd[j * kDim + 2 * lane + 1] = (double)v.y;
+    }
+}
+
+template <int kQ>
+__device__ __forceinline__ void exact_scores(double const* __restrict__ qd, float const* __restrict__ c, int nRows,
+                                             float* __restrict__ stage, int lane, float (&out)[kQ])
+{
+    double acc[kQ];
+#pragma unroll
+    for (int j = 0; j < kQ; ++j) acc[j] = 0.0;
+    v4f v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = exact_chunk(c, min(8 * u + (lane >> 3), nRows - 1), lane & 7);
+    float const* const mine = stage + lane * kExactRow;
+#pragma unroll 1
+    for (int p = 0; p < 4; ++p) {
+        // LDS operations of one wave are in order: the fences only keep the compiler's order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            *reinterpret_cast<v4f*>(stage + (8 * u + (lane >> 3)) * kExactRow + 4 * (lane & 7)) = v[u];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        int const next = min(p + 1, 3);  // (the last quarter once more, unused)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = exact_chunk(c, min(8 * u + (lane >> 3), nRows - 1), 8 * next + (lane & 7));
+#pragma unroll 4
+        for (int k = 0; k < 8; ++k) {
+            float4 const x = *reinterpret_cast<float4 const*>(mine + 4 * k);
+            double const x0 = x.x, x1 = x.y, x2 = x.z, x3 = x.w;
+#pragma unroll
+            for (int j = 0; j < kQ; ++j) {
+                double const* const y = qd + j * kDim + 32 * p + 4 * k;
+                acc[j] += y[0] * x0;
+                acc[j] += y[1] * x1;
+                acc[j] += y[2] * x2;
+                acc[j] += y[3] * x3;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kQ; ++j) out[j] = (float)acc[j];
+}
+
+// One wave's partial top-2 of an open query, published to the device (part[c] of the query's
+// nCh partials), and the query's ticket; returns whether this wave is the last of the query,
+// whose partials it may then merge (merge_partials).  The ticket is left at zero.
+__device__ __forceinline__ bool publish_partial(Top2 s, Top2* part, int c, int nCh, int* ticket, int lane)
+{
+    int last = 0;
+    if (lane == 0) {
+        int* const p = reinterpret_cast<int*>(part + c);
+        __hip_atomic_store(p + 0, __float_as_int(s.b1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p + 1, __float_as_int(s.b2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p + 2, s.a1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nCh - 1;
+        if (last) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return __shfl(last, 0) != 0;
+}
+
+__device__ __forceinline__ Top2 merge_partials(Top2 const* part, int nCh, int lane)
+{
+    Top2 s = top2_init();
+    for (int c = lane; c < nCh; c += 64) {
+        int const* const p = reinterpret_cast<int const*>(part + c);
+        Top2 t;
+        t.b1 = __int_as_float(__hip_atomic_load(p + 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        t.b2 = __int_as_float(__hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        t.a1 = __hip_atomic_load(p + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s = top2_merge(s, t);
+    }
+    for (int o = 32; o > 0; o >>= 1) s = top2_merge(s, top2_shfl_xor(s, o));
+    return s;
+}
+
 }  // namespace v3dm

@@ -35,6 +35,7 @@ struct ExtState {
     int* sDecHost = nullptr;   // the same memory as the host addresses it
     int* sFlags = nullptr;     // open-query list of the samples
     Top2* sRpart = nullptr;    // re-check partials
+    int* sTickets = nullptr;   // re-check tickets
     int* sCounters = nullptr;  // kNumCounters
     int* sHost = nullptr;      // learned decisions of the samples (pinned, mapped, coherent)
     int* sHostDev = nullptr;   // sHost as the kernels address it
@@ -150,6 +151,8 @@ int ensure_sample(v3dm_context* h, ExtState* e)
     EXTCHECK(h, hipHostGetDevicePointer((void**)&e->sDec, e->sDecHost, 0));
     EXTCHECK(h, hipMalloc(&e->sFlags, (kSampleRows + 1) * sizeof(int)));
     EXTCHECK(h, hipMalloc(&e->sRpart, (size_t)(kSampleRows + 1) * kRecheckMaxChunks * sizeof(Top2)));
+    EXTCHECK(h, hipMalloc(&e->sTickets, (kSampleRows + 1) * sizeof(int)));
+    EXTCHECK(h, hipMemset(e->sTickets, 0, (kSampleRows + 1) * sizeof(int)));
     EXTCHECK(h, hipMalloc(&e->sCounters, kNumCounters * sizeof(int)));
     EXTCHECK(h, hipHostMalloc(&e->sHost, kSampleRows * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     EXTCHECK(h, hipHostGetDevicePointer((void**)&e->sHostDev, e->sHost, 0));
@@ -182,8 +185,8 @@ int enqueue_sample_check(v3dm_context* h, ExtState* e, float minScore, float min
     launch_fused_fp32(e->sL, h->dR, S, nR, p, e->sColPart, kSampleRows, nullptr, 0, st);  // left decisions only
     launch_sample_decide(e->sColPart, p.splits, kSampleRows, S, e->sNorm, h->maxNormBits, h->epsRel, minScore,
                          minRatio, e->sDec, e->sFlags, e->sCounters, st);
-    launch_recheck_exact(e->sL, h->dR, S, nR, e->sFlags, kSampleRows, e->sCounters, minScore, minRatio, e->sDec,
-                         e->sDec + kSampleRows, e->sRpart, kRecheckGrid, st);
+    launch_recheck_exact(e->sL, h->dR, S, nR, e->sFlags, kSampleRows, 1, e->sCounters, minScore, minRatio, e->sDec,
+                         e->sDec + kSampleRows, e->sRpart, e->sTickets, kRecheckGrid, st);
     e->sSamples = S;
     return V3DM_OK;
 }
@@ -411,7 +414,7 @@ void ext_release(ExtState* e)
     e->cLValid = e->cRValid = false;
     if (e->side) (void)hipStreamSynchronize(e->side);
     for (void* p : {(void*)e->sL, (void*)e->sNorm, (void*)e->sIdx, (void*)e->sColPart, (void*)e->sFlags,
-                    (void*)e->sRpart, (void*)e->sCounters})
+                    (void*)e->sRpart, (void*)e->sTickets, (void*)e->sCounters})
         if (p) (void)hipFree(p);
     if (e->sHost) (void)hipHostFree(e->sHost);
     if (e->sDecHost) (void)hipHostFree(e->sDecHost);
@@ -423,6 +426,7 @@ void ext_release(ExtState* e)
     e->sL = e->sNorm = nullptr;
     e->sIdx = e->sDec = e->sDecHost = e->sFlags = e->sCounters = e->sHost = e->sHostDev = nullptr;
     e->sColPart = e->sRpart = nullptr;
+    e->sTickets = nullptr;
     e->sPending = false;
     e->f8L = e->f8R = e->eL = e->eR = nullptr;
     e->f8LValid = e->f8RValid = false;

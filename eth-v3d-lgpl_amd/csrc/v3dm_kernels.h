@@ -23,7 +23,7 @@ constexpr double kFallbackAlpha = 0.05;  // level of the sampled check's one-sid
 constexpr int kFallbackMaxAccepted = 1 << 24;  // largest count v3dm_fallback_allowed_misses takes  // ... its right features split into up to 256 work-groups
 constexpr int kStripes = 64;
 constexpr int kStripeStride = 32;  // ints (128 bytes)
-constexpr int kRecheckMaxChunks = 64;  // candidate chunks per re-checked query
+constexpr int kRecheckMaxChunks = 64;  // re-check partials per row of either side
 constexpr int kRowPad = 128;      // device descriptor buffers hold a multiple of 128 rows
 constexpr int kRecheckGrid = 1024;
 // |approximate score - exact score| <= epsRel * ||q|| * max||c|| + kEpsAbs for the FP32
@@ -32,11 +32,6 @@ constexpr int kRecheckGrid = 1024;
 // sends every query to the exact re-check.
 constexpr float kEpsRelFp32 = 3.0517578125e-05f;  // 2^-15
 constexpr float kEpsAbs = 1e-30f;
-
-struct RecheckPlan {
-    int nChunks = 1;
-    int per = 1;  // candidates per thread of one chunk
-};
 
 struct FusedPlan {
     int leftBlocks = 0;
@@ -50,12 +45,13 @@ void launch_merge_decide(Top2 const* colPart, int nColParts, int ldc, Top2 const
                          int nL, int nR, float const* normL, float const* normR, unsigned int const* maxNormBits,
                          float epsRel, float minScore, float minRatio, int* colMax, int* rowMax, int* flagList,
                          int flagOffR, int* counters, hipStream_t st);
-RecheckPlan plan_recheck(int nC);
-// flagList: open left queries at [0, ...), open right queries at [flagOffR, ...).  gbits:
-// guided-matching bitmap (pairs scored -1e20), or null.
-void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int const* flagList, int flagOffR,
+// flagList: open left queries at [0, ...) (at most rowsL), open right queries at [rowsL, ...)
+// (at most rowsR); part: (rowsL + rowsR) * kRecheckMaxChunks partials; tickets: rowsL + rowsR
+// ints, zero before the first call and left zero.  gbits: guided-matching bitmap (pairs scored
+// -1e20), or null.
+void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int const* flagList, int rowsL, int rowsR,
                           int const* counters, float minScore, float minRatio, int* colMax, int* rowMax, Top2* part,
-                          int grid, hipStream_t st, unsigned const* gbits = nullptr, int ldi = 0);
+                          int* tickets, int grid, hipStream_t st, unsigned const* gbits = nullptr, int ldi = 0);
 // The learned decisions of the S sampled left features of the sampled exact check:
 // out[k] = colMax[sample_row(k, nL, S)], k < S.  out may be mapped host memory.  S = 0:
 // nothing to write.

@@ -49,7 +49,8 @@ constexpr size_t kOffStatus = kOffRpart + alignUp((size_t)2 * kNoAllocCap * kRec
 constexpr size_t kOffStripes =
     kOffStatus + alignUp((size_t)(kNoAllocCap / kMutualSlice + 1) * sizeof(unsigned long long));
 constexpr size_t kOffCounters = kOffStripes + alignUp((size_t)kStripes * kStripeStride * sizeof(int));
-constexpr size_t kNoAllocScratchBytes = kOffCounters + kAlign;
+constexpr size_t kOffTickets = kOffCounters + kAlign;
+constexpr size_t kNoAllocScratchBytes = kOffTickets + alignUp((size_t)2 * kNoAllocCap * sizeof(int));
 
 static_assert(kNoAllocCap % 128 == 0, "the cap is a whole number of 128-row blocks");
 
@@ -173,8 +174,8 @@ int v3dm_match_device_noalloc(const float* leftDesc, int nLeft, const float* rig
         launch_fused_fp32(L, R, nL, nR, p, colPart, capL, rowPart, capR, st);
         launch_merge_decide(colPart, p.splits, capL, rowPart, p.leftBlocks, capR, nL, nR, normL, normR, maxNorm,
                             kEpsRelFp32, minScore, minRatio, colMax, rowMax, flagList, capL, counters, st);
-        launch_recheck_exact(L, R, nL, nR, flagList, capL, counters, minScore, minRatio, colMax, rowMax, rpart,
-                             kRecheckGrid, st);
+        launch_recheck_exact(L, R, nL, nR, flagList, capL, capR, counters, minScore, minRatio, colMax, rowMax,
+                             rpart, reinterpret_cast<int*>(b + kOffTickets), kRecheckGrid, st);
     }
     launch_mutual_compact(colMax, rowMax, work ? nL : 0, nR, status, ep, stripes, reinterpret_cast<int2*>(pairs),
                           counters, st);

@@ -241,181 +241,127 @@ void launch_merge_decide(Top2 const* colPart, int nColParts, int ldc, Top2 const
 
 // ------------------------------------------------------------------------------ exact re-check
 // Open queries are listed per direction (left queries at flagList[0..), right queries at
-// flagList[flagOffR..)).  Pass 1: a work item is (group of up to kRecheckGroup queries of
-// one direction, chunk of 256*per candidates); grid-stride over all items.  Each thread
-// scores its candidate against every query of the group: fl32(sum_k double(q_k) *
-// double(c_k)) in ascending k (products of floats are exact in FP64, so fused
-// multiply-adds give the same sum), the group's queries being independent FP64 chains.
-// The chunk's top-2 per query (first index on ties) goes to part[(row) * kRecheckMaxChunks
-// + chunk].  Pass 2: one wave per open query merges its chunk partials and takes the IEEE
-// FP32 decision.  The kernel boundary between the passes orders the partial writes.
-constexpr int kRecheckGroup = 16;
-constexpr int kRecheckSub = 64;     // candidates staged in LDS at a time
-constexpr int kRecheckRow = 132;    // floats per staged candidate row (528 bytes: conflict-free b128 reads)
+// flagList[flagOffR..)).  A work unit is (one or up to kRecheckGroup queries of one direction, chunk of 64 *
+// subs candidates), one wave each, grid-stride over all units; the last wave of a query
+// merges its partials and takes the IEEE FP32 decision.  Chunks are as short as the partials'
+// buffer allows (kRecheckMaxChunks per listed row of either side, so the fewer queries are
+// open, the more chunks each gets): with the usual tens of open queries every unit is one
+// step of 64 candidates, 14 us for a few open queries of 16384 x 16384 in one launch (a chain of
+// loads, 64 dependent FP64 steps a quarter and the tickets; nothing is near a rate) against
+// 38 + 5 us in two.  With every query open (a zero error bound) it is 1.3 times the earlier
+// 16 queries a group: 3.7 against 2.8 ms at 8192 x 8192.
+constexpr int kRecheckGroup = 4;  // queries per unit: they share the candidates' loads
 
-__global__ __launch_bounds__(256) void k_recheck_chunks(float const* __restrict__ L, float const* __restrict__ R,
-                                                        int nL, int nR, int const* __restrict__ flagList,
-                                                        int flagOffR, int const* __restrict__ counters,
-                                                        int nChunksL, int perL, int nChunksR, int perR,
-                                                        Top2* __restrict__ part, unsigned const* __restrict__ gbits,
-                                                        int ldi)
+struct RecheckDir {
+    float const* Q;
+    float const* C;
+    int* sel;
+    int nC, cnt, base;  // base: first list entry and row of the partials
+    int subs, nCh;
+};
+
+__device__ __forceinline__ RecheckDir recheck_dir(bool left, float const* L, float const* R, int nL, int nR, int cnt,
+                                                  int rowsL, int rowsR, int* colMax, int* rowMax)
 {
-    __shared__ __attribute__((aligned(16))) double qd[kRecheckGroup][kDim];
-    __shared__ __attribute__((aligned(16))) float cand[kRecheckSub * kRecheckRow];
-    __shared__ int qidx[kRecheckGroup];
-    int const tid = threadIdx.x;
-    int const lane = tid & 63;
-    int const wave = tid >> 6;
-    int const cntL = counters[kCntFlag];
-    int const cntR = counters[kCntFlagR];
-    int const grpL = (cntL + kRecheckGroup - 1) / kRecheckGroup;
-    int const grpR = (cntR + kRecheckGroup - 1) / kRecheckGroup;
-    int const itemsL = grpL * nChunksL;
-    int const items = itemsL + grpR * nChunksR;
-    for (int w = blockIdx.x; w < items; w += gridDim.x) {
-        bool const left = w < itemsL;
-        int const wl = left ? w : w - itemsL;
-        int const nCh = left ? nChunksL : nChunksR;
-        int const per = left ? perL : perR;
-        int const g = wl / nCh;
-        int const c = wl - g * nCh;
-        int const cnt = left ? cntL : cntR;
-        int const base = left ? 0 : flagOffR;
-        int const nq = min(kRecheckGroup, cnt - g * kRecheckGroup);
-        float const* Qs = left ? L : R;
-        float const* C = left ? R : L;
-        int const nC = left ? nR : nL;
-        __syncthreads();
-        if (tid < kRecheckGroup) qidx[tid] = (tid < nq) ? flagList[base + g * kRecheckGroup + tid] : -1;
-        __syncthreads();
-        {
-            // 16 queries x 128 floats = 512 float4: two independent float4 loads per thread
-            float4 v[2];
-            int qi[2], k4[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                int const x = u * 256 + tid;
-                qi[u] = x >> 5;
-                k4[u] = x & 31;
-                int const row = qidx[qi[u]];
-                v[u] = (row >= 0) ? reinterpret_cast<float4 const*>(Qs + (size_t)row * kDim)[k4[u]]
-                                  : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                qd[qi[u]][4 * k4[u] + 0] = v[u].x;
-                qd[qi[u]][4 * k4[u] + 1] = v[u].y;
-                qd[qi[u]][4 * k4[u] + 2] = v[u].z;
-                qd[qi[u]][4 * k4[u] + 3] = v[u].w;
-            }
-        }
-        // wave w scores queries 4w .. 4w+3 of the group; lane = candidate of the sub-tile
-        Top2 s[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s[j] = top2_init();
-        int const cbeg = c * 256 * per;
-        int const cend = min(cbeg + 256 * per, nC);
-        for (int c0 = cbeg; c0 < cend; c0 += kRecheckSub) {
-            __syncthreads();  // previous sub-tile consumed (and qd written, first time)
-            {
-                float4 v[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    int const x = u * 256 + tid;
-                    int const row = x >> 5, k4 = x & 31;
-                    v[u] = (c0 + row < nC) ? reinterpret_cast<float4 const*>(C + (size_t)(c0 + row) * kDim)[k4]
-                                           : make_float4(0.f, 0.f, 0.f, 0.f);
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    int const x = u * 256 + tid;
-                    int const row = x >> 5, k4 = x & 31;
-                    *reinterpret_cast<float4*>(&cand[row * kRecheckRow + 4 * k4]) = v[u];
-                }
-            }
-            __syncthreads();
-            double acc[4] = {0.0, 0.0, 0.0, 0.0};
-            float const* cr = &cand[lane * kRecheckRow];
-#pragma unroll 4
-            for (int k4 = 0; k4 < 32; ++k4) {
-                float4 const v = *reinterpret_cast<float4 const*>(cr + 4 * k4);
-                double const x0 = v.x, x1 = v.y, x2 = v.z, x3 = v.w;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    double const* q = &qd[4 * wave + j][4 * k4];
-                    acc[j] += q[0] * x0;
-                    acc[j] += q[1] * x1;
-                    acc[j] += q[2] * x2;
-                    acc[j] += q[3] * x3;
-                }
-            }
-            int const ci = c0 + lane;
-            if (ci < nC) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float v = (float)acc[j];
-                    int const qrow = qidx[4 * wave + j];
-                    if (gbits && qrow >= 0) {
-                        // guided matching: a removed (left, right) pair scores -1e20
-                        int const li = left ? qrow : ci;
-                        int const rj = left ? ci : qrow;
-                        v = ((gbits[(size_t)(rj >> 5) * ldi + li] >> (rj & 31)) & 1u) ? -1e20f : v;
-                    }
-                    top2_push(s[j], v, ci);
-                }
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            Top2 t = s[j];
-            for (int o = 32; o > 0; o >>= 1) t = top2_merge(t, top2_shfl_xor(t, o));
-            int const qg = 4 * wave + j;
-            if (lane == 0 && qg < nq) part[(size_t)(base + g * kRecheckGroup + qg) * kRecheckMaxChunks + c] = t;
-        }
-    }
+    RecheckDir d;
+    d.Q = left ? L : R;
+    d.C = left ? R : L;
+    d.sel = left ? colMax : rowMax;
+    d.nC = left ? nR : nL;
+    d.cnt = cnt;
+    d.base = left ? 0 : rowsL;
+    int const nSub = (d.nC + 63) / 64;
+    long long const room = (long long)(left ? rowsL : rowsR) * kRecheckMaxChunks / max(cnt, 1);
+    int const most = (int)min(room, (long long)nSub);
+    d.subs = (nSub + most - 1) / max(most, 1);
+    d.nCh = (nSub + d.subs - 1) / d.subs;
+    return d;
 }
 
-__global__ __launch_bounds__(256) void k_recheck_finish(int const* __restrict__ flagList, int flagOffR,
-                                                        int const* __restrict__ counters, int nChunksL,
-                                                        int nChunksR, Top2 const* __restrict__ part,
-                                                        float minScore, float minRatio, int* __restrict__ colMax,
-                                                        int* __restrict__ rowMax)
+template <int kQ>
+__device__ __forceinline__ void recheck_units(RecheckDir const& dl, RecheckDir const& dr, int const* flagList,
+                                              Top2* __restrict__ part, int* __restrict__ tickets,
+                                              unsigned const* __restrict__ gbits, int ldi, float minScore,
+                                              float minRatio, float* __restrict__ stage, double* __restrict__ qd)
 {
     int const lane = threadIdx.x & 63;
-    int const cntL = counters[kCntFlag];
-    int const cnt = cntL + counters[kCntFlagR];
-    for (int e = blockIdx.x * 4 + (threadIdx.x >> 6); e < cnt; e += gridDim.x * 4) {
-        bool const left = e < cntL;
-        int const row = left ? e : flagOffR + (e - cntL);
-        int const nCh = left ? nChunksL : nChunksR;
-        Top2 s = top2_init();
-        for (int c = lane; c < nCh; c += 64) s = top2_merge(s, part[(size_t)row * kRecheckMaxChunks + c]);
-        for (int o = 32; o > 0; o >>= 1) s = top2_merge(s, top2_shfl_xor(s, o));
-        if (lane == 0) (left ? colMax : rowMax)[flagList[row]] = decide_exact(s, minScore, minRatio);
+    int const wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * 256 + threadIdx.x) >> 6));
+    int const unitsL = (dl.cnt + kQ - 1) / kQ * dl.nCh;
+    int const units = unitsL + (dr.cnt + kQ - 1) / kQ * dr.nCh;
+    for (int w = wave; w < units; w += gridDim.x * 4) {
+        bool const left = w < unitsL;
+        RecheckDir const& d = left ? dl : dr;
+        int const wl = left ? w : w - unitsL;
+        int const g = wl / d.nCh, c = wl - g * d.nCh;
+        float const* q[kQ];
+        int row[kQ];
+        Top2 s[kQ];
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+            int const e = min(g * kQ + j, d.cnt - 1);  // past the end: the last query again, not published
+            row[j] = __builtin_amdgcn_readfirstlane(flagList[d.base + e]);
+            q[j] = d.Q + (size_t)row[j] * kDim;
+            s[j] = top2_init();
+        }
+        exact_queries<kQ>(q, qd, lane);
+        int const c1 = min((c + 1) * d.subs * 64, d.nC);
+        for (int c0 = c * d.subs * 64; c0 < c1; c0 += 64) {
+            int const ci = c0 + lane;
+            float v[kQ];
+            exact_scores<kQ>(qd, d.C + (size_t)c0 * kDim, d.nC - c0, stage, lane, v);
+#pragma unroll
+            for (int j = 0; j < kQ; ++j) {
+                if (gbits) {
+                    // guided matching: a removed (left, right) pair scores -1e20
+                    int const li = left ? row[j] : min(ci, d.nC - 1), rj = left ? min(ci, d.nC - 1) : row[j];
+                    v[j] = ((gbits[(size_t)(rj >> 5) * ldi + li] >> (rj & 31)) & 1u) ? -1e20f : v[j];
+                }
+                if (ci < c1) top2_push(s[j], v[j], ci);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kQ; ++j) {
+            int const e = g * kQ + j;
+            if (e >= d.cnt) break;  // uniform
+            for (int o = 32; o > 0; o >>= 1) s[j] = top2_merge(s[j], top2_shfl_xor(s[j], o));
+            Top2* const p = part + (size_t)d.base * kRecheckMaxChunks + (size_t)e * d.nCh;
+            if (publish_partial(s[j], p, c, d.nCh, tickets + d.base + e, lane)) {
+                Top2 const t = merge_partials(p, d.nCh, lane);
+                if (lane == 0) d.sel[row[j]] = decide_exact(t, minScore, minRatio);
+            }
+        }
     }
 }
 
-RecheckPlan plan_recheck(int nC)
+__global__ __launch_bounds__(256) void k_recheck(float const* __restrict__ L, float const* __restrict__ R, int nL,
+                                                 int nR, int const* __restrict__ flagList, int rowsL, int rowsR,
+                                                 int const* __restrict__ counters, Top2* __restrict__ part,
+                                                 int* __restrict__ tickets, unsigned const* __restrict__ gbits,
+                                                 int ldi, float minScore, float minRatio, int* __restrict__ colMax,
+                                                 int* __restrict__ rowMax)
 {
-    RecheckPlan p;
-    p.per = (nC + 256 * kRecheckMaxChunks - 1) / (256 * kRecheckMaxChunks);
-    if (p.per < 1) p.per = 1;
-    p.nChunks = (nC + 256 * p.per - 1) / (256 * p.per);
-    if (p.nChunks < 1) p.nChunks = 1;
-    return p;
+    __shared__ __attribute__((aligned(16))) float stage[4][kExactLds];
+    __shared__ __attribute__((aligned(16))) double qd[4][kRecheckGroup * kDim];
+    int const cntL = __builtin_amdgcn_readfirstlane(counters[kCntFlag]);
+    int const cntR = __builtin_amdgcn_readfirstlane(counters[kCntFlagR]);
+    RecheckDir const dl = recheck_dir(true, L, R, nL, nR, cntL, rowsL, rowsR, colMax, rowMax);
+    RecheckDir const dr = recheck_dir(false, L, R, nL, nR, cntR, rowsL, rowsR, colMax, rowMax);
+    int const wv = threadIdx.x >> 6;
+    // a query per wave while the grid holds a wave for every unit
+    if ((long long)cntL * dl.nCh + (long long)cntR * dr.nCh <= 4LL * gridDim.x)
+        recheck_units<1>(dl, dr, flagList, part, tickets, gbits, ldi, minScore, minRatio, stage[wv], qd[wv]);
+    else
+        recheck_units<kRecheckGroup>(dl, dr, flagList, part, tickets, gbits, ldi, minScore, minRatio, stage[wv],
+                                     qd[wv]);
 }
 
-void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int const* flagList, int flagOffR,
-                          int const* counters, float minScore, float minRatio, int* colMax, int* rowMax,
-                          Top2* part, int grid, hipStream_t st, unsigned const* gbits, int ldi)
+void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int const* flagList, int rowsL, int rowsR,
+                          int const* counters, float minScore, float minRatio, int* colMax, int* rowMax, Top2* part,
+                          int* tickets, int grid, hipStream_t st, unsigned const* gbits, int ldi)
 {
     if (nL <= 0 || nR <= 0) return;
-    RecheckPlan const pl = plan_recheck(nR);  // left queries scan the right features
-    RecheckPlan const pr = plan_recheck(nL);
-    hipLaunchKernelGGL(k_recheck_chunks, dim3(grid), dim3(256), 0, st, L, R, nL, nR, flagList, flagOffR, counters,
-                       pl.nChunks, pl.per, pr.nChunks, pr.per, part, gbits, ldi);
-    hipLaunchKernelGGL(k_recheck_finish, dim3(256), dim3(256), 0, st, flagList, flagOffR, counters, pl.nChunks,
-                       pr.nChunks, part, minScore, minRatio, colMax, rowMax);
+    hipLaunchKernelGGL(k_recheck, dim3(grid), dim3(256), 0, st, L, R, nL, nR, flagList, rowsL, rowsR, counters, part,
+                       tickets, gbits, ldi, minScore, minRatio, colMax, rowMax);
 }
 
 // ------------------------------------------------------------------------------ mutual + compaction

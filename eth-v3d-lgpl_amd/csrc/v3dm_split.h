@@ -21,6 +21,13 @@ namespace v3dm {
 // ||q|| ||c|| + 2^-39 sqrt(128) (||q|| + ||c||), and with norms of at least 2^-10 the last
 // term is below 2^-24 ||q|| max||c||: within the 2^-15 that the certified decisions assume.
 // Measured on unit descriptors it is below the FP32 instruction's (v3dm_split.hip).
+//
+// The certified decisions take epsRel (2^-15 unless the caller sets it), the FP32 instruction's
+// bound with a factor 2, times kSplitEps for split rows (2^-17: a factor 2 on the bound above)
+// and kIntEps for integer rows (2^-21: |score - exact| <= 5.01 * 2^-24 score), so that fewer
+// queries are left open (16384 x 16384: 16 of 32768 at 2^-15).
+constexpr float kSplitEps = 0.25f;
+constexpr float kIntEps = 0.015625f;
 constexpr float kSplitScale = 16384.0f;
 constexpr float kSplitBack = 3.7252902984619140625e-09f;  // 2^-28
 constexpr float kSplitNormMin = 0.0009765625f;            // 2^-10

@@ -107,8 +107,10 @@ int v3dm_run_guided_H(v3dm_handle h, const double H[9], float distanceThreshold,
 int v3dm_set_precision(v3dm_handle h, int mode);
 /* Error-bound scale of the certified FP32 decisions: a query is settled from the MFMA
  * scores only when every exact score set within epsRel * ||q|| * max||c|| gives the same
- * decision; otherwise it is re-checked exactly in FP64.  Default 2^-15; 0 re-checks every
- * query (the whole selection then runs on exact FP64 scores). */
+ * decision; otherwise it is re-checked exactly in FP64.  Scores from two FP16 parts take a
+ * quarter of it, scores from uint8 components a 64th (their error bounds are that much
+ * smaller).  Default 2^-15; 0 re-checks every query (the whole selection then runs on exact
+ * FP64 scores). */
 int v3dm_set_certification(v3dm_handle h, float epsRel);
 /* Candidates per query scored exactly in the learned mode (the best k by code score;
  * default 6, at most 32). */
