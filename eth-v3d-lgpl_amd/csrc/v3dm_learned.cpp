@@ -35,6 +35,8 @@ struct LearnedState {
     __bf16 *X = nullptr, *XT = nullptr, *HT = nullptr, *dZ = nullptr, *dZT = nullptr, *dHT = nullptr;
     float *Z = nullptr, *dC = nullptr, *dZf = nullptr, *part = nullptr, *lossPart = nullptr;
     int* hard = nullptr;
+    float* hardVal = nullptr;  // hardest positives per chunk of the search
+    int* hardIdx = nullptr;
 };
 
 namespace {
@@ -75,6 +77,8 @@ int ensure_workspace(v3dm_context* h, LearnedState* L, int Rp)
     for (__bf16** p : {&L->X, &L->XT, &L->HT, &L->dZ, &L->dZT, &L->dHT}) freeDev(*p);
     for (float** p : {&L->Z, &L->dC, &L->dZf, &L->part, &L->lossPart}) freeDev(*p);
     freeDev(L->hard);
+    freeDev(L->hardVal);
+    freeDev(L->hardIdx);
     size_t const r = (size_t)Rp;
     LCHECK(h, hipMalloc(&L->X, r * 128 * sizeof(__bf16)));
     LCHECK(h, hipMalloc(&L->XT, r * 128 * sizeof(__bf16)));
@@ -88,6 +92,8 @@ int ensure_workspace(v3dm_context* h, LearnedState* L, int Rp)
     LCHECK(h, hipMalloc(&L->part, (size_t)mlp_wgrad_chunks(Rp) * kParams * sizeof(float)));
     LCHECK(h, hipMalloc(&L->lossPart, (r / 64 + 1) * sizeof(float)));
     LCHECK(h, hipMalloc(&L->hard, r * sizeof(int)));
+    LCHECK(h, hipMalloc(&L->hardVal, mlp_hard_slots(Rp) * sizeof(float)));
+    LCHECK(h, hipMalloc(&L->hardIdx, mlp_hard_slots(Rp) * sizeof(int)));
     L->capRp = Rp;
     return V3DM_OK;
 }
@@ -105,7 +111,7 @@ int enqueue_step(v3dm_context* h, LearnedState* L, int orderOff, int B, float lr
     launch_mlp_gather(L->pool, L->tri, L->order, orderOff, B, Rp, L->X, L->XT, st);
     launch_mlp_forward(L->X, Rp, L->w, L->HT, L->Z, st);
     launch_fill(L->dC, (size_t)Rp * kCode, 0.0f, st);
-    launch_mlp_loss(L->Z, B, tau, L->dC, L->hard, L->lossPart, st);
+    launch_mlp_loss(L->Z, B, tau, L->hardVal, L->hardIdx, L->dC, L->hard, L->lossPart, st);
     launch_mlp_norm_backward(L->Z, L->dC, R, Rp, L->dZf, L->dZ, L->dZT, st);
     launch_mlp_backward_h(L->dZ, Rp, L->w, L->HT, L->dHT, st);
     launch_mlp_wgrad(L->XT, L->HT, L->dZT, L->dHT, L->dZf, Rp, L->part, st);
@@ -138,6 +144,8 @@ void learned_destroy(LearnedState*& L)
     freeDev(L->tri);
     freeDev(L->order);
     freeDev(L->hard);
+    freeDev(L->hardVal);
+    freeDev(L->hardIdx);
     delete L;
     L = nullptr;
 }

@@ -38,7 +38,11 @@ void launch_mlp_codes_u8(uint8_t const* Q, float const* denom, int rows128, MlpW
 // two feature sets in one launch (row counts multiples of 128; either may be 0)
 void launch_mlp_codes2_f32(float const* X0, int rows0, signed char* codes0, float const* X1, int rows1,
                            signed char* codes1, MlpWeights const& w, float scale, hipStream_t st);
-void launch_mlp_loss(float const* Z, int B, float tau, float* dC, int* hard, float* lossPart, hipStream_t st);
+// hardVal, hardIdx: room for mlp_hard_slots(B) entries (the hardest positives per chunk)
+constexpr int kMlpHardGroups = 512;  // work-groups of the hardest-positive search
+inline size_t mlp_hard_slots(int B) { return (size_t)B + 128 * kMlpHardGroups; }
+void launch_mlp_loss(float const* Z, int B, float tau, float* hardVal, int* hardIdx, float* dC, int* hard,
+                     float* lossPart, hipStream_t st);
 void launch_mlp_norm_backward(float const* Z, float const* dC, int R, int Rp, float* dZf, __bf16* dZ, __bf16* dZT,
                               hipStream_t st);
 void launch_mlp_backward_h(__bf16 const* dZ, int Rp, MlpWeights const& w, __bf16 const* HT, __bf16* dHT,

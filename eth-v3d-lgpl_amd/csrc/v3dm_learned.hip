@@ -19,6 +19,8 @@
 #include "v3dm_device.h"
 #include "v3dm_learned.h"
 
+#include <algorithm>
+
 namespace v3dm {
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
@@ -39,26 +41,42 @@ __device__ __forceinline__ void store4_bf16(__bf16* p, float a, float b, float c
 }
 
 // ------------------------------------------------------------------------------ gather
-// One wave per row: row r of the minibatch is pool row tri[3*(r % B) + r / B] (anchors,
-// then positives, then negatives); rows >= R are zero.
+// Row r of the minibatch is pool row tri[3*(r % B) + r / B] (anchors, then positives, then
+// negatives); rows >= 3 B are zero.  Work-group: 64 rows, a wave per row 16 times, transposed
+// through LDS so that XT is written in runs of 64 rows (one 2-byte store per element and row
+// otherwise: 15 us for 12288 rows).
+constexpr int kGatherRow = kDim + 2;  // bf16 per staged row
+
 __global__ __launch_bounds__(256) void k_mlp_gather(float const* __restrict__ pool, int const* __restrict__ tri,
                                                     int const* __restrict__ order, int orderOff, int B, int Rp,
                                                     __bf16* __restrict__ X, __bf16* __restrict__ XT)
 {
+    __shared__ __bf16 rows[64 * kGatherRow];
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
     int const lane = threadIdx.x & 63;
-    int const r = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= Rp) return;
-    float2 v = make_float2(0.0f, 0.0f);
-    if (r < 3 * B) {
-        int const t = order[orderOff + r % B];
-        int const row = tri[3 * t + r / B];
-        v = reinterpret_cast<float2 const*>(pool + (size_t)row * kDim)[lane];
+    int const wave = threadIdx.x >> 6;
+    int const r0 = blockIdx.x * 64;  // Rp is a multiple of kRowPadMlp
+    int row[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        int const r = r0 + wave * 16 + k;
+        row[k] = r < 3 * B ? tri[3 * order[orderOff + r % B] + r / B] : -1;
     }
-    __bf16 const a = (__bf16)v.x, b = (__bf16)v.y;
-    X[(size_t)r * kDim + 2 * lane] = a;
-    X[(size_t)r * kDim + 2 * lane + 1] = b;
-    XT[(size_t)(2 * lane) * Rp + r] = a;
-    XT[(size_t)(2 * lane + 1) * Rp + r] = b;
+    float2 v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+        v[k] = row[k] >= 0 ? reinterpret_cast<float2 const*>(pool + (size_t)row[k] * kDim)[lane]
+                           : make_float2(0.0f, 0.0f);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        v2bf const p = {(__bf16)v[k].x, (__bf16)v[k].y};
+        int const rl = wave * 16 + k;
+        reinterpret_cast<v2bf*>(X + (size_t)(r0 + rl) * kDim)[lane] = p;
+        *reinterpret_cast<v2bf*>(rows + rl * kGatherRow + 2 * lane) = p;
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int d = wave; d < kDim; d += 4) XT[(size_t)d * Rp + r0 + lane] = rows[lane * kGatherRow + d];
 }
 
 // FP32 rows -> bf16 rows (inference input), rows >= n zero.
@@ -160,52 +178,59 @@ __global__ __launch_bounds__(256) void k_mlp_forward(TIn const* __restrict__ X, 
 }
 
 // ------------------------------------------------------------------------------ loss
-// 64 anchors per work-group, 4 threads per anchor (quarter q of each 64-row positive tile).
-// Codes are normalised on the fly.  The in-batch hardest positive of anchor t is the
-// argmax over t' != t of c_t . c_{p_t'} (first index on ties).  Gradients with respect to
-// the normalised codes go to dC: anchor and negative rows are owned by their triplet,
-// positive rows also receive the hardest-negative terms of other anchors (atomic adds on a
-// zeroed dC).
+// Codes are normalised on the fly.  The in-batch hardest positive of anchor t is the argmax
+// over t' != t of c_t . c_{p_t'} (first index on ties): k_mlp_hardest searches chunks of the
+// positives, k_mlp_loss takes the best of the chunks (the dot products and the winner do not
+// depend on the chunks).  Gradients with respect to the normalised codes go to dC: anchor and
+// negative rows are owned by their triplet, positive rows also receive the hardest-negative
+// terms of other anchors (atomic adds on a zeroed dC).
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-__global__ __launch_bounds__(256) void k_mlp_loss(float const* __restrict__ Z, int B, float invTau,
-                                                  float* __restrict__ dC, int* __restrict__ hardOut,
-                                                  float* __restrict__ lossPart)
+// The normalised code of row r (8 components per thread of the row's four, gathered to all 32
+// by shuffles); rows >= R read as row 0.
+__device__ __forceinline__ void mlp_unit_code(float const* __restrict__ Z, int r, int R, int q, int lane,
+                                              float (&c)[kCode])
 {
-    __shared__ float tile[64][kCode + 1];
-    __shared__ float wl[4];
+    int const rr = r < R ? r : 0;
+    float s = 0.0f;
+    float part[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        part[e] = Z[(size_t)rr * kCode + 8 * q + e];
+        s += part[e] * part[e];
+    }
+    s += __shfl_xor(s, 1);
+    s += __shfl_xor(s, 2);
+    float const inv = 1.0f / fmaxf(sqrtf(s), 1e-12f);
+#pragma unroll
+    for (int qq = 0; qq < 4; ++qq)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c[8 * qq + e] = __shfl(part[e], (lane & ~3) | qq) * inv;
+}
+
+// The best positive of each anchor among tiles [y * tiles, (y + 1) * tiles) of 64 positives ->
+// hardVal / hardIdx[y * B + t] (-1: none).  Work-group: 128 anchors, two per thread and four
+// threads per anchor (quarter q of each tile), so a row read from LDS (8 reads of 16 bytes,
+// broadcast to the threads of a quarter) serves 64 multiply-adds; the positives are split until
+// about 512 work-groups run.  One work-group per 64 anchors over all positives, a 4-byte LDS
+// read per multiply-add: 345 us for 4096 triplets in 64 work-groups.
+constexpr int kHardRow = kCode + 4;  // floats per staged row (16-byte reads, distinct banks)
+
+__global__ __launch_bounds__(256) void k_mlp_hardest(float const* __restrict__ Z, int B, int tiles,
+                                                     float* __restrict__ hardVal, int* __restrict__ hardIdx)
+{
+    __shared__ __attribute__((aligned(16))) float tile[64 * kHardRow];
     int const tid = threadIdx.x;
     int const q = tid & 3;
-    int const al = tid >> 2;
-    int const t = blockIdx.x * 64 + al;
-    bool const valid = t < B;
-
-    // normalised anchor code (8 components per thread, gathered to all 32 by shuffles)
-    float ca[kCode];
-    {
-        int const tt = valid ? t : 0;
-        float s = 0.0f;
-        float part[8];
+    int const t0 = blockIdx.x * 128 + (tid >> 2);
+    float ca[2][kCode];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            part[e] = Z[(size_t)tt * kCode + 8 * q + e];
-            s += part[e] * part[e];
-        }
-        s += __shfl_xor(s, 1);
-        s += __shfl_xor(s, 2);
-        float const inv = 1.0f / fmaxf(sqrtf(s), 1e-12f);
-#pragma unroll
-        for (int qq = 0; qq < 4; ++qq)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float const v = __shfl(part[e], ((tid & 63) & ~3) | qq) * inv;
-                ca[8 * qq + e] = v;
-            }
-    }
-    float best = -INFINITY;
-    int bestIdx = -1;
-    for (int p0 = 0; p0 < B; p0 += 64) {
+    for (int a = 0; a < 2; ++a) mlp_unit_code(Z, t0 + 64 * a, B, q, tid & 63, ca[a]);
+    float best[2] = {-INFINITY, -INFINITY};
+    int idx[2] = {-1, -1};
+    int const p1 = min((int)(blockIdx.y + 1) * tiles * 64, B);
+    for (int p0 = blockIdx.y * tiles * 64; p0 < p1; p0 += 64) {
         __syncthreads();
         {
             // stage positives p0 .. p0+63, normalised (4 threads per row, 8 components each)
@@ -222,19 +247,74 @@ __global__ __launch_bounds__(256) void k_mlp_loss(float const* __restrict__ Z, i
             s += __shfl_xor(s, 2);
             float const inv = 1.0f / fmaxf(sqrtf(s), 1e-12f);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) tile[pr][8 * q + e] = part[e] * inv;
+            for (int e = 0; e < 8; ++e) tile[pr * kHardRow + 8 * q + e] = part[e] * inv;
         }
         __syncthreads();
         for (int j = q; j < 64; j += 4) {
             int const pj = p0 + j;
-            if (pj >= B || pj == t) continue;
-            float d = 0.0f;
+            float d[2] = {0.0f, 0.0f};
 #pragma unroll
-            for (int e = 0; e < kCode; ++e) d += ca[e] * tile[j][e];
-            if (d > best) {
-                best = d;
-                bestIdx = pj;
+            for (int e = 0; e < kCode; e += 4) {
+                float4 const x = *reinterpret_cast<float4 const*>(tile + j * kHardRow + e);
+#pragma unroll
+                for (int a = 0; a < 2; ++a) {
+                    d[a] += ca[a][e + 0] * x.x;
+                    d[a] += ca[a][e + 1] * x.y;
+                    d[a] += ca[a][e + 2] * x.z;
+                    d[a] += ca[a][e + 3] * x.w;
+                }
             }
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+                if (pj < B && pj != t0 + 64 * a && d[a] > best[a]) {
+                    best[a] = d[a];
+                    idx[a] = pj;
+                }
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        // combine the 4 quarters (first index on ties)
+#pragma unroll
+        for (int o = 1; o < 4; o <<= 1) {
+            float const ob = __shfl_xor(best[a], o);
+            int const oi = __shfl_xor(idx[a], o);
+            bool const take = ob > best[a] || (ob == best[a] && oi >= 0 && (idx[a] < 0 || oi < idx[a]));
+            best[a] = take ? ob : best[a];
+            idx[a] = take ? oi : idx[a];
+        }
+        int const t = t0 + 64 * a;
+        if (q == 0 && t < B) {
+            hardVal[(size_t)blockIdx.y * B + t] = best[a];
+            hardIdx[(size_t)blockIdx.y * B + t] = idx[a];
+        }
+    }
+}
+
+// 64 anchors per work-group, 4 threads per anchor: the chunks' best positive, loss and code
+// gradients.
+__global__ __launch_bounds__(256) void k_mlp_loss(float const* __restrict__ Z, int B, float invTau,
+                                                  float const* __restrict__ hardVal, int const* __restrict__ hardIdx,
+                                                  int chunks, float* __restrict__ dC, int* __restrict__ hardOut,
+                                                  float* __restrict__ lossPart)
+{
+    __shared__ float wl[4];
+    int const tid = threadIdx.x;
+    int const q = tid & 3;
+    int const al = tid >> 2;
+    int const t = blockIdx.x * 64 + al;
+    bool const valid = t < B;
+
+    float ca[kCode];
+    mlp_unit_code(Z, t, B, q, tid & 63, ca);
+    float best = -INFINITY;
+    int bestIdx = -1;
+    for (int c = q; c < chunks && valid; c += 4) {
+        float const ob = hardVal[(size_t)c * B + t];
+        int const oi = hardIdx[(size_t)c * B + t];
+        if (oi >= 0 && (ob > best || bestIdx < 0)) {  // ascending chunks: the first index on ties
+            best = ob;
+            bestIdx = oi;
         }
     }
     // combine the 4 quarters (first index on ties)
@@ -309,12 +389,12 @@ __global__ __launch_bounds__(256) void k_mlp_loss(float const* __restrict__ Z, i
 }
 
 // Code gradient through the normalisation: dz = (dc - c (c . dc)) / |z|.  One thread per
-// row; rows >= R get zeros.
-__global__ __launch_bounds__(256) void k_mlp_norm_backward(float const* __restrict__ Z, float const* __restrict__ dC,
+// row (a wave per work-group: a minibatch is a few hundred waves); rows >= R get zeros.
+__global__ __launch_bounds__(64) void k_mlp_norm_backward(float const* __restrict__ Z, float const* __restrict__ dC,
                                                            int R, int Rp, float* __restrict__ dZf,
                                                            __bf16* __restrict__ dZ, __bf16* __restrict__ dZT)
 {
-    int const r = blockIdx.x * 256 + threadIdx.x;
+    int const r = blockIdx.x * 64 + threadIdx.x;
     if (r >= Rp) return;
     float z[kCode], d[kCode];
     float s2 = 0.0f, cd = 0.0f;
@@ -386,10 +466,11 @@ __global__ __launch_bounds__(256) void k_mlp_backward_h(__bf16 const* __restrict
     }
 }
 
-// Weight gradients over a chunk of kWgChunk rows: grid (chunks, 5); y < 4: dW1 blocks (unit
+// Weight gradients over a chunk of kWgChunk rows: grid (chunks, 6); y < 4: dW1 blocks (unit
 // block 2y + w/2 ... ) -- each wave computes 2 of the 32 dW1 blocks of its y, y == 4: the 8
-// dW2 blocks (2 per wave).  Bias gradients: y == 4 also sums dZf (db2) and dHT (db1) over
-// the chunk.  Partials -> part[chunk][param].
+// dW2 blocks (2 per wave), y == 5: the bias gradients, sums of dZf (db2) and dHT (db1) over
+// the chunk.  Partials -> part[chunk][param].  Bound by load latency (a chunk is 32 dependent
+// steps): eight steps' loads in flight, and the bias sums in work-groups of their own
 constexpr int kWgChunk = 512;
 
 __global__ __launch_bounds__(256) void k_mlp_wgrad(__bf16 const* __restrict__ XT, __bf16 const* __restrict__ HT,
@@ -414,6 +495,7 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(__bf16 const* __restrict__ XT
             ub[s] = b >> 2;
             db[s] = b & 3;
         }
+#pragma unroll 8
         for (int ks = 0; ks < kWgChunk / 16; ++ks) {
             int const i = i0 + ks * 16 + 8 * h;
 #pragma unroll
@@ -431,8 +513,9 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(__bf16 const* __restrict__ XT
                 int const d = db[s] * 32 + c32;
                 out[kOffW1 + u * kDim + d] = acc[s][r];
             }
-    } else {
+    } else if (y == 4) {
         // dW2 blocks: unit block ub = 2*wave + s; D[code][unit]
+#pragma unroll 8
         for (int ks = 0; ks < kWgChunk / 16; ++ks) {
             int const i = i0 + ks * 16 + 8 * h;
             v8bf const a = load8(dZT + (size_t)c32 * Rp + i);
@@ -450,13 +533,21 @@ __global__ __launch_bounds__(256) void k_mlp_wgrad(__bf16 const* __restrict__ XT
                 int const u = (2 * wave + s) * 32 + c32;
                 out[kOffW2 + c * kHid + u] = acc[s][r];
             }
-        // bias gradients of the chunk: thread t < 256 -> db1[t], t < 32 also db2[t]
+    } else {
+        // bias gradients of the chunk: thread t < 256 -> db1[t], t < 32 also db2[t], in
+        // ascending rows (loads of 8 rows and 16 rows ahead of the sums)
         int const t = threadIdx.x;
         float s1 = 0.0f;
-        for (int i = 0; i < kWgChunk; ++i) s1 += (float)dHT[(size_t)t * Rp + i0 + i];
+#pragma unroll 8
+        for (int i = 0; i < kWgChunk; i += 8) {
+            v8bf const v = load8(dHT + (size_t)t * Rp + i0 + i);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s1 += (float)v[e];
+        }
         out[kOffB1 + t] = s1;
         if (t < kCode) {
             float s2 = 0.0f;
+#pragma unroll 16
             for (int i = 0; i < kWgChunk; ++i) s2 += dZf[(size_t)(i0 + i) * kCode + t];
             out[kOffB2 + t] = s2;
         }
@@ -951,7 +1042,7 @@ __global__ void k_fill_f32(float* __restrict__ p, size_t n, float v)
 void launch_mlp_gather(float const* pool, int const* tri, int const* order, int orderOff, int B, int Rp,
                        __bf16* X, __bf16* XT, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_mlp_gather, dim3((Rp + 3) / 4), dim3(256), 0, st, pool, tri, order, orderOff, B, Rp, X, XT);
+    hipLaunchKernelGGL(k_mlp_gather, dim3(Rp / 64), dim3(256), 0, st, pool, tri, order, orderOff, B, Rp, X, XT);
 }
 
 void launch_mlp_rows_bf16(float const* src, int n, int Rp, __bf16* X, hipStream_t st)
@@ -967,15 +1058,22 @@ void launch_mlp_forward(__bf16 const* X, int Rp, MlpWeights const& w, __bf16* HT
 
 
 
-void launch_mlp_loss(float const* Z, int B, float tau, float* dC, int* hard, float* lossPart, hipStream_t st)
+void launch_mlp_loss(float const* Z, int B, float tau, float* hardVal, int* hardIdx, float* dC, int* hard,
+                     float* lossPart, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_mlp_loss, dim3((B + 63) / 64), dim3(256), 0, st, Z, B, 1.0f / tau, dC, hard, lossPart);
+    int const blocks = (B + 127) / 128, nTiles = (B + 63) / 64;
+    int const want = std::min((kMlpHardGroups + blocks - 1) / blocks, nTiles);
+    int const tiles = (nTiles + want - 1) / want;
+    int const chunks = (nTiles + tiles - 1) / tiles;
+    hipLaunchKernelGGL(k_mlp_hardest, dim3(blocks, chunks), dim3(256), 0, st, Z, B, tiles, hardVal, hardIdx);
+    hipLaunchKernelGGL(k_mlp_loss, dim3((B + 63) / 64), dim3(256), 0, st, Z, B, 1.0f / tau, hardVal, hardIdx, chunks,
+                       dC, hard, lossPart);
 }
 
 void launch_mlp_norm_backward(float const* Z, float const* dC, int R, int Rp, float* dZf, __bf16* dZ, __bf16* dZT,
                               hipStream_t st)
 {
-    hipLaunchKernelGGL(k_mlp_norm_backward, dim3((Rp + 255) / 256), dim3(256), 0, st, Z, dC, R, Rp, dZf, dZ, dZT);
+    hipLaunchKernelGGL(k_mlp_norm_backward, dim3((Rp + 63) / 64), dim3(64), 0, st, Z, dC, R, Rp, dZf, dZ, dZT);
 }
 
 void launch_mlp_backward_h(__bf16 const* dZ, int Rp, MlpWeights const& w, __bf16 const* HT, __bf16* dHT,
@@ -989,7 +1087,7 @@ int mlp_wgrad_chunks(int Rp) { return (Rp + kWgChunk - 1) / kWgChunk; }
 void launch_mlp_wgrad(__bf16 const* XT, __bf16 const* HT, __bf16 const* dZT, __bf16 const* dHT, float const* dZf,
                       int Rp, float* part, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_mlp_wgrad, dim3(Rp / kWgChunk, 5), dim3(256), 0, st, XT, HT, dZT, dHT, dZf, Rp, part);
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(Rp / kWgChunk, 6), dim3(256), 0, st, XT, HT, dZT, dHT, dZf, Rp, part);
 }
 
 void launch_mlp_adam(float const* part, int nChunks, float* grad, MlpWeights const& w, float* M, float* V, float lr,
