@@ -274,49 +274,70 @@ void launch_vt_score(float const* keys, float const* keyNorm, int n, float const
 // against its running best (start: the -1e30 floor); the lanes' bests combine to the
 // first child of maximal score.  No valid child gives -1, so the key moves to node
 // c0 - 1, as the reference's leafId = nextLeafId + bestNode does.
+//
+// The 64 children of a step are loaded whole lines at a time and pass through the wave's own
+// LDS a quarter of their dims at a time (exact_chunk, v3dm_device.h); the key is read from LDS
+// by broadcast.  With every lane loading its own child's row, each line was fetched eight
+// times: 180-205 us a level for 10^6 keys of a <50,3> tree, 70-76 us a level so.
 __global__ __launch_bounds__(256) void k_vt_exact(float const* __restrict__ keys, float const* __restrict__ nodes,
                                                   long long nNodes, int branch, int level,
                                                   int const* __restrict__ exactList, int* __restrict__ node,
                                                   int* __restrict__ counters)
 {
-    __shared__ float keyRow[4][kDim];
+    __shared__ __attribute__((aligned(16))) float keyRows[4][kDim];
+    __shared__ __attribute__((aligned(16))) float stages[4][kExactLds];
     int const lane = threadIdx.x & 63;
+    int const wave = threadIdx.x >> 6;
     int const cnt = counters[kVtCntExact];
-    for (int e = blockIdx.x * 4 + (threadIdx.x >> 6); e < cnt; e += gridDim.x * 4) {
+    float* const kw = keyRows[wave];
+    float* const stage = stages[wave];
+    float const* const mine = stage + lane * kExactRow;
+    int done = 0;
+    for (int e = blockIdx.x * 4 + wave; e < cnt; e += gridDim.x * 4) {
         int const kk = exactList[e];
+        done += 1;
         long long const c0 = (level == 0) ? 0 : ((long long)node[kk] + 1) * branch;
         if (c0 < 0 || c0 + branch > nNodes) {
             if (lane == 0) node[kk] = kVtNone;
+            done -= 1;
             continue;
         }
-        // the key in LDS (one row per wave), each child row in registers 32 floats at a
-        // time: the loads are issued together instead of one per step of the sum
-        float* kw = keyRow[threadIdx.x >> 6];
-        __builtin_amdgcn_wave_barrier();  // the previous key's reads are done
+        // LDS operations of one wave are in order: the fences only keep the compiler's order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         reinterpret_cast<float2*>(kw)[lane] = reinterpret_cast<float2 const*>(keys + (size_t)kk * kDim)[lane];
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         float bestS = -INFINITY;
         int bestJ = -1;
-        for (int j = lane; j < branch; j += 64) {
-            float4 const* c = reinterpret_cast<float4 const*>(nodes + (size_t)(c0 + j) * kDim);
+        for (int j0 = 0; j0 < branch; j0 += 64) {
+            float const* const c = nodes + (size_t)(c0 + j0) * kDim;
+            int const nRows = branch - j0;  // of which this step takes 64; the rest repeat the last
             float score = 0.0f;
-            for (int q0 = 0; q0 < 32; q0 += 8) {
-                float4 v[8];
+            v4f v[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = c[q0 + u];
+            for (int u = 0; u < 8; ++u) v[u] = exact_chunk(c, min(8 * u + (lane >> 3), nRows - 1), lane & 7);
+#pragma unroll 1
+            for (int p = 0; p < 4; ++p) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    float const* kq = kw + 4 * (q0 + u);
-                    score = add_nc(score, mul_nc(kq[0], v[u].x));
-                    score = add_nc(score, mul_nc(kq[1], v[u].y));
-                    score = add_nc(score, mul_nc(kq[2], v[u].z));
-                    score = add_nc(score, mul_nc(kq[3], v[u].w));
+                for (int u = 0; u < 8; ++u)
+                    *reinterpret_cast<v4f*>(stage + (8 * u + (lane >> 3)) * kExactRow + 4 * (lane & 7)) = v[u];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                int const next = min(p + 1, 3);  // (the last quarter once more, unused)
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    v[u] = exact_chunk(c, min(8 * u + (lane >> 3), nRows - 1), 8 * next + (lane & 7));
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    float4 const x = *reinterpret_cast<float4 const*>(mine + 4 * k);
+                    float4 const y = *reinterpret_cast<float4 const*>(kw + 32 * p + 4 * k);
+                    score = add_nc(score, mul_nc(y.x, x.x));
+                    score = add_nc(score, mul_nc(y.y, x.y));
+                    score = add_nc(score, mul_nc(y.z, x.z));
+                    score = add_nc(score, mul_nc(y.w, x.w));
                 }
             }
-            if (score > -1e30f && score > bestS) {
+            if (lane < nRows && score > -1e30f && score > bestS) {
                 bestS = score;
-                bestJ = j;
+                bestJ = j0 + lane;
             }
         }
         for (int o = 32; o > 0; o >>= 1) {
@@ -326,17 +347,16 @@ __global__ __launch_bounds__(256) void k_vt_exact(float const* __restrict__ keys
             bestS = take ? os : bestS;
             bestJ = take ? oj : bestJ;
         }
-        if (lane == 0) {
-            node[kk] = (int)(c0 + bestJ);
-            atomicAdd(&counters[kVtCntFlagged], 1);
-        }
+        if (lane == 0) node[kk] = (int)(c0 + bestJ);
     }
+    // one atomic a wave (they share an address)
+    if (lane == 0 && done > 0) atomicAdd(&counters[kVtCntFlagged], done);
 }
 
 void launch_vt_exact(float const* keys, float const* nodes, VtLevel const& lv, int const* exactList, int* node,
                      int* counters, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_vt_exact, dim3(512), dim3(256), 0, st, keys, nodes, lv.nNodes, lv.branch, lv.level,
+    hipLaunchKernelGGL(k_vt_exact, dim3(1024), dim3(256), 0, st, keys, nodes, lv.nNodes, lv.branch, lv.level,
                        exactList, node, counters);
 }
 
