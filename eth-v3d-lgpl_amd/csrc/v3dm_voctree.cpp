@@ -30,13 +30,15 @@ struct v3dm_voctree_s {
     std::vector<long long> levelStarts;  // depth + 1 entries
     long long maxParents = 1;            // nodes of the widest parent level (branch^(depth-1))
     float* dNodes = nullptr;             // (nNodes + 32) x 128, the last 32 rows zero
+    unsigned char* dSplit = nullptr;     // the same rows in two FP16 parts
     float maxNodeNorm = 0.0f;
+    int nodeExp = 0;                     // maxNodeNorm in [2^nodeExp, 2^(nodeExp + 1))
+    bool usable = false;                 // maxNodeNorm in [2^-60, 2^60]: certified scores
     bool haveNodes = false;
 
     int cap = 0;
     float* dKeys = nullptr;
     float* keyNorm = nullptr;
-    unsigned* maxBits = nullptr;
     int* node = nullptr;
     int* order = nullptr;
     int* exactList = nullptr;
@@ -70,7 +72,6 @@ void releaseKeys(v3dm_voctree_s* t)
 {
     vfree(t->dKeys);
     vfree(t->keyNorm);
-    vfree(t->maxBits);
     vfree(t->node);
     vfree(t->order);
     vfree(t->exactList);
@@ -87,7 +88,6 @@ int ensureCapacity(v3dm_voctree_s* t, int n)
     int const c = std::max(n, 1024);
     VTCHECK(hipMalloc(&t->dKeys, (size_t)c * kDim * sizeof(float)));
     VTCHECK(hipMalloc(&t->keyNorm, (size_t)c * sizeof(float)));
-    VTCHECK(hipMalloc(&t->maxBits, 4 * sizeof(unsigned)));
     VTCHECK(hipMalloc(&t->node, (size_t)c * sizeof(int)));
     VTCHECK(hipMalloc(&t->order, (size_t)orderCapacity(c, t->maxParents) * sizeof(int)));
     VTCHECK(hipMalloc(&t->exactList, (size_t)c * sizeof(int)));
@@ -102,8 +102,6 @@ int enqueueTraverse(v3dm_voctree_s* t, int n, float const* dKeys, int32_t* dLeav
     hipStream_t const st = t->stream;
     launch_vt_reset(t->counters, true, st);
     if (n <= 0) return V3DM_OK;
-    VTCHECK(hipMemsetAsync(t->maxBits, 0, sizeof(unsigned), st));
-    launch_norms(dKeys, n, t->keyNorm, t->maxBits, st);
     VtLevel lv;
     lv.branch = t->branch;
     lv.nNodes = t->nNodes;
@@ -112,16 +110,16 @@ int enqueueTraverse(v3dm_voctree_s* t, int n, float const* dKeys, int32_t* dLeav
         if (d == 0) {
             lv.parentStart = 0;
             lv.nParents = 1;
-            launch_vt_score(dKeys, t->keyNorm, n, t->dNodes, t->maxNodeNorm, lv, nullptr, true, (n + 31) / 32,
-                            t->node, t->exactList, t->counters, st);
+            launch_vt_score(dKeys, t->keyNorm, n, t->dSplit, t->maxNodeNorm, t->nodeExp, t->usable, lv, nullptr,
+                            true, (n + 31) / 32, t->node, t->exactList, t->counters, st);
         } else {
             launch_vt_reset(t->counters, false, st);
             lv.parentStart = t->levelStarts[d - 1];
             lv.nParents = (int)(t->levelStarts[d] - t->levelStarts[d - 1]);
             long long const oc = orderCapacity(n, lv.nParents) - 32;
             launch_vt_bucket(t->node, n, lv, t->cnt, t->cursor, t->order, (int)oc, t->exactList, t->counters, st);
-            launch_vt_score(dKeys, t->keyNorm, n, t->dNodes, t->maxNodeNorm, lv, t->order, false,
-                            (int)((oc + 31) / 32), t->node, t->exactList, t->counters, st);
+            launch_vt_score(dKeys, t->keyNorm, n, t->dSplit, t->maxNodeNorm, t->nodeExp, t->usable, lv, t->order,
+                            false, (int)((oc + 31) / 32), t->node, t->exactList, t->counters, st);
         }
         launch_vt_exact(dKeys, t->dNodes, lv, t->exactList, t->node, t->counters, st);
     }
@@ -179,6 +177,13 @@ int v3dm_voctree_create(v3dm_voctree* out, int device, int branchFactor, int dep
     if (e == hipSuccess) e = hipMalloc(&t->cnt, (size_t)t->maxParents * kVtBinStride * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&t->cursor, (size_t)t->maxParents * kVtBinStride * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&t->counters, kVtCounters * sizeof(int));
+    size_t const splitBytes = (size_t)((nodes + 63) / 32) * kVtTileBytes;  // 32 rows of padding here too
+    // a tree whose second copy does not fit still works: every key is decided exactly
+    if (e == hipSuccess && hipMalloc(&t->dSplit, splitBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        t->dSplit = nullptr;
+    }
+    if (t->dSplit) e = hipMemset(t->dSplit, 0, splitBytes);
     if (e != hipSuccess) {
         v3dm_voctree_destroy(t);
         return vfail(e == hipErrorOutOfMemory ? V3DM_ERR_NOMEM : V3DM_ERR_HIP,
@@ -195,6 +200,7 @@ void v3dm_voctree_destroy(v3dm_voctree t)
     if (t->stream) (void)hipStreamSynchronize(t->stream);
     releaseKeys(t);
     vfree(t->dNodes);
+    vfree(t->dSplit);
     vfree(t->cnt);
     vfree(t->cursor);
     vfree(t->counters);
@@ -222,6 +228,12 @@ int v3dm_voctree_set_nodes(v3dm_voctree t, const float* nodes)
     t->maxNodeNorm = finite ? (float)(std::sqrt(mx) * (1.0 + 1e-6)) : INFINITY;
     VTCHECK(hipMemcpyAsync(t->dNodes, nodes, (size_t)t->nNodes * kDim * sizeof(float), hipMemcpyHostToDevice,
                            t->stream));
+    t->usable = t->dSplit && finite && t->maxNodeNorm >= std::ldexp(1.0f, -60) && t->maxNodeNorm <= std::ldexp(1.0f, 60);
+    if (t->usable) {
+        t->nodeExp = std::ilogb(t->maxNodeNorm);
+        launch_vt_split_nodes(t->dNodes, t->nNodes, std::ldexp(1.0f, 14 - t->nodeExp), t->dSplit, t->stream);
+        VTCHECK(hipGetLastError());
+    }
     VTCHECK(hipStreamSynchronize(t->stream));
     t->haveNodes = true;
     return V3DM_OK;

@@ -19,6 +19,8 @@ constexpr int kVtNone = INT32_MIN;  // child range outside the node array
 constexpr int kVtBinStride = 32;    // ints between bucket counters (one 128-byte line each)
 constexpr int kVtLdsBins = 16384;   // parent levels up to this many nodes are counted in LDS
 
+constexpr int kVtTileBytes = 32 * 512;  // 32 node rows in two FP16 parts
+
 struct VtLevel {
     int branch;
     int level;              // 0 .. depth - 1
@@ -36,9 +38,13 @@ void launch_vt_bucket(int const* node, int n, VtLevel const& lv, int* cnt, int* 
                       int* exactList, int* counters, hipStream_t st);
 // certified MFMA scores of every key against the children of its parent; settled keys get
 // their child, the others go to the exact list
-void launch_vt_score(float const* keys, float const* keyNorm, int n, float const* nodes, float maxNodeNorm,
-                     VtLevel const& lv, int const* order, bool identity, int maxSlots, int* node,
-                     int* exactList, int* counters, hipStream_t st);
+// keyNorm: written at level 0 (identity), read below it; nodes: tiles of split rows scaled by
+// 2^(14 - nodeExp), maxNodeNorm in [2^nodeExp, 2^(nodeExp + 1)); usable = false: every key goes
+// to the exact list
+void launch_vt_score(float const* keys, float* keyNorm, int n, unsigned char const* nodes, float maxNodeNorm,
+                     int nodeExp, bool usable, VtLevel const& lv, int const* order, bool identity, int maxSlots,
+                     int* node, int* exactList, int* counters, hipStream_t st);
+void launch_vt_split_nodes(float const* nodes, long long rows, float scale, unsigned char* split, hipStream_t st);
 // exact decision (sequential FP32 sums, the reference's scan) of the listed keys
 void launch_vt_exact(float const* keys, float const* nodes, VtLevel const& lv, int const* exactList,
                      int* node, int* counters, hipStream_t st);

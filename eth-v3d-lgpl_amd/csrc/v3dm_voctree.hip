@@ -4,16 +4,19 @@
 //
 // Per level the keys are bucketed by their current node (a counting sort into buckets
 // padded to 32 keys), so that a wave takes 32 keys with the same parent and scores them
-// against the parent's children with v_mfma_f32_32x32x2_f32: the children are the A
-// operand (32 per block, read straight from L2), the keys the resident B operand (64
-// VGPRs per lane, as in the matcher's fused kernel).  The reference's choice is the first
-// child of maximal sequential-FP32 score; the MFMA score differs from that score by at most
-// eps = 2^-15 * ||key|| * max||node|| (a 128-term FP32 dot product in any order errs by
-// <= ~129 * 2^-24 * sum|k_i c_i| <= 2^-17 * ||k|| ||c|| against the exact value; two of
-// them differ by less than 2^-16 ||k|| ||c||), so a key whose best approximate score leads
-// the second by more than 2 eps has the reference's child.  The other keys (near ties,
-// non-finite values, scores near the -1e30 floor) are decided exactly: sequential FP32
-// sums with IEEE products, the scan's strict '>' (first index on ties, NaN never wins).
+// against the parent's children with v_mfma_f32_32x32x16_f16 on two FP16 parts of every
+// component, as the matcher's split pass does (v3dm_split.h): the children are the A operand
+// (32 per block, split once per tree, read straight from L2), the keys the resident B operand,
+// split as they are loaded.  Keys are scaled by the power of two that puts their norm in
+// [1, 2), nodes by the one that puts the largest node norm there.  The reference's choice is
+// the first child of maximal sequential-FP32 score, which differs from the exact product by
+// at most 128 * 2^-24 ||key|| ||node|| = 2^-17 ||key|| ||node||; the split score differs from it
+// by at most (3 * 2^-22 + 24 * 2^-23) ||key|| ||node|| + 2^-39 sqrt(128) * 2 ||key|| max||node||
+// < 2^-18 ||key|| max||node||; together less than eps = 2^-16 * ||key|| * max||node||, so a key
+// whose best approximate score leads the second by more than 2 eps has the reference's child.
+// The other keys (near ties, non-finite values, norms outside [2^-60, 2^60], scores near the
+// -1e30 floor) are decided exactly: sequential FP32 sums with IEEE products, the scan's strict
+// '>' (first index on ties, NaN never wins).
 #include <algorithm>
 
 #include "v3dm_device.h"
@@ -21,7 +24,48 @@
 
 namespace v3dm {
 
-constexpr float kVtEpsRel = 3.0517578125e-05f;  // 2^-15
+constexpr float kVtEpsRel = 1.52587890625e-05f;  // 2^-16
+constexpr float kVtNormMin = 8.673617379884035e-19f, kVtNormMax = 1.152921504606847e18f;  // 2^-60, 2^60
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+// x * scale = hi + lo (8 components)
+__device__ __forceinline__ void vt_split8(float4 a, float4 b, float scale, v8h& hi, v8h& lo)
+{
+    float const f[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        float const x = f[k] * scale;
+        hi[k] = (_Float16)x;
+        lo[k] = (_Float16)(x - (float)hi[k]);
+    }
+}
+
+// Node rows -> FP16 parts in the order in which the score kernel's lanes read them: tiles of 32
+// rows, in a tile [matrix step s][part][half h][row] of 8 components, the dims
+// 32 (s / 2) + 16 h + 8 (s % 2) + v.  One load of a wave is then one run of 1 KiB (two when the
+// children straddle tiles).
+__global__ __launch_bounds__(256) void k_vt_split_nodes(float const* __restrict__ nodes, long long rows, float scale,
+                                                        unsigned char* __restrict__ split)
+{
+    int const c = threadIdx.x >> 4;  // dims [8 c, 8 c + 8)
+    for (long long row = (long long)blockIdx.x * 16 + (threadIdx.x & 15); row < rows;
+         row += (long long)gridDim.x * 16) {
+        float4 const* x = reinterpret_cast<float4 const*>(nodes + (size_t)row * kDim) + 2 * c;
+        v8h hi, lo;
+        vt_split8(x[0], x[1], scale, hi, lo);
+        int const s = 2 * (c >> 2) + (c & 1), h = (c >> 1) & 1;
+        unsigned char* const o = split + (size_t)(row >> 5) * kVtTileBytes + s * 2048 + h * 512 + (row & 31) * 16;
+        *reinterpret_cast<v8h*>(o) = hi;
+        *reinterpret_cast<v8h*>(o + 1024) = lo;
+    }
+}
+
+void launch_vt_split_nodes(float const* nodes, long long rows, float scale, unsigned char* split, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_vt_split_nodes, dim3((unsigned)std::min((rows + 15) / 16, 65536LL)), dim3(256), 0, st, nodes, rows, scale,
+                       split);
+}
 
 __global__ void k_vt_reset(int* counters, int all)
 {
@@ -188,84 +232,133 @@ void launch_vt_bucket(int const* node, int n, VtLevel const& lv, int* cnt, int* 
 }
 
 // ------------------------------------------------------------------------------ certified scores
-// Wave = one slot of 32 keys with the same parent.  Lane l holds key l % 32, dims
-// [64 h, 64 h + 64) (h = l / 32) as the B operand; the A operand of MFMA step 4 s4 + q is
-// dim 64 h + 4 s4 + q of child row l % 32 of the block (same k map on both sides).
-// Accumulator element r of lane l: child 8 (r / 4) + 4 h + r % 4 of the block, key l % 32.
-__global__ __launch_bounds__(256) void k_vt_score(float const* __restrict__ keys, float const* __restrict__ keyNorm,
-                                                  int n, float const* __restrict__ nodes, float maxNodeNorm,
-                                                  int branch, int identity, int const* __restrict__ order,
-                                                  int* __restrict__ node, int* __restrict__ exactList,
-                                                  int* __restrict__ counters, float inf)
+// One block of 32 children as the A operand: a[2 s] the low, a[2 s + 1] the high parts.
+__device__ __forceinline__ void vt_load_block(v8h (&a)[16], unsigned char const* __restrict__ nodes, long long row,
+                                              int h)
 {
+    unsigned char const* const ap = nodes + (size_t)(row >> 5) * kVtTileBytes + h * 512 + (row & 31) * 16;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        a[2 * q] = *reinterpret_cast<v8h const*>(ap + q * 2048 + 1024);
+        a[2 * q + 1] = *reinterpret_cast<v8h const*>(ap + q * 2048);
+    }
+}
+
+// Wave = one slot of 32 keys with the same parent.  Lane l holds key l % 32 as the B operand;
+// element v of matrix step s is dim 32 (s / 2) + 16 h + 8 (s % 2) + v (h = l / 32) on both
+// sides.  Accumulator element r of lane l: child 8 (r / 4) + 4 h + r % 4 of the block, key
+// l % 32.  Level 0 (identity) also forms the keys' norms.
+//
+// What bounds it: the keys' rows (512 bytes each, gathered in bucket order: 100 us for 10^6 at
+// the card's copy rate).  The keys are loaded whole lines at a time and turned into operands
+// through the wave's own LDS, a quarter of their dims at a time; the children come in operand
+// order.  With every lane loading from its own row, for keys and children, the same kernel
+// took 264-306 us a level (64 lines an instruction, each line fetched eight times), and the FP32
+// matrix instructions 281-305 us besides a pass of 213 us for the norms; 121-150 us so.
+__global__ __launch_bounds__(256, 3) void k_vt_score(float const* __restrict__ keys, float* __restrict__ keyNorm,
+                                                     int n, unsigned char const* __restrict__ nodes,
+                                                     float maxNodeNorm, int nodeExp, int usable, int branch,
+                                                     int identity, int const* __restrict__ order,
+                                                     int* __restrict__ node, int* __restrict__ exactList,
+                                                     int* __restrict__ counters, float inf)
+{
+    __shared__ __attribute__((aligned(16))) float stages[4][32 * kExactRow];
     int const lane = threadIdx.x & 63;
     int const h = lane >> 5;
     int const c32 = lane & 31;
     int const slot = blockIdx.x * 4 + (threadIdx.x >> 6);
     int const nSlots = identity ? (n + 31) / 32 : counters[kVtCntSlots];
-    if (slot >= nSlots) return;  // uniform per wave
+    if (slot >= nSlots) return;  // uniform per wave; the waves of a group share nothing
+    float* const stage = stages[threadIdx.x >> 6];
     int kk;
-    long long c0;
+    if (identity) kk = (slot * 32 + c32 < n) ? slot * 32 + c32 : -1;
+    else kk = order[slot * 32 + c32];
+    // an absent key repeats the slot's first one (read with all lanes active: lane 0 holds a key)
+    int const first = __builtin_amdgcn_readfirstlane(kk);
+    int const kr = kk >= 0 ? kk : first;
+    // load u of a quarter: rows 8 u + l / 8, 16 bytes at column l % 8
+    v4f in[16];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        float const* const row = keys + (size_t)__shfl(kr, 8 * u + (lane >> 3)) * kDim + 4 * (lane & 7);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) in[4 * p + u] = *reinterpret_cast<v4f const*>(row + 32 * p);
+    }
+    long long const c0 = identity ? 0 : ((long long)node[first] + 1) * branch;
+    float norm = identity ? 0.0f : keyNorm[kr];
+    int const nb = usable ? (branch + 31) / 32 : 0;  // an unusable tree may have no split rows
+    // rows past the last child exist (the tiles have 32 rows of padding)
+    v8h a[16] = {};
+    if (nb > 0) vt_load_block(a, nodes, c0 + c32, h);
+    float4 raw[16];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        // LDS operations of one wave are in order: the fences only keep the compiler's order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            *reinterpret_cast<v4f*>(stage + (8 * u + (lane >> 3)) * kExactRow + 4 * (lane & 7)) = in[4 * p + u];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            raw[4 * p + q] = *reinterpret_cast<float4 const*>(stage + c32 * kExactRow + 16 * h + 4 * q);
+    }
     if (identity) {
-        kk = (slot * 32 + c32 < n) ? slot * 32 + c32 : -1;
-        c0 = 0;
-    } else {
-        kk = order[slot * 32 + c32];
-        c0 = ((long long)node[order[slot * 32]] + 1) * branch;  // a slot's first entry is a key
-    }
-    float bfrag[64];
-    if (kk >= 0) {
-        float4 const* kp = reinterpret_cast<float4 const*>(keys + (size_t)kk * kDim + h * 64);
+        float s = 0.0f;
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            float4 const v = kp[q];
-            bfrag[4 * q + 0] = v.x;
-            bfrag[4 * q + 1] = v.y;
-            bfrag[4 * q + 2] = v.z;
-            bfrag[4 * q + 3] = v.w;
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < 64; ++q) bfrag[q] = 0.0f;
+        for (int q = 0; q < 16; ++q)
+            s += raw[q].x * raw[q].x + raw[q].y * raw[q].y + raw[q].z * raw[q].z + raw[q].w * raw[q].w;
+        norm = sqrtf(s + __shfl_xor(s, 32));
+        if (h == 0 && kk >= 0) keyNorm[kk] = norm;
     }
+    bool const inRange = usable && norm >= kVtNormMin && norm <= kVtNormMax;
+    int const keyExp = inRange ? (int)(__float_as_uint(norm) >> 23) - 127 : 0;
+    float const scale = __uint_as_float((unsigned)(127 + 14 - keyExp) << 23);  // 2^(14 - keyExp)
+    v8h bh[8], bl[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) vt_split8(raw[2 * s], raw[2 * s + 1], scale, bh[s], bl[s]);
     Top2 s = top2_init();
-    int const nb = (branch + 31) / 32;
     for (int cb = 0; cb < nb; ++cb) {
-        // rows past the last child exist (the node array has 32 zero rows of padding)
-        float4 const* ap = reinterpret_cast<float4 const*>(nodes + (size_t)(c0 + cb * 32 + c32) * kDim + h * 64);
-        float4 a[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) a[q] = ap[q];
         v16f acc = {};
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].x, bfrag[4 * q + 0], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].y, bfrag[4 * q + 1], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].z, bfrag[4 * q + 2], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q].w, bfrag[4 * q + 3], acc, 0, 0, 0);
+        for (int q = 0; q < 8; ++q) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[2 * q], bh[q], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[2 * q + 1], bl[q], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[2 * q + 1], bh[q], acc, 0, 0, 0);
         }
+        // the next block's loads are in flight during the selection
+        if (cb + 1 < nb) vt_load_block(a, nodes, c0 + (cb + 1) * 32 + c32, h);
+        __builtin_amdgcn_sched_barrier(0);
+        if (cb * 32 + 32 <= branch) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            int const j = cb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-            top2_push_fast(s, (j < branch) ? acc[r] : -INFINITY, j, inf);
+            for (int r = 0; r < 16; ++r)
+                top2_push_fast(s, acc[r], cb * 32 + 8 * (r >> 2) + 4 * h + (r & 3), inf);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                int const j = cb * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                top2_push_fast(s, (j < branch) ? acc[r] : -INFINITY, j, inf);
+            }
         }
     }
     s = top2_merge(s, top2_shfl_xor(s, 32));
     if (h != 0 || kk < 0) return;
-    float const eps = kVtEpsRel * keyNorm[kk] * maxNodeNorm + 1e-30f;
-    bool const settled = (eps < 3.0e38f) && (s.b1 == s.b1) && (s.b2 == s.b2) && s.a1 >= 0 &&
-                         (s.b1 - s.b2 > 2.0f * eps) && (s.b1 - eps > -1e30f);
+    float const b1 = ldexpf(s.b1, keyExp + nodeExp - 28);
+    float const b2 = s.b2 > -1e29f ? ldexpf(s.b2, keyExp + nodeExp - 28) : kInit;
+    float const eps = kVtEpsRel * norm * maxNodeNorm + 1e-30f;
+    bool const settled = inRange && (eps < 3.0e38f) && s.a1 >= 0 && (b1 - b2 > 2.0f * eps) && (b1 - eps > -1e30f);
     if (settled) node[kk] = (int)(c0 + s.a1);
     else exactList[atomicAdd(&counters[kVtCntExact], 1)] = kk;
 }
 
-void launch_vt_score(float const* keys, float const* keyNorm, int n, float const* nodes, float maxNodeNorm,
-                     VtLevel const& lv, int const* order, bool identity, int maxSlots, int* node, int* exactList,
-                     int* counters, hipStream_t st)
+void launch_vt_score(float const* keys, float* keyNorm, int n, unsigned char const* nodes, float maxNodeNorm,
+                     int nodeExp, bool usable, VtLevel const& lv, int const* order, bool identity, int maxSlots,
+                     int* node, int* exactList, int* counters, hipStream_t st)
 {
     if (n <= 0 || maxSlots <= 0) return;
     hipLaunchKernelGGL(k_vt_score, dim3((maxSlots + 3) / 4), dim3(256), 0, st, keys, keyNorm, n, nodes, maxNodeNorm,
-                       lv.branch, identity ? 1 : 0, order, node, exactList, counters, INFINITY);
+                       nodeExp, usable ? 1 : 0, lv.branch, identity ? 1 : 0, order, node, exactList, counters,
+                       INFINITY);
 }
 
 // ------------------------------------------------------------------------------ exact decisions
