@@ -100,7 +100,7 @@ int ensureCapacity(v3dm_voctree_s* t, int n)
 int enqueueTraverse(v3dm_voctree_s* t, int n, float const* dKeys, int32_t* dLeaves, bool globalIds)
 {
     hipStream_t const st = t->stream;
-    launch_vt_reset(t->counters, true, st);
+    launch_vt_reset(t->counters, st);
     if (n <= 0) return V3DM_OK;
     VtLevel lv;
     lv.branch = t->branch;
@@ -113,7 +113,6 @@ int enqueueTraverse(v3dm_voctree_s* t, int n, float const* dKeys, int32_t* dLeav
             launch_vt_score(dKeys, t->keyNorm, n, t->dSplit, t->maxNodeNorm, t->nodeExp, t->usable, lv, nullptr,
                             true, (n + 31) / 32, t->node, t->exactList, t->counters, st);
         } else {
-            launch_vt_reset(t->counters, false, st);
             lv.parentStart = t->levelStarts[d - 1];
             lv.nParents = (int)(t->levelStarts[d] - t->levelStarts[d - 1]);
             long long const oc = orderCapacity(n, lv.nParents) - 32;

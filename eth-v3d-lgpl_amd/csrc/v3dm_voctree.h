@@ -30,7 +30,7 @@ struct VtLevel {
 };
 
 // reset the per-level counters (a kernel, so that no memset node is needed)
-void launch_vt_reset(int* counters, bool all, hipStream_t st);
+void launch_vt_reset(int* counters, hipStream_t st);
 // bucket keys by their parent node (level >= 1); keys whose parent is not a node of level
 // - 1 go straight to the exact list
 // cnt, cursor: nParents * kVtBinStride ints

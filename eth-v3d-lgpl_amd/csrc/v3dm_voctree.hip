@@ -67,20 +67,26 @@ void launch_vt_split_nodes(float const* nodes, long long rows, float scale, unsi
                        split);
 }
 
-__global__ void k_vt_reset(int* counters, int all)
+__global__ void k_vt_reset(int* counters)
 {
-    if (threadIdx.x < kVtCounters && (all || threadIdx.x != kVtCntFlagged)) counters[threadIdx.x] = 0;
+    if (threadIdx.x < kVtCounters) counters[threadIdx.x] = 0;
 }
 
-void launch_vt_reset(int* counters, bool all, hipStream_t st)
+void launch_vt_reset(int* counters, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_vt_reset, dim3(1), dim3(64), 0, st, counters, all ? 1 : 0);
+    hipLaunchKernelGGL(k_vt_reset, dim3(1), dim3(64), 0, st, counters);
 }
 
 // ------------------------------------------------------------------------------ bucketing
-__global__ __launch_bounds__(256) void k_vt_zero(int* a, int n, int value)
+// Bucket counts and the level's counters to zero, the order to "no key": one launch (three took
+// 15 us a level).
+__global__ __launch_bounds__(256) void k_vt_clear(int* __restrict__ cnt, int nCnt, int* __restrict__ order,
+                                                  int nOrder, int* __restrict__ counters)
 {
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) a[i] = value;
+    int const t0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+    if (t0 < kVtCounters && t0 != kVtCntFlagged) counters[t0] = 0;
+    for (int i = t0; i < nCnt; i += step) cnt[i] = 0;
+    for (int i = t0; i < nOrder; i += step) order[i] = -1;
 }
 
 // Bucket counts live kVtBinStride ints apart (one L2 line per bucket): the global atomics
@@ -88,13 +94,16 @@ __global__ __launch_bounds__(256) void k_vt_zero(int* a, int n, int value)
 // work-group first counts its kVtKeysPerGroup keys in LDS and adds one total per bucket it
 // saw; the scatter reserves each bucket's range for the work-group with one atomic and
 // places the keys by their LDS rank.  Wider parent levels use one global atomic per key.
-constexpr int kVtKeysPerThread = 16;
-constexpr int kVtKeysPerGroup = 256 * kVtKeysPerThread;
+// What bounds both is the groups' atomics and latency: 1024 threads load their 8 keys together
+// (count and scatter of 10^6 keys over 2500 parents 14 and 23 us); with 4 keys a thread, so
+// twice the atomics, 21 and 31 us, with 256 threads taking 16 keys in turn 25 and 31 us.
+constexpr int kVtGroup = 1024;
+constexpr int kVtKeysPerThread = 8;
+constexpr int kVtKeysPerGroup = kVtGroup * kVtKeysPerThread;
 
-__device__ __forceinline__ int vt_bucket(int const* __restrict__ node, int k, long long parentStart, int nParents,
+__device__ __forceinline__ int vt_bucket(int nd, int k, long long parentStart, int nParents,
                                          int* __restrict__ exactList, int* __restrict__ counters)
 {
-    int const nd = node[k];
     if (nd == kVtNone) return -1;
     long long const b = (long long)nd - parentStart;
     if (b >= 0 && b < nParents) return (int)b;
@@ -102,60 +111,63 @@ __device__ __forceinline__ int vt_bucket(int const* __restrict__ node, int k, lo
     return -1;
 }
 
-__global__ __launch_bounds__(256) void k_vt_count_lds(int const* __restrict__ node, int n, long long parentStart,
-                                                      int nParents, int* __restrict__ cnt,
-                                                      int* __restrict__ exactList, int* __restrict__ counters)
+__global__ __launch_bounds__(kVtGroup) void k_vt_count_lds(int const* __restrict__ node, int n,
+                                                           long long parentStart, int nParents,
+                                                           int* __restrict__ cnt, int* __restrict__ exactList,
+                                                           int* __restrict__ counters)
 {
     extern __shared__ int hist[];
     int const tid = threadIdx.x;
-    for (int b = tid; b < nParents; b += 256) hist[b] = 0;
+    for (int b = tid; b < nParents; b += kVtGroup) hist[b] = 0;
     __syncthreads();
     int const k0 = blockIdx.x * kVtKeysPerGroup;
+    int nd[kVtKeysPerThread];
+#pragma unroll
     for (int i = 0; i < kVtKeysPerThread; ++i) {
-        int const k = k0 + i * 256 + tid;
-        if (k >= n) break;
-        int const b = vt_bucket(node, k, parentStart, nParents, exactList, counters);
+        int const k = k0 + i * kVtGroup + tid;
+        nd[i] = k < n ? node[k] : kVtNone;
+    }
+#pragma unroll
+    for (int i = 0; i < kVtKeysPerThread; ++i) {
+        int const b = vt_bucket(nd[i], k0 + i * kVtGroup + tid, parentStart, nParents, exactList, counters);
         if (b >= 0) atomicAdd(&hist[b], 1);
     }
     __syncthreads();
-    for (int b = tid; b < nParents; b += 256) {
+    for (int b = tid; b < nParents; b += kVtGroup) {
         int const c = hist[b];
         if (c) atomicAdd(&cnt[(size_t)b * kVtBinStride], c);
     }
 }
 
-__global__ __launch_bounds__(256) void k_vt_scatter_lds(int const* __restrict__ node, int n, long long parentStart,
-                                                        int nParents, int* __restrict__ cursor,
-                                                        int* __restrict__ order)
+__global__ __launch_bounds__(kVtGroup) void k_vt_scatter_lds(int const* __restrict__ node, int n,
+                                                             long long parentStart, int nParents,
+                                                             int* __restrict__ cursor, int* __restrict__ order)
 {
     extern __shared__ int hist[];
     int const tid = threadIdx.x;
-    for (int b = tid; b < nParents; b += 256) hist[b] = 0;
+    for (int b = tid; b < nParents; b += kVtGroup) hist[b] = 0;
     __syncthreads();
     int const k0 = blockIdx.x * kVtKeysPerGroup;
     int bin[kVtKeysPerThread], rank[kVtKeysPerThread];
 #pragma unroll
     for (int i = 0; i < kVtKeysPerThread; ++i) {
-        int const k = k0 + i * 256 + tid;
-        bin[i] = -1;
-        if (k < n) {
-            int const nd = node[k];
-            long long const b = (long long)nd - parentStart;
-            if (nd != kVtNone && b >= 0 && b < nParents) {
-                bin[i] = (int)b;
-                rank[i] = atomicAdd(&hist[b], 1);
-            }
-        }
+        int const k = k0 + i * kVtGroup + tid;
+        int const nd = k < n ? node[k] : kVtNone;
+        long long const b = (long long)nd - parentStart;
+        bin[i] = (nd != kVtNone && b >= 0 && b < nParents) ? (int)b : -1;
     }
+#pragma unroll
+    for (int i = 0; i < kVtKeysPerThread; ++i)
+        if (bin[i] >= 0) rank[i] = atomicAdd(&hist[bin[i]], 1);
     __syncthreads();
-    for (int b = tid; b < nParents; b += 256) {
+    for (int b = tid; b < nParents; b += kVtGroup) {
         int const c = hist[b];
         if (c) hist[b] = atomicAdd(&cursor[(size_t)b * kVtBinStride], c);  // the group's range in the bucket
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kVtKeysPerThread; ++i)
-        if (bin[i] >= 0) order[hist[bin[i]] + rank[i]] = k0 + i * 256 + tid;
+        if (bin[i] >= 0) order[hist[bin[i]] + rank[i]] = k0 + i * kVtGroup + tid;
 }
 
 __global__ __launch_bounds__(256) void k_vt_count(int const* __restrict__ node, int n, long long parentStart,
@@ -164,7 +176,7 @@ __global__ __launch_bounds__(256) void k_vt_count(int const* __restrict__ node, 
 {
     int const k = blockIdx.x * 256 + threadIdx.x;
     if (k >= n) return;
-    int const b = vt_bucket(node, k, parentStart, nParents, exactList, counters);
+    int const b = vt_bucket(node[k], k, parentStart, nParents, exactList, counters);
     if (b >= 0) atomicAdd(&cnt[(size_t)b * kVtBinStride], 1);
 }
 
@@ -210,16 +222,15 @@ void launch_vt_bucket(int const* node, int n, VtLevel const& lv, int* cnt, int* 
                       int* exactList, int* counters, hipStream_t st)
 {
     int const binInts = lv.nParents * kVtBinStride;
-    hipLaunchKernelGGL(k_vt_zero, dim3(std::min((binInts + 255) / 256, 4096)), dim3(256), 0, st, cnt, binInts, 0);
-    hipLaunchKernelGGL(k_vt_zero, dim3(std::min((orderCap + 255) / 256, 4096)), dim3(256), 0, st, order, orderCap,
-                       -1);
+    hipLaunchKernelGGL(k_vt_clear, dim3(std::min((std::max(orderCap, binInts) + 255) / 256, 4096)), dim3(256), 0, st,
+                       cnt, binInts, order, orderCap, counters);
     if (lv.nParents <= kVtLdsBins) {
         int const g = (n + kVtKeysPerGroup - 1) / kVtKeysPerGroup;
         size_t const lds = (size_t)lv.nParents * sizeof(int);
-        hipLaunchKernelGGL(k_vt_count_lds, dim3(g), dim3(256), lds, st, node, n, lv.parentStart, lv.nParents, cnt,
+        hipLaunchKernelGGL(k_vt_count_lds, dim3(g), dim3(kVtGroup), lds, st, node, n, lv.parentStart, lv.nParents, cnt,
                            exactList, counters);
         hipLaunchKernelGGL(k_vt_scan, dim3(1), dim3(1024), 0, st, cnt, lv.nParents, cursor, counters);
-        hipLaunchKernelGGL(k_vt_scatter_lds, dim3(g), dim3(256), lds, st, node, n, lv.parentStart, lv.nParents,
+        hipLaunchKernelGGL(k_vt_scatter_lds, dim3(g), dim3(kVtGroup), lds, st, node, n, lv.parentStart, lv.nParents,
                            cursor, order);
     } else {
         int const g = (n + 255) / 256;
@@ -371,7 +382,8 @@ void launch_vt_score(float const* keys, float* keyNorm, int n, unsigned char con
 // The 64 children of a step are loaded whole lines at a time and pass through the wave's own
 // LDS a quarter of their dims at a time (exact_chunk, v3dm_device.h); the key is read from LDS
 // by broadcast.  With every lane loading its own child's row, each line was fetched eight
-// times: 180-205 us a level for 10^6 keys of a <50,3> tree, 70-76 us a level so.
+// times: 180-205 us a level for 10^6 keys of a <50,3> tree, 70-76 us so; counting the keys with
+// one atomic instead of one a wave left 6-27 us.
 __global__ __launch_bounds__(256) void k_vt_exact(float const* __restrict__ keys, float const* __restrict__ nodes,
                                                   long long nNodes, int branch, int level,
                                                   int const* __restrict__ exactList, int* __restrict__ node,
@@ -385,14 +397,16 @@ __global__ __launch_bounds__(256) void k_vt_exact(float const* __restrict__ keys
     float* const kw = keyRows[wave];
     float* const stage = stages[wave];
     float const* const mine = stage + lane * kExactRow;
-    int done = 0;
+    // atomics of one address take about 10 ns each: the whole list is counted by one
+    if (blockIdx.x == 0 && threadIdx.x == 0 && cnt > 0) atomicAdd(&counters[kVtCntFlagged], cnt);
     for (int e = blockIdx.x * 4 + wave; e < cnt; e += gridDim.x * 4) {
         int const kk = exactList[e];
-        done += 1;
         long long const c0 = (level == 0) ? 0 : ((long long)node[kk] + 1) * branch;
         if (c0 < 0 || c0 + branch > nNodes) {
-            if (lane == 0) node[kk] = kVtNone;
-            done -= 1;
+            if (lane == 0) {
+                node[kk] = kVtNone;
+                atomicSub(&counters[kVtCntFlagged], 1);
+            }
             continue;
         }
         // LDS operations of one wave are in order: the fences only keep the compiler's order
@@ -442,8 +456,6 @@ __global__ __launch_bounds__(256) void k_vt_exact(float const* __restrict__ keys
         }
         if (lane == 0) node[kk] = (int)(c0 + bestJ);
     }
-    // one atomic a wave (they share an address)
-    if (lane == 0 && done > 0) atomicAdd(&counters[kVtCntFlagged], done);
 }
 
 void launch_vt_exact(float const* keys, float const* nodes, VtLevel const& lv, int const* exactList, int* node,
