@@ -53,6 +53,9 @@ void launch_mlp_wgrad(__bf16 const* XT, __bf16 const* HT, __bf16 const* dZT, __b
 // apply = 0: only sums the gradient (and refreshes the bf16 copies from the masters)
 void launch_mlp_adam(float const* part, int nChunks, float* grad, MlpWeights const& w, float* M, float* V, float lr,
                      int step, int apply, hipStream_t st);
+// gradients, loss parts and hardest positives -> one block of pinned host memory
+void launch_mlp_results(float const* grad, float const* lossPart, int nLoss, int const* hard, int B, int* host,
+                        hipStream_t st);
 void launch_fill(float* p, size_t n, float v, hipStream_t st);
 
 }  // namespace v3dm

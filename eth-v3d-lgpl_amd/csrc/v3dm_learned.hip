@@ -1032,6 +1032,17 @@ void launch_mlp_codes_u8(uint8_t const* Q, float const* denom, int rows128, MlpW
                        w.P + kOffB1, w.W2p, w.P + kOffB2, scale);
 }
 
+// The results of a gradient call, written across the link in one launch.
+__global__ __launch_bounds__(256) void k_mlp_results(int const* __restrict__ grad, int const* __restrict__ lossPart,
+                                                     int nLoss, int const* __restrict__ hard, int B,
+                                                     int* __restrict__ host)
+{
+    int const i = blockIdx.x * 256 + threadIdx.x;
+    if (i < kParams) host[i] = grad[i];
+    else if (i < kParams + nLoss) host[i] = lossPart[i - kParams];
+    else if (i < kParams + nLoss + B) host[i] = hard[i - kParams - nLoss];
+}
+
 __global__ void k_fill_f32(float* __restrict__ p, size_t n, float v)
 {
     size_t const i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -1098,6 +1109,14 @@ void launch_mlp_adam(float const* part, int nChunks, float* grad, MlpWeights con
     hipLaunchKernelGGL(k_mlp_adam, dim3((kParams + 255) / 256), dim3(256), 0, st, part, nChunks, grad, w.P, M, V,
                        lr, beta1, beta2, eps, apply ? bc1 : 1.0f, apply ? bc2 : 1.0f, apply, w.W1b, w.W2b, w.W2Tb,
                        w.W2p);
+}
+
+void launch_mlp_results(float const* grad, float const* lossPart, int nLoss, int const* hard, int B, int* host,
+                        hipStream_t st)
+{
+    int const n = kParams + nLoss + B;
+    hipLaunchKernelGGL(k_mlp_results, dim3((n + 255) / 256), dim3(256), 0, st, reinterpret_cast<int const*>(grad),
+                       reinterpret_cast<int const*>(lossPart), nLoss, hard, B, host);
 }
 
 void launch_fill(float* p, size_t n, float v, hipStream_t st)
