@@ -29,6 +29,7 @@ HIP_FLAGS = [
 # extra moves per tile); the split pass takes finite sets only, and without NaN semantics its
 # maxima need no canonicalising instruction per operand
 HIP_SOURCE_FLAGS = {"v3dm_check.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                    "v3dm_sieve.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
                     "v3dm_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-fno-honor-nans"]}
 HIP_SOURCES = ["v3dm_fp32.hip", "v3dm_select.hip", "v3dm_short.hip", "v3dm_api.cpp", "v3dm_ext.cpp", "v3dm_batch.cpp",
                "v3dm_learned.cpp", "v3dm_features.cpp",

@@ -19,6 +19,7 @@
 #include "v3dm_kernels.h"
 #include "v3dm_ext.h"
 #include "v3dm_context.h"
+#include "v3dm_sieve.h"
 #include "v3dm_split.h"
 
 using namespace v3dm;
@@ -69,6 +70,12 @@ void releaseBuffers(v3dm_context* h)
     freeDev(h->normR);
     freeDev(h->splitL);
     freeDev(h->splitR);
+    freeDev(h->q8L);
+    freeDev(h->q8R);
+    freeDev(h->resL);
+    freeDev(h->resR);
+    freeDev(h->sieveBest);
+    freeDev(h->sieveSecond);
     freeDev(h->intL);
     freeDev(h->intR);
     freeDev(h->intScaleL);
@@ -186,6 +193,48 @@ void launch_score_pass(v3dm_context* h, FusedPlan const& p, unsigned const* bits
         launch_fused_fp32(h->dL, h->dR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, st);
 }
 
+// Whether a plain (or guided) call goes through the sieve, with its bound.
+bool sieve_fits(v3dm_context const* h, float minScore, float minRatio, float* T)
+{
+    return split_fits(h) && h->epsRel > 0.0f && sieve_bound(minScore, minRatio, T);
+}
+
+SieveBest sieve_best(v3dm_context const* h) { return SieveBest{h->sieveBest, h->sieveSecond, h->capL}; }
+
+void launch_sieve_pass(v3dm_context* h, float T, unsigned const* bits)
+{
+    launch_sieve(SieveSet{h->q8L, h->resL, h->dL, h->nL}, SieveSet{h->q8R, h->resR, h->dR, h->nR},
+                 plan_sieve(h->nL, h->nR), h->maxNormBits, T, sieve_best(h), bits, h->capL, h->stream);
+}
+
+// Scores, decisions and the exact re-check of open queries of the current features (bits: the
+// guided bitmap or null); colMax / rowMax are decided on the stream.
+int enqueue_decisions(v3dm_context* h, unsigned const* bits, float minScore, float minRatio)
+{
+    hipStream_t const st = h->stream;
+    int const nL = h->nL, nR = h->nR;
+    int rc;
+    float T = 0.0f;
+    if (sieve_fits(h, minScore, minRatio, &T)) {
+        if ((rc = prof_begin(h))) return rc;
+        launch_sieve_pass(h, T, bits);
+        if ((rc = prof_end(h))) return rc;
+        launch_sieve_decide(sieve_best(h), nL, nR, minScore, minRatio, h->colMax, h->rowMax, h->flagList, h->capL,
+                            h->results, st);
+    } else {
+        FusedPlan const p = score_plan(h);
+        if ((rc = prof_begin(h))) return rc;
+        launch_score_pass(h, p, bits, minScore);
+        if ((rc = prof_end(h))) return rc;
+        launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
+                            h->normR, h->maxNormBits, score_eps(h, bits), minScore, minRatio, h->colMax, h->rowMax,
+                            h->flagList, h->capL, h->results, st);
+    }
+    launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore, minRatio,
+                         h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st, bits, h->capL);
+    return V3DM_OK;
+}
+
 // Enqueue the plain FP32 exact path for the current features; leaves colMax/rowMax
 // decided and the compacted pairs + counters in h->results.
 int enqueue_plain(v3dm_context* h, float minScore, float minRatio)
@@ -193,17 +242,9 @@ int enqueue_plain(v3dm_context* h, float minScore, float minRatio)
     hipStream_t const st = h->stream;
     int const nL = h->nL, nR = h->nR;
     bool const work = nL > 0 && nR > 0;
-    int rc;
     if (work) {
-        FusedPlan const p = score_plan(h);
-        if ((rc = prof_begin(h))) return rc;
-        launch_score_pass(h, p, nullptr, minScore);
-        if ((rc = prof_end(h))) return rc;
-        launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
-                            h->normR, h->maxNormBits, score_eps(h, nullptr), minScore, minRatio, h->colMax, h->rowMax,
-                            h->flagList, h->capL, h->results, st);
-        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore,
-                             minRatio, h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st);
+        int const rc = enqueue_decisions(h, nullptr, minScore, minRatio);
+        if (rc) return rc;
     }
     launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
                           reinterpret_cast<int2*>(h->results + kNumCounters), h->results, st, {}, h->mutualWait);
@@ -285,6 +326,14 @@ int v3dm_allocate(v3dm_handle h, int nMaxLeft, int nMaxRight, int useGuidedMatch
     auto split_rows = [](int cap) { return (size_t)roundUp(cap, kSplitRowPad); };
     HIPCHECK(h, hipMalloc(&h->splitL, split_rows(h->capL) * kSplitRowBytes));
     HIPCHECK(h, hipMalloc(&h->splitR, split_rows(h->capR) * kSplitRowBytes));
+    HIPCHECK(h, hipMalloc(&h->q8L, split_rows(h->capL) * kDim));
+    HIPCHECK(h, hipMalloc(&h->q8R, split_rows(h->capR) * kDim));
+    HIPCHECK(h, hipMalloc(&h->resL, split_rows(h->capL) / kSieveGroup * sizeof(float)));
+    HIPCHECK(h, hipMalloc(&h->resR, split_rows(h->capR) / kSieveGroup * sizeof(float)));
+    HIPCHECK(h, hipMalloc(&h->sieveBest, (cl + cr) * sizeof(unsigned long long)));
+    HIPCHECK(h, hipMalloc(&h->sieveSecond, (cl + cr) * sizeof(unsigned)));
+    HIPCHECK(h, hipMemsetAsync(h->sieveBest, 0, (cl + cr) * sizeof(unsigned long long), h->stream));
+    HIPCHECK(h, hipMemsetAsync(h->sieveSecond, 0, (cl + cr) * sizeof(unsigned), h->stream));
     HIPCHECK(h, hipMalloc(&h->splitInfo, kPrepInfo * sizeof(int)));
     HIPCHECK(h, hipMemsetAsync(h->splitInfo, 0, kPrepInfo * sizeof(int), h->stream));
     HIPCHECK(h, hipHostMalloc(&h->splitFitHost, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
@@ -393,7 +442,8 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
     }
     launch_split_rows(from, from == kRowsU8 ? (void const*)h->dQ : src, dst, n, left ? h->normL : h->normR,
                       h->maxNormBits + (left ? 0 : 1), left ? h->splitL : h->splitR,
-                      left ? h->intL : h->intR, left ? h->intScaleL : h->intScaleR, h->splitInfo,
+                      left ? h->intL : h->intR, left ? h->intScaleL : h->intScaleR,
+                      left ? h->q8L : h->q8R, left ? h->resL : h->resR, h->splitInfo,
                       h->splitFitDev + (left ? 0 : 1), h->stream);
     (left ? h->haveIntL : h->haveIntR) = from == kRowsU8;
     HIPCHECK(h, hipGetLastError());
@@ -480,17 +530,9 @@ int runGuided(v3dm_context* h, int kind, const double M[9], float distanceThresh
     for (int t = 0; t < 9; ++t) gm.m[t] = m[t];
     gm.sqrThreshold = sqrThreshold;
     h->masks.push_back(gm);
-    int rc;
     if (work) {
-        FusedPlan const p = score_plan(h);
-        if ((rc = prof_begin(h))) return rc;
-        launch_score_pass(h, p, h->guidedBits, minScore);
-        if ((rc = prof_end(h))) return rc;
-        launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
-                            h->normR, h->maxNormBits, score_eps(h, h->guidedBits), minScore, minRatio, h->colMax, h->rowMax,
-                            h->flagList, h->capL, h->results, st);
-        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore, minRatio,
-                             h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st, h->guidedBits, h->capL);
+        int const rc = enqueue_decisions(h, h->guidedBits, minScore, minRatio);
+        if (rc) return rc;
     }
     launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
                           reinterpret_cast<int2*>(h->results + kNumCounters), h->results, st, {}, h->mutualWait);
@@ -772,9 +814,19 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
     if (h->precision == V3DM_PREC_FP32) {
         if (h->nL > 0 && h->nR > 0) {
             FusedPlan const p = score_plan(h);
+            float T = 0.0f;
+            bool const sieve = sieve_fits(h, h->lastMinScore, h->lastMinRatio, &T);
             e = hipEventRecord(a, h->stream);
-            for (int r = 0; r < reps && e == hipSuccess; ++r) launch_score_pass(h, p, nullptr, h->lastMinScore);
+            for (int r = 0; r < reps && e == hipSuccess; ++r) {
+                if (sieve) launch_sieve_pass(h, T, nullptr);
+                else launch_score_pass(h, p, nullptr, h->lastMinScore);
+            }
             if (e == hipSuccess) e = hipEventRecord(b, h->stream);
+            if (sieve) {  // no decisions follow that would leave the bests at zero
+                size_t const n = (size_t)h->capL + h->capR;
+                if (e == hipSuccess) e = hipMemsetAsync(h->sieveBest, 0, n * sizeof(unsigned long long), h->stream);
+                if (e == hipSuccess) e = hipMemsetAsync(h->sieveSecond, 0, n * sizeof(unsigned), h->stream);
+            }
             launches = reps;
         }
     } else {

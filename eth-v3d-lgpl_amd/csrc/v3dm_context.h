@@ -44,6 +44,10 @@ struct v3dm_context {
     float* intScaleL = nullptr;       // ... and the rows' scales (allocated by the first uint8 upload)
     float* intScaleR = nullptr;
     bool haveIntL = false, haveIntR = false;  // the current set has them
+    signed char *q8L = nullptr, *q8R = nullptr;   // the sieve's rows and residuals
+    float *resL = nullptr, *resR = nullptr;
+    unsigned long long* sieveBest = nullptr;      // of capL left, then capR right features
+    unsigned* sieveSecond = nullptr;
     int* splitInfo = nullptr;         // scratch of launch_split_rows
     int* splitFitHost = nullptr;      // mapped: [0] left, [1] right set in the split pass's range
     int* splitFitDev = nullptr;       // the same memory as the kernels address it

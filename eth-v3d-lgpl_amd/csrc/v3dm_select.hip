@@ -7,6 +7,7 @@
 // mutual check).
 #include "v3dm_device.h"
 #include "v3dm_kernels.h"
+#include "v3dm_sieve.h"
 #include "v3dm_split.h"
 
 namespace v3dm {
@@ -68,11 +69,34 @@ __device__ __forceinline__ void split_pair(float2 v, unsigned& hi, unsigned& lo)
     lo = __builtin_bit_cast(unsigned, l);
 }
 
+// The sum of each of 8 values over the wave's lanes, the largest of them in every lane: the
+// first three steps halve the values a lane carries.
+__device__ __forceinline__ float max_of_sums(float (&s)[8], int lane)
+{
+#pragma unroll
+    for (int n = 4, o = 32; n >= 1; n >>= 1, o >>= 1) {
+        bool const up = lane & o;
+#pragma unroll
+        for (int k = 0; k < n; ++k) {
+            float const other = __shfl_xor(up ? s[k] : s[n + k], o);
+            s[k] = (up ? s[n + k] : s[k]) + other;
+        }
+    }
+    float x = s[0];
+    x += __shfl_xor(x, 4);
+    x += __shfl_xor(x, 2);
+    x += __shfl_xor(x, 1);
+    x = fmaxf(x, __shfl_xor(x, 32));
+    x = fmaxf(x, __shfl_xor(x, 16));
+    return fmaxf(x, __shfl_xor(x, 8));
+}
+
 template <int kFrom>
 __global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src, float* __restrict__ X, int n,
                                                     float* __restrict__ norm, unsigned int* __restrict__ maxNormBits,
                                                     unsigned char* __restrict__ split,
                                                     unsigned char* __restrict__ ints, float* __restrict__ scale,
+                                                    signed char* __restrict__ q8, float* __restrict__ res,
                                                     int* __restrict__ info, int* __restrict__ hostFit)
 {
     __shared__ unsigned int wmax[4];
@@ -129,6 +153,21 @@ __global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src
             o[lane & 31] = hi;
             o[32 + (lane & 31)] = lo;
         }
+        // the sieve's rows (past n: inside the padded buffer, never read)
+        float e2[kPrepRows];
+#pragma unroll
+        for (int k = 0; k < kPrepRows; ++k) {
+            float const qx = fminf(fmaxf(rintf(v[k].x * kSieveScale), -127.0f), 127.0f);
+            float const qy = fminf(fmaxf(rintf(v[k].y * kSieveScale), -127.0f), 127.0f);
+            float const ex = v[k].x - qx * (1.0f / kSieveScale), ey = v[k].y - qy * (1.0f / kSieveScale);
+            e2[k] = ex * ex + ey * ey;
+            int const row = row0 + k;
+            *reinterpret_cast<char2*>(q8 + (size_t)(row / kSieveTile) * kSieveTileBytes + (lane >> 3) * 512 +
+                                      (row % kSieveTile) * 16 + (lane & 7) * 2) =
+                make_char2((signed char)(int)qx, (signed char)(int)qy);
+        }
+        float const r2 = max_of_sums(e2, lane);
+        if (lane == 0) res[row0 / kSieveGroup] = sqrtf(r2) * 1.001f + 1e-6f;  // rounded up
     }
     if (lane == 0) {
         wmax[wave] = mx;
@@ -170,21 +209,21 @@ __global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src
 }
 
 void launch_split_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNormBits,
-                       unsigned char* split, unsigned char* ints, float* scale, int* info, int* hostFit,
-                       hipStream_t st)
+                       unsigned char* split, unsigned char* ints, float* scale, signed char* q8, float* res, int* info,
+                       int* hostFit, hipStream_t st)
 {
     if (n <= 0) return;
     int const per = 4 * kPrepRows;
     dim3 const grid(min((n + per - 1) / per, kPrepGroups));
     if (from == kRowsU8)
         hipLaunchKernelGGL(k_split_rows<kRowsU8>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, ints,
-                           scale, info, hostFit);
+                           scale, q8, res, info, hostFit);
     else if (from == kRowsF32)
         hipLaunchKernelGGL(k_split_rows<kRowsF32>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, ints,
-                           scale, info, hostFit);
+                           scale, q8, res, info, hostFit);
     else
         hipLaunchKernelGGL(k_split_rows<kRowsInPlace>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split,
-                           ints, scale, info, hostFit);
+                           ints, scale, q8, res, info, hostFit);
 }
 
 // ------------------------------------------------------------------------------ merge + decide

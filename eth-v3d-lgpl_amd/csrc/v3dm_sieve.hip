@@ -1,0 +1,258 @@
+// The sieve of plain putative matching (gfx950): int8 score pass, exact scores of its
+// candidates, decisions.
+//
+// Reference path: V3D_CUDA::SIFT_Matching::findPutativeMatches
+// (V3D/CUDA/v3d_cudamatching.cu:522-552); best and second best are those of the exact scores
+// fl32(sum of the FP64 products), as the exact re-check decides open queries of the other passes.
+#include <algorithm>
+#include <cmath>
+
+#include "v3dm_device.h"
+#include "v3dm_sieve.h"
+
+namespace v3dm {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+bool sieve_bound(float minScore, float minRatio, float* T)
+{
+    double t = minScore;
+    // the rule's own roundings (2 - 2 b, the quotient) are below 2^-21 of its values
+    if (minRatio >= 0.0f) t = std::min(t, 1.0 - (1.0 - (double)minScore) * (1.0 + 1e-5) / (double)minRatio);
+    t -= 1e-5;
+    *T = (float)t;
+    return t >= kSieveMin && t < 1e6;  // NaN, and a ratio of zero, are out
+}
+
+// ------------------------------------------------------------------------------ score pass
+// Wave = 128 left features (four 32-column blocks, their int8 rows the resident B operands, 64
+// VGPRs) against a run of 32-row tiles of right features, four v_mfma_i32_32x32x32_i8 a block
+// and tile.  The rows lie in operand order, so a tile is four loads of 1 KiB straight from L1 /
+// L2 (the four waves of a group take the same tiles), two tiles ahead; there is no LDS staging
+// and no barrier.  Per block the 16 scores of a lane are reduced by 8 max3 and compared with
+// the lane's bound; only a block with a score above it looks at single scores and lists them
+// (LDS, kSieveList per wave).  After its last tile the wave scores its list exactly, a pair per
+// lane, and enters each score for both features: an atomic maximum of (score, ~index) returns the
+// smaller of two keys, which goes to the second best's maximum; so every key but the largest
+// reaches it, and equal scores keep the smallest index.  A wave whose list overflows marks all
+// its features for the exact re-check instead.
+//
+// What bounds it: the int8 matrix instructions (16384 x 16384: 2^20 of them, 20 us of the 37),
+// then the tail, where each wave waits for the rows and the atomics of its few candidates
+// (512 x 512, nothing but tail: 9 us).  16384 x 16384: 37 us for the pass and 5 for the decisions
+// against 182 + 6 + 14 of the FP16 split pass, its merge and its re-check (605 of the FP32
+// instruction); 4096 x 4096: 12 + 3 against 24 + 5 + 4; 480 x 512: 9 + 2 against 8 + 5 + 4.
+constexpr int kSieveBlocks = 4;
+constexpr int kSieveList = 512;
+constexpr unsigned long long kSieveFlood = ~0ull;
+
+__device__ __forceinline__ int max3i(int a, int b, int c) { return max(max(a, b), c); }
+
+__device__ __forceinline__ int max16(v16i const& a)
+{
+    int const x = max3i(a[0], a[1], a[2]), y = max3i(a[3], a[4], a[5]), z = max3i(a[6], a[7], a[8]);
+    int const u = max3i(a[9], a[10], a[11]), v = max3i(a[12], a[13], a[14]);
+    return max3i(max3i(x, y, z), max(u, v), a[15]);
+}
+
+__device__ __forceinline__ void sieve_tile(v4i (&a)[4], signed char const* __restrict__ q, int t, int lane)
+{
+    v4i const* const p = reinterpret_cast<v4i const*>(q + (size_t)t * kSieveTileBytes) + lane;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) a[s] = p[64 * s];
+}
+
+// fl32 of the FP64 sum in ascending order, as exact_scores (v3dm_device.h).
+__device__ __forceinline__ float sieve_exact(float const* __restrict__ x, float const* __restrict__ y)
+{
+    float4 const* const a = reinterpret_cast<float4 const*>(x);
+    float4 const* const b = reinterpret_cast<float4 const*>(y);
+    double acc = 0.0;
+#pragma unroll 1
+    for (int p = 0; p < 4; ++p) {
+        float4 u[8], v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            u[k] = a[8 * p + k];
+            v[k] = b[8 * p + k];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            acc += (double)u[k].x * (double)v[k].x;
+            acc += (double)u[k].y * (double)v[k].y;
+            acc += (double)u[k].z * (double)v[k].z;
+            acc += (double)u[k].w * (double)v[k].w;
+        }
+    }
+    return (float)acc;
+}
+
+__device__ __forceinline__ void sieve_enter(unsigned long long* best, unsigned* second, unsigned long long key)
+{
+    unsigned long long const old = atomicMax(best, key);
+    unsigned const loser = (unsigned)((old < key ? old : key) >> 32);
+    if (loser) atomicMax(second, loser);
+}
+
+__global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SievePlan p,
+                                                  unsigned const* __restrict__ maxNormBits, float T, SieveBest out,
+                                                  unsigned const* __restrict__ bits, int ldi)
+{
+    __shared__ int lists[4][kSieveList];
+    int const lane = threadIdx.x & 63;
+    int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int const h = lane >> 5;
+    int const c32 = lane & 31;
+    int* const list = lists[wv];
+    // neighbouring work-groups of one XCD share a split's right tiles in its L2
+    int const b = xcd_block(blockIdx.x, gridDim.x);
+    int const split = b / p.groups;
+    int const i0 = ((b - split * p.groups) * 4 + wv) * (32 * kSieveBlocks);
+    if (i0 >= L.n) return;  // the waves of a group share nothing
+    int const t0 = split * p.tiles;
+    int const t1 = min(t0 + p.tiles, R.n / kSieveTile);
+    float const ML = __uint_as_float(maxNormBits[0]), MR = __uint_as_float(maxNormBits[1]);
+
+    // blocks past L.n (a multiple of 32) repeat the last one with a bound that nothing exceeds
+    v4i B[kSieveBlocks][4];
+    float base[kSieveBlocks], arm[kSieveBlocks];
+#pragma unroll
+    for (int cb = 0; cb < kSieveBlocks; ++cb) {
+        int const blk = min(i0 / 32 + cb, L.n / 32 - 1);
+        sieve_tile(B[cb], L.q, blk, lane);
+        float const r = L.res[(blk * 32 + c32) / kSieveGroup];
+        bool const exists = i0 + 32 * cb < L.n;
+        // score units * 65536; the 2 covers the roundings here and below
+        base[cb] = exists ? (T - r * MR) * 65536.0f - 2.0f : INFINITY;
+        arm[cb] = (ML + r) * 65536.0f;
+    }
+    int cnt = 0;  // uniform
+    auto tile = [&](v4i(&a)[4], int t) {
+        float const* const rt = R.res + t * (kSieveTile / kSieveGroup);
+        float const r = fmaxf(fmaxf(rt[0], rt[1]), fmaxf(rt[2], rt[3]));
+        // two blocks at a time: four would not fit beside the operands
+#pragma unroll
+        for (int c0 = 0; c0 < kSieveBlocks; c0 += 2) {
+            v16i acc[2] = {};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+                    acc[k] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[s], B[c0 + k][s], acc[k], 0, 0, 0);
+            if (c0 + 2 == kSieveBlocks) sieve_tile(a, R.q, min(t + 2, t1 - 1), lane);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                int const cb = c0 + k;
+                float const thr = fmaf(-arm[cb], r, base[cb]);
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64((float)max16(acc[k]) > thr) == 0, 1)) continue;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    bool const hit = (float)acc[k][e] > thr;
+                    unsigned long long const m = __builtin_amdgcn_ballot_w64(hit);
+                    if (m == 0) continue;
+                    int const at = cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                    int const j = t * kSieveTile + 8 * (e >> 2) + 4 * h + (e & 3);
+                    if (hit && at < kSieveList) list[at] = ((cb * 32 + c32) << 20) | j;
+                    cnt += __builtin_popcountll(m);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    {
+        v4i a0[4], a1[4];
+        sieve_tile(a0, R.q, t0, lane);
+        sieve_tile(a1, R.q, min(t0 + 1, t1 - 1), lane);
+        int t = t0;
+        for (; t + 1 < t1; t += 2) {
+            tile(a0, t);
+            tile(a1, t + 1);
+        }
+        if (t < t1) tile(a0, t);
+    }
+    if (cnt > kSieveList) {
+        for (int i = lane; i < min(32 * kSieveBlocks, L.n - i0); i += 64) atomicMax(out.best + i0 + i, kSieveFlood);
+        for (int j = t0 * kSieveTile + lane; j < t1 * kSieveTile; j += 64)
+            atomicMax(out.best + out.offR + j, kSieveFlood);
+        return;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // LDS operations of one wave are in order
+    for (int c = lane; c < cnt; c += 64) {
+        int const e = list[c];
+        int const i = i0 + (e >> 20), j = e & 0xfffff;
+        if (bits && ((bits[(size_t)(j >> 5) * ldi + i] >> (j & 31)) & 1u)) continue;  // a removed pair
+        float const s = sieve_exact(L.X + (size_t)i * kDim, R.X + (size_t)j * kDim);
+        if (!(s > 0.0f)) continue;  // T > 0: cannot matter
+        unsigned long long const v = (unsigned long long)__float_as_uint(s) << 32;
+        sieve_enter(out.best + i, out.second + i, v | (0xffffffffu - (unsigned)j));
+        sieve_enter(out.best + out.offR + j, out.second + out.offR + j, v | (0xffffffffu - (unsigned)i));
+    }
+}
+
+// Splits of the right features: three work-groups of four waves per CU run at a time, and a
+// wave's operand load and exact scores cost about four tiles.
+SievePlan plan_sieve(int nL, int nR)
+{
+    SievePlan p;
+    p.groups = (nL + 128 * kSieveBlocks - 1) / (128 * kSieveBlocks);
+    int const nTiles = nR / kSieveTile;
+    long long best = 1LL << 60;
+    for (int s = 1; s <= nTiles && s <= 1024; ++s) {
+        int const tiles = (nTiles + s - 1) / s;
+        int const splits = (nTiles + tiles - 1) / tiles;
+        long long const cost = ((long long)p.groups * splits + 767) / 768 * (tiles + 4);
+        if (cost < best) {
+            best = cost;
+            p.splits = splits;
+            p.tiles = tiles;
+        }
+    }
+    return p;
+}
+
+void launch_sieve(SieveSet const& L, SieveSet const& R, SievePlan const& p, unsigned const* maxNormBits, float T,
+                  SieveBest const& b, unsigned const* bits, int ldi, hipStream_t st)
+{
+    if (L.n <= 0 || R.n <= 0) return;
+    hipLaunchKernelGGL(k_sieve, dim3(p.groups * p.splits), dim3(256), 0, st, L, R, p, maxNormBits, T, b, bits, ldi);
+}
+
+// ------------------------------------------------------------------------------ decisions
+__global__ __launch_bounds__(256) void k_sieve_decide(SieveBest b, int nL, int nR, float minScore, float minRatio,
+                                                      int* __restrict__ colMax, int* __restrict__ rowMax,
+                                                      int* __restrict__ flagList, int flagOffR,
+                                                      int* __restrict__ counters)
+{
+    int const g = blockIdx.x * 256 + threadIdx.x;
+    if (g >= nL + nR) return;
+    bool const left = g < nL;
+    int const q = left ? g : g - nL;
+    int const at = left ? q : b.offR + q;
+    unsigned long long const k = b.best[at];
+    unsigned const s2 = b.second[at];
+    int d = -1;
+    if (k == kSieveFlood) {
+        int const slot = atomicAdd(&counters[left ? kCntFlag : kCntFlagR], 1);
+        flagList[left ? slot : flagOffR + slot] = q;
+        d = kFlag;
+    } else if (k) {
+        Top2 const s{__uint_as_float((unsigned)(k >> 32)), s2 ? __uint_as_float(s2) : kInit,
+                     (int)(0xffffffffu - (unsigned)k)};
+        d = decide_exact(s, minScore, minRatio);
+    }
+    if (k) b.best[at] = 0;
+    if (s2) b.second[at] = 0;
+    (left ? colMax : rowMax)[q] = d;
+}
+
+void launch_sieve_decide(SieveBest const& b, int nL, int nR, float minScore, float minRatio, int* colMax, int* rowMax,
+                         int* flagList, int flagOffR, int* counters, hipStream_t st)
+{
+    if (nL + nR <= 0) return;
+    hipLaunchKernelGGL(k_sieve_decide, dim3((nL + nR + 255) / 256), dim3(256), 0, st, b, nL, nR, minScore, minRatio,
+                       colMax, rowMax, flagList, flagOffR, counters);
+}
+
+}  // namespace v3dm

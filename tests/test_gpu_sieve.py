@@ -1,0 +1,95 @@
+"""The sieved plain path (int8 score pass, exact scores of its candidates) against the CPU
+oracle: matches of pairs at block and tile edges, uneven sizes, minimum scores and ratios on
+both sides of the rule that takes the path, rows the int8 form holds badly (large components,
+negative components, norms other than one), equal scores, and sets that overflow the candidate
+lists.  Matches are whole numbers: they equal the oracle's."""
+import numpy as np
+import pytest
+
+import v3dmatch
+from oracle import oracle
+from v3dmatch import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def matcher():
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(4096, 4096)
+    yield m
+    m.close()
+
+
+def _unit(x):
+    return (x / np.linalg.norm(x, axis=1, keepdims=True)).astype(np.float32)
+
+
+def _same(m, L, R, min_score, min_ratio):
+    m.setLeftFeatures(L.shape[0], L)
+    m.setRightFeatures(R.shape[0], R)
+    got = m.find_putative_matches_array(min_score, min_ratio)
+    assert np.array_equal(got, oracle.find_putative_matches(L, R, min_score, min_ratio))
+
+
+@pytest.mark.parametrize("nL,nR", [(32, 32), (32, 4096), (4096, 32), (96, 160), (128, 512), (512, 128), (544, 1056),
+                                   (2016, 2080), (4096, 4096)])
+@pytest.mark.parametrize("min_score,min_ratio", [(0.9, 0.8), (0.85, 0.7), (0.8, -1.0), (0.75, 0.9), (0.2, 0.8)])
+def test_sizes(matcher, nL, nR, min_score, min_ratio):
+    print(f"case sieve {nL} x {nR} min {min_score} ratio {min_ratio}", flush=True)
+    a, b, _ = synth.make_pair(nL, nR, 0.4, config=7, pair=nL + nR)
+    _same(matcher, synth.dequantise(a), synth.dequantise(b), min_score, min_ratio)
+
+
+@pytest.mark.parametrize("kind", ["sparse", "signed", "norms", "ties"])
+def test_rows(matcher, kind):
+    """sparse: components up to 1 (the int8 rows clip); signed: both signs; norms: 2^-3 to 1.9;
+    ties: equal rows on both sides."""
+    print(f"case sieve rows {kind}", flush=True)
+    rng = np.random.default_rng(3)
+    n = 640
+    if kind == "sparse":
+        L = np.zeros((n, 128), np.float32)
+        for i in range(n):
+            L[i, rng.choice(128, 3, replace=False)] = rng.uniform(0.3, 1.0, 3)
+        L = _unit(L)
+    else:
+        L = _unit(rng.standard_normal((n, 128)))
+    R = _unit(L[rng.permutation(n)] + 0.02 * rng.standard_normal((n, 128)))
+    if kind == "norms":
+        L = L * rng.uniform(0.125, 1.9, (n, 1)).astype(np.float32)
+        R = R * rng.uniform(0.125, 1.9, (n, 1)).astype(np.float32)
+    if kind == "ties":
+        R[200:232] = R[100]
+        L[300:340] = L[17]
+        R[5] = L[17]
+        R[630] = L[17]
+    for ms, mr in ((0.9, 0.8), (0.8, -1.0), (0.8, 0.95)):
+        _same(matcher, L, R, ms, mr)
+
+
+@pytest.mark.parametrize("share", [0.3, 1.0])
+def test_flooded_lists(matcher, share):
+    """Nearly equal rows: every pair of them is a candidate and the lists overflow."""
+    print(f"case sieve flooded {share}", flush=True)
+    rng = np.random.default_rng(4)
+    n = 1024
+    a, b, _ = synth.make_pair(n, n, 0.4, config=7, pair=3)
+    L, R = synth.dequantise(a), synth.dequantise(b)
+    k = int(share * n)
+    c = _unit(np.abs(rng.standard_normal((1, 128))))
+    L[:k] = _unit(c + 0.01 * rng.standard_normal((k, 128)))
+    R[n - k:] = _unit(c + 0.01 * rng.standard_normal((k, 128)))
+    _same(matcher, L, R, 0.9, 0.8)
+    assert matcher.stats()["nRechecked"] > 0
+    _same(matcher, L, R, 0.9, -1.0)
+
+
+def test_timing_leaves_no_state(matcher):
+    print("case sieve timing", flush=True)
+    a, b, _ = synth.make_pair(1024, 992, 0.4, config=7, pair=9)
+    L, R = synth.dequantise(a), synth.dequantise(b)
+    _same(matcher, L, R, 0.9, 0.8)
+    assert matcher.time_dominant_kernel(3) > 0
+    _same(matcher, L, R, 0.9, 0.8)
