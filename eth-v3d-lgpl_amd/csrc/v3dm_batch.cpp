@@ -18,6 +18,7 @@
 #include "v3dm_batch.h"
 #include "v3dm_context.h"
 #include "v3dm_learned.h"
+#include "v3dm_sieve.h"
 #include "v3dm_split.h"
 
 namespace v3dm {
@@ -75,6 +76,18 @@ struct BatchState {
     int* notFit = nullptr;           // device: set by the norms of a row outside the range
     bool splitValid = false;
     bool splitFit = false;           // every row is in the split pass's range
+    signed char* q8 = nullptr;       // the sieve's rows and residuals, made by a run that takes it
+    float* res = nullptr;
+    size_t q8Cap = 0, resCap = 0;
+    bool q8Valid = false;
+    unsigned long long* sieveBest = nullptr;  // per query row, zero between runs
+    unsigned* sieveSecond = nullptr;
+    int sieveCap = 0;
+    int4* sieveItems = nullptr;
+    int nSieveItems = 0, sieveItemCap = 0;
+    bool sieveValid = false;  // sieveItems hold the current pairs
+    bool lastSieve = false;   // the last run took the sieve, with this bound
+    float lastT = 0.0f;
     bool codesValid = false;
     float codesScale = 0.0f;
     int* imgBase = nullptr;
@@ -232,6 +245,8 @@ BatchDev dev_view(BatchState* b, int form)
     d.u8 = b->haveU8 ? b->imgU8 : nullptr;
     d.denom = b->denom;
     d.split = b->split;
+    d.q8 = b->q8;
+    d.res = b->res;
     d.imgBase = b->imgBase;
     d.norm = b->norm;
     d.maxNorm = b->maxNorm;
@@ -629,6 +644,67 @@ int ensure_split(v3dm_context* h, BatchState* b)
     return grow(h, b->split, b->splitCap, need);
 }
 
+// Whether the plain decisions of a run come from the sieve, with its bound (v3dm_sieve.h).
+bool sieve_run(v3dm_context const* h, BatchState const* b, float minScore, float minRatio, float* T)
+{
+    return b->splitFit && h->epsRel > 0.0f && sieve_bound(minScore, minRatio, T);
+}
+
+// Rows, entries and items of the sieve.  An item is 512 left features against a run of 32-row
+// right tiles: 64 tiles (a wave's operand loads and its exact scores cost about four), fewer
+// where that would leave under four rounds of 768 work-groups.
+int ensure_sieve(v3dm_context* h, BatchState* b)
+{
+    int rc;
+    if (!b->q8 || !b->res || b->q8Cap < (size_t)b->imgRows * kDim || b->resCap < (size_t)b->imgRows / kSieveGroup) {
+        drop_graphs(b);  // captured runs hold the old buffers
+        b->q8Valid = false;
+        if ((rc = grow(h, b->q8, b->q8Cap, (size_t)b->imgRows * kDim))) return rc;
+        if ((rc = grow(h, b->res, b->resCap, (size_t)b->imgRows / kSieveGroup))) return rc;
+    }
+    if (!b->sieveBest || !b->sieveSecond || b->sieveCap < b->qRows) {
+        drop_graphs(b);
+        for (void* p : {(void*)b->sieveBest, (void*)b->sieveSecond})
+            if (p) (void)hipFree(p);
+        b->sieveBest = nullptr;
+        b->sieveSecond = nullptr;
+        b->sieveCap = 0;
+        size_t const n = (size_t)std::max(b->qRows, 1);
+        BCHECK(h, hipMalloc(&b->sieveBest, n * sizeof(unsigned long long)));
+        BCHECK(h, hipMalloc(&b->sieveSecond, n * sizeof(unsigned)));
+        BCHECK(h, hipMemsetAsync(b->sieveBest, 0, n * sizeof(unsigned long long), h->stream));
+        BCHECK(h, hipMemsetAsync(b->sieveSecond, 0, n * sizeof(unsigned), h->stream));
+        b->sieveCap = b->qRows;
+    }
+    if (b->sieveValid) return V3DM_OK;
+    drop_graphs(b);
+    long long total = 0;
+    for (int p = 0; p < b->nPairs; ++p)
+        total += (long long)((b->imgN[b->pa[p]] + 511) / 512) * (b->imgN[b->pb[p]] / kSieveTile);
+    int const tiles = (int)std::min<long long>(64, std::max<long long>(8, total / (4 * 768)));
+    std::vector<std::pair<int, int4>> work;
+    for (int p = 0; p < b->nPairs; ++p) {
+        int const groups = (b->imgN[b->pa[p]] + 511) / 512, nTiles = b->imgN[b->pb[p]] / kSieveTile;
+        for (int g = 0; g < groups; ++g)
+            for (int s = 0; s * tiles < nTiles; ++s)
+                work.push_back({std::min(tiles, nTiles - s * tiles), make_int4(p, g, s, tiles)});
+    }
+    std::stable_sort(work.begin(), work.end(),
+                     [](std::pair<int, int4> const& x, std::pair<int, int4> const& y) { return x.first > y.first; });
+    std::vector<int4> items;
+    items.reserve(work.size());
+    for (auto& w : work) items.push_back(w.second);
+    if ((rc = growi(h, b->sieveItems, b->sieveItemCap, items.size()))) return rc;
+    if (!items.empty())
+        BCHECK(h, hipMemcpyAsync(b->sieveItems, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice,
+                                 h->stream));
+    BCHECK(h, hipStreamSynchronize(h->stream));
+    b->nSieveItems = (int)items.size();
+    b->sieveValid = true;
+    b->version += 1;
+    return V3DM_OK;
+}
+
 // The certified decisions' error bound for the scores of launch_plain_pass.
 float plain_eps(v3dm_context const* h, BatchState const* b)
 {
@@ -656,8 +732,19 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
     BatchDev const d = dev_view(b, form);
     Plan const& pl = b->plan[form];
     launch_batch_reset(b->counters, b->pairCount, b->nPairs, st);
-    if (!h->cacheDerived) enqueue_derived(h, b, form);
-    if (form == 0) {
+    float T = 0.0f;
+    bool const sieve = form != 1 && sieve_run(h, b, minScore, minRatio, &T);
+    if (!h->cacheDerived) {
+        if (form == 0 && sieve) launch_batch_sieve_rows(d, b->imgRows, b->q8, b->res, st);
+        else enqueue_derived(h, b, form);
+    }
+    if (form == 0 && sieve) {
+        launch_batch_sieve(d, b->sieveItems, b->nSieveItems, T, b->sieveBest, b->sieveSecond, nullptr, st);
+        launch_batch_sieve_decide(d, b->sieveBest, b->sieveSecond, minScore, minRatio, b->sel, b->flagList,
+                                  b->counters, nullptr, st);
+        launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio,
+                             b->sel, 1024, st);
+    } else if (form == 0) {
         launch_plain_pass(b, 0, b->items[0], (int)pl.items.size(), b->counters + 0, minScore, st);
         launch_batch_merge_decide(d, b->partF, plain_eps(h, b), minScore, minRatio, b->sel, b->flagList, b->counters, st);
         launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio,
@@ -703,12 +790,19 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
             BatchDev const d0 = dev_view(b, 3);
             launch_batch_fb_filter(b->items[3], np, b->pairFlag, b->nPairs, b->fbItems, b->counters + kBCntFbItems,
                                    b->segMask, st);
-            // (the split rows of a plain run may be there already, of the same images)
-            if (b->splitFit && !(h->cacheDerived && b->splitValid))
-                launch_batch_split_masked(d0, b->segMask, b->split, 2 * cus, st);
-            launch_plain_pass(b, 3, b->fbItems, np, b->counters + 0, minScore, st, b->counters + kBCntFbItems);
-            launch_batch_merge_masked(d0, b->partF, plain_eps(h, b), minScore, minRatio, b->sel, b->flagList, b->counters,
-                                      b->segMask, 2 * cus, st);
+            // (the rows of a plain run may be there already, of the same images)
+            if (sieve) {
+                if (!(h->cacheDerived && b->q8Valid)) launch_batch_sieve_masked(d0, b->segMask, b->q8, b->res, st);
+                launch_batch_sieve(d0, b->sieveItems, b->nSieveItems, T, b->sieveBest, b->sieveSecond, b->pairFlag, st);
+                launch_batch_sieve_decide(d0, b->sieveBest, b->sieveSecond, minScore, minRatio, b->sel, b->flagList,
+                                          b->counters, b->segMask, st);
+            } else {
+                if (b->splitFit && !(h->cacheDerived && b->splitValid))
+                    launch_batch_split_masked(d0, b->segMask, b->split, 2 * cus, st);
+                launch_plain_pass(b, 3, b->fbItems, np, b->counters + 0, minScore, st, b->counters + kBCntFbItems);
+                launch_batch_merge_masked(d0, b->partF, plain_eps(h, b), minScore, minRatio, b->sel, b->flagList,
+                                          b->counters, b->segMask, 2 * cus, st);
+            }
             launch_batch_recheck(d0, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore,
                                  minRatio, b->sel, 1024, st);
         }
@@ -888,7 +982,7 @@ int set_images(v3dm_context* h, int nImages, int32_t const* counts, void const* 
     }
     if (totalRaw > (size_t)0x7fffffff / kDim) return ctx_fail(h, V3DM_ERR_INVALID, "batch too large");
     drop_graphs(b);
-    b->planValid[0] = b->planValid[1] = b->planValid[2] = b->planValid[3] = false;
+    b->planValid[0] = b->planValid[1] = b->planValid[2] = b->planValid[3] = b->sieveValid = false;
     b->nPairs = 0;
     b->pending = false;
     b->nImages = nImages;
@@ -976,6 +1070,7 @@ int set_images(v3dm_context* h, int nImages, int32_t const* counts, void const* 
     b->bfValid = false;
     b->codesValid = false;
     b->splitValid = false;
+    b->q8Valid = false;
     BCHECK(h, hipGetLastError());
     int notFit = 1;
     BCHECK(h, hipMemcpyAsync(&notFit, b->notFit, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -990,7 +1085,8 @@ void batch_destroy(BatchState*& b)
 {
     if (!b) return;
     drop_graphs(b);
-    for (void* p : {(void*)b->split, (void*)b->notFit, (void*)b->img, (void*)b->imgB, (void*)b->codes, (void*)b->imgU8, (void*)b->denom, (void*)b->imgBase, (void*)b->blkImg, (void*)b->nImgD,
+    for (void* p : {(void*)b->split, (void*)b->q8, (void*)b->res, (void*)b->sieveBest, (void*)b->sieveSecond,
+                    (void*)b->sieveItems, (void*)b->notFit, (void*)b->img, (void*)b->imgB, (void*)b->codes, (void*)b->imgU8, (void*)b->denom, (void*)b->imgBase, (void*)b->blkImg, (void*)b->nImgD,
                     (void*)b->srcRow, (void*)b->norm, (void*)b->maxNorm, b->upload, (void*)b->segOfBlock,
                     (void*)b->items[0], (void*)b->items[1], (void*)b->items[2], (void*)b->items[3],
                     (void*)b->segD[0], (void*)b->segD[1], (void*)b->segD[2], (void*)b->segD[3], (void*)b->blkInfo[0],
@@ -1037,7 +1133,7 @@ int v3dm_batch_set_pairs(v3dm_handle h, int nPairs, const int32_t* left, const i
         if (left[p] < 0 || left[p] >= b->nImages || right[p] < 0 || right[p] >= b->nImages)
             return ctx_fail(h, V3DM_ERR_INVALID, "pair refers to an image outside the batch");
     drop_graphs(b);
-    b->planValid[0] = b->planValid[1] = b->planValid[2] = b->planValid[3] = false;
+    b->planValid[0] = b->planValid[1] = b->planValid[2] = b->planValid[3] = b->sieveValid = false;
     b->pending = false;
     b->nPairs = nPairs;
     b->pa.assign(left, left + nPairs);
@@ -1134,9 +1230,18 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
         if (b->codesScale != learned_code_scale(L)) b->codesValid = false;
         b->codesScale = learned_code_scale(L);
     }
-    if ((form == 0 || (form == 2 && h->fallbackSamples > 0)) && (rc = ensure_split(h, b))) return rc;
+    bool const plain = form == 0 || (form == 2 && h->fallbackSamples > 0);
+    float T = 0.0f;
+    bool const sieve = plain && sieve_run(h, b, minScore, minRatio, &T);
+    bool const split = plain && (!sieve || (form == 0 && !b->planValid[0]));  // (the tuner times the full pass)
+    if (sieve && (rc = ensure_sieve(h, b))) return rc;
+    if (split && (rc = ensure_split(h, b))) return rc;
     // derived copies outside the run when they are cached (else every run derives them)
-    if (h->cacheDerived && form == 0 && !b->splitValid) {
+    if (h->cacheDerived && form == 0 && sieve && !b->q8Valid) {
+        launch_batch_sieve_rows(dev_view(b, 0), b->imgRows, b->q8, b->res, st);
+        b->q8Valid = true;
+    }
+    if (h->cacheDerived && form == 0 && split && !b->splitValid) {
         enqueue_derived(h, b, 0);
         b->splitValid = true;
     }
@@ -1149,7 +1254,7 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
         b->codesValid = true;
     }
     if (!h->cacheDerived && !b->planValid[form]) enqueue_derived(h, b, form);  // for the tuner
-    if (!h->cacheDerived) b->splitValid = false;  // a learned run rewrites the rows of its failing pairs
+    if (!h->cacheDerived) b->splitValid = b->q8Valid = false;  // a learned run rewrites rows of its failing pairs
     if ((rc = ensure_plan(h, b, form))) return rc;
     if (form == 2 && h->fallbackSamples > 0 && (rc = ensure_fallback_plan(h, b))) return rc;
     BCHECK(h, hipEventRecord(b->evA, st));
@@ -1157,7 +1262,7 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
         BatchState::GraphKey const key{mode, minScore, minRatio, h->epsRel, b->version * 2 + (h->cacheDerived ? 1 : 0),
                                        h->learnedTopK, form == 2 ? learned_margin(h) : 0.0f,
                                        form == 2 ? h->fallbackSamples : 0, form == 2 ? h->fallbackRecall : 0.0f,
-                                       form == 2 && b->splitValid};
+                                       form == 2 && (sieve ? b->q8Valid : b->splitValid)};
         auto it = b->graphs.find(key);
         if (it == b->graphs.end()) {
             hipGraph_t g = nullptr;
@@ -1190,6 +1295,8 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
     b->lastMinRatio = minRatio;
     b->pending = true;
     b->lastMode = mode;
+    b->lastSieve = form == 0 && sieve;
+    b->lastT = T;
     return V3DM_OK;
 }
 
@@ -1263,11 +1370,17 @@ int v3dm_batch_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
     if (e == hipSuccess) e = hipEventRecord(b->evA, st);
     for (int r = 0; r < reps && e == hipSuccess; ++r) {
         int const n = (int)pl.items.size();
-        if (form == 0) launch_plain_pass(b, 0, b->items[0], n, q + r, b->lastMinScore, st);
+        if (form == 0 && b->lastSieve)
+            launch_batch_sieve(d, b->sieveItems, b->nSieveItems, b->lastT, b->sieveBest, b->sieveSecond, nullptr, st);
+        else if (form == 0) launch_plain_pass(b, 0, b->items[0], n, q + r, b->lastMinScore, st);
         else if (form == 1) launch_batch_pass_bf16(d, b->items[1], n, q + r, b->partB, pl.grid, pl.qRows, st);
         else launch_batch_pass_code(d, b->items[2], n, q + r, b->partB, pl.grid, pl.qRows, st);
     }
     if (e == hipSuccess) e = hipEventRecord(b->evB, st);
+    if (form == 0 && b->lastSieve) {  // no decisions follow that would leave the entries at zero
+        if (e == hipSuccess) e = hipMemsetAsync(b->sieveBest, 0, b->sieveCap * sizeof(unsigned long long), st);
+        if (e == hipSuccess) e = hipMemsetAsync(b->sieveSecond, 0, b->sieveCap * sizeof(unsigned), st);
+    }
     if (e == hipSuccess) e = hipEventSynchronize(b->evB);
     float ms = 0.0f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, b->evA, b->evB);

@@ -75,6 +75,8 @@ struct BatchDev {
     uint8_t const* u8;            // uint8 rows (images uploaded as uint8) or null
     float const* denom;           // their scales: element k = (float)u8[k] * denom
     unsigned char const* split;   // split rows of the images, or the uint8 components in FP16 (v3dm_split.h)
+    signed char const* q8;        // the sieve's rows and residuals (v3dm_sieve.h)
+    float const* res;
     int const* imgBase;
     float const* norm;            // per image row
     unsigned int const* maxNorm;  // per image (float bits)
@@ -174,5 +176,15 @@ void launch_batch_fb_filter(int4 const* items, int nItems, int const* pairFlag, 
                             int* fbCount, int* segMask, hipStream_t st);
 void launch_batch_mutual(BatchDev const& b, int const* sel, int leftRows, int2* tmp, int* blockCount, int2* pairs,
                          int* pairCount, int* stripes, int* counters, hipStream_t st);
+
+// The sieve over a batch (v3dm_sieve.hip): rows, score pass and decisions; best / second: one
+// entry per query row, zero before a pass and after the decisions.
+void launch_batch_sieve_rows(BatchDev const& b, int rows, signed char* q8, float* res, hipStream_t st);
+void launch_batch_sieve_masked(BatchDev const& b, int const* segMask, signed char* q8, float* res, hipStream_t st);
+void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
+                        unsigned* second, int const* pairFlag, hipStream_t st);
+void launch_batch_sieve_decide(BatchDev const& b, unsigned long long* best, unsigned* second, float minScore,
+                               float minRatio, int* sel, int* flagList, int* counters, int const* segMask,
+                               hipStream_t st);
 
 }  // namespace v3dm

@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "v3dm_batch.h"
 #include "v3dm_device.h"
 #include "v3dm_sieve.h"
 
@@ -32,11 +33,11 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // L2 (the four waves of a group take the same tiles), two tiles ahead; there is no LDS staging
 // and no barrier.  Per block the 16 scores of a lane are reduced by 8 max3 and compared with
 // the lane's bound; only a block with a score above it looks at single scores and lists them
-// (LDS, kSieveList per wave).  After its last tile the wave scores its list exactly, a pair per
-// lane, and enters each score for both features: an atomic maximum of (score, ~index) returns the
-// smaller of two keys, which goes to the second best's maximum; so every key but the largest
-// reaches it, and equal scores keep the smallest index.  A wave whose list overflows marks all
-// its features for the exact re-check instead.
+// (LDS, kSieveList per wave; sets hold less than 2^24 rows).  After its last tile the wave
+// scores its list exactly, a pair per lane, and enters each score for both features: an atomic
+// maximum of (score, ~index) returns the smaller of two keys, which goes to the second best's
+// maximum; so every key but the largest reaches it, and equal scores keep the smallest index.
+// A wave whose list overflows marks all its features for the exact re-check instead.
 //
 // What bounds it: the int8 matrix instructions (16384 x 16384: 2^20 of them, 20 us of the 37),
 // then the tail, where each wave waits for the rows and the atomics of its few candidates
@@ -95,28 +96,19 @@ __device__ __forceinline__ void sieve_enter(unsigned long long* best, unsigned* 
     if (loser) atomicMax(second, loser);
 }
 
-__global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SievePlan p,
-                                                  unsigned const* __restrict__ maxNormBits, float T, SieveBest out,
-                                                  unsigned const* __restrict__ bits, int ldi)
+// One wave: left features [i0, i0 + 128) against right tiles [t0, t1).  ML, MR: the sets' largest
+// norms; bestL / secondL, bestR / secondR: the features' entries.
+__device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R, int i0, int t0, int t1, float ML,
+                                           float MR, float T, unsigned long long* __restrict__ bestL,
+                                           unsigned* __restrict__ secondL, unsigned long long* __restrict__ bestR,
+                                           unsigned* __restrict__ secondR, unsigned const* __restrict__ bits, int ldi,
+                                           int* list, int lane)
 {
-    __shared__ int lists[4][kSieveList];
-    int const lane = threadIdx.x & 63;
-    int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int const h = lane >> 5;
     int const c32 = lane & 31;
-    int* const list = lists[wv];
-    // neighbouring work-groups of one XCD share a split's right tiles in its L2
-    int const b = xcd_block(blockIdx.x, gridDim.x);
-    int const split = b / p.groups;
-    int const i0 = ((b - split * p.groups) * 4 + wv) * (32 * kSieveBlocks);
-    if (i0 >= L.n) return;  // the waves of a group share nothing
-    int const t0 = split * p.tiles;
-    int const t1 = min(t0 + p.tiles, R.n / kSieveTile);
-    float const ML = __uint_as_float(maxNormBits[0]), MR = __uint_as_float(maxNormBits[1]);
-
     // blocks past L.n (a multiple of 32) repeat the last one with a bound that nothing exceeds
     v4i B[kSieveBlocks][4];
-    float base[kSieveBlocks], arm[kSieveBlocks];
+    float base[kSieveBlocks], arm = ML;
 #pragma unroll
     for (int cb = 0; cb < kSieveBlocks; ++cb) {
         int const blk = min(i0 / 32 + cb, L.n / 32 - 1);
@@ -125,8 +117,9 @@ __global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SieveP
         bool const exists = i0 + 32 * cb < L.n;
         // score units * 65536; the 2 covers the roundings here and below
         base[cb] = exists ? (T - r * MR) * 65536.0f - 2.0f : INFINITY;
-        arm[cb] = (ML + r) * 65536.0f;
+        arm = fmaxf(arm, ML + r);
     }
+    arm *= 65536.0f;
     int cnt = 0;  // uniform
     auto tile = [&](v4i(&a)[4], int t) {
         float const* const rt = R.res + t * (kSieveTile / kSieveGroup);
@@ -144,8 +137,9 @@ __global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SieveP
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 int const cb = c0 + k;
-                float const thr = fmaf(-arm[cb], r, base[cb]);
+                float const thr = fmaf(-arm, r, base[cb]);
                 if (__builtin_expect(__builtin_amdgcn_ballot_w64((float)max16(acc[k]) > thr) == 0, 1)) continue;
+                int const entry = ((cb * 32 + c32) << 24) | (t * kSieveTile) | (h << 4);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     bool const hit = (float)acc[k][e] > thr;
@@ -153,8 +147,7 @@ __global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SieveP
                     if (m == 0) continue;
                     int const at = cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                                    __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-                    int const j = t * kSieveTile + 8 * (e >> 2) + 4 * h + (e & 3);
-                    if (hit && at < kSieveList) list[at] = ((cb * 32 + c32) << 20) | j;
+                    if (hit && at < kSieveList) list[at] = entry | e;
                     cnt += __builtin_popcountll(m);
                 }
             }
@@ -173,22 +166,72 @@ __global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SieveP
         if (t < t1) tile(a0, t);
     }
     if (cnt > kSieveList) {
-        for (int i = lane; i < min(32 * kSieveBlocks, L.n - i0); i += 64) atomicMax(out.best + i0 + i, kSieveFlood);
-        for (int j = t0 * kSieveTile + lane; j < t1 * kSieveTile; j += 64)
-            atomicMax(out.best + out.offR + j, kSieveFlood);
+        for (int i = lane; i < min(32 * kSieveBlocks, L.n - i0); i += 64) atomicMax(bestL + i0 + i, kSieveFlood);
+        for (int j = t0 * kSieveTile + lane; j < t1 * kSieveTile; j += 64) atomicMax(bestR + j, kSieveFlood);
         return;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // LDS operations of one wave are in order
     for (int c = lane; c < cnt; c += 64) {
+        // accumulator element r of lane half h: row 8 (r / 4) + 4 h + r % 4 of the tile
         int const e = list[c];
-        int const i = i0 + (e >> 20), j = e & 0xfffff;
+        int const i = i0 + (e >> 24), j = (e & 0xffffe0) + 8 * ((e >> 2) & 3) + 4 * ((e >> 4) & 1) + (e & 3);
         if (bits && ((bits[(size_t)(j >> 5) * ldi + i] >> (j & 31)) & 1u)) continue;  // a removed pair
         float const s = sieve_exact(L.X + (size_t)i * kDim, R.X + (size_t)j * kDim);
         if (!(s > 0.0f)) continue;  // T > 0: cannot matter
         unsigned long long const v = (unsigned long long)__float_as_uint(s) << 32;
-        sieve_enter(out.best + i, out.second + i, v | (0xffffffffu - (unsigned)j));
-        sieve_enter(out.best + out.offR + j, out.second + out.offR + j, v | (0xffffffffu - (unsigned)i));
+        sieve_enter(bestL + i, secondL + i, v | (0xffffffffu - (unsigned)j));
+        sieve_enter(bestR + j, secondR + j, v | (0xffffffffu - (unsigned)i));
     }
+}
+
+__global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SievePlan p,
+                                                  unsigned const* __restrict__ maxNormBits, float T, SieveBest out,
+                                                  unsigned const* __restrict__ bits, int ldi)
+{
+    __shared__ int lists[4][kSieveList];
+    int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    // neighbouring work-groups of one XCD share a split's right tiles in its L2
+    int const b = xcd_block(blockIdx.x, gridDim.x);
+    int const split = b / p.groups;
+    int const i0 = ((b - split * p.groups) * 4 + wv) * (32 * kSieveBlocks);
+    if (i0 >= L.n) return;  // the waves of a group share nothing
+    int const t0 = split * p.tiles;
+    sieve_wave(L, R, i0, t0, min(t0 + p.tiles, R.n / kSieveTile), __uint_as_float(maxNormBits[0]),
+               __uint_as_float(maxNormBits[1]), T, out.best, out.second, out.best + out.offR, out.second + out.offR,
+               bits, ldi, lists[wv], threadIdx.x & 63);
+}
+
+// Over a batch: item = (pair, group of 512 left features, split, tiles per split), one
+// work-group each.  pairFlag: only the flagged pairs (a learned run's fallback), or null.
+// 256 uneven uint8 pairs: 531 us (2.9 TB/s would read the rows, 3.4 POPS of int8 products) + 13 for
+// the decisions, against 2358 + 167 + 23 of the integer-row pass, its merge and its re-check.
+__global__ __launch_bounds__(256, 3) void k_batch_sieve(BatchDev b, int4 const* __restrict__ items, float T,
+                                                        unsigned long long* __restrict__ best,
+                                                        unsigned* __restrict__ second,
+                                                        int const* __restrict__ pairFlag)
+{
+    __shared__ int lists[4][kSieveList];
+    int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int4 const w = items[blockIdx.x];
+    if (pairFlag && !pairFlag[w.x]) return;
+    BatchSeg const sl = b.seg[w.x];
+    BatchSeg const sr = b.seg[b.nPairs + w.x];
+    int const i0 = (w.y * 4 + wv) * (32 * kSieveBlocks);
+    if (i0 >= sl.n) return;
+    size_t const l0 = b.imgBase[sl.img], r0 = b.imgBase[sr.img];
+    SieveSet const L{b.q8 + l0 * kDim, b.res + l0 / kSieveGroup, b.img + l0 * kDim, sl.n};
+    SieveSet const R{b.q8 + r0 * kDim, b.res + r0 / kSieveGroup, b.img + r0 * kDim, sr.n};
+    int const t0 = w.z * w.w;
+    sieve_wave(L, R, i0, t0, min(t0 + w.w, sr.n / kSieveTile), __uint_as_float(b.maxNorm[sl.img]),
+               __uint_as_float(b.maxNorm[sr.img]), T, best + sl.qOff, second + sl.qOff, best + sr.qOff,
+               second + sr.qOff, nullptr, 0, lists[wv], threadIdx.x & 63);
+}
+
+void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
+                        unsigned* second, int const* pairFlag, hipStream_t st)
+{
+    if (nItems <= 0) return;
+    hipLaunchKernelGGL(k_batch_sieve, dim3(nItems), dim3(256), 0, st, b, items, T, best, second, pairFlag);
 }
 
 // Splits of the right features: three work-groups of four waves per CU run at a time, and a
@@ -220,6 +263,20 @@ void launch_sieve(SieveSet const& L, SieveSet const& R, SievePlan const& p, unsi
 }
 
 // ------------------------------------------------------------------------------ decisions
+__device__ __forceinline__ int sieve_decision(unsigned long long* best, unsigned* second, float minScore,
+                                              float minRatio)
+{
+    unsigned long long const k = *best;
+    unsigned const s2 = *second;
+    if (k) *best = 0;
+    if (s2) *second = 0;
+    if (k == kSieveFlood) return kFlag;
+    if (!k) return -1;
+    Top2 const s{__uint_as_float((unsigned)(k >> 32)), s2 ? __uint_as_float(s2) : kInit,
+                 (int)(0xffffffffu - (unsigned)k)};
+    return decide_exact(s, minScore, minRatio);
+}
+
 __global__ __launch_bounds__(256) void k_sieve_decide(SieveBest b, int nL, int nR, float minScore, float minRatio,
                                                       int* __restrict__ colMax, int* __restrict__ rowMax,
                                                       int* __restrict__ flagList, int flagOffR,
@@ -230,20 +287,11 @@ __global__ __launch_bounds__(256) void k_sieve_decide(SieveBest b, int nL, int n
     bool const left = g < nL;
     int const q = left ? g : g - nL;
     int const at = left ? q : b.offR + q;
-    unsigned long long const k = b.best[at];
-    unsigned const s2 = b.second[at];
-    int d = -1;
-    if (k == kSieveFlood) {
+    int const d = sieve_decision(b.best + at, b.second + at, minScore, minRatio);
+    if (d == kFlag) {
         int const slot = atomicAdd(&counters[left ? kCntFlag : kCntFlagR], 1);
         flagList[left ? slot : flagOffR + slot] = q;
-        d = kFlag;
-    } else if (k) {
-        Top2 const s{__uint_as_float((unsigned)(k >> 32)), s2 ? __uint_as_float(s2) : kInit,
-                     (int)(0xffffffffu - (unsigned)k)};
-        d = decide_exact(s, minScore, minRatio);
     }
-    if (k) b.best[at] = 0;
-    if (s2) b.second[at] = 0;
     (left ? colMax : rowMax)[q] = d;
 }
 
@@ -253,6 +301,114 @@ void launch_sieve_decide(SieveBest const& b, int nL, int nR, float minScore, flo
     if (nL + nR <= 0) return;
     hipLaunchKernelGGL(k_sieve_decide, dim3((nL + nR + 255) / 256), dim3(256), 0, st, b, nL, nR, minScore, minRatio,
                        colMax, rowMax, flagList, flagOffR, counters);
+}
+
+__global__ __launch_bounds__(256) void k_batch_sieve_decide(BatchDev b, unsigned long long* __restrict__ best,
+                                                            unsigned* __restrict__ second, float minScore,
+                                                            float minRatio, int* __restrict__ sel,
+                                                            int* __restrict__ flagList, int* __restrict__ counters,
+                                                            int const* __restrict__ segMask)
+{
+    int const si = b.segOfBlock[blockIdx.x];  // 256 queries of one segment
+    if (segMask && !segMask[si]) return;
+    int const g = blockIdx.x * kBatchRowAlign + threadIdx.x;
+    int const d = sieve_decision(best + g, second + g, minScore, minRatio);
+    if (d == kFlag) flagList[atomicAdd(&counters[kBCntFlag], 1)] = g;
+    sel[g] = d;
+}
+
+void launch_batch_sieve_decide(BatchDev const& b, unsigned long long* best, unsigned* second, float minScore,
+                               float minRatio, int* sel, int* flagList, int* counters, int const* segMask,
+                               hipStream_t st)
+{
+    static_assert(kBatchRowAlign == 256, "a work-group per query block");
+    if (b.qRows <= 0) return;
+    hipLaunchKernelGGL(k_batch_sieve_decide, dim3(b.qRows / kBatchRowAlign), dim3(256), 0, st, b, best, second,
+                       minScore, minRatio, sel, flagList, counters, segMask);
+}
+
+// ------------------------------------------------------------------------------ rows of a batch
+// The int8 tiles and residuals (as the single pair's, v3dm_select.hip): 8 rows per wave, lane =
+// 8 * (16 components) + row, so that a store is 8 runs of 128 bytes.  What bounds it: the rows
+// (128 bytes in, 128 out) and some 150 vector instructions per 8 rows: 108 us for 2.4 * 10^6 rows of
+// uint8 (139 for the FP16 integers of the full pass).
+template <bool kU8>
+__device__ __forceinline__ void sieve_rows8(BatchDev const& b, size_t row0, signed char* __restrict__ q8,
+                                            float* __restrict__ res)
+{
+    int const lane = threadIdx.x & 63;
+    int const c = lane >> 3;
+    size_t const row = row0 + (lane & 7);
+    float x[16];
+    if (kU8) {
+        uint4 const w = reinterpret_cast<uint4 const*>(b.u8 + row * kDim)[c];
+        float const d = b.denom[row];
+        unsigned const u[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = dequant_u8_value((unsigned char)(u[k >> 2] >> (8 * (k & 3))), d);
+    } else {
+        float4 const* const p = reinterpret_cast<float4 const*>(b.img + row * kDim) + 4 * c;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float4 const v = p[k];
+            x[4 * k] = v.x, x[4 * k + 1] = v.y, x[4 * k + 2] = v.z, x[4 * k + 3] = v.w;
+        }
+    }
+    unsigned o[4] = {0, 0, 0, 0};
+    float r2 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        float const q = fminf(fmaxf(rintf(x[k] * kSieveScale), -127.0f), 127.0f);
+        float const e = x[k] - q * (1.0f / kSieveScale);
+        r2 += e * e;
+        o[k >> 2] |= ((unsigned)(int)q & 0xffu) << (8 * (k & 3));
+    }
+    *reinterpret_cast<uint4*>(q8 + (row / kSieveTile) * kSieveTileBytes + c * 512 + (row % kSieveTile) * 16) =
+        make_uint4(o[0], o[1], o[2], o[3]);
+    r2 += __shfl_xor(r2, 8);
+    r2 += __shfl_xor(r2, 16);
+    r2 += __shfl_xor(r2, 32);
+    r2 = fmaxf(r2, __shfl_xor(r2, 1));
+    r2 = fmaxf(r2, __shfl_xor(r2, 2));
+    r2 = fmaxf(r2, __shfl_xor(r2, 4));
+    if (lane == 0) res[row0 / kSieveGroup] = sqrtf(r2) * 1.001f + 1e-6f;
+}
+
+template <bool kU8>
+__global__ __launch_bounds__(256) void k_batch_sieve_rows(BatchDev b, signed char* __restrict__ q8,
+                                                          float* __restrict__ res)
+{
+    sieve_rows8<kU8>(b, ((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 8, q8, res);
+}
+
+// The rows of the flagged segments' images (a learned run's fallback).
+template <bool kU8>
+__global__ __launch_bounds__(256) void k_batch_sieve_masked(BatchDev b, int const* __restrict__ segMask,
+                                                            signed char* __restrict__ q8, float* __restrict__ res)
+{
+    int const si = b.segOfBlock[blockIdx.x];
+    if (!segMask[si]) return;
+    BatchSeg const sg = b.seg[si];
+    int const q0 = blockIdx.x * kBatchRowAlign - sg.qOff;
+    size_t const row0 = (size_t)b.imgBase[sg.img] + q0;
+    for (int r = 8 * (threadIdx.x >> 6); r < kBatchRowAlign && q0 + r < sg.n; r += 32)
+        sieve_rows8<kU8>(b, row0 + r, q8, res);
+}
+
+void launch_batch_sieve_rows(BatchDev const& b, int rows, signed char* q8, float* res, hipStream_t st)
+{
+    if (rows <= 0) return;
+    dim3 const g(rows / 32);  // images are padded to 256 rows
+    if (b.u8) hipLaunchKernelGGL(k_batch_sieve_rows<true>, g, dim3(256), 0, st, b, q8, res);
+    else hipLaunchKernelGGL(k_batch_sieve_rows<false>, g, dim3(256), 0, st, b, q8, res);
+}
+
+void launch_batch_sieve_masked(BatchDev const& b, int const* segMask, signed char* q8, float* res, hipStream_t st)
+{
+    if (b.qRows <= 0) return;
+    dim3 const g(b.qRows / kBatchRowAlign);
+    if (b.u8) hipLaunchKernelGGL(k_batch_sieve_masked<true>, g, dim3(256), 0, st, b, segMask, q8, res);
+    else hipLaunchKernelGGL(k_batch_sieve_masked<false>, g, dim3(256), 0, st, b, segMask, q8, res);
 }
 
 }  // namespace v3dm

@@ -93,3 +93,30 @@ def test_timing_leaves_no_state(matcher):
     _same(matcher, L, R, 0.9, 0.8)
     assert matcher.time_dominant_kernel(3) > 0
     _same(matcher, L, R, 0.9, 0.8)
+
+
+SIZES = [(33, 70), (512, 31), (256, 256), (300, 1700), (1056, 96), (32, 32), (640, 513), (513, 2080)]
+
+
+@pytest.mark.parametrize("dtype", ["u8", "f32"])
+@pytest.mark.parametrize("cache", [False, True])
+def test_batch(dtype, cache):
+    """Uneven pairs, with minimum scores that take the sieve and one that does not, in turn on
+    one batch (runs, graph replays, and rows made by every run or kept)."""
+    images = []
+    for p, (nL, nR) in enumerate(SIZES):
+        images += list(synth.make_pair(nL, nR, 0.5, config=3, pair=700 + p)[:2])
+    left = np.arange(0, 2 * len(SIZES), 2, dtype=np.int32)
+    rows = np.concatenate(images if dtype == "u8" else [synth.dequantise(q) for q in images])
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([len(q) for q in images], rows)
+    m.batch_set_pairs(left, left + 1)
+    m.set_derived_cache(cache)
+    for ms, mr in ((0.9, 0.8), (0.2, 0.8), (0.85, -1.0), (0.9, 0.8), (0.2, 0.8)):
+        print(f"case sieve batch {dtype} cache {cache} min {ms} ratio {mr}", flush=True)
+        got = m.batch_match(ms, mr)
+        for p in range(len(SIZES)):
+            L, R = (synth.dequantise(images[2 * p + k][:len(images[2 * p + k]) // 32 * 32]) for k in (0, 1))
+            want = oracle.find_putative_matches(L, R, ms, mr) if len(L) and len(R) else np.zeros((0, 2), np.int32)
+            assert np.array_equal(np.asarray(got[p]).reshape(-1, 2), want.reshape(-1, 2)), (p, ms, mr)
+    m.close()
