@@ -81,7 +81,6 @@ void releaseBuffers(v3dm_context* h)
     freeDev(h->intScaleL);
     freeDev(h->intScaleR);
     h->haveIntL = h->haveIntR = false;
-    freeDev(h->splitInfo);
     if (h->splitFitHost) (void)hipHostFree(h->splitFitHost);
     h->splitFitHost = h->splitFitDev = nullptr;
     freeDev(h->maxNormBits);
@@ -180,9 +179,19 @@ FusedPlan score_plan(v3dm_context const* h)
     return split_fits(h) ? plan_split(h->nL, h->nR) : plan_fused_fp32(h->nL, h->nR, 512);
 }
 
+// The rows of the split pass, made once for the current sets.
+void ensure_split_rows(v3dm_context* h)
+{
+    if (h->haveSplit) return;
+    launch_split_sets(SplitRowsOf{h->dL, h->intScaleL, h->splitL, h->haveIntL ? h->intL : nullptr, h->nL},
+                      SplitRowsOf{h->dR, h->intScaleR, h->splitR, h->haveIntR ? h->intR : nullptr, h->nR}, h->stream);
+    h->haveSplit = true;
+}
+
 void launch_score_pass(v3dm_context* h, FusedPlan const& p, unsigned const* bits, float minScore)
 {
     hipStream_t const st = h->stream;
+    if (split_fits(h)) ensure_split_rows(h);
     if (split_fits(h))
         launch_split_pass(SplitSet{h->splitL, h->haveIntL ? h->intL : nullptr, h->intScaleL, h->nL},
                           SplitSet{h->splitR, h->haveIntR ? h->intR : nullptr, h->intScaleR, h->nR}, p, h->colPart,
@@ -334,8 +343,6 @@ int v3dm_allocate(v3dm_handle h, int nMaxLeft, int nMaxRight, int useGuidedMatch
     HIPCHECK(h, hipMalloc(&h->sieveSecond, (cl + cr) * sizeof(unsigned)));
     HIPCHECK(h, hipMemsetAsync(h->sieveBest, 0, (cl + cr) * sizeof(unsigned long long), h->stream));
     HIPCHECK(h, hipMemsetAsync(h->sieveSecond, 0, (cl + cr) * sizeof(unsigned), h->stream));
-    HIPCHECK(h, hipMalloc(&h->splitInfo, kPrepInfo * sizeof(int)));
-    HIPCHECK(h, hipMemsetAsync(h->splitInfo, 0, kPrepInfo * sizeof(int), h->stream));
     HIPCHECK(h, hipHostMalloc(&h->splitFitHost, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     HIPCHECK(h, hipHostGetDevicePointer((void**)&h->splitFitDev, h->splitFitHost, 0));
     h->splitFitHost[0] = h->splitFitHost[1] = 0;
@@ -440,11 +447,16 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
             from = kRowsU8;
         }
     }
-    launch_split_rows(from, from == kRowsU8 ? (void const*)h->dQ : src, dst, n, left ? h->normL : h->normR,
-                      h->maxNormBits + (left ? 0 : 1), left ? h->splitL : h->splitR,
-                      left ? h->intL : h->intR, left ? h->intScaleL : h->intScaleR,
-                      left ? h->q8L : h->q8R, left ? h->resL : h->resR, h->splitInfo,
-                      h->splitFitDev + (left ? 0 : 1), h->stream);
+    if (++h->prepEpoch == 0) {
+        HIPCHECK(h, hipMemsetAsync(h->maxNormBits, 0, 4 * sizeof(unsigned int), h->stream));
+        h->prepEpoch = 1;
+    }
+    // the previous call's launch has ended (every call waits for its own)
+    if (n > 0) __atomic_store_n(h->splitFitHost + (left ? 0 : 1), 1, __ATOMIC_RELEASE);
+    launch_prep_rows(from, from == kRowsU8 ? (void const*)h->dQ : src, dst, n, left ? h->normL : h->normR,
+                     h->maxNormBits + (left ? 0 : kMaxNormR), h->prepEpoch, left ? h->intScaleL : h->intScaleR,
+                     left ? h->q8L : h->q8R, left ? h->resL : h->resR, h->splitFitDev + (left ? 0 : 1), h->stream);
+    h->haveSplit = false;
     (left ? h->haveIntL : h->haveIntR) = from == kRowsU8;
     HIPCHECK(h, hipGetLastError());
     HIPCHECK(h, hipStreamSynchronize(h->stream));
@@ -784,10 +796,12 @@ int v3dm_score_block(v3dm_handle h, int mode, int nRows, int nCols, float* score
     float* d = nullptr;
     size_t const bytes = (size_t)nRows * nCols * sizeof(float);
     HIPCHECK(h, hipMalloc(&d, bytes));
-    if (mode == V3DM_PREC_FP32 && split_fits(h))
+    if (mode == V3DM_PREC_FP32 && split_fits(h)) {
+        ensure_split_rows(h);
         launch_score_block_split(h->splitL, h->splitR, nRows, nCols, d, h->stream);
-    else
+    } else {
         launch_score_block(mode, h->dL, h->dR, nRows, nCols, d, h->stream);
+    }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipMemcpyAsync(scores, d, bytes, hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);

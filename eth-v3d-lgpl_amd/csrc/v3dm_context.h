@@ -37,21 +37,22 @@ struct v3dm_context {
     float* dR = nullptr;
     float* normL = nullptr;
     float* normR = nullptr;
-    unsigned char* splitL = nullptr;  // rows in two FP16 parts (v3dm_split.h), written with the norms
+    unsigned char* splitL = nullptr;  // rows in two FP16 parts (v3dm_split.h), made by the first full pass
     unsigned char* splitR = nullptr;
     unsigned char* intL = nullptr;    // uint8 sets: the components as FP16 integers ...
     unsigned char* intR = nullptr;
     float* intScaleL = nullptr;       // ... and the rows' scales (allocated by the first uint8 upload)
     float* intScaleR = nullptr;
     bool haveIntL = false, haveIntR = false;  // the current set has them
+    bool haveSplit = false;           // the split and integer rows of the current sets are made
     signed char *q8L = nullptr, *q8R = nullptr;   // the sieve's rows and residuals
     float *resL = nullptr, *resR = nullptr;
     unsigned long long* sieveBest = nullptr;      // of capL left, then capR right features
     unsigned* sieveSecond = nullptr;
-    int* splitInfo = nullptr;         // scratch of launch_split_rows
     int* splitFitHost = nullptr;      // mapped: [0] left, [1] right set in the split pass's range
     int* splitFitDev = nullptr;       // the same memory as the kernels address it
-    unsigned int* maxNormBits = nullptr;  // [0] = left, [1] = right
+    unsigned int* maxNormBits = nullptr;  // [0] = left, [kMaxNormR] = right, with epochs above
+    unsigned prepEpoch = 0;               // of the last launch_prep_rows
     v3dm::Top2* colPart = nullptr;
     v3dm::Top2* rowPart = nullptr;
     int* colMax = nullptr;

@@ -124,12 +124,14 @@ __device__ __forceinline__ float sub_nc(float a, float b)
 // as SIFT_Feature::normalizeDescriptor (V3D/Base/v3d_feature.h:30-38): the sum of squares
 // of integers <= 255 over 128 terms stays below 2^24, so it is exact in FP32 in any order,
 // and the scale is 1/sqrt with IEEE rounding.
+__device__ __forceinline__ float dequant_u8_scale(float s) { return __fdiv_rn(1.0f, __fsqrt_rn(s)); }
+
 __device__ __forceinline__ float dequant_u8_denom(uchar2 v)
 {
     float const a = (float)v.x, b = (float)v.y;
     float s = a * a + b * b;
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    return __fdiv_rn(1.0f, __fsqrt_rn(s));
+    return dequant_u8_scale(s);
 }
 
 // element value: the IEEE product (float)q * denom, the same in every kernel that forms it

@@ -31,6 +31,9 @@ constexpr int kRecheckGrid = 1024;
 // sum|q_k c_k| <= ||q|| ||c||; epsRel = 2^-15 leaves a factor 2 on top.  epsRel <= 0
 // sends every query to the exact re-check.
 constexpr float kEpsRelFp32 = 3.0517578125e-05f;  // 2^-15
+// The largest norms of a pair: float bits of the left set at [0], of the right at [kMaxNormR] (an
+// odd word above each is the epoch of launch_prep_rows).
+constexpr int kMaxNormR = 2;
 constexpr float kEpsAbs = 1e-30f;
 
 struct FusedPlan {
@@ -97,7 +100,7 @@ void launch_score_block(int mode, float const* L, float const* R, int nRows, int
 // (also zeroes the check's counters)
 void launch_sample_gather(float const* L, float const* normL, int nL, int S, float* Ls, float* normS, int* idx,
                           int* counters, hipStream_t st);
-// merge + certified decision of the S sampled rows (maxNormBits[1]: max right norm)
+// merge + certified decision of the S sampled rows (maxNormBits[kMaxNormR]: max right norm)
 void launch_sample_decide(Top2 const* colPart, int nParts, int ldc, int S, float const* normS,
                           unsigned int const* maxNormBits, float epsRel, float minScore, float minRatio, int* dec,
                           int* flagList, int* counters, hipStream_t st);

@@ -76,7 +76,7 @@ __global__ void k_noalloc_clear(int* __restrict__ counters, unsigned int* __rest
 {
     int const t = threadIdx.x;
     if (t < kNumCounters) counters[t] = 0;
-    if (t < 2) maxNorm[t] = 0u;
+    if (t <= kMaxNormR) maxNorm[t] = 0u;
 }
 
 // the match count, or -1 when the mutual check's ordering wait ran out (its epoch in
@@ -169,7 +169,7 @@ int v3dm_match_device_noalloc(const float* leftDesc, int nLeft, const float* rig
         hipLaunchKernelGGL(k_noalloc_copy_pad, dim3((capR * (kDim / 4) + 255) / 256), dim3(256), 0, st, rightDesc, nR,
                            capR, R);
         launch_norms(L, nL, normL, maxNorm + 0, st);
-        launch_norms(R, nR, normR, maxNorm + 1, st);
+        launch_norms(R, nR, normR, maxNorm + kMaxNormR, st);
         FusedPlan const p = plan_fused_fp32(nL, nR, 512);
         launch_fused_fp32(L, R, nL, nR, p, colPart, capL, rowPart, capR, st);
         launch_merge_decide(colPart, p.splits, capL, rowPart, p.leftBlocks, capR, nL, nR, normL, normR, maxNorm,

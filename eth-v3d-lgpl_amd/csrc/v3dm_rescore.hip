@@ -350,7 +350,7 @@ __global__ __launch_bounds__(256) void k_shortlist_finish(float const* __restric
         int const q = left ? g : g - nL;
         Top2x const s = finish_query<false>((left ? partL : partR) + (size_t)q * 2, 2 * (size_t)(left ? ldqL : ldqR),
                                             left ? nPartL : nPartR, left ? spanL : spanR, left ? normL[q] : normR[q],
-                                            __uint_as_float(maxNormBits[left ? 1 : 0]), winRel, topK, margin,
+                                            __uint_as_float(maxNormBits[left ? kMaxNormR : 0]), winRel, topK, margin,
                                             (left ? L : R) + (size_t)q * kDim, left ? R : L, nullptr, nullptr, sub,
                                             slots[threadIdx.x >> 3], qrow[threadIdx.x >> 3], n);
         if (sub == 0) {

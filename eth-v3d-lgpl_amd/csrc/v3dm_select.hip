@@ -48,30 +48,23 @@ void launch_norms(float const* X, int n, float* norm, unsigned int* maxNormBits,
 }
 
 // ------------------------------------------------------------------------------ row preparation
-// Per row: the FP32 row (from a device array, from uint8 components, or in place), its norm
-// (summed as k_norms does) and its split parts, in one launch: the set is read once, where a
-// copy or a dequantisation, a fill of the maximum and k_norms took three launches.  A wave
-// takes 8 rows at a time, all loads in flight before the first reduction (k_norms waits for
-// each row's load in its turn: 14 us for any set up to 16384 rows).  Every work-group leaves
-// its largest norm and range flag in a slot and takes a ticket; the last one publishes the
-// set's (at most kPrepGroups work-groups, so one thread each reads a slot).  The slots are
-// device-coherent stores waited for before the ticket, not fenced: a fence would write back
-// the XCD's whole L2 (22 us for 512 work-groups).
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+// Per row: the FP32 row (from a device array, from uint8 components, or in place), its norm and
+// its int8 row for the sieve, in one launch: the set is read once, where a copy or a
+// dequantisation, a fill of the maximum and k_norms took three launches.  A wave takes 8 rows at
+// a time, all loads in flight before the first reduction (k_norms waits for each row's load in
+// its turn: 14 us for any set up to 16384 rows), and reduces the 8 rows' sums together.  The
+// split rows of the full pass are made where that pass runs (k_split_sets).  The set's largest
+// norm is an atomic maximum under the call's epoch, so nothing is cleared and no work-group waits
+// for another; a row out of range clears the host's flag, which the host has set.
+//
+// What bounds it: latency (the loads, two reductions, the stores: 7 us for any small set); a set
+// of 32768 rows moves 38 MB in 12 us.  With the split rows made here and a ticket for the last
+// work-group, which published the maximum: 8 us for small sets, 18 for 32768 rows.
 constexpr int kPrepRows = 8;  // rows per wave and round
 
-__device__ __forceinline__ void split_pair(float2 v, unsigned& hi, unsigned& lo)
-{
-    float const x = v.x * kSplitScale, y = v.y * kSplitScale;
-    v2h const h = {(_Float16)x, (_Float16)y};
-    v2h const l = {(_Float16)(x - (float)h.x), (_Float16)(y - (float)h.y)};
-    hi = __builtin_bit_cast(unsigned, h);
-    lo = __builtin_bit_cast(unsigned, l);
-}
-
-// The sum of each of 8 values over the wave's lanes, the largest of them in every lane: the
-// first three steps halve the values a lane carries.
-__device__ __forceinline__ float max_of_sums(float (&s)[8], int lane)
+// The sums of 8 values over the wave's lanes: lane l gets the sum of value l / 8.  The first
+// three steps halve the values a lane carries (10 shuffles instead of 48).
+__device__ __forceinline__ float sums_of8(float (&s)[8], int lane)
 {
 #pragma unroll
     for (int n = 4, o = 32; n >= 1; n >>= 1, o >>= 1) {
@@ -85,78 +78,51 @@ __device__ __forceinline__ float max_of_sums(float (&s)[8], int lane)
     float x = s[0];
     x += __shfl_xor(x, 4);
     x += __shfl_xor(x, 2);
-    x += __shfl_xor(x, 1);
-    x = fmaxf(x, __shfl_xor(x, 32));
-    x = fmaxf(x, __shfl_xor(x, 16));
-    return fmaxf(x, __shfl_xor(x, 8));
+    return x + __shfl_xor(x, 1);
 }
 
-template <int kFrom>
-__global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src, float* __restrict__ X, int n,
-                                                    float* __restrict__ norm, unsigned int* __restrict__ maxNormBits,
-                                                    unsigned char* __restrict__ split,
-                                                    unsigned char* __restrict__ ints, float* __restrict__ scale,
-                                                    signed char* __restrict__ q8, float* __restrict__ res,
-                                                    int* __restrict__ info, int* __restrict__ hostFit)
+template <int kFrom, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) void k_prep_rows(void const* __restrict__ src, float* __restrict__ X, int n,
+                                                   float* __restrict__ norm, unsigned long long* __restrict__ maxNorm,
+                                                   unsigned epoch, float* __restrict__ scale,
+                                                   signed char* __restrict__ q8, float* __restrict__ res,
+                                                   int* __restrict__ hostFit)
 {
-    __shared__ unsigned int wmax[4];
-    __shared__ int wbad[4];
-    __shared__ int last;
+    __shared__ unsigned int wmax[kWaves];
     int const lane = threadIdx.x & 63;
     int const wave = threadIdx.x >> 6;
     unsigned int mx = 0;
-    bool bad = false;
-    for (int row0 = (blockIdx.x * 4 + wave) * kPrepRows; row0 < n; row0 += gridDim.x * 4 * kPrepRows) {
+    int bad = 0;
+    for (int row0 = (blockIdx.x * kWaves + wave) * kPrepRows; row0 < n;
+         row0 += gridDim.x * kWaves * kPrepRows) {
+        // n is a multiple of 32: no round is partial
         float2 v[kPrepRows];
         if constexpr (kFrom == kRowsU8) {
             uchar2 q[kPrepRows];
 #pragma unroll
-            for (int k = 0; k < kPrepRows; ++k)
-                q[k] = (row0 + k < n) ? static_cast<uchar2 const*>(src)[(size_t)(row0 + k) * 64 + lane]
-                                      : make_uchar2(0, 0);
+            for (int k = 0; k < kPrepRows; ++k) q[k] = static_cast<uchar2 const*>(src)[(size_t)(row0 + k) * 64 + lane];
+            // the sums of squares are exact in any order (dequant_u8_denom)
+            float s[kPrepRows];
+#pragma unroll
+            for (int k = 0; k < kPrepRows; ++k) s[k] = (float)q[k].x * (float)q[k].x + (float)q[k].y * (float)q[k].y;
+            float const mine = dequant_u8_scale(sums_of8(s, lane));
+            if ((lane & 7) == 0) scale[row0 + (lane >> 3)] = mine;
 #pragma unroll
             for (int k = 0; k < kPrepRows; ++k) {
-                float const d = dequant_u8_denom(q[k]);
-                v[k] = (row0 + k < n) ? make_float2(dequant_u8_value(q[k].x, d), dequant_u8_value(q[k].y, d))
-                                      : make_float2(0.0f, 0.0f);
-                if (row0 + k < n) {
-                    v2h const i = {(_Float16)(float)q[k].x, (_Float16)(float)q[k].y};
-                    reinterpret_cast<v2h*>(ints + (size_t)(row0 + k) * kIntRowBytes)[lane] = i;
-                    if (lane == 0) scale[row0 + k] = d;
-                }
+                float const d = __shfl(mine, 8 * k);
+                v[k] = make_float2(dequant_u8_value(q[k].x, d), dequant_u8_value(q[k].y, d));
             }
         } else {
             float2 const* const rows = kFrom == kRowsF32 ? static_cast<float2 const*>(src)
                                                          : reinterpret_cast<float2 const*>(X);
 #pragma unroll
-            for (int k = 0; k < kPrepRows; ++k)
-                v[k] = (row0 + k < n) ? rows[(size_t)(row0 + k) * 64 + lane] : make_float2(0.0f, 0.0f);
+            for (int k = 0; k < kPrepRows; ++k) v[k] = rows[(size_t)(row0 + k) * 64 + lane];
         }
-        float s[kPrepRows];
-#pragma unroll
-        for (int k = 0; k < kPrepRows; ++k) s[k] = v[k].x * v[k].x + v[k].y * v[k].y;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-            for (int k = 0; k < kPrepRows; ++k) s[k] += __shfl_xor(s[k], o);
+        float s[kPrepRows], e2[kPrepRows];
 #pragma unroll
         for (int k = 0; k < kPrepRows; ++k) {
-            float const nr = sqrtf(s[k]);
-            mx = max(mx, __float_as_uint(nr));  // norms are >= 0 or NaN: a NaN wins
-            bad = bad || !(nr == 0.0f || (nr >= kSplitNormMin && nr < kSplitNormMax));
-            if (row0 + k >= n) break;  // uniform over the wave; rows past n are zero above
-            if (lane == 0) norm[row0 + k] = nr;
+            s[k] = v[k].x * v[k].x + v[k].y * v[k].y;
             if (kFrom != kRowsInPlace) reinterpret_cast<float2*>(X)[(size_t)(row0 + k) * 64 + lane] = v[k];
-            unsigned hi, lo;
-            split_pair(v[k], hi, lo);
-            unsigned* o = reinterpret_cast<unsigned*>(split + (size_t)(row0 + k) * kSplitRowBytes + (lane >> 5) * 256);
-            o[lane & 31] = hi;
-            o[32 + (lane & 31)] = lo;
-        }
-        // the sieve's rows (past n: inside the padded buffer, never read)
-        float e2[kPrepRows];
-#pragma unroll
-        for (int k = 0; k < kPrepRows; ++k) {
             float const qx = fminf(fmaxf(rintf(v[k].x * kSieveScale), -127.0f), 127.0f);
             float const qy = fminf(fmaxf(rintf(v[k].y * kSieveScale), -127.0f), 127.0f);
             float const ex = v[k].x - qx * (1.0f / kSieveScale), ey = v[k].y - qy * (1.0f / kSieveScale);
@@ -166,64 +132,102 @@ __global__ __launch_bounds__(256) void k_split_rows(void const* __restrict__ src
                                       (row % kSieveTile) * 16 + (lane & 7) * 2) =
                 make_char2((signed char)(int)qx, (signed char)(int)qy);
         }
-        float const r2 = max_of_sums(e2, lane);
+        float const nr = sqrtf(sums_of8(s, lane));
+        if ((lane & 7) == 0) norm[row0 + (lane >> 3)] = nr;
+        mx = max(mx, __float_as_uint(nr));  // norms are >= 0 or NaN: a NaN wins
+        bad |= !(nr == 0.0f || (nr >= kSplitNormMin && nr < kSplitNormMax));
+        float r2 = sums_of8(e2, lane);
+#pragma unroll
+        for (int o = 32; o >= 8; o >>= 1) r2 = fmaxf(r2, __shfl_xor(r2, o));
         if (lane == 0) res[row0 / kSieveGroup] = sqrtf(r2) * 1.001f + 1e-6f;  // rounded up
+    }
+#pragma unroll
+    for (int o = 32; o >= 8; o >>= 1) {
+        mx = max(mx, __shfl_xor(mx, o));
+        bad |= __shfl_xor(bad, o);
     }
     if (lane == 0) {
         wmax[wave] = mx;
-        wbad[wave] = bad;
+        if (bad) *hostFit = 0;
     }
     __syncthreads();
-    int* const slot = info + kPrepSlot;  // two ints per work-group
-    if (threadIdx.x == 0) {
-        unsigned int const m = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
-        int const f = wbad[0] | wbad[1] | wbad[2] | wbad[3];
-        __hip_atomic_store(slot + 2 * blockIdx.x, (int)m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(slot + 2 * blockIdx.x + 1, f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        int const t = __hip_atomic_fetch_add(info, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = t == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    unsigned int m = 0;
-    int f = 0;
-    if (threadIdx.x < gridDim.x) {
-        m = (unsigned int)__hip_atomic_load(slot + 2 * threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        f = __hip_atomic_load(slot + 2 * threadIdx.x + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        m = max(m, __shfl_xor(m, o));
-        f |= __shfl_xor(f, o);
-    }
-    __syncthreads();
-    if (lane == 0) {
-        wmax[wave] = m;
-        wbad[wave] = f;
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    *maxNormBits = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
-    *hostFit = !(wbad[0] | wbad[1] | wbad[2] | wbad[3]);
-    __hip_atomic_store(info, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x >= kWaves) return;
+    mx = wmax[threadIdx.x];
+#pragma unroll
+    for (int o = kWaves / 2; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o));
+    // atomics of one address take about 10 ns each: one a work-group, and only with a new maximum
+    unsigned long long const word = ((unsigned long long)epoch << 32) | mx;
+    if (threadIdx.x == 0 && __hip_atomic_load(maxNorm, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < word)
+        atomicMax(maxNorm, word);
 }
 
-void launch_split_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNormBits,
-                       unsigned char* split, unsigned char* ints, float* scale, signed char* q8, float* res, int* info,
-                       int* hostFit, hipStream_t st)
+template <int kFrom>
+void launch_prep_from(void const* src, float* X, int n, float* norm, unsigned long long* maxNorm, unsigned epoch,
+                      float* scale, signed char* q8, float* res, int* hostFit, hipStream_t st)
+{
+    int const small = (n + 4 * kPrepRows - 1) / (4 * kPrepRows), large = (n + 16 * kPrepRows - 1) / (16 * kPrepRows);
+    if (small <= kPrepGroups)
+        hipLaunchKernelGGL((k_prep_rows<kFrom, 4>), dim3(small), dim3(256), 0, st, src, X, n, norm, maxNorm, epoch,
+                           scale, q8, res, hostFit);
+    else
+        hipLaunchKernelGGL((k_prep_rows<kFrom, 16>), dim3(min(large, kPrepGroups)), dim3(1024), 0, st, src, X, n, norm,
+                           maxNorm, epoch, scale, q8, res, hostFit);
+}
+
+// Work-groups of 4 waves while one round of kPrepGroups of them holds the set (8192 rows), of 16
+// above: a maximum's atomic a work-group is what the larger ones save (16384 rows 14 -> 11 us,
+// 32768 rows 17 -> 12 us), and below they would leave compute units idle (1920 rows of uint8 8.5
+// against 10.5 us).
+void launch_prep_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNorm,
+                      unsigned epoch, float* scale, signed char* q8, float* res, int* hostFit, hipStream_t st)
 {
     if (n <= 0) return;
-    int const per = 4 * kPrepRows;
-    dim3 const grid(min((n + per - 1) / per, kPrepGroups));
-    if (from == kRowsU8)
-        hipLaunchKernelGGL(k_split_rows<kRowsU8>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, ints,
-                           scale, q8, res, info, hostFit);
-    else if (from == kRowsF32)
-        hipLaunchKernelGGL(k_split_rows<kRowsF32>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split, ints,
-                           scale, q8, res, info, hostFit);
-    else
-        hipLaunchKernelGGL(k_split_rows<kRowsInPlace>, grid, dim3(256), 0, st, src, X, n, norm, maxNormBits, split,
-                           ints, scale, q8, res, info, hostFit);
+    auto* const mx = reinterpret_cast<unsigned long long*>(maxNorm);
+    if (from == kRowsU8) launch_prep_from<kRowsU8>(src, X, n, norm, mx, epoch, scale, q8, res, hostFit, st);
+    else if (from == kRowsF32) launch_prep_from<kRowsF32>(src, X, n, norm, mx, epoch, scale, q8, res, hostFit, st);
+    else launch_prep_from<kRowsInPlace>(src, X, n, norm, mx, epoch, scale, q8, res, hostFit, st);
+}
+
+// The rows of the full pass for both sets in one launch, a chunk of 8 components per thread:
+// the split parts, and where a set has scales (uint8 uploads) its components as FP16 integers
+// (x = fl(q d) with d > 0, so q is the integer next to x / d).  Made when the full pass first
+// needs them: with the sieve few calls do.
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+__global__ __launch_bounds__(256) void k_split_sets(SplitRowsOf a, SplitRowsOf b)
+{
+    int const t = blockIdx.x * 256 + threadIdx.x;
+    bool const first = (t >> 4) < a.n;
+    SplitRowsOf const& s = first ? a : b;
+    int const row = first ? t >> 4 : (t >> 4) - a.n;
+    int const c = t & 15;
+    if (row >= s.n) return;
+    float4 const* const p = reinterpret_cast<float4 const*>(s.X + (size_t)row * kDim) + 2 * c;
+    float4 const u = p[0], w = p[1];
+    float const x[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+    v8h hi, lo;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        float const y = x[k] * kSplitScale;
+        hi[k] = (_Float16)y;
+        lo[k] = (_Float16)(y - (float)hi[k]);
+    }
+    unsigned char* const o = s.split + (size_t)row * kSplitRowBytes + (c >> 3) * 256 + (c & 7) * 16;
+    *reinterpret_cast<v8h*>(o) = hi;
+    *reinterpret_cast<v8h*>(o + 128) = lo;
+    if (!s.ints) return;
+    float const d = s.scale[row];
+    v8h q;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) q[k] = x[k] == 0.0f ? (_Float16)0.0f : (_Float16)rintf(__fdiv_rn(x[k], d));
+    *reinterpret_cast<v8h*>(s.ints + (size_t)row * kIntRowBytes + c * 16) = q;
+}
+
+void launch_split_sets(SplitRowsOf const& a, SplitRowsOf const& b, hipStream_t st)
+{
+    int const rows = a.n + b.n;
+    if (rows <= 0) return;
+    hipLaunchKernelGGL(k_split_sets, dim3((rows + 15) / 16), dim3(256), 0, st, a, b);
 }
 
 // ------------------------------------------------------------------------------ merge + decide
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(256) void k_merge_decide(Top2 const* __restrict__ c
     s = top2_merge(s, top2_shfl_xor(s, 4));
     if (!valid || sub != 0) return;
     float const nq = left ? normL[q] : normR[q];
-    float const mo = __uint_as_float(maxNormBits[left ? 1 : 0]);
+    float const mo = __uint_as_float(maxNormBits[left ? kMaxNormR : 0]);
     float const eps = epsRel * nq * mo + kEpsAbs;
     int const d = (epsRel > 0.0f) ? decide_certified(s, eps, minScore, minRatio) : kFlag;
     if (d == kFlag) {
@@ -594,7 +598,7 @@ __global__ __launch_bounds__(256) void k_sample_decide(Top2 const* __restrict__ 
     for (int p = lane; p < nParts; p += 64) s = top2_merge(s, colPart[(size_t)p * ldc + q]);
     for (int o = 32; o > 0; o >>= 1) s = top2_merge(s, top2_shfl_xor(s, o));
     if (lane != 0) return;
-    float const eps = epsRel * normS[q] * __uint_as_float(maxNormBits[1]) + kEpsAbs;
+    float const eps = epsRel * normS[q] * __uint_as_float(maxNormBits[kMaxNormR]) + kEpsAbs;
     int const d = (epsRel > 0.0f) ? decide_certified(s, eps, minScore, minRatio) : kFlag;
     if (d == kFlag) flagList[atomicAdd(&counters[kCntFlag], 1)] = q;
     dec[q] = d;

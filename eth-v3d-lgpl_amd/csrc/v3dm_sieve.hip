@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SieveP
     if (i0 >= L.n) return;  // the waves of a group share nothing
     int const t0 = split * p.tiles;
     sieve_wave(L, R, i0, t0, min(t0 + p.tiles, R.n / kSieveTile), __uint_as_float(maxNormBits[0]),
-               __uint_as_float(maxNormBits[1]), T, out.best, out.second, out.best + out.offR, out.second + out.offR,
+               __uint_as_float(maxNormBits[kMaxNormR]), T, out.best, out.second, out.best + out.offR, out.second + out.offR,
                bits, ldi, lists[wv], threadIdx.x & 63);
 }
 

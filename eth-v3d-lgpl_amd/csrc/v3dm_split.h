@@ -39,17 +39,25 @@ constexpr int kSplitTile = 32;       // right features per tile
 
 // One feature set in one launch: its FP32 rows X (copied from the device array src, or
 // dequantised from the uint8 rows src as SIFT_Feature::normalizeDescriptor, or in place), the
-// norms and the set's largest norm (as launch_norms), the split rows, (uint8 rows) the
-// integer rows and their scales, and the sieve's int8 rows and residuals (v3dm_sieve.h).  info (device,
-// kPrepInfo ints, zero before the first call, left ready for the next): scratch; *hostFit
-// (mapped host memory): 1 when the set is in the range of the split pass.
+// norms and the set's largest norm (as launch_norms), the sieve's int8 rows and residuals
+// (v3dm_sieve.h) and the scales of uint8 rows.  n: a multiple of 32.  maxNorm: 8 bytes, the norm's
+// bits under the epoch, which grows from call to call (the 8 bytes start at zero); *hostFit
+// (mapped host memory): set to 0 when the set is out of the split pass's range.
 enum RowSource { kRowsInPlace, kRowsF32, kRowsU8 };
 constexpr int kPrepGroups = 256;
-constexpr int kPrepSlot = 32;
-constexpr int kPrepInfo = kPrepSlot + 2 * kPrepGroups;
-void launch_split_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNormBits,
-                       unsigned char* split, unsigned char* ints, float* scale, signed char* q8, float* res, int* info,
-                       int* hostFit, hipStream_t st);
+void launch_prep_rows(RowSource from, void const* src, float* X, int n, float* norm, unsigned int* maxNorm,
+                      unsigned epoch, float* scale, signed char* q8, float* res, int* hostFit, hipStream_t st);
+
+// The rows of the full pass of two sets in range: split rows, and of sets with scales the
+// components as FP16 integers (ints null: none).
+struct SplitRowsOf {
+    float const* X;
+    float const* scale;
+    unsigned char* split;
+    unsigned char* ints;
+    int n;
+};
+void launch_split_sets(SplitRowsOf const& a, SplitRowsOf const& b, hipStream_t st);
 
 // One side of a score pass: n split rows, and for sets uploaded as uint8 their components as
 // FP16 integers with the rows' scales (else null).  All padded to kSplitRowPad rows.
