@@ -70,12 +70,8 @@ void releaseBuffers(v3dm_context* h)
     freeDev(h->normR);
     freeDev(h->splitL);
     freeDev(h->splitR);
-    freeDev(h->q8L);
-    freeDev(h->q8R);
-    freeDev(h->resL);
-    freeDev(h->resR);
-    freeDev(h->sieveBest);
-    freeDev(h->sieveSecond);
+    freeDev(h->sieveBuf);
+    h->haveSplit = false;
     freeDev(h->intL);
     freeDev(h->intR);
     freeDev(h->intScaleL);
@@ -180,18 +176,25 @@ FusedPlan score_plan(v3dm_context const* h)
 }
 
 // The rows of the split pass, made once for the current sets.
-void ensure_split_rows(v3dm_context* h)
+int ensure_split_rows(v3dm_context* h)
 {
-    if (h->haveSplit) return;
+    if (h->haveSplit) return V3DM_OK;
+    for (bool left : {true, false}) {
+        size_t const rows = (size_t)roundUp(left ? h->capL : h->capR, kSplitRowPad);
+        unsigned char*& split = left ? h->splitL : h->splitR;
+        unsigned char*& ints = left ? h->intL : h->intR;
+        if (!split) HIPCHECK(h, hipMalloc(&split, rows * kSplitRowBytes));
+        if (!ints && (left ? h->haveIntL : h->haveIntR)) HIPCHECK(h, hipMalloc(&ints, rows * kIntRowBytes));
+    }
     launch_split_sets(SplitRowsOf{h->dL, h->intScaleL, h->splitL, h->haveIntL ? h->intL : nullptr, h->nL},
                       SplitRowsOf{h->dR, h->intScaleR, h->splitR, h->haveIntR ? h->intR : nullptr, h->nR}, h->stream);
     h->haveSplit = true;
+    return V3DM_OK;
 }
 
 void launch_score_pass(v3dm_context* h, FusedPlan const& p, unsigned const* bits, float minScore)
 {
     hipStream_t const st = h->stream;
-    if (split_fits(h)) ensure_split_rows(h);
     if (split_fits(h))
         launch_split_pass(SplitSet{h->splitL, h->haveIntL ? h->intL : nullptr, h->intScaleL, h->nL},
                           SplitSet{h->splitR, h->haveIntR ? h->intR : nullptr, h->intScaleR, h->nR}, p, h->colPart,
@@ -208,7 +211,11 @@ bool sieve_fits(v3dm_context const* h, float minScore, float minRatio, float* T)
     return split_fits(h) && h->epsRel > 0.0f && sieve_bound(minScore, minRatio, T);
 }
 
-SieveBest sieve_best(v3dm_context const* h) { return SieveBest{h->sieveBest, h->sieveSecond, h->capL}; }
+SieveBest sieve_best(v3dm_context const* h)
+{
+    return SieveBest{h->sieveBest, h->sieveSecond, h->capL, h->flagList, h->results + kCntFlag,
+                     h->results + kCntFlagR};
+}
 
 void launch_sieve_pass(v3dm_context* h, float T, unsigned const* bits)
 {
@@ -228,19 +235,20 @@ int enqueue_decisions(v3dm_context* h, unsigned const* bits, float minScore, flo
         if ((rc = prof_begin(h))) return rc;
         launch_sieve_pass(h, T, bits);
         if ((rc = prof_end(h))) return rc;
-        launch_sieve_decide(sieve_best(h), nL, nR, minScore, minRatio, h->colMax, h->rowMax, h->flagList, h->capL,
-                            h->results, st);
+        launch_sieve_finish(h->dL, h->dR, nL, nR, sieve_best(h), h->flagList, h->capL, h->capR, h->results, minScore,
+                            minRatio, h->colMax, h->rowMax, h->rpart, h->rtickets, bits, h->capL, st);
     } else {
         FusedPlan const p = score_plan(h);
+        if (split_fits(h) && (rc = ensure_split_rows(h))) return rc;
         if ((rc = prof_begin(h))) return rc;
         launch_score_pass(h, p, bits, minScore);
         if ((rc = prof_end(h))) return rc;
         launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
                             h->normR, h->maxNormBits, score_eps(h, bits), minScore, minRatio, h->colMax, h->rowMax,
                             h->flagList, h->capL, h->results, st);
+        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore, minRatio,
+                             h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st, bits, h->capL);
     }
-    launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore, minRatio,
-                         h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st, bits, h->capL);
     return V3DM_OK;
 }
 
@@ -256,7 +264,8 @@ int enqueue_plain(v3dm_context* h, float minScore, float minRatio)
         if (rc) return rc;
     }
     launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
-                          reinterpret_cast<int2*>(h->results + kNumCounters), h->results, st, {}, h->mutualWait);
+                          reinterpret_cast<int2*>(h->results + kNumCounters), h->results, h->hostStage, st,
+                          {}, h->mutualWait);
     HIPCHECK(h, hipGetLastError());
     return V3DM_OK;
 }
@@ -332,17 +341,19 @@ int v3dm_allocate(v3dm_handle h, int nMaxLeft, int nMaxRight, int useGuidedMatch
     HIPCHECK(h, hipMemsetAsync(h->dR, 0, cr * kDim * sizeof(float), h->stream));
     HIPCHECK(h, hipMalloc(&h->normL, cl * sizeof(float)));
     HIPCHECK(h, hipMalloc(&h->normR, cr * sizeof(float)));
-    auto split_rows = [](int cap) { return (size_t)roundUp(cap, kSplitRowPad); };
-    HIPCHECK(h, hipMalloc(&h->splitL, split_rows(h->capL) * kSplitRowBytes));
-    HIPCHECK(h, hipMalloc(&h->splitR, split_rows(h->capR) * kSplitRowBytes));
-    HIPCHECK(h, hipMalloc(&h->q8L, split_rows(h->capL) * kDim));
-    HIPCHECK(h, hipMalloc(&h->q8R, split_rows(h->capR) * kDim));
-    HIPCHECK(h, hipMalloc(&h->resL, split_rows(h->capL) / kSieveGroup * sizeof(float)));
-    HIPCHECK(h, hipMalloc(&h->resR, split_rows(h->capR) / kSieveGroup * sizeof(float)));
-    HIPCHECK(h, hipMalloc(&h->sieveBest, (cl + cr) * sizeof(unsigned long long)));
-    HIPCHECK(h, hipMalloc(&h->sieveSecond, (cl + cr) * sizeof(unsigned)));
-    HIPCHECK(h, hipMemsetAsync(h->sieveBest, 0, (cl + cr) * sizeof(unsigned long long), h->stream));
-    HIPCHECK(h, hipMemsetAsync(h->sieveSecond, 0, (cl + cr) * sizeof(unsigned), h->stream));
+    {
+        // bests, second bests, rows, residuals; row counts (multiples of 128) keep each aligned
+        size_t const best = (cl + cr) * sizeof(unsigned long long), second = (cl + cr) * sizeof(unsigned);
+        HIPCHECK(h, hipMalloc(&h->sieveBuf, best + second + (cl + cr) * kDim + (cl + cr) / kSieveGroup * sizeof(float)));
+        HIPCHECK(h, hipMemsetAsync(h->sieveBuf, 0, best + second, h->stream));
+        unsigned char* p = h->sieveBuf;
+        h->sieveBest = reinterpret_cast<unsigned long long*>(p);
+        h->sieveSecond = reinterpret_cast<unsigned*>(p += best);
+        h->q8L = reinterpret_cast<signed char*>(p += second);
+        h->q8R = h->q8L + cl * kDim;
+        h->resL = reinterpret_cast<float*>(p += (cl + cr) * kDim);
+        h->resR = h->resL + cl / kSieveGroup;
+    }
     HIPCHECK(h, hipHostMalloc(&h->splitFitHost, 2 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     HIPCHECK(h, hipHostGetDevicePointer((void**)&h->splitFitDev, h->splitFitHost, 0));
     h->splitFitHost[0] = h->splitFitHost[1] = 0;
@@ -365,6 +376,7 @@ int v3dm_allocate(v3dm_handle h, int nMaxLeft, int nMaxRight, int useGuidedMatch
     HIPCHECK(h, hipMalloc(&h->results, (kNumCounters + 2 * (size_t)h->pairCap) * sizeof(int)));
     HIPCHECK(h, hipMemsetAsync(h->results, 0, (kNumCounters + 2 * (size_t)h->pairCap) * sizeof(int), h->stream));
     HIPCHECK(h, hipHostMalloc(&h->hostStage, (kNumCounters + 2 * (size_t)h->pairCap) * sizeof(int)));
+    memset(h->hostStage, 0, kNumCounters * sizeof(int));
     if (h->useGuided) {
         HIPCHECK(h, hipMalloc(&h->dLeftXY, cl * 2 * sizeof(float)));
         HIPCHECK(h, hipMalloc(&h->dRightXY, cr * 2 * sizeof(float)));
@@ -439,8 +451,7 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
                 HIPCHECK(h, hipMalloc(&h->dQ, qb));
                 h->dQBytes = qb;
             }
-            size_t const rows = (size_t)roundUp(left ? h->capL : h->capR, kSplitRowPad);
-            if (!(left ? h->intL : h->intR)) HIPCHECK(h, hipMalloc(left ? &h->intL : &h->intR, rows * kIntRowBytes));
+            size_t const rows = (size_t)(left ? h->capL : h->capR);
             if (!(left ? h->intScaleL : h->intScaleR))
                 HIPCHECK(h, hipMalloc(left ? &h->intScaleL : &h->intScaleR, rows * sizeof(float)));
             HIPCHECK(h, hipMemcpyAsync(h->dQ, src, (size_t)n * kDim, hipMemcpyHostToDevice, h->stream));
@@ -471,28 +482,13 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
 int copyResults(v3dm_context* h, int32_t* pairs, int cap, int* nPairs)
 {
     if (!h->haveResult) return fail(h, V3DM_ERR_STATE, "no result: call findPutativeMatches first");
-    // One copy of the counters and of as many pairs as the previous result held (plus a
-    // margin), enqueued before the wait for the sampled check so that both end in one round
-    // trip; the rest only when the result is larger.
-    size_t const headBytes = kNumCounters * sizeof(int);
-    size_t const prev = (size_t)std::max(h->stats.nMatches, 0);
-    size_t const guess = std::min((size_t)h->pairCap, prev + prev / 4 + 1024);
-    HIPCHECK(h, hipMemcpyAsync(h->hostStage, h->results, headBytes + guess * 2 * sizeof(int), hipMemcpyDeviceToHost,
-                               h->stream));
+    // the mutual check wrote the counts and the pairs to the pinned block
     int const rcf = ext_finish(h);
     if (rcf) return rcf;
-    if (h->stats.nFallback)  // the plain form's result replaced the learned one
-        HIPCHECK(h, hipMemcpyAsync(h->hostStage, h->results, headBytes + guess * 2 * sizeof(int),
-                                   hipMemcpyDeviceToHost, h->stream));
     HIPCHECK(h, hipStreamSynchronize(h->stream));
     if (h->hostStage[kCntMutualError] == (int)h->mutualEpoch)
         return fail(h, V3DM_ERR_HIP, "mutual check: ordering wait between work-groups ran out");
     int const n = h->hostStage[kCntPairs];
-    if ((size_t)n > guess) {
-        HIPCHECK(h, hipMemcpyAsync(h->hostStage + kNumCounters + 2 * guess, h->results + kNumCounters + 2 * guess,
-                                   ((size_t)n - guess) * 2 * sizeof(int), hipMemcpyDeviceToHost, h->stream));
-        HIPCHECK(h, hipStreamSynchronize(h->stream));
-    }
     h->stats.nMatches = n;
     h->stats.nRechecked = h->hostStage[kCntFlagDone];
     h->stats.nRescored = h->hostStage[kCntRescoredDone];
@@ -547,7 +543,8 @@ int runGuided(v3dm_context* h, int kind, const double M[9], float distanceThresh
         if (rc) return rc;
     }
     launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
-                          reinterpret_cast<int2*>(h->results + kNumCounters), h->results, st, {}, h->mutualWait);
+                          reinterpret_cast<int2*>(h->results + kNumCounters), h->results, h->hostStage, st,
+                          {}, h->mutualWait);
     HIPCHECK(h, hipGetLastError());
     h->lastMinScore = minScore;
     h->lastMinRatio = minRatio;
@@ -797,7 +794,11 @@ int v3dm_score_block(v3dm_handle h, int mode, int nRows, int nCols, float* score
     size_t const bytes = (size_t)nRows * nCols * sizeof(float);
     HIPCHECK(h, hipMalloc(&d, bytes));
     if (mode == V3DM_PREC_FP32 && split_fits(h)) {
-        ensure_split_rows(h);
+        int const rc = ensure_split_rows(h);
+        if (rc) {
+            (void)hipFree(d);
+            return rc;
+        }
         launch_score_block_split(h->splitL, h->splitR, nRows, nCols, d, h->stream);
     } else {
         launch_score_block(mode, h->dL, h->dR, nRows, nCols, d, h->stream);
@@ -830,7 +831,9 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
             FusedPlan const p = score_plan(h);
             float T = 0.0f;
             bool const sieve = sieve_fits(h, h->lastMinScore, h->lastMinRatio, &T);
-            e = hipEventRecord(a, h->stream);
+            if (!sieve && split_fits(h)) rc = ensure_split_rows(h);
+            if (rc) e = hipErrorOutOfMemory;
+            if (e == hipSuccess) e = hipEventRecord(a, h->stream);
             for (int r = 0; r < reps && e == hipSuccess; ++r) {
                 if (sieve) launch_sieve_pass(h, T, nullptr);
                 else launch_score_pass(h, p, nullptr, h->lastMinScore);
@@ -840,6 +843,8 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
                 size_t const n = (size_t)h->capL + h->capR;
                 if (e == hipSuccess) e = hipMemsetAsync(h->sieveBest, 0, n * sizeof(unsigned long long), h->stream);
                 if (e == hipSuccess) e = hipMemsetAsync(h->sieveSecond, 0, n * sizeof(unsigned), h->stream);
+                if (e == hipSuccess) e = hipMemsetAsync(h->results + kCntFlag, 0, sizeof(int), h->stream);
+                if (e == hipSuccess) e = hipMemsetAsync(h->results + kCntFlagR, 0, sizeof(int), h->stream);
             }
             launches = reps;
         }

@@ -45,7 +45,8 @@ struct v3dm_context {
     float* intScaleR = nullptr;
     bool haveIntL = false, haveIntR = false;  // the current set has them
     bool haveSplit = false;           // the split and integer rows of the current sets are made
-    signed char *q8L = nullptr, *q8R = nullptr;   // the sieve's rows and residuals
+    unsigned char* sieveBuf = nullptr;            // one allocation of the sieve's arrays:
+    signed char *q8L = nullptr, *q8R = nullptr;   // rows and residuals
     float *resL = nullptr, *resR = nullptr;
     unsigned long long* sieveBest = nullptr;      // of capL left, then capR right features
     unsigned* sieveSecond = nullptr;

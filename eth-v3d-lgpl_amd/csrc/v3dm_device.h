@@ -312,4 +312,20 @@ __device__ __forceinline__ Top2 merge_partials(Top2 const* part, int nCh, int la
     return s;
 }
 
+// A query's decision from its sieve entries (v3dm_sieve.h), which are left at zero; kFlag: it
+// goes to the exact re-check.
+__device__ __forceinline__ int sieve_decision(unsigned long long* best, unsigned* second, float minScore,
+                                              float minRatio)
+{
+    unsigned long long const k = *best;
+    unsigned const s2 = *second;
+    if (k) *best = 0;
+    if (s2) *second = 0;
+    if (k == ~0ull) return kFlag;
+    if (!k) return -1;
+    Top2 const s{__uint_as_float((unsigned)(k >> 32)), s2 ? __uint_as_float(s2) : kInit,
+                 (int)(0xffffffffu - (unsigned)k)};
+    return decide_exact(s, minScore, minRatio);
+}
+
 }  // namespace v3dm

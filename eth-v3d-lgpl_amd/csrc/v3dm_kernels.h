@@ -74,8 +74,9 @@ struct MutualWait {
     unsigned spinLimit = kMutualSpinLimit;
     unsigned readXor = 0;
 };
+// host: pinned block that also gets the counters and the pairs behind them, or null
 void launch_mutual_compact(int const* colMax, int const* rowMax, int nL, int nR, unsigned long long* status,
-                           unsigned epoch, int* stripes, int2* pairs, int* counters, hipStream_t st,
+                           unsigned epoch, int* stripes, int2* pairs, int* counters, int* host, hipStream_t st,
                            SampleOut const& so = {}, MutualWait const& mw = {});
 
 // plain FP32 fused score + top-2 kernel (v3dm_fp32.hip)

@@ -178,7 +178,7 @@ int v3dm_match_device_noalloc(const float* leftDesc, int nLeft, const float* rig
                              rpart, reinterpret_cast<int*>(b + kOffTickets), kRecheckGrid, st);
     }
     launch_mutual_compact(colMax, rowMax, work ? nL : 0, nR, status, ep, stripes, reinterpret_cast<int2*>(pairs),
-                          counters, st);
+                          counters, nullptr, st);
     hipLaunchKernelGGL(k_noalloc_count, dim3(1), dim3(64), 0, st, counters, ep, count);
     e = hipGetLastError();
     if (e != hipSuccess) return noalloc_fail(V3DM_ERR_HIP, "launch", e);

@@ -376,15 +376,25 @@ __device__ __forceinline__ void recheck_units(RecheckDir const& dl, RecheckDir c
     }
 }
 
+template <bool kSieve>
 __global__ __launch_bounds__(256) void k_recheck(float const* __restrict__ L, float const* __restrict__ R, int nL,
                                                  int nR, int const* __restrict__ flagList, int rowsL, int rowsR,
                                                  int const* __restrict__ counters, Top2* __restrict__ part,
                                                  int* __restrict__ tickets, unsigned const* __restrict__ gbits,
                                                  int ldi, float minScore, float minRatio, int* __restrict__ colMax,
-                                                 int* __restrict__ rowMax)
+                                                 int* __restrict__ rowMax, SieveBest sieve)
 {
     __shared__ __attribute__((aligned(16))) float stage[4][kExactLds];
     __shared__ __attribute__((aligned(16))) double qd[4][kRecheckGroup * kDim];
+    if constexpr (kSieve) {
+        // the other queries' decisions; the listed ones' follow below
+        for (int g = blockIdx.x * 256 + threadIdx.x; g < nL + nR; g += gridDim.x * 256) {
+            int const q = g < nL ? g : g - nL;
+            int const at = g < nL ? q : sieve.offR + q;
+            int const d = sieve_decision(sieve.best + at, sieve.second + at, minScore, minRatio);
+            if (d != kFlag) (g < nL ? colMax : rowMax)[q] = d;
+        }
+    }
     int const cntL = __builtin_amdgcn_readfirstlane(counters[kCntFlag]);
     int const cntR = __builtin_amdgcn_readfirstlane(counters[kCntFlagR]);
     RecheckDir const dl = recheck_dir(true, L, R, nL, nR, cntL, rowsL, rowsR, colMax, rowMax);
@@ -403,8 +413,19 @@ void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int co
                           int* tickets, int grid, hipStream_t st, unsigned const* gbits, int ldi)
 {
     if (nL <= 0 || nR <= 0) return;
-    hipLaunchKernelGGL(k_recheck, dim3(grid), dim3(256), 0, st, L, R, nL, nR, flagList, rowsL, rowsR, counters, part,
-                       tickets, gbits, ldi, minScore, minRatio, colMax, rowMax);
+    hipLaunchKernelGGL(k_recheck<false>, dim3(grid), dim3(256), 0, st, L, R, nL, nR, flagList, rowsL, rowsR, counters,
+                       part, tickets, gbits, ldi, minScore, minRatio, colMax, rowMax, SieveBest{});
+}
+
+// A thread per query; hardly ever is a query listed, and then the units take the grid in turn.
+void launch_sieve_finish(float const* L, float const* R, int nL, int nR, SieveBest const& b, int const* flagList,
+                         int rowsL, int rowsR, int const* counters, float minScore, float minRatio, int* colMax,
+                         int* rowMax, Top2* part, int* tickets, unsigned const* gbits, int ldi, hipStream_t st)
+{
+    if (nL <= 0 || nR <= 0) return;
+    int const grid = min(max((nL + nR + 255) / 256, 128), kRecheckGrid);
+    hipLaunchKernelGGL(k_recheck<true>, dim3(grid), dim3(256), 0, st, L, R, nL, nR, flagList, rowsL, rowsR, counters,
+                       part, tickets, gbits, ldi, minScore, minRatio, colMax, rowMax, b);
 }
 
 // ------------------------------------------------------------------------------ mutual + compaction
@@ -419,7 +440,8 @@ void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int co
 // are dispatched before it; the wait is bounded (mw.spinLimit sleeps), and a work-group
 // that runs out of it stores the epoch in counters[kCntMutualError] (its matches then land
 // below their place, inside the buffer).  The last work-group also publishes the match,
-// re-check and rescoring counts and clears the per-call counters.
+// re-check and rescoring counts and clears the per-call counters.  Matches and counts also go
+// straight to the handle's pinned host block: a copy after the kernel cost about 10 us a call.
 
 // Left feature sampled as sample k of S (evenly spaced over [0, nL)).
 __device__ __forceinline__ int sample_row(int k, int nL, int S) { return (int)(((long long)k * nL) / S); }
@@ -432,8 +454,8 @@ __device__ __forceinline__ unsigned long long mutual_word(unsigned epoch, unsign
 __global__ __launch_bounds__(256) void k_mutual(int const* __restrict__ colMax, int const* __restrict__ rowMax,
                                                 int nL, int nR, unsigned long long* __restrict__ status,
                                                 unsigned epoch, int* __restrict__ stripes,
-                                                int2* __restrict__ pairs, int* __restrict__ counters, SampleOut so,
-                                                MutualWait mw)
+                                                int2* __restrict__ pairs, int* __restrict__ counters,
+                                                int* __restrict__ host, SampleOut so, MutualWait mw)
 {
     __shared__ int wsum[4];
     __shared__ int sBase;
@@ -514,7 +536,10 @@ __global__ __launch_bounds__(256) void k_mutual(int const* __restrict__ colMax, 
             if (b > 0)
                 __hip_atomic_store(&status[b], mutual_word(epoch, 2u, (unsigned)(excl + total)), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-            if (failed) counters[kCntMutualError] = (int)epoch;
+            if (failed) {
+                counters[kCntMutualError] = (int)epoch;
+                if (host) host[kCntMutualError] = (int)epoch;
+            }
             sBase = excl;
         }
     }
@@ -522,7 +547,11 @@ __global__ __launch_bounds__(256) void k_mutual(int const* __restrict__ colMax, 
     int pos = sBase + off + incl - cnt;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-        if (m[u]) pairs[pos++] = make_int2(i0 + u, l[u]);
+        if (m[u]) {
+            int2 const pr = make_int2(i0 + u, l[u]);
+            if (host) reinterpret_cast<int2*>(host + kNumCounters)[pos] = pr;
+            pairs[pos++] = pr;
+        }
     // work-group 0 (off the look-back chain by now): the sampled learned decisions
     if (b == 0 && tid < so.S) so.out[tid] = colMax[sample_row(tid, nL, so.S)];  // vector stores
     if (b != (int)gridDim.x - 1) return;
@@ -535,22 +564,28 @@ __global__ __launch_bounds__(256) void k_mutual(int const* __restrict__ colMax, 
         }
         for (int o = 32; o > 0; o >>= 1) rescored += __shfl_xor(rescored, o);
         if (tid == 0) {
+            int const open = counters[kCntFlag] + counters[kCntFlagR];
             counters[kCntPairs] = sBase + total;
-            counters[kCntFlagDone] = counters[kCntFlag] + counters[kCntFlagR];
+            counters[kCntFlagDone] = open;
             counters[kCntFlag] = 0;
             counters[kCntFlagR] = 0;
             counters[kCntRescoredDone] = rescored;
+            if (host) {
+                host[kCntPairs] = sBase + total;
+                host[kCntFlagDone] = open;
+                host[kCntRescoredDone] = rescored;
+            }
         }
     }
 }
 
 void launch_mutual_compact(int const* colMax, int const* rowMax, int nL, int nR, unsigned long long* status,
-                           unsigned epoch, int* stripes, int2* pairs, int* counters, hipStream_t st,
+                           unsigned epoch, int* stripes, int2* pairs, int* counters, int* host, hipStream_t st,
                            SampleOut const& so, MutualWait const& mw)
 {
     int const nb = (nL + kMutualSlice - 1) / kMutualSlice;
     hipLaunchKernelGGL(k_mutual, dim3(nb > 0 ? nb : 1), dim3(256), 0, st, colMax, rowMax, nL, nR, status, epoch,
-                       stripes, pairs, counters, so, mw);
+                       stripes, pairs, counters, host, so, mw);
 }
 
 // ------------------------------------------------------------------------------ sampled check

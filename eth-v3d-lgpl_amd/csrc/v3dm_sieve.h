@@ -38,11 +38,19 @@ struct SieveSet {
 };
 
 // Per query (left, then right at offR): the candidates' best as score bits << 32 | ~index, and
-// the second best's bits.  Zero before a pass; sieve_decide leaves them zero.
+// the second best's bits.  Zero before a pass; the decisions leave them zero.  Features of a
+// block whose list overflowed hold kSieveFlood and are listed for the exact re-check (flags:
+// left ones from 0, right ones from offR, counted at cntL and cntR; null: the decisions list
+// them).
+constexpr unsigned long long kSieveFlood = ~0ull;
+
 struct SieveBest {
     unsigned long long* best;
     unsigned* second;
     int offR;
+    int* flags;
+    int* cntL;
+    int* cntR;
 };
 
 struct SievePlan {
@@ -53,9 +61,10 @@ SievePlan plan_sieve(int nL, int nR);
 // bits: guided-matching bitmap (removed pairs are no candidates), or null.
 void launch_sieve(SieveSet const& L, SieveSet const& R, SievePlan const& p, unsigned const* maxNormBits, float T,
                   SieveBest const& b, unsigned const* bits, int ldi, hipStream_t st);
-// Decisions of all queries; queries of a flooded block go to the exact re-check (flagList as
-// launch_merge_decide).
-void launch_sieve_decide(SieveBest const& b, int nL, int nR, float minScore, float minRatio, int* colMax, int* rowMax,
-                         int* flagList, int flagOffR, int* counters, hipStream_t st);
+// Decisions of all queries and the exact re-check of the listed ones, in one launch (buffers as
+// launch_recheck_exact).
+void launch_sieve_finish(float const* L, float const* R, int nL, int nR, SieveBest const& b, int const* flagList,
+                         int rowsL, int rowsR, int const* counters, float minScore, float minRatio, int* colMax,
+                         int* rowMax, Top2* part, int* tickets, unsigned const* gbits, int ldi, hipStream_t st);
 
 }  // namespace v3dm

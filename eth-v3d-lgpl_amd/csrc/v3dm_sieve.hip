@@ -46,7 +46,6 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // instruction); 4096 x 4096: 12 + 3 against 24 + 5 + 4; 480 x 512: 9 + 2 against 8 + 5 + 4.
 constexpr int kSieveBlocks = 4;
 constexpr int kSieveList = 512;
-constexpr unsigned long long kSieveFlood = ~0ull;
 
 __device__ __forceinline__ int max3i(int a, int b, int c) { return max(max(a, b), c); }
 
@@ -102,7 +101,7 @@ __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R,
                                            float MR, float T, unsigned long long* __restrict__ bestL,
                                            unsigned* __restrict__ secondL, unsigned long long* __restrict__ bestR,
                                            unsigned* __restrict__ secondR, unsigned const* __restrict__ bits, int ldi,
-                                           int* list, int lane)
+                                           SieveBest const& flood, int* list, int lane)
 {
     int const h = lane >> 5;
     int const c32 = lane & 31;
@@ -166,8 +165,12 @@ __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R,
         if (t < t1) tile(a0, t);
     }
     if (cnt > kSieveList) {
-        for (int i = lane; i < min(32 * kSieveBlocks, L.n - i0); i += 64) atomicMax(bestL + i0 + i, kSieveFlood);
-        for (int j = t0 * kSieveTile + lane; j < t1 * kSieveTile; j += 64) atomicMax(bestR + j, kSieveFlood);
+        for (int i = i0 + lane; i < min(i0 + 32 * kSieveBlocks, L.n); i += 64)
+            if (atomicMax(bestL + i, kSieveFlood) != kSieveFlood && flood.flags)
+                flood.flags[atomicAdd(flood.cntL, 1)] = i;
+        for (int j = t0 * kSieveTile + lane; j < t1 * kSieveTile; j += 64)
+            if (atomicMax(bestR + j, kSieveFlood) != kSieveFlood && flood.flags)
+                flood.flags[flood.offR + atomicAdd(flood.cntR, 1)] = j;
         return;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // LDS operations of one wave are in order
@@ -198,7 +201,7 @@ __global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SieveP
     int const t0 = split * p.tiles;
     sieve_wave(L, R, i0, t0, min(t0 + p.tiles, R.n / kSieveTile), __uint_as_float(maxNormBits[0]),
                __uint_as_float(maxNormBits[kMaxNormR]), T, out.best, out.second, out.best + out.offR, out.second + out.offR,
-               bits, ldi, lists[wv], threadIdx.x & 63);
+               bits, ldi, out, lists[wv], threadIdx.x & 63);
 }
 
 // Over a batch: item = (pair, group of 512 left features, split, tiles per split), one
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(256, 3) void k_batch_sieve(BatchDev b, int4 const* 
     int const t0 = w.z * w.w;
     sieve_wave(L, R, i0, t0, min(t0 + w.w, sr.n / kSieveTile), __uint_as_float(b.maxNorm[sl.img]),
                __uint_as_float(b.maxNorm[sr.img]), T, best + sl.qOff, second + sl.qOff, best + sr.qOff,
-               second + sr.qOff, nullptr, 0, lists[wv], threadIdx.x & 63);
+               second + sr.qOff, nullptr, 0, SieveBest{}, lists[wv], threadIdx.x & 63);
 }
 
 void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
@@ -263,46 +266,6 @@ void launch_sieve(SieveSet const& L, SieveSet const& R, SievePlan const& p, unsi
 }
 
 // ------------------------------------------------------------------------------ decisions
-__device__ __forceinline__ int sieve_decision(unsigned long long* best, unsigned* second, float minScore,
-                                              float minRatio)
-{
-    unsigned long long const k = *best;
-    unsigned const s2 = *second;
-    if (k) *best = 0;
-    if (s2) *second = 0;
-    if (k == kSieveFlood) return kFlag;
-    if (!k) return -1;
-    Top2 const s{__uint_as_float((unsigned)(k >> 32)), s2 ? __uint_as_float(s2) : kInit,
-                 (int)(0xffffffffu - (unsigned)k)};
-    return decide_exact(s, minScore, minRatio);
-}
-
-__global__ __launch_bounds__(256) void k_sieve_decide(SieveBest b, int nL, int nR, float minScore, float minRatio,
-                                                      int* __restrict__ colMax, int* __restrict__ rowMax,
-                                                      int* __restrict__ flagList, int flagOffR,
-                                                      int* __restrict__ counters)
-{
-    int const g = blockIdx.x * 256 + threadIdx.x;
-    if (g >= nL + nR) return;
-    bool const left = g < nL;
-    int const q = left ? g : g - nL;
-    int const at = left ? q : b.offR + q;
-    int const d = sieve_decision(b.best + at, b.second + at, minScore, minRatio);
-    if (d == kFlag) {
-        int const slot = atomicAdd(&counters[left ? kCntFlag : kCntFlagR], 1);
-        flagList[left ? slot : flagOffR + slot] = q;
-    }
-    (left ? colMax : rowMax)[q] = d;
-}
-
-void launch_sieve_decide(SieveBest const& b, int nL, int nR, float minScore, float minRatio, int* colMax, int* rowMax,
-                         int* flagList, int flagOffR, int* counters, hipStream_t st)
-{
-    if (nL + nR <= 0) return;
-    hipLaunchKernelGGL(k_sieve_decide, dim3((nL + nR + 255) / 256), dim3(256), 0, st, b, nL, nR, minScore, minRatio,
-                       colMax, rowMax, flagList, flagOffR, counters);
-}
-
 __global__ __launch_bounds__(256) void k_batch_sieve_decide(BatchDev b, unsigned long long* __restrict__ best,
                                                             unsigned* __restrict__ second, float minScore,
                                                             float minRatio, int* __restrict__ sel,
