@@ -120,3 +120,37 @@ def test_batch(dtype, cache):
             want = oracle.find_putative_matches(L, R, ms, mr) if len(L) and len(R) else np.zeros((0, 2), np.int32)
             assert np.array_equal(np.asarray(got[p]).reshape(-1, 2), want.reshape(-1, 2)), (p, ms, mr)
     m.close()
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-8, 1e-20, 1e12])
+@pytest.mark.parametrize("threshold", [0.0, 1e-3, 1.5, 40.0])
+def test_guided_mask(matcher_guided, scale, threshold):
+    """The epipolar mask at scales of F that take the comparison of products and that leave
+    single pairs or every pair to the division, on positions of which some lie on the lines."""
+    print(f"case guided mask scale {scale} threshold {threshold}", flush=True)
+    m = matcher_guided
+    rng = np.random.default_rng(12)
+    nL, nR = 352, 288
+    a, b, _ = synth.make_pair(nL, nR, 0.5, config=7, pair=44)
+    L, R = synth.dequantise(a), synth.dequantise(b)
+    lxy = rng.uniform(0, 1000, (nL, 2)).astype(np.float32)
+    rxy = rng.uniform(0, 1000, (nR, 2)).astype(np.float32)
+    rxy[::3, 1] = lxy[:len(rxy[::3]), 1]                    # on the lines of a sideways motion
+    F = np.array([[0, 0, 0], [0, 0, -1.0], [0, 1.0, 0]]) + 1e-4 * rng.standard_normal((3, 3))
+    m.setLeftFeatures(nL, L)
+    m.setRightFeatures(nR, R)
+    m.find_putative_matches_array(0.9, 0.8)
+    S = oracle.scores(L, R)
+    for min_score in (0.9, 0.2):
+        got = m.run_guided_array(False, scale * F, threshold, lxy, rxy, min_score, -1.0)
+        want = oracle.guided(S, 0, scale * F, np.float32(threshold), lxy, rxy, min_score, -1.0)
+        assert np.array_equal(got, want)
+
+
+@pytest.fixture(scope="module")
+def matcher_guided():
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(512, 512, True)
+    yield m
+    m.close()
