@@ -146,9 +146,9 @@ def bench_batch(args):
            "pairs": BATCH_PAIRS, "features": int(counts.sum()), "score_pairs": score_pairs}
     log("bench: batch plain_fp32")
     plain, out["plain_fp32"] = time_batch(m, v3dmatch.PREC_FP32, args.steps, args.warmup)
-    out["plain_fp32"]["kernel"] = "k_batch_fused_fp32"
+    out["plain_fp32"]["kernel"] = "k_batch_sieve"
     out["plain_fp32"]["kernel_ms"] = m.batch_time_dominant_kernel(3)
-    out["plain_fp32"]["flop_per_launch"] = 2.0 * score_pairs * 128
+    out["plain_fp32"]["ops_per_launch"] = 2.0 * score_pairs * 128  # int8 products, one per score
     ex = _sets(plain)
     log("bench: batch bf16_shortlist")
     bf, out["bf16_shortlist"] = time_batch(m, v3dmatch.PREC_BF16, args.steps, args.warmup)
@@ -271,9 +271,9 @@ def bench_pair(args):
     log("bench: pair plain FP32")
     ms, kms, st = time_form(m, args.steps, args.warmup)
     exact = m.get_matches()
-    forms = {"plain_fp32": {"pairs_per_s": 1e3 / ms, "ms_per_step": ms, "kernel": "k_fused_fp32",
-                            "kernel_ms": kms, "kernel_tflops": flop / (kms * 1e-3) / 1e12,
-                            "frac": flop / (kms * 1e-3) / PEAK_FP32_MFMA, "matches": int(len(exact)),
+    forms = {"plain_fp32": {"pairs_per_s": 1e3 / ms, "ms_per_step": ms, "kernel": "k_sieve",
+                            "kernel_ms": kms, "kernel_tops": flop / (kms * 1e-3) / 1e12,
+                            "frac": flop / (kms * 1e-3) / PEAK_INT8_MFMA, "matches": int(len(exact)),
                             "rechecked_queries": int(st["nRechecked"]),
                             "ms_per_call_read_back": time_read_back(m, args.steps)}}
     ex = set(map(tuple, exact.tolist()))
@@ -363,8 +363,8 @@ def bench_small_pair(args):
     m.close()
     flop = 2.0 * N_SMALL * N_SMALL * 128
     out = {"workload": f"one pair of {N_SMALL}x{N_SMALL} descriptors, 40% noisy copies, plain FP32 form",
-           "ms_per_step": ms, "pairs_per_s": 1e3 / ms, "ms_per_call_read_back": rb, "kernel": "k_fused_fp32",
-           "kernel_ms": kms, "frac_fp32_peak": flop / (kms * 1e-3) / PEAK_FP32_MFMA, "matches": int(len(got))}
+           "ms_per_step": ms, "pairs_per_s": 1e3 / ms, "ms_per_call_read_back": rb, "kernel": "k_sieve",
+           "kernel_ms": kms, "frac_int8_peak": flop / (kms * 1e-3) / PEAK_INT8_MFMA, "matches": int(len(got))}
     if not args.no_cpu:
         cb, cpu_pairs = cpu_baseline_pair(L, R, budget_s=5.0)
         cb["match_set_identical_to_gpu"] = bool(np.array_equal(cpu_pairs, got))
@@ -479,7 +479,8 @@ def bench_voctree(steps, warmup, cpu, branch=50, depth=3, n=1_000_000):
     hip.free(dw)
     flop = 2.0 * n * branch * depth * 128
     res.update({"ms_per_run": dt * 1e3, "keys_per_s": n / dt, "exact_keys": int(exact),
-                "tflops": flop / dt / 1e12, "frac_fp32_mfma": flop / dt / PEAK_FP32_MFMA})
+                "tflops": flop / dt / 1e12,
+                "frac_f16_mfma": 3.0 * flop / dt / PEAK_BF16_MFMA})  # three FP16 products per score
     if cpu:
         from oracle import oracle
         s = 20000

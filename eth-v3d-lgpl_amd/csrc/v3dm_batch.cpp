@@ -844,7 +844,8 @@ int time_pass(v3dm_context* h, BatchState* b, int form, Plan const& pl, float& m
 }
 
 // Choose (tiles per item, persistent grid, and the work-group's tile shape: 128 or 256 query
-// rows against 64-candidate tiles, i.e. 4 or 8 waves for the plain form, 2 or 4 waves for
+// rows against 64-candidate tiles, i.e. 2 or 4 waves (FP32 rows: 4 or 8) for the plain form's
+// full pass, 2 or 4 waves for
 // the BF16 and code passes) for a form: the given override, or the fastest candidate
 // measured on this batch, or the default when tuning is off.
 int ensure_plan(v3dm_context* h, BatchState* b, int form)
@@ -917,7 +918,8 @@ int ensure_fallback_plan(v3dm_context* h, BatchState* b)
         (void)hipGetDevice(&dev);
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         drop_graphs(b);
-        // 256 left features an item on split rows (109 -> see k_batch_split), 128 on FP32 rows
+        // 256 left features an item on split rows (the fallback pass of the
+        // 256-pair uint8 batch 109 us with 128, 78 so), 128 on FP32 rows
         Plan pl = plan_plain(b, kFallbackTiles, 2 * cus, b->splitFit ? 256 : 128);
         if ((rc = upload_plan(h, b, 3, pl))) return rc;
         b->plan[3] = std::move(pl);

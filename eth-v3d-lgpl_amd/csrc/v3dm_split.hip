@@ -24,15 +24,15 @@ typedef __attribute__((address_space(3))) void lds_void;
 // two LDS stages filled by direct global->LDS loads.  Why this shape: a tile's parts (16 KiB)
 // are read from LDS once per wave for two column blocks, so 48 matrix instructions (1536
 // cycles) stand against 16 KiB of operand reads, 16 KiB of the score transpose below (256
-// LDS cycles a wave together, 1024 of the CU's per tile) and about 300 vector instructions
-// (1200 cycles) that the SIMD's other wave overlaps; 256 VGPRs leave two waves per SIMD, and
-// the 70 KiB of LDS two work-groups per CU, which drift apart and fill each other's gaps.
+// LDS cycles a wave together, 1024 of the CU's per tile) and about 190 vector instructions
+// (760 cycles) that the SIMD's other wave overlaps; 256 VGPRs leave two waves per SIMD, and
+// the 76 KiB of LDS two work-groups per CU, which drift apart and fill each other's gaps.
 // Counts are multiples of 32, so no tile and no column block is partial; a wave's second (or
 // every) block past nL is skipped.
 //
 // Lane l holds column c = l % 32 and rows j = 8 (r / 4) + 4 (l / 32) + r % 4 of each 32x32
-// block.  Per left feature the running top-2 stays in registers (the position inside the tile
-// as r, the tile noted once per tile when the best changed); per right feature each wave
+// block.  Per left feature the running top-2 stays in registers (the position
+// looked for only where it can matter, see Selection); per right feature each wave
 // writes its scores to its own LDS rows, reads them back a row per lane pair, and the waves'
 // partial top-2 of a tile are merged by one of them after the next tile's barrier, so a tile
 // costs one barrier.
@@ -41,12 +41,14 @@ typedef __attribute__((address_space(3))) void lds_void;
 // small products first (lo hi, hi lo, then hi hi) step by step.
 //
 // What bounds it: matrix instructions on real descriptors, which draw the card's power limit
-// (three products of 16384 x 16384 run at 1.05 PFLOP/s here; a loop of nothing but the
-// instruction reaches 1.48, the library's 8192^3 product 1.2), then the selection beside them
-// (the products and operand reads alone take 164 us of the 196).
-// 16384 x 16384: 196 us against 605-635 us of k_fused_fp32; 8192 x 7936: 59 against 185 us.
-// One tile's selection after its products instead of beside the next tile's: 210 us; every
-// position tracked instead of looked for: 215 against 195 us (same box).
+// (the three products of 16384 x 16384 run at 1.13 PFLOP/s here; a loop of nothing but the
+// instruction reaches 1.48, the library's 8192^3 product 1.2); the products and operand reads
+// alone take 164 us of the 182.  16384 x 16384: 182 us against 605-635 us of k_fused_fp32;
+// 8192 x 7936: 58 against 185 us.  One tile's selection after its products instead of beside
+// the next tile's: 210 against 196 us; every position tracked instead of looked for: 215
+// against 195 us; second bests left to the compiler's order (spills): 196 against 182 us.
+// Most calls take the sieve (v3dm_sieve.h: 37 us); this pass serves low minimum scores, a zero
+// error bound and blocks of scores.
 //
 // Integer rows (kInt): descriptors uploaded as uint8 are their integer components q times the
 // row's scale d, the scale leaves the sum, and FP16 holds the integers exactly: ONE product per

@@ -49,7 +49,8 @@ enum {
 typedef struct v3dm_stats {
     int nLeft, nRight;        /* feature counts used (after rounding / clamping) */
     int nMatches;             /* matches found */
-    int nRechecked;           /* queries whose decision was settled by the exact re-check */
+    int nRechecked;           /* queries whose decision was settled by the exact re-check
+                                 (the sieve of plain calls leaves hardly any) */
     int precision;            /* V3DM_PREC_* used */
     int nFallback;            /* pairs that fell back to the exact path (shortlist modes) */
     double kernelMs;          /* accumulated time of the dominant kernel since the last reset
@@ -299,8 +300,8 @@ int v3dm_batch_match(v3dm_handle h, float minScore, float minRatio, int32_t* off
  * per query): it changes which candidates are listed, so it is never tuned. */
 int v3dm_batch_set_tuning(v3dm_handle h, int autotune, int mode, int tilesPerItem, int grid);
 /* The work-group tile shape of a form's pass: queries (plain: left features) per work-group
- * x candidate rows per tile, 128 x 64 or 256 x 64 in every form (plain FP32: 4 or 8 waves;
- * BF16 and learned codes: 2 or 4 waves), chosen by the autotuner with the tiles per item and
+ * x candidate rows per tile, 128 x 64 or 256 x 64 in every form (FP32 instruction: 4 or 8
+ * waves; else 2 or 4; the plain form's full pass, which runs where its sieve does not apply), chosen by the autotuner with the tiles per item and
  * the grid (no shape changes the result: the plain form's match set is the exact one in
  * every shape, and the shortlist forms list the same candidates).  set: queryRows 128 or 256
  * fixes the shape of the form of `mode`, 0 lets the tuner choose (default without tuning:
