@@ -739,7 +739,7 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
         else enqueue_derived(h, b, form);
     }
     if (form == 0 && sieve) {
-        launch_batch_sieve(d, b->sieveItems, b->nSieveItems, T, b->sieveBest, b->sieveSecond, nullptr, st);
+        launch_batch_sieve(d, b->sieveItems, b->nSieveItems, T, b->sieveBest, b->sieveSecond, st);
         launch_batch_sieve_decide(d, b->sieveBest, b->sieveSecond, minScore, minRatio, b->sel, b->flagList,
                                   b->counters, nullptr, st);
         launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio,
@@ -788,12 +788,13 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
             Plan const& pp = b->plan[3];
             int const np = (int)pp.items.size();
             BatchDev const d0 = dev_view(b, 3);
-            launch_batch_fb_filter(b->items[3], np, b->pairFlag, b->nPairs, b->fbItems, b->counters + kBCntFbItems,
-                                   b->segMask, st);
+            launch_batch_fb_filter(sieve ? b->sieveItems : b->items[3], sieve ? b->nSieveItems : np, b->pairFlag,
+                                   b->nPairs, b->fbItems, b->counters + kBCntFbItems, b->segMask, st);
             // (the rows of a plain run may be there already, of the same images)
             if (sieve) {
                 if (!(h->cacheDerived && b->q8Valid)) launch_batch_sieve_masked(d0, b->segMask, b->q8, b->res, st);
-                launch_batch_sieve(d0, b->sieveItems, b->nSieveItems, T, b->sieveBest, b->sieveSecond, b->pairFlag, st);
+                launch_batch_sieve_listed(d0, b->fbItems, b->counters + kBCntFbItems, T, b->sieveBest, b->sieveSecond,
+                                          st);
                 launch_batch_sieve_decide(d0, b->sieveBest, b->sieveSecond, minScore, minRatio, b->sel, b->flagList,
                                           b->counters, b->segMask, st);
             } else {
@@ -926,7 +927,7 @@ int ensure_fallback_plan(v3dm_context* h, BatchState* b)
         b->planValid[3] = true;
         b->version += 1;
     }
-    size_t const need = std::max<size_t>(b->plan[3].items.size(), 1);
+    size_t const need = std::max<size_t>({b->plan[3].items.size(), (size_t)b->nSieveItems, 1});
     if ((size_t)b->fbItemCap < need) {
         drop_graphs(b);  // captured runs hold the old buffer
         if ((rc = growi(h, b->fbItems, b->fbItemCap, need))) return rc;
@@ -1373,7 +1374,7 @@ int v3dm_batch_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
     for (int r = 0; r < reps && e == hipSuccess; ++r) {
         int const n = (int)pl.items.size();
         if (form == 0 && b->lastSieve)
-            launch_batch_sieve(d, b->sieveItems, b->nSieveItems, b->lastT, b->sieveBest, b->sieveSecond, nullptr, st);
+            launch_batch_sieve(d, b->sieveItems, b->nSieveItems, b->lastT, b->sieveBest, b->sieveSecond, st);
         else if (form == 0) launch_plain_pass(b, 0, b->items[0], n, q + r, b->lastMinScore, st);
         else if (form == 1) launch_batch_pass_bf16(d, b->items[1], n, q + r, b->partB, pl.grid, pl.qRows, st);
         else launch_batch_pass_code(d, b->items[2], n, q + r, b->partB, pl.grid, pl.qRows, st);

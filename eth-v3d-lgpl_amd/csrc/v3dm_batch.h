@@ -182,7 +182,9 @@ void launch_batch_mutual(BatchDev const& b, int const* sel, int leftRows, int2* 
 void launch_batch_sieve_rows(BatchDev const& b, int rows, signed char* q8, float* res, hipStream_t st);
 void launch_batch_sieve_masked(BatchDev const& b, int const* segMask, signed char* q8, float* res, hipStream_t st);
 void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
-                        unsigned* second, int const* pairFlag, hipStream_t st);
+                        unsigned* second, hipStream_t st);
+void launch_batch_sieve_listed(BatchDev const& b, int4 const* items, int const* nItems, float T,
+                               unsigned long long* best, unsigned* second, hipStream_t st);
 void launch_batch_sieve_decide(BatchDev const& b, unsigned long long* best, unsigned* second, float minScore,
                                float minRatio, int* sel, int* flagList, int* counters, int const* segMask,
                                hipStream_t st);

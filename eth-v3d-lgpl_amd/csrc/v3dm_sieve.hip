@@ -204,39 +204,6 @@ __global__ __launch_bounds__(256, 3) void k_sieve(SieveSet L, SieveSet R, SieveP
                bits, ldi, out, lists[wv], threadIdx.x & 63);
 }
 
-// Over a batch: item = (pair, group of 512 left features, split, tiles per split), one
-// work-group each.  pairFlag: only the flagged pairs (a learned run's fallback), or null.
-// 256 uneven uint8 pairs: 531 us (2.9 TB/s would read the rows, 3.4 POPS of int8 products) + 13 for
-// the decisions, against 2358 + 167 + 23 of the integer-row pass, its merge and its re-check.
-__global__ __launch_bounds__(256, 3) void k_batch_sieve(BatchDev b, int4 const* __restrict__ items, float T,
-                                                        unsigned long long* __restrict__ best,
-                                                        unsigned* __restrict__ second,
-                                                        int const* __restrict__ pairFlag)
-{
-    __shared__ int lists[4][kSieveList];
-    int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    int4 const w = items[blockIdx.x];
-    if (pairFlag && !pairFlag[w.x]) return;
-    BatchSeg const sl = b.seg[w.x];
-    BatchSeg const sr = b.seg[b.nPairs + w.x];
-    int const i0 = (w.y * 4 + wv) * (32 * kSieveBlocks);
-    if (i0 >= sl.n) return;
-    size_t const l0 = b.imgBase[sl.img], r0 = b.imgBase[sr.img];
-    SieveSet const L{b.q8 + l0 * kDim, b.res + l0 / kSieveGroup, b.img + l0 * kDim, sl.n};
-    SieveSet const R{b.q8 + r0 * kDim, b.res + r0 / kSieveGroup, b.img + r0 * kDim, sr.n};
-    int const t0 = w.z * w.w;
-    sieve_wave(L, R, i0, t0, min(t0 + w.w, sr.n / kSieveTile), __uint_as_float(b.maxNorm[sl.img]),
-               __uint_as_float(b.maxNorm[sr.img]), T, best + sl.qOff, second + sl.qOff, best + sr.qOff,
-               second + sr.qOff, nullptr, 0, SieveBest{}, lists[wv], threadIdx.x & 63);
-}
-
-void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
-                        unsigned* second, int const* pairFlag, hipStream_t st)
-{
-    if (nItems <= 0) return;
-    hipLaunchKernelGGL(k_batch_sieve, dim3(nItems), dim3(256), 0, st, b, items, T, best, second, pairFlag);
-}
-
 // Splits of the right features: three work-groups of four waves per CU run at a time, and a
 // wave's operand load and exact scores cost about four tiles.
 SievePlan plan_sieve(int nL, int nR)
@@ -263,6 +230,74 @@ void launch_sieve(SieveSet const& L, SieveSet const& R, SievePlan const& p, unsi
 {
     if (L.n <= 0 || R.n <= 0) return;
     hipLaunchKernelGGL(k_sieve, dim3(p.groups * p.splits), dim3(256), 0, st, L, R, p, maxNormBits, T, b, bits, ldi);
+}
+
+// Over a batch: item = (pair, group of 512 left features, split, tiles per split), one
+// work-group each.
+// 256 uneven uint8 pairs: 531 us (2.9 TB/s would read the rows, 3.4 POPS of int8 products) + 13 for
+// the decisions, against 2358 + 167 + 23 of the integer-row pass, its merge and its re-check.
+__device__ __forceinline__ void sieve_item(BatchDev const& b, int4 w, int t0, int t1, float T,
+                                           unsigned long long* __restrict__ best, unsigned* __restrict__ second,
+                                           int* list, int wv)
+{
+    BatchSeg const sl = b.seg[w.x];
+    BatchSeg const sr = b.seg[b.nPairs + w.x];
+    int const i0 = (w.y * 4 + wv) * (32 * kSieveBlocks);
+    t1 = min(t1, sr.n / kSieveTile);
+    if (i0 >= sl.n || t0 >= t1) return;
+    size_t const l0 = b.imgBase[sl.img], r0 = b.imgBase[sr.img];
+    SieveSet const L{b.q8 + l0 * kDim, b.res + l0 / kSieveGroup, b.img + l0 * kDim, sl.n};
+    SieveSet const R{b.q8 + r0 * kDim, b.res + r0 / kSieveGroup, b.img + r0 * kDim, sr.n};
+    sieve_wave(L, R, i0, t0, t1, __uint_as_float(b.maxNorm[sl.img]), __uint_as_float(b.maxNorm[sr.img]), T,
+               best + sl.qOff, second + sl.qOff, best + sr.qOff, second + sr.qOff, nullptr, 0, SieveBest{}, list,
+               threadIdx.x & 63);
+}
+
+__global__ __launch_bounds__(256, 3) void k_batch_sieve(BatchDev b, int4 const* __restrict__ items, float T,
+                                                        unsigned long long* __restrict__ best,
+                                                        unsigned* __restrict__ second)
+{
+    __shared__ int lists[4][kSieveList];
+    int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int4 const w = items[blockIdx.x];
+    sieve_item(b, w, w.z * w.w, (w.z + 1) * w.w, T, best, second, lists[wv], wv);
+}
+
+// The items of the pairs that a learned run hands over (counted by an earlier kernel): few, so
+// each is cut into runs of kSieveRun tiles, taken by a fixed grid: a run is a wave's shortest
+// useful chain.  Whole items, one work-group each, of which the others leave at once: 56 us on the
+// 256-pair batch, 31 so.
+constexpr int kSieveRun = 8;
+
+__global__ __launch_bounds__(256, 3) void k_batch_sieve_listed(BatchDev b, int4 const* __restrict__ items,
+                                                               int const* __restrict__ nItems, float T,
+                                                               unsigned long long* __restrict__ best,
+                                                               unsigned* __restrict__ second)
+{
+    __shared__ int lists[4][kSieveList];
+    int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int const n = __builtin_amdgcn_readfirstlane(*nItems);
+    if (n == 0) return;
+    int const runs = (items[0].w + kSieveRun - 1) / kSieveRun;  // every item has the same tiles per split
+    for (int u = blockIdx.x; u < n * runs; u += gridDim.x) {
+        int4 const w = items[u / runs];
+        int const t0 = w.z * w.w + (u % runs) * kSieveRun;
+        sieve_item(b, w, t0, min(t0 + kSieveRun, (w.z + 1) * w.w), T, best, second, lists[wv], wv);
+    }
+}
+
+void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
+                        unsigned* second, hipStream_t st)
+{
+    if (nItems <= 0) return;
+    hipLaunchKernelGGL(k_batch_sieve, dim3(nItems), dim3(256), 0, st, b, items, T, best, second);
+}
+
+void launch_batch_sieve_listed(BatchDev const& b, int4 const* items, int const* nItems, float T,
+                               unsigned long long* best, unsigned* second, hipStream_t st)
+{
+    if (b.nPairs <= 0) return;
+    hipLaunchKernelGGL(k_batch_sieve_listed, dim3(768), dim3(256), 0, st, b, items, nItems, T, best, second);
 }
 
 // ------------------------------------------------------------------------------ decisions
