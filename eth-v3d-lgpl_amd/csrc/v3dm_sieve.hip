@@ -38,6 +38,9 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // maximum of (score, ~index) returns the smaller of two keys, which goes to the second best's
 // maximum; so every key but the largest reaches it, and equal scores keep the smallest index.
 // A wave whose list overflows marks all its features for the exact re-check instead.
+// With 512 entries a tenth of 8192 x 8192 rows in one cluster of nearly equal ones overflowed some
+// lists; with 2048 (32 KiB a group, no group fewer per CU) the call takes 0.25 ms there, as the
+// FP32 instruction did, and the lists overflow from about a sixth of both sets on.
 //
 // What bounds it: the int8 matrix instructions (16384 x 16384: 2^20 of them, 20 us of the 37),
 // then the tail, where each wave waits for the rows and the atomics of its few candidates
@@ -45,7 +48,7 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // against 182 + 6 + 14 of the FP16 split pass, its merge and its re-check (605 of the FP32
 // instruction); 4096 x 4096: 12 + 3 against 24 + 5 + 4; 480 x 512: 9 + 2 against 8 + 5 + 4.
 constexpr int kSieveBlocks = 4;
-constexpr int kSieveList = 512;
+constexpr int kSieveList = 2048;
 
 __device__ __forceinline__ int max3i(int a, int b, int c) { return max(max(a, b), c); }
 
