@@ -303,6 +303,7 @@ void layout_segments(BatchState* b, std::vector<BatchSeg>& seg)
 // Plain plan: items (pair, left block of leftRows features, split, tiles per split).
 Plan plan_plain(BatchState* b, int tiles, int grid, int leftRows = 128)
 {
+    tiles = std::min(tiles, kSplitMaxTiles / 2);  // (64-row tiles; the split pass's have 32)
     Plan pl;
     pl.tiles = tiles;
     pl.grid = grid;

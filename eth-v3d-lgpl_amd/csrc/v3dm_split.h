@@ -36,6 +36,7 @@ constexpr int kIntRowBytes = 256;    // integer components in FP16
 constexpr int kSplitRowBytes = 512;  // per half (64 components): 128 B of hi, 128 B of lo
 constexpr int kSplitRowPad = 256;    // split buffers hold a multiple of 256 rows
 constexpr int kSplitTile = 32;       // right features per tile
+constexpr int kSplitMaxTiles = 1 << 16;  // tiles of one work unit: their byte offsets fit 32 bits
 
 // One feature set in one launch: its FP32 rows X (copied from the device array src, or
 // dequantised from the uint8 rows src as SIFT_Feature::normalizeDescriptor, or in place), the

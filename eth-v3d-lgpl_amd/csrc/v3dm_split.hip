@@ -282,6 +282,7 @@ __device__ __forceinline__ void split_block(unsigned char const* __restrict__ L,
                                             float thr)
 {
     using Rows = SplitRows<kInt>;
+    static_assert((long long)kSplitMaxTiles * Rows::kTileBytes < (1LL << 31), "32-bit offsets of a unit's tiles");
     // an opaque copy of the thread index: in the persistent kernel it keeps the per-lane
     // offsets derived from it inside the item loop instead of live across it
     int tid = threadIdx.x;
@@ -294,8 +295,11 @@ __device__ __forceinline__ void split_block(unsigned char const* __restrict__ L,
     int const nBlk = min(max((nL - i0) / 32, 0), 2);  // column blocks of this wave that exist
 
     int const src = split_src<kInt>(tid);
-    int const bytes = t1 * Rows::kTileBytes;
-    split_stage<kInt, kW>(R, bytes, t0, lds.stage[0], src, wv);
+    // the resource spans the unit's own tiles: their offsets fit 32 bits (kSplitMaxTiles), an
+    // image's need not (a tile of split rows is 16 KiB: from 2^17 tiles on they would not)
+    R += (size_t)t0 * Rows::kTileBytes;
+    int const bytes = (t1 - t0) * Rows::kTileBytes;
+    split_stage<kInt, kW>(R, bytes, 0, lds.stage[0], src, wv);
 
     // rows past nL are inside the buffer (a multiple of kSplitRowPad rows) and never used
     v8h bh[2][8], bl[2][8];
@@ -338,7 +342,7 @@ __device__ __forceinline__ void split_block(unsigned char const* __restrict__ L,
         wait_lds_loads();
         __syncthreads();  // tile t is staged; every wave is done with the other stage
         int const cur = (t - t0) & 1;
-        if (t + 1 < t1) split_stage<kInt, kW>(R, bytes, t + 1, lds.stage[cur ^ 1], src, wv);
+        if (t + 1 < t1) split_stage<kInt, kW>(R, bytes, t + 1 - t0, lds.stage[cur ^ 1], src, wv);
         // the partials of tile t - 2 were written before this barrier
         if (t >= t0 + 2 && wv == t % kW) split_merge_rows<kInt, kW>(lds, t - 2, lane, rowPart);
         TileSide<kInt> now{};

@@ -223,3 +223,27 @@ def test_batch_fallback_split(dtype, cache, plain_first):
                 assert np.array_equal(res[p], w)
     assert flags.sum() >= 1
     m.close()
+
+
+@pytest.mark.parametrize("tiles", [64, 1 << 30])
+def test_batch_image_of_many_rows(tiles):
+    """An image whose split rows span more than 4 GiB: features past row 2^23 are scored by their
+    own rows (the zero rows between score 0 and change no decision).  One work unit's tiles are
+    bounded whatever the caller asks for."""
+    n, far = 2 ** 23 + 96, 2 ** 23
+    qL, qR, _ = synth.make_pair(96, 96, 0.6, config=1, pair=71)
+    _, near, _ = synth.make_pair(96, 96, 0.6, config=1, pair=72)
+    L, R = synth.dequantise(qL), np.concatenate([synth.dequantise(near), synth.dequantise(qR)])
+    rows = np.zeros((96 + n, 128), np.float32)
+    rows[:96], rows[96:192], rows[96 + far:] = L, R[:96], R[96:]
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([96, n], rows)
+    del rows
+    m.batch_set_pairs([0], [1])
+    m.batch_set_tuning(False, v3dmatch.PREC_FP32, tiles, 512)
+    print(f"case split image of 2^23 + 96 rows, {tiles} tiles an item", flush=True)
+    got = m.batch_match(0.2, 0.8)[0]
+    m.close()
+    want = oracle.find_putative_matches(L, R, 0.2, 0.8)
+    want[:, 1] += np.where(want[:, 1] >= 96, far - 96, 0)
+    assert len(want) > 20 and np.array_equal(got, want)
