@@ -451,7 +451,8 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
                 HIPCHECK(h, hipMalloc(&h->dQ, qb));
                 h->dQBytes = qb;
             }
-            size_t const rows = (size_t)(left ? h->capL : h->capR);
+            // the full pass loads the scales of whole blocks of left features
+            size_t const rows = (size_t)roundUp(left ? h->capL : h->capR, kSplitRowPad);
             if (!(left ? h->intScaleL : h->intScaleR))
                 HIPCHECK(h, hipMalloc(left ? &h->intScaleL : &h->intScaleR, rows * sizeof(float)));
             HIPCHECK(h, hipMemcpyAsync(h->dQ, src, (size_t)n * kDim, hipMemcpyHostToDevice, h->stream));

@@ -247,3 +247,20 @@ def test_batch_image_of_many_rows(tiles):
     want = oracle.find_putative_matches(L, R, 0.2, 0.8)
     want[:, 1] += np.where(want[:, 1] >= 96, far - 96, 0)
     assert len(want) > 20 and np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("capacity", [96, 384, 2085])
+def test_u8_odd_capacity(capacity):
+    """uint8 pairs of a handle whose buffers hold an odd number of 128-row blocks, at thresholds
+    that take the full pass on integer rows: its last work-group loads whole blocks of scales."""
+    print(f"case integer rows, capacity {capacity}", flush=True)
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(capacity, capacity)
+    n = capacity // 32 * 32
+    qL, qR, _ = synth.make_pair(n, n, 0.5, config=1, pair=capacity)
+    m.set_left_u8(qL)
+    m.set_right_u8(qR)
+    _check(m, synth.dequantise(qL), synth.dequantise(qR), 0.4, 0.99)
+    _check(m, synth.dequantise(qL), synth.dequantise(qR), -2.0, -1.0)
+    m.close()
