@@ -459,15 +459,18 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
             from = kRowsU8;
         }
     }
-    if (++h->prepEpoch == 0) {
-        HIPCHECK(h, hipMemsetAsync(h->maxNormBits, 0, 4 * sizeof(unsigned int), h->stream));
-        h->prepEpoch = 1;
+    // a side's own epoch and its own two words: the other side's norm stays valid over a wrap
+    unsigned int* const maxNorm = h->maxNormBits + (left ? 0 : kMaxNormR);
+    unsigned& epoch = h->prepEpoch[left ? 0 : 1];
+    if (++epoch == 0) {
+        HIPCHECK(h, hipMemsetAsync(maxNorm, 0, 2 * sizeof(unsigned int), h->stream));
+        epoch = 1;
     }
     // the previous call's launch has ended (every call waits for its own)
     if (n > 0) __atomic_store_n(h->splitFitHost + (left ? 0 : 1), 1, __ATOMIC_RELEASE);
     launch_prep_rows(from, from == kRowsU8 ? (void const*)h->dQ : src, dst, n, left ? h->normL : h->normR,
-                     h->maxNormBits + (left ? 0 : kMaxNormR), h->prepEpoch, left ? h->intScaleL : h->intScaleR,
-                     left ? h->q8L : h->q8R, left ? h->resL : h->resR, h->splitFitDev + (left ? 0 : 1), h->stream);
+                     maxNorm, epoch, left ? h->intScaleL : h->intScaleR, left ? h->q8L : h->q8R,
+                     left ? h->resL : h->resR, h->splitFitDev + (left ? 0 : 1), h->stream);
     h->haveSplit = false;
     (left ? h->haveIntL : h->haveIntR) = from == kRowsU8;
     HIPCHECK(h, hipGetLastError());
@@ -630,6 +633,15 @@ int v3dm_debug_mutual_wait(v3dm_handle h, int spinLimit, int neverReady)
     if (!h) return fail(nullptr, V3DM_ERR_INVALID, "null handle");
     h->mutualWait.spinLimit = spinLimit < 0 ? kMutualSpinLimit : (unsigned)spinLimit;
     h->mutualWait.readXor = neverReady ? 0x80000000u : 0u;
+    return V3DM_OK;
+}
+
+int v3dm_debug_prep_epoch(v3dm_handle h, unsigned epoch)
+{
+    if (!h) return fail(nullptr, V3DM_ERR_INVALID, "null handle");
+    if (epoch < h->prepEpoch[0] || epoch < h->prepEpoch[1])  // the words hold the present epochs
+        return fail(h, V3DM_ERR_INVALID, "epochs only grow");
+    h->prepEpoch[0] = h->prepEpoch[1] = epoch;
     return V3DM_OK;
 }
 

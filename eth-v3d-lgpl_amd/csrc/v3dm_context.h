@@ -53,7 +53,7 @@ struct v3dm_context {
     int* splitFitHost = nullptr;      // mapped: [0] left, [1] right set in the split pass's range
     int* splitFitDev = nullptr;       // the same memory as the kernels address it
     unsigned int* maxNormBits = nullptr;  // [0] = left, [kMaxNormR] = right, with epochs above
-    unsigned prepEpoch = 0;               // of the last launch_prep_rows
+    unsigned prepEpoch[2] = {0, 0};       // of the sides' last launch_prep_rows
     v3dm::Top2* colPart = nullptr;
     v3dm::Top2* rowPart = nullptr;
     int* colMax = nullptr;

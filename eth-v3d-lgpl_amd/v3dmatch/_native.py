@@ -70,6 +70,7 @@ SIGNATURES = {
     "v3dm_batch_set_tile_shape": (_I, [_P, _I, _I]),
     "v3dm_batch_get_tile_shape": (_I, [_P, _I, _IP, _IP]),
     "v3dm_debug_mutual_wait": (_I, [_P, _I, _I]),
+    "v3dm_debug_prep_epoch": (_I, [_P, C.c_uint]),
     "v3dm_set_left_device": (_I, [_P, _I, _FP]),
     "v3dm_set_right_device": (_I, [_P, _I, _FP]),
     "v3dm_set_left_u8": (_I, [_P, _I, _FP]),

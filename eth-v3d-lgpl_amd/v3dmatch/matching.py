@@ -184,6 +184,10 @@ class SIFT_Matching:
         debug_mutual_wait(8, True) makes the next calls fail; debug_mutual_wait() restores."""
         self._check(self._lib.v3dm_debug_mutual_wait(self._h, int(spin_limit), int(bool(never_ready))))
 
+    def debug_prep_epoch(self, epoch):
+        """Test hook: moves the upload counters forward (v3dm_debug_prep_epoch)."""
+        self._check(self._lib.v3dm_debug_prep_epoch(self._h, int(epoch)))
+
     @staticmethod
     def fallback_allowed_misses(accepted, min_recall=0.995, rule=0):
         """Misses a sampled check of `accepted` exact matches tolerates before the plain

@@ -144,6 +144,9 @@ int v3dm_set_fallback_rule(v3dm_handle h, int rule);
  * count visible, so every work-group but the first runs out of its wait (with several
  * work-groups, i.e. more than 1024 left features).  0, -1 restores normal operation. */
 int v3dm_debug_mutual_wait(v3dm_handle h, int spinLimit, int neverReady);
+/* Test hook (for tests only): moves both sides' upload counters forward to `epoch`, so that a
+ * test reaches their 32-bit wrap.  V3DM_ERR_INVALID for a value that has been passed. */
+int v3dm_debug_prep_epoch(v3dm_handle h, unsigned epoch);
 /* The misses a sampled check of `accepted` exact matches tolerates at recall minRecall
  * under the threshold rule: the largest m with (float)(accepted - m) / (float)accepted not
  * below minRecall (0 for minRecall 1, `accepted` for minRecall 0); -1 when accepted is

@@ -154,3 +154,36 @@ def matcher_guided():
     m.allocate(512, 512, True)
     yield m
     m.close()
+
+
+@pytest.mark.parametrize("first", [0xfffffffe, 0xffffffff])
+@pytest.mark.parametrize("order", ["left right", "right left", "left right left", "right left right"])
+def test_upload_counters_wrap(first, order):
+    """The sets' largest norms are kept under the number of the upload; past its 32-bit wrap each
+    side still has its own.  The side uploaded second holds rows whose int8 rounding errors all
+    point the same way, the other side rows that int8 holds exactly, and the scores lie within
+    those errors above the minimum: with a norm of 0 for the exact side the bound would drop them."""
+    print(f"case sieve upload counter {first} order {order}", flush=True)
+    rng = np.random.default_rng(8)
+    n = 512
+    X = np.rint(256 * _unit(rng.gamma(0.5, 1.0, (n, 128)))).clip(0, 120)
+    X = (X / 256).astype(np.float32)
+    Y = np.empty_like(X)
+    for i in range(n):  # the largest multiple of row i below a score of 0.903
+        for a in np.linspace(0.8, 1.3, 201):
+            y = ((np.floor(a * 256 * X[i]) + 0.45) / 256).astype(np.float32)
+            if float(y @ X[i]) > 0.903:
+                break
+            Y[i] = y
+    L, R = (X, Y) if order.split()[0] == "left" else (Y, X)
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(n, n)
+    m.debug_prep_epoch(first)
+    for side in order.split():
+        (m.setLeftFeatures if side == "left" else m.setRightFeatures)(n, L if side == "left" else R)
+    want = oracle.find_putative_matches(L, R, 0.9, -1.0)
+    assert len(want) > 100 and np.array_equal(m.find_putative_matches_array(0.9, -1.0), want)
+    with pytest.raises(v3dmatch.V3DMError):
+        m.debug_prep_epoch(0)
+    m.close()
