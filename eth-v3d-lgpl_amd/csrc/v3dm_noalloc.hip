@@ -13,8 +13,8 @@
 // v3dm_find_putative_matches on the same descriptors.
 //
 // All calls on one GPU share its array: calls that overlap in time on one GPU (other
-// streams, other threads) race.  Counters and norm maxima are cleared by a kernel at the
-// start of every call; the status words carry a per-device epoch.
+// streams, other threads) race, and only they: counters, norm maxima and tickets are cleared by a
+// kernel at the start of every call; the status words carry a per-device epoch.
 #include <algorithm>
 #include <atomic>
 #include <cstdio>
@@ -72,11 +72,21 @@ __global__ __launch_bounds__(256) void k_noalloc_copy_pad(float const* __restric
     reinterpret_cast<float4*>(dst)[i] = v;
 }
 
-__global__ void k_noalloc_clear(int* __restrict__ counters, unsigned int* __restrict__ maxNorm)
+// Counters, norm maxima and the re-check's tickets of nRows listed queries.  The tickets too: a
+// call that overlapped another on this GPU may have left some above zero.
+__global__ __launch_bounds__(256) void k_noalloc_clear(int* __restrict__ counters, unsigned int* __restrict__ maxNorm,
+                                                       int* __restrict__ tickets, int nRows)
 {
-    int const t = threadIdx.x;
+    int const t = blockIdx.x * 256 + threadIdx.x;
     if (t < kNumCounters) counters[t] = 0;
     if (t <= kMaxNormR) maxNorm[t] = 0u;
+    if (t < nRows) tickets[t] = 0;
+}
+
+__global__ __launch_bounds__(256) void k_noalloc_fill(int* __restrict__ p, int n, int v)
+{
+    int const t = blockIdx.x * 256 + threadIdx.x;
+    if (t < n) p[t] = v;
 }
 
 // the match count, or -1 when the mutual check's ordering wait ran out (its epoch in
@@ -157,12 +167,15 @@ int v3dm_match_device_noalloc(const float* leftDesc, int nLeft, const float* rig
     unsigned long long* const status = reinterpret_cast<unsigned long long*>(b + kOffStatus);
     int* const stripes = reinterpret_cast<int*>(b + kOffStripes);
     int* const counters = reinterpret_cast<int*>(b + kOffCounters);
+    int* const tickets = reinterpret_cast<int*>(b + kOffTickets);
 
     unsigned ep = ds->epoch.fetch_add(1) + 1;
     if (ep == 0) ep = ds->epoch.fetch_add(1) + 1;  // epoch 0 marks never-written status words
     int const capL = std::max(128, (nL + 127) / 128 * 128), capR = std::max(128, (nR + 127) / 128 * 128);
     bool const work = nL > 0 && nR > 0;
-    hipLaunchKernelGGL(k_noalloc_clear, dim3(1), dim3(64), 0, st, counters, maxNorm);
+    static_assert(kNumCounters <= 256 && kMaxNormR < 256, "cleared by the first work-group");
+    hipLaunchKernelGGL(k_noalloc_clear, dim3((capL + capR + 255) / 256), dim3(256), 0, st, counters, maxNorm, tickets,
+                       capL + capR);
     if (work) {
         hipLaunchKernelGGL(k_noalloc_copy_pad, dim3((capL * (kDim / 4) + 255) / 256), dim3(256), 0, st, leftDesc, nL,
                            capL, L);
@@ -175,7 +188,7 @@ int v3dm_match_device_noalloc(const float* leftDesc, int nLeft, const float* rig
         launch_merge_decide(colPart, p.splits, capL, rowPart, p.leftBlocks, capR, nL, nR, normL, normR, maxNorm,
                             kEpsRelFp32, minScore, minRatio, colMax, rowMax, flagList, capL, counters, st);
         launch_recheck_exact(L, R, nL, nR, flagList, capL, capR, counters, minScore, minRatio, colMax, rowMax,
-                             rpart, reinterpret_cast<int*>(b + kOffTickets), kRecheckGrid, st);
+                             rpart, tickets, kRecheckGrid, st);
     }
     launch_mutual_compact(colMax, rowMax, work ? nL : 0, nR, status, ep, stripes, reinterpret_cast<int2*>(pairs),
                           counters, nullptr, st);
@@ -183,6 +196,18 @@ int v3dm_match_device_noalloc(const float* leftDesc, int nLeft, const float* rig
     e = hipGetLastError();
     if (e != hipSuccess) return noalloc_fail(V3DM_ERR_HIP, "launch", e);
     return V3DM_OK;
+}
+
+int v3dm_debug_noalloc_tickets(int value)
+{
+    DeviceScratch* ds = nullptr;
+    hipError_t e = scratch_of_current_device(ds);
+    if (e != hipSuccess) return noalloc_fail(V3DM_ERR_HIP, "hipGetSymbolAddress(scratch)", e);
+    hipLaunchKernelGGL(k_noalloc_fill, dim3((2 * kNoAllocCap + 255) / 256), dim3(256), 0, nullptr,
+                       reinterpret_cast<int*>(ds->base + kOffTickets), 2 * kNoAllocCap, value);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipDeviceSynchronize();
+    return e == hipSuccess ? V3DM_OK : noalloc_fail(V3DM_ERR_HIP, "tickets", e);
 }
 
 const char* v3dm_noalloc_last_error(void) { return gNoAllocErr; }

@@ -181,6 +181,9 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch);
 int v3dm_match_device_noalloc(const float* leftDesc, int nLeft, const float* rightDesc, int nRight, float minScore,
                               float minRatio, int32_t* pairs, int32_t* count, void* stream);
 const char* v3dm_noalloc_last_error(void);
+/* Test hook (for tests only): fills the re-check's tickets in the current device's array with
+ * `value`, as calls that overlapped may leave them; waits for the device. */
+int v3dm_debug_noalloc_tickets(int value);
 /* Measurement helper (no reference analogue): the approximate scores the pass of mode
  * V3DM_PREC_FP32 / BF16 / FP8 computes for the first nRows left x nCols right features of
  * the current sets (same instruction, operand rounding and summation order as the pass,

@@ -122,3 +122,19 @@ def test_noalloc_rejects_sizes_above_the_maximum():
     qL, qR, _ = synth.make_pair(64, 64, 0.4, config=1, pair=4)
     L = synth.dequantise(qL)
     assert _noalloc(lib, hip, L, np.zeros((31, 128), np.float32)).shape == (0, 2)
+
+
+@pytest.mark.parametrize("value", [0, 1, -3, 1000])
+@pytest.mark.parametrize("n", [64, 2048])
+def test_noalloc_tickets_of_spoiled_calls(n, value):
+    """Tickets that overlapping calls left behind do not reach a later call (copies score 1: every
+    query goes to the exact re-check)."""
+    say(f"case noalloc tickets {value} n {n}")
+    lib, hip = _lib(), _Hip()
+    qL, _, _ = synth.make_pair(n, n, 0.4, config=1, pair=8)
+    L = synth.dequantise(qL)
+    R = np.ascontiguousarray(L[np.random.default_rng(1).permutation(n)])
+    assert lib.v3dm_debug_noalloc_tickets(value) == 0
+    want = oracle.find_putative_matches(L, R, 0.9, 0.8)
+    assert len(want) > n // 2
+    assert np.array_equal(_noalloc(lib, hip, L, R), want)
