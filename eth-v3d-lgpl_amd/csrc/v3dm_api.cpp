@@ -20,6 +20,7 @@
 #include "v3dm_ext.h"
 #include "v3dm_context.h"
 #include "v3dm_sieve.h"
+#include "v3dm_source.h"
 #include "v3dm_split.h"
 
 using namespace v3dm;
@@ -432,15 +433,15 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
         if (kind == kHostF32) {
             HIPCHECK(h, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream));
         } else if (kind == kDeviceF32) {
-            // the row kernel reads this device's own memory, apart from the set's buffer and
-            // aligned for its loads; any other pointer the copy engine takes is copied first
-            char const *s0 = static_cast<char const*>(src), *d0 = reinterpret_cast<char const*>(dst);
-            bool const apart = s0 + bytes <= d0 || d0 + bytes <= s0;
             hipPointerAttribute_t at{};
-            bool const known = hipPointerGetAttributes(&at, src) == hipSuccess;
+            void* base = nullptr;
+            size_t size = 0;
+            bool const known = hipPointerGetAttributes(&at, src) == hipSuccess &&
+                               hipMemGetAddressRange((hipDeviceptr_t*)&base, &size, (hipDeviceptr_t)src) == hipSuccess;
             if (!known) (void)hipGetLastError();
-            if (known && at.type == hipMemoryTypeDevice && at.device == h->device && apart &&
-                (reinterpret_cast<uintptr_t>(src) & 7) == 0)
+            if (known && rows_readable(reinterpret_cast<uintptr_t>(src), bytes,
+                                       at.type == hipMemoryTypeDevice && at.device == h->device,
+                                       reinterpret_cast<uintptr_t>(base), size, reinterpret_cast<uintptr_t>(dst)))
                 from = kRowsF32;
             else
                 HIPCHECK(h, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, h->stream));
