@@ -555,7 +555,7 @@ int ensure_sample_plan(v3dm_context* h, BatchState* b)
     }
     BCHECK(h, hipMalloc(&b->pairFlag, 5 * P * sizeof(int)));
     BCHECK(h, hipMalloc(&b->segMask, 2 * P * sizeof(int)));
-    BCHECK(h, hipMemset(b->pairFlag, 0, 5 * P * sizeof(int)));
+    BCHECK(h, hipMemsetAsync(b->pairFlag, 0, 5 * P * sizeof(int), h->stream));  // the runs' stream
     BCHECK(h, hipHostMalloc(&b->hostChk, 5 * P * sizeof(int), hipHostMallocDefault));
     std::memset(b->hostChk, 0, 5 * P * sizeof(int));
     b->checkPending = false;

@@ -153,7 +153,9 @@ int ensure_sample(v3dm_context* h, ExtState* e)
     EXTCHECK(h, hipMalloc(&e->sFlags, (kSampleRows + 1) * sizeof(int)));
     EXTCHECK(h, hipMalloc(&e->sRpart, (size_t)(kSampleRows + 1) * kRecheckMaxChunks * sizeof(Top2)));
     EXTCHECK(h, hipMalloc(&e->sTickets, (kSampleRows + 1) * sizeof(int)));
-    EXTCHECK(h, hipMemset(e->sTickets, 0, (kSampleRows + 1) * sizeof(int)));
+    // on the handle's stream, which the side stream waits for before its first check (evFork): a
+    // memset of the null stream is not ordered before a non-blocking stream's kernels
+    EXTCHECK(h, hipMemsetAsync(e->sTickets, 0, (kSampleRows + 1) * sizeof(int), h->stream));
     EXTCHECK(h, hipMalloc(&e->sCounters, kNumCounters * sizeof(int)));
     EXTCHECK(h, hipHostMalloc(&e->sHost, kSampleRows * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     EXTCHECK(h, hipHostGetDevicePointer((void**)&e->sHostDev, e->sHost, 0));

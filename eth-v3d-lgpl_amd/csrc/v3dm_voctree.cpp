@@ -172,7 +172,8 @@ int v3dm_voctree_create(v3dm_voctree* out, int device, int branchFactor, int dep
     t->maxParents = depth > 1 ? t->levelStarts[depth - 1] - t->levelStarts[depth - 2] : 1;
     hipError_t e = hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&t->dNodes, (size_t)(nodes + 32) * kDim * sizeof(float));
-    if (e == hipSuccess) e = hipMemset(t->dNodes, 0, (size_t)(nodes + 32) * kDim * sizeof(float));
+    // on the tree's stream: a memset of the null stream is not ordered before a non-blocking one's work
+    if (e == hipSuccess) e = hipMemsetAsync(t->dNodes, 0, (size_t)(nodes + 32) * kDim * sizeof(float), t->stream);
     if (e == hipSuccess) e = hipMalloc(&t->cnt, (size_t)t->maxParents * kVtBinStride * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&t->cursor, (size_t)t->maxParents * kVtBinStride * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&t->counters, kVtCounters * sizeof(int));
@@ -182,7 +183,7 @@ int v3dm_voctree_create(v3dm_voctree* out, int device, int branchFactor, int dep
         (void)hipGetLastError();
         t->dSplit = nullptr;
     }
-    if (t->dSplit) e = hipMemset(t->dSplit, 0, splitBytes);
+    if (t->dSplit) e = hipMemsetAsync(t->dSplit, 0, splitBytes, t->stream);
     if (e != hipSuccess) {
         v3dm_voctree_destroy(t);
         return vfail(e == hipErrorOutOfMemory ? V3DM_ERR_NOMEM : V3DM_ERR_HIP,
