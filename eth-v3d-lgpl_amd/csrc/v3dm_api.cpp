@@ -235,9 +235,11 @@ int enqueue_decisions(v3dm_context* h, unsigned const* bits, float minScore, flo
     if (sieve_fits(h, minScore, minRatio, &T)) {
         if ((rc = prof_begin(h))) return rc;
         launch_sieve_pass(h, T, bits);
-        if ((rc = prof_end(h))) return rc;
+        rc = prof_end(h);
+        // also after an error: the decisions leave the sieve's entries at zero for the next call
         launch_sieve_finish(h->dL, h->dR, nL, nR, sieve_best(h), h->flagList, h->capL, h->capR, h->results, minScore,
                             minRatio, h->colMax, h->rowMax, h->rpart, h->rtickets, bits, h->capL, st);
+        if (rc) return rc;
     } else {
         FusedPlan const p = score_plan(h);
         if (split_fits(h) && (rc = ensure_split_rows(h))) return rc;
@@ -853,12 +855,14 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
                 else launch_score_pass(h, p, nullptr, h->lastMinScore);
             }
             if (e == hipSuccess) e = hipEventRecord(b, h->stream);
-            if (sieve) {  // no decisions follow that would leave the bests at zero
+            if (sieve) {  // no decisions follow that would leave the bests at zero (also after an error)
                 size_t const n = (size_t)h->capL + h->capR;
-                if (e == hipSuccess) e = hipMemsetAsync(h->sieveBest, 0, n * sizeof(unsigned long long), h->stream);
-                if (e == hipSuccess) e = hipMemsetAsync(h->sieveSecond, 0, n * sizeof(unsigned), h->stream);
-                if (e == hipSuccess) e = hipMemsetAsync(h->results + kCntFlag, 0, sizeof(int), h->stream);
-                if (e == hipSuccess) e = hipMemsetAsync(h->results + kCntFlagR, 0, sizeof(int), h->stream);
+                for (hipError_t const c :
+                     {hipMemsetAsync(h->sieveBest, 0, n * sizeof(unsigned long long), h->stream),
+                      hipMemsetAsync(h->sieveSecond, 0, n * sizeof(unsigned), h->stream),
+                      hipMemsetAsync(h->results + kCntFlag, 0, sizeof(int), h->stream),
+                      hipMemsetAsync(h->results + kCntFlagR, 0, sizeof(int), h->stream)})
+                    if (e == hipSuccess) e = c;
             }
             launches = reps;
         }

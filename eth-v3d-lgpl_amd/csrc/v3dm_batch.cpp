@@ -1381,10 +1381,10 @@ int v3dm_batch_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
         else launch_batch_pass_code(d, b->items[2], n, q + r, b->partB, pl.grid, pl.qRows, st);
     }
     if (e == hipSuccess) e = hipEventRecord(b->evB, st);
-    if (form == 0 && b->lastSieve) {  // no decisions follow that would leave the entries at zero
-        if (e == hipSuccess) e = hipMemsetAsync(b->sieveBest, 0, b->sieveCap * sizeof(unsigned long long), st);
-        if (e == hipSuccess) e = hipMemsetAsync(b->sieveSecond, 0, b->sieveCap * sizeof(unsigned), st);
-    }
+    if (form == 0 && b->lastSieve)  // no decisions follow that would leave the entries at zero (also after an error)
+        for (hipError_t const c : {hipMemsetAsync(b->sieveBest, 0, b->sieveCap * sizeof(unsigned long long), st),
+                                   hipMemsetAsync(b->sieveSecond, 0, b->sieveCap * sizeof(unsigned), st)})
+            if (e == hipSuccess) e = c;
     if (e == hipSuccess) e = hipEventSynchronize(b->evB);
     float ms = 0.0f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, b->evA, b->evB);
