@@ -115,6 +115,7 @@ struct BatchState {
     // so that a few pairs still spread over the whole GPU)
     Plan plan[4];
     bool planValid[4] = {false, false, false, false};
+    bool planPass[4] = {false, false, false, false};  // ... and is ready for its pass (else the layout alone)
     int4* items[4] = {nullptr, nullptr, nullptr, nullptr};
     int itemCap[4] = {0, 0, 0, 0};
     BatchSeg* segD[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -416,7 +417,8 @@ Plan plan_short_batch(BatchState* b, int tiles, int grid, int maxSplits, bool wh
     return pl;
 }
 
-int upload_plan(v3dm_context* h, BatchState* b, int form, Plan const& pl)
+// pass: with room for the partials of the plan's pass (else the layout of the queries alone).
+int upload_plan(v3dm_context* h, BatchState* b, int form, Plan const& pl, bool pass = true)
 {
     int rc;
     if ((rc = growi(h, b->items[form], b->itemCap[form], pl.items.size()))) return rc;
@@ -424,7 +426,10 @@ int upload_plan(v3dm_context* h, BatchState* b, int form, Plan const& pl)
     if ((rc = growi(h, b->blkInfo[form], b->blkInfoCap[form], pl.blocks.size()))) return rc;
     if (form == 0 || form == 3) {
         // at least one slot per query row: the re-check's partials go there after the merge
-        if ((rc = grow(h, b->partF, b->partFCap, std::max(pl.partSlots, (size_t)b->qRows)))) return rc;
+        if ((rc = grow(h, b->partF, b->partFCap, std::max(pass ? pl.partSlots : 0, (size_t)b->qRows)))) {
+            b->planValid[0] = b->planValid[3] = false;  // the buffer is both plans'
+            return rc;
+        }
     } else {
         if ((rc = grow(h, b->partB, b->partBCap, pl.partSlots * 2))) return rc;
     }
@@ -849,10 +854,15 @@ int time_pass(v3dm_context* h, BatchState* b, int form, Plan const& pl, float& m
 // rows against 64-candidate tiles, i.e. 2 or 4 waves (FP32 rows: 4 or 8) for the plain form's
 // full pass, 2 or 4 waves for
 // the BF16 and code passes) for a form: the given override, or the fastest candidate
-// measured on this batch, or the default when tuning is off.
-int ensure_plan(v3dm_context* h, BatchState* b, int form)
+// measured on this batch, or the default when tuning is off.  pass = false: for a run that takes
+// the sieve and of this plan needs the query layout alone; nothing is timed (the 16 candidates
+// of the plain form took 0.23 s on the 256-pair batch, whose run takes 0.9 ms) and no partials
+// are allocated, until a run takes the pass.
+int ensure_plan(v3dm_context* h, BatchState* b, int form, bool pass)
 {
-    if (b->planValid[form]) return V3DM_OK;
+    if (b->planValid[form] && (b->planPass[form] || !pass)) return V3DM_OK;
+    b->planValid[form] = false;  // (should this fail, the next run plans again)
+    drop_graphs(b);              // captured runs hold the old buffers
     int dev = 0;
     (void)hipGetDevice(&dev);
     int cus = 256;
@@ -881,7 +891,7 @@ int ensure_plan(v3dm_context* h, BatchState* b, int form)
         bestT = b->forceTiles[form] > 0 ? b->forceTiles[form] : bestT;
         bestQ = b->forceQRows[form] > 0 ? b->forceQRows[form] : bestQ;
         bestG = b->forceGrid[form] > 0 ? b->forceGrid[form] : gridCands(bestQ)[0];
-    } else if (b->autotune) {
+    } else if (b->autotune && pass) {
         for (int q : shapeCands)
             for (int t : tileCands)
                 for (int g : gridCands(q)) {
@@ -896,13 +906,13 @@ int ensure_plan(v3dm_context* h, BatchState* b, int form)
                     }
                 }
     }
-    drop_graphs(b);
     Plan pl = make(bestT, bestG, bestQ);
     pl.passMs = bestMs;
-    int const rc = upload_plan(h, b, form, pl);
+    int const rc = upload_plan(h, b, form, pl, pass);
     if (rc) return rc;
     b->plan[form] = std::move(pl);
     b->planValid[form] = true;
+    b->planPass[form] = pass;
     b->version += 1;
     return V3DM_OK;
 }
@@ -1237,7 +1247,8 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
     bool const plain = form == 0 || (form == 2 && h->fallbackSamples > 0);
     float T = 0.0f;
     bool const sieve = plain && sieve_run(h, b, minScore, minRatio, &T);
-    bool const split = plain && (!sieve || (form == 0 && !b->planValid[0]));  // (the tuner times the full pass)
+    bool const split = plain && !sieve;
+    bool const pass = !(form == 0 && sieve);  // the run takes the pass of its form's plan
     if (sieve && (rc = ensure_sieve(h, b))) return rc;
     if (split && (rc = ensure_split(h, b))) return rc;
     // derived copies outside the run when they are cached (else every run derives them)
@@ -1257,9 +1268,10 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
         enqueue_derived(h, b, 2);
         b->codesValid = true;
     }
-    if (!h->cacheDerived && !b->planValid[form]) enqueue_derived(h, b, form);  // for the tuner
+    if (!h->cacheDerived && pass && !(b->planValid[form] && b->planPass[form]))
+        enqueue_derived(h, b, form);  // for the tuner
     if (!h->cacheDerived) b->splitValid = b->q8Valid = false;  // a learned run rewrites rows of its failing pairs
-    if ((rc = ensure_plan(h, b, form))) return rc;
+    if ((rc = ensure_plan(h, b, form, pass))) return rc;
     if (form == 2 && h->fallbackSamples > 0 && (rc = ensure_fallback_plan(h, b))) return rc;
     BCHECK(h, hipEventRecord(b->evA, st));
     if (b->useGraph) {

@@ -300,8 +300,8 @@ int v3dm_batch_get_matches(v3dm_handle h, int32_t* offsets, int32_t* pairs, int 
 int v3dm_batch_match(v3dm_handle h, float minScore, float minRatio, int32_t* offsets, int32_t* pairs, int cap,
                      int* nTotal);
 /* Work-item tuning of the persistent kernels: autotune != 0 measures the candidate
- * (tiles per item, grid) settings on the batch at its first run; tilesPerItem / grid > 0
- * fix them for the form of `mode` instead.  In the learned form tilesPerItem is the minimum
+ * (tiles per item, grid) settings on the batch at the first run that takes them (a plain run
+ * that its sieve serves does not); tilesPerItem / grid > 0 fix them for the form of `mode` instead.  In the learned form tilesPerItem is the minimum
  * split size of the candidate lists (default 32 tiles of 64 candidates, at most 8 splits
  * per query): it changes which candidates are listed, so it is never tuned. */
 int v3dm_batch_set_tuning(v3dm_handle h, int autotune, int mode, int tilesPerItem, int grid);

@@ -187,3 +187,31 @@ def test_upload_counters_wrap(first, order):
     with pytest.raises(v3dmatch.V3DMError):
         m.debug_prep_epoch(0)
     m.close()
+
+
+@pytest.mark.parametrize("cache", [False, True])
+@pytest.mark.parametrize("dtype", ["u8", "f32"])
+def test_batch_tunes_the_pass_it_takes(dtype, cache):
+    """A run that takes the sieve times no candidate of the full pass and still reports its
+    setting; the first run that takes the pass tunes it, also after sieved runs of the same pairs,
+    and every result is the oracle's."""
+    print(f"case batch tuning with the sieve {dtype} cache {cache}", flush=True)
+    images = []
+    for p, (nL, nR) in enumerate(SIZES):
+        images += list(synth.make_pair(nL, nR, 0.5, config=3, pair=800 + p)[:2])
+    left = np.arange(0, 2 * len(SIZES), 2, dtype=np.int32)
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([len(q) for q in images],
+                       np.concatenate(images if dtype == "u8" else [synth.dequantise(q) for q in images]))
+    m.batch_set_pairs(left, left + 1)
+    m.set_derived_cache(cache)
+    for ms, mr, timed in ((0.9, 0.8, False), (0.9, 0.8, False), (0.2, 0.8, True), (0.9, 0.8, True), (0.2, 0.8, True)):
+        got = m.batch_match(ms, mr)
+        t = m.batch_get_tuning(v3dmatch.PREC_FP32)
+        assert (t["pass_ms"] > 0) == timed and t["tiles_per_item"] > 0 and t["grid"] > 0 and t["items"] > 0
+        for p in range(len(SIZES)):
+            L, R = (synth.dequantise(images[2 * p + k][:len(images[2 * p + k]) // 32 * 32]) for k in (0, 1))
+            want = oracle.find_putative_matches(L, R, ms, mr) if len(L) and len(R) else np.zeros((0, 2), np.int32)
+            assert np.array_equal(np.asarray(got[p]).reshape(-1, 2), want.reshape(-1, 2)), (p, ms, mr)
+    assert m.batch_time_dominant_kernel(2) > 0
+    m.close()
