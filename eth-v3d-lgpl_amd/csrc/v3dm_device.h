@@ -226,21 +226,22 @@ __device__ __forceinline__ v4f exact_chunk(float const* __restrict__ c, int row,
     return reinterpret_cast<v4f const*>(c + (size_t)row * kDim)[chunk];
 }
 
-// The wave's query rows into its LDS.
-template <int kQ>
-__device__ __forceinline__ void exact_queries(float const* const (&q)[kQ], double* __restrict__ qd, int lane)
+// The wave's query rows into its LDS, as doubles or as the floats they are (with many queries a
+// unit the LDS reads bound the kernel, and a float read brings twice the components).
+template <int kQ, class T>
+__device__ __forceinline__ void exact_queries(float const* const (&q)[kQ], T* __restrict__ qd, int lane)
 {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the previous unit's reads come first
 #pragma unroll
     for (int j = 0; j < kQ; ++j) {
         float2 const v = reinterpret_cast<float2 const*>(q[j])[lane];
-        qd[j * kDim + 2 * lane] = (double)v.x;
-        qd[j * kDim + 2 * lane + 1] = (double)v.y;
+        qd[j * kDim + 2 * lane] = (T)v.x;
+        qd[j * kDim + 2 * lane + 1] = (T)v.y;
     }
 }
 
-template <int kQ>
-__device__ __forceinline__ void exact_scores(double const* __restrict__ qd, float const* __restrict__ c, int nRows,
+template <int kQ, class T>
+__device__ __forceinline__ void exact_scores(T const* __restrict__ qd, float const* __restrict__ c, int nRows,
                                              float* __restrict__ stage, int lane, float (&out)[kQ])
 {
     double acc[kQ];
@@ -261,17 +262,17 @@ __device__ __forceinline__ void exact_scores(double const* __restrict__ qd, floa
         int const next = min(p + 1, 3);  // (the last quarter once more, unused)
 #pragma unroll
         for (int u = 0; u < 8; ++u) v[u] = exact_chunk(c, min(8 * u + (lane >> 3), nRows - 1), 8 * next + (lane & 7));
-#pragma unroll 4
+#pragma unroll(kQ > 4 ? 1 : 4)
         for (int k = 0; k < 8; ++k) {
             float4 const x = *reinterpret_cast<float4 const*>(mine + 4 * k);
             double const x0 = x.x, x1 = x.y, x2 = x.z, x3 = x.w;
 #pragma unroll
             for (int j = 0; j < kQ; ++j) {
-                double const* const y = qd + j * kDim + 32 * p + 4 * k;
-                acc[j] += y[0] * x0;
-                acc[j] += y[1] * x1;
-                acc[j] += y[2] * x2;
-                acc[j] += y[3] * x3;
+                T const* const y = qd + j * kDim + 32 * p + 4 * k;
+                acc[j] += (double)y[0] * x0;
+                acc[j] += (double)y[1] * x1;
+                acc[j] += (double)y[2] * x2;
+                acc[j] += (double)y[3] * x3;
             }
         }
     }

@@ -25,7 +25,7 @@ constexpr int kStripes = 64;
 constexpr int kStripeStride = 32;  // ints (128 bytes)
 constexpr int kRecheckMaxChunks = 64;  // re-check partials per row of either side
 constexpr int kRowPad = 128;      // device descriptor buffers hold a multiple of 128 rows
-constexpr int kRecheckGrid = 1024;
+constexpr int kRecheckGrid = 768;  // one generation: three work-groups per CU beside their LDS
 // |approximate score - exact score| <= epsRel * ||q|| * max||c|| + kEpsAbs for the FP32
 // MFMA path: 128-term FP32 dot products err by at most ~129 * 2^-23 * sum|q_k c_k|, and
 // sum|q_k c_k| <= ||q|| ||c||; epsRel = 2^-15 leaves a factor 2 on top.  epsRel <= 0

@@ -291,9 +291,13 @@ void launch_merge_decide(Top2 const* colPart, int nColParts, int ldc, Top2 const
 // open, the more chunks each gets): with the usual tens of open queries every unit is one
 // step of 64 candidates, 14 us for a few open queries of 16384 x 16384 in one launch (a chain of
 // loads, 64 dependent FP64 steps a quarter and the tickets; nothing is near a rate) against
-// 38 + 5 us in two.  With every query open (a zero error bound) it is 1.3 times the earlier
-// 16 queries a group: 3.7 against 2.8 ms at 8192 x 8192.
+// 38 + 5 us in two.  With every query open (a zero error bound, or equal rows) LDS reads bound
+// it, with conversions close behind: eight queries a unit, kept as floats, and no more units than
+// four a wave (each loads its queries and publishes its partials): 8192 x 8192 2.1 ms, 4096 x 4096
+// 0.6; four queries as doubles in units of 64 or 128 candidates 3.7 and 1.3, 16 queries a
+// work-group 2.8 and 0.8.
 constexpr int kRecheckGroup = 4;  // queries per unit: they share the candidates' loads
+constexpr int kRecheckWide = 8;   // ... where every wave has two such units
 
 struct RecheckDir {
     float const* Q;
@@ -304,7 +308,7 @@ struct RecheckDir {
 };
 
 __device__ __forceinline__ RecheckDir recheck_dir(bool left, float const* L, float const* R, int nL, int nR, int cnt,
-                                                  int rowsL, int rowsR, int* colMax, int* rowMax)
+                                                  int rowsL, int rowsR, int* colMax, int* rowMax, int target)
 {
     RecheckDir d;
     d.Q = left ? L : R;
@@ -315,17 +319,17 @@ __device__ __forceinline__ RecheckDir recheck_dir(bool left, float const* L, flo
     d.base = left ? 0 : rowsL;
     int const nSub = (d.nC + 63) / 64;
     long long const room = (long long)(left ? rowsL : rowsR) * kRecheckMaxChunks / max(cnt, 1);
-    int const most = (int)min(room, (long long)nSub);
+    int const most = (int)min(room, (long long)min(nSub, target));
     d.subs = (nSub + most - 1) / max(most, 1);
     d.nCh = (nSub + d.subs - 1) / d.subs;
     return d;
 }
 
-template <int kQ>
+template <int kQ, class T>
 __device__ __forceinline__ void recheck_units(RecheckDir const& dl, RecheckDir const& dr, int const* flagList,
                                               Top2* __restrict__ part, int* __restrict__ tickets,
                                               unsigned const* __restrict__ gbits, int ldi, float minScore,
-                                              float minRatio, float* __restrict__ stage, double* __restrict__ qd)
+                                              float minRatio, float* __restrict__ stage, T* __restrict__ qd)
 {
     int const lane = threadIdx.x & 63;
     int const wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * 256 + threadIdx.x) >> 6));
@@ -377,7 +381,7 @@ __device__ __forceinline__ void recheck_units(RecheckDir const& dl, RecheckDir c
 }
 
 template <bool kSieve>
-__global__ __launch_bounds__(256) void k_recheck(float const* __restrict__ L, float const* __restrict__ R, int nL,
+__global__ __launch_bounds__(256, 3) void k_recheck(float const* __restrict__ L, float const* __restrict__ R, int nL,
                                                  int nR, int const* __restrict__ flagList, int rowsL, int rowsR,
                                                  int const* __restrict__ counters, Top2* __restrict__ part,
                                                  int* __restrict__ tickets, unsigned const* __restrict__ gbits,
@@ -397,15 +401,22 @@ __global__ __launch_bounds__(256) void k_recheck(float const* __restrict__ L, fl
     }
     int const cntL = __builtin_amdgcn_readfirstlane(counters[kCntFlag]);
     int const cntR = __builtin_amdgcn_readfirstlane(counters[kCntFlagR]);
-    RecheckDir const dl = recheck_dir(true, L, R, nL, nR, cntL, rowsL, rowsR, colMax, rowMax);
-    RecheckDir const dr = recheck_dir(false, L, R, nL, nR, cntR, rowsL, rowsR, colMax, rowMax);
+    // with many queries open no more chunks than give every wave four wide units
+    int const target = max(16 * kRecheckWide * (int)gridDim.x / max(cntL + cntR, 1), 1);
+    RecheckDir const dl = recheck_dir(true, L, R, nL, nR, cntL, rowsL, rowsR, colMax, rowMax, target);
+    RecheckDir const dr = recheck_dir(false, L, R, nL, nR, cntR, rowsL, rowsR, colMax, rowMax, target);
     int const wv = threadIdx.x >> 6;
     // a query per wave while the grid holds a wave for every unit
-    if ((long long)cntL * dl.nCh + (long long)cntR * dr.nCh <= 4LL * gridDim.x)
+    long long const single = (long long)cntL * dl.nCh + (long long)cntR * dr.nCh;
+    static_assert(kRecheckWide * sizeof(float) <= kRecheckGroup * sizeof(double), "the queries' room");
+    if (single <= 4LL * gridDim.x)
         recheck_units<1>(dl, dr, flagList, part, tickets, gbits, ldi, minScore, minRatio, stage[wv], qd[wv]);
+    else if (single >= 8LL * kRecheckWide * gridDim.x)
+        recheck_units<kRecheckWide>(dl, dr, flagList, part, tickets, gbits, ldi, minScore, minRatio, stage[wv],
+                                    reinterpret_cast<float*>(qd[wv]));
     else
         recheck_units<kRecheckGroup>(dl, dr, flagList, part, tickets, gbits, ldi, minScore, minRatio, stage[wv],
-                                     qd[wv]);
+                                     reinterpret_cast<float*>(qd[wv]));
 }
 
 void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int const* flagList, int rowsL, int rowsR,

@@ -264,3 +264,31 @@ def test_u8_odd_capacity(capacity):
     _check(m, synth.dequantise(qL), synth.dequantise(qR), 0.4, 0.99)
     _check(m, synth.dequantise(qL), synth.dequantise(qR), -2.0, -1.0)
     m.close()
+
+
+@pytest.mark.parametrize("n,copies", [(256, 33), (1536, 1001), (4096, 3001), (2304, 2304)])
+@pytest.mark.parametrize("guided", [False, True])
+def test_many_open_queries(n, copies, guided):
+    """Exact copies score 1, which the certified rule leaves open: re-checks of one, four and eight
+    queries a unit, with a partial last group, and with removed pairs of a guided call."""
+    print(f"case open queries {copies} of {n} guided {guided}", flush=True)
+    L, R = _pair(n, n, 12)
+    R[:copies] = L[np.random.default_rng(5).permutation(n)[:copies]]
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(n, n, guided)
+    _set(m, L, R)
+    got = m.find_putative_matches_array(0.2, 0.8)
+    S = oracle.scores(L, R)
+    assert np.array_equal(got, oracle.find_putative_matches(L, R, 0.2, 0.8))
+    assert m.stats()["nRechecked"] >= 2 * copies
+    if guided:
+        rng = np.random.default_rng(6)
+        lxy, rxy = (rng.uniform(0, 1000, (n, 2)).astype(np.float32) for _ in range(2))
+        H = np.eye(3)
+        got = m.run_guided_array(True, H, 600.0, lxy, rxy, 0.2, 0.8)
+        assert np.array_equal(got, oracle.guided(S, 1, H, np.float32(600.0), lxy, rxy, 0.2, 0.8))
+    m.set_certification(0.0)
+    assert np.array_equal(m.find_putative_matches_array(0.9, 0.8), oracle.find_putative_matches(L, R, 0.9, 0.8))
+    assert m.stats()["nRechecked"] == 2 * n
+    m.close()
