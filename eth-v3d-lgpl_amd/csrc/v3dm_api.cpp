@@ -101,6 +101,7 @@ void releaseBuffers(v3dm_context* h)
     h->allocated = false;
     h->nL = h->nR = 0;
     h->haveResult = false;
+    h->sieveDeferred = h->deviceReaders = false;
     h->masks.clear();
     ext_release(h->ext);
 }
@@ -165,10 +166,10 @@ int prof_end(v3dm_context* h)
 bool split_fits(v3dm_context const* h) { return h->splitFitHost[0] && h->splitFitHost[1]; }
 
 // The certified decisions' error bound for the scores of launch_score_pass.
-float score_eps(v3dm_context const* h, unsigned const* bits)
+float score_eps(v3dm_context const* h, unsigned const* bits, float epsRel)
 {
-    if (!split_fits(h)) return h->epsRel;
-    return h->epsRel * (h->haveIntL && h->haveIntR && !bits ? kIntEps : kSplitEps);
+    if (!split_fits(h)) return epsRel;
+    return epsRel * (h->haveIntL && h->haveIntR && !bits ? kIntEps : kSplitEps);
 }
 
 FusedPlan score_plan(v3dm_context const* h)
@@ -176,10 +177,9 @@ FusedPlan score_plan(v3dm_context const* h)
     return split_fits(h) ? plan_split(h->nL, h->nR) : plan_fused_fp32(h->nL, h->nR, 512);
 }
 
-// The rows of the split pass, made once for the current sets.
-int ensure_split_rows(v3dm_context* h)
+// Room for the rows of the split pass of the current sets.
+int ensure_split_room(v3dm_context* h)
 {
-    if (h->haveSplit) return V3DM_OK;
     for (bool left : {true, false}) {
         size_t const rows = (size_t)roundUp(left ? h->capL : h->capR, kSplitRowPad);
         unsigned char*& split = left ? h->splitL : h->splitR;
@@ -187,19 +187,43 @@ int ensure_split_rows(v3dm_context* h)
         if (!split) HIPCHECK(h, hipMalloc(&split, rows * kSplitRowBytes));
         if (!ints && (left ? h->haveIntL : h->haveIntR)) HIPCHECK(h, hipMalloc(&ints, rows * kIntRowBytes));
     }
+    return V3DM_OK;
+}
+
+// The same for a caller that goes on without.
+bool have_split_room(v3dm_context* h)
+{
+    if (ensure_split_room(h) == V3DM_OK) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+void launch_split_rows(v3dm_context* h, int* gated)
+{
     launch_split_sets(SplitRowsOf{h->dL, h->intScaleL, h->splitL, h->haveIntL ? h->intL : nullptr, h->nL},
-                      SplitRowsOf{h->dR, h->intScaleR, h->splitR, h->haveIntR ? h->intR : nullptr, h->nR}, h->stream);
+                      SplitRowsOf{h->dR, h->intScaleR, h->splitR, h->haveIntR ? h->intR : nullptr, h->nR}, gated,
+                      h->stream);
+}
+
+// The rows of the split pass, made once for the current sets.
+int ensure_split_rows(v3dm_context* h)
+{
+    if (h->haveSplit) return V3DM_OK;
+    int const rc = ensure_split_room(h);
+    if (rc) return rc;
+    launch_split_rows(h, nullptr);
     h->haveSplit = true;
     return V3DM_OK;
 }
 
-void launch_score_pass(v3dm_context* h, FusedPlan const& p, unsigned const* bits, float minScore)
+void launch_score_pass(v3dm_context* h, FusedPlan const& p, unsigned const* bits, float minScore,
+                       int const* gate = nullptr)
 {
     hipStream_t const st = h->stream;
     if (split_fits(h))
         launch_split_pass(SplitSet{h->splitL, h->haveIntL ? h->intL : nullptr, h->intScaleL, h->nL},
                           SplitSet{h->splitR, h->haveIntR ? h->intR : nullptr, h->intScaleR, h->nR}, p, h->colPart,
-                          h->capL, h->rowPart, h->capR, bits, h->capL, minScore, st);
+                          h->capL, h->rowPart, h->capR, bits, h->capL, minScore, st, gate);
     else if (bits)
         launch_guided_fp32(h->dL, h->dR, h->nL, h->nR, p, h->colPart, h->capL, h->rowPart, h->capR, bits, h->capL, st);
     else
@@ -212,64 +236,136 @@ bool sieve_fits(v3dm_context const* h, float minScore, float minRatio, float* T)
     return split_fits(h) && h->epsRel > 0.0f && sieve_bound(minScore, minRatio, T);
 }
 
-SieveBest sieve_best(v3dm_context const* h)
+// bounded: the call's candidates have a bound past which the sieve gives it to the full pass.
+SieveBest sieve_best(v3dm_context const* h, SievePlan const& p, bool bounded)
 {
-    return SieveBest{h->sieveBest, h->sieveSecond, h->capL, h->flagList, h->results + kCntFlag,
-                     h->results + kCntFlagR};
+    double const pairs = (double)h->nL * h->nR;
+    SieveBest b{};
+    b.best = h->sieveBest;
+    b.second = h->sieveSecond;
+    b.offR = h->capL;
+    b.limit = sieve_limit((long long)p.tiles * kSieveTile * 128);
+    b.flags = h->flagList;
+    b.cntL = h->results + kCntFlag;
+    b.cntR = h->results + kCntFlagR;
+    b.scored = reinterpret_cast<unsigned*>(h->results + kCntScored);
+    b.mostScored = sieve_most_scored(pairs);
+    b.mostListed = sieve_most_listed(pairs);
+    b.gate = bounded ? h->results + kCntGate : nullptr;
+    return b;
 }
 
-void launch_sieve_pass(v3dm_context* h, float T, unsigned const* bits)
+void launch_sieve_pass(v3dm_context* h, float T, unsigned const* bits, bool bounded)
 {
-    launch_sieve(SieveSet{h->q8L, h->resL, h->dL, h->nL}, SieveSet{h->q8R, h->resR, h->dR, h->nR},
-                 plan_sieve(h->nL, h->nR), h->maxNormBits, T, sieve_best(h), bits, h->capL, h->stream);
+    SievePlan const p = plan_sieve(h->nL, h->nR);
+    launch_sieve(SieveSet{h->q8L, h->resL, h->dL, h->nL}, SieveSet{h->q8R, h->resR, h->dR, h->nR}, p, h->maxNormBits,
+                 T, sieve_best(h, p, bounded), bits, h->capL, h->stream);
 }
 
-// Scores, decisions and the exact re-check of open queries of the current features (bits: the
-// guided bitmap or null); colMax / rowMax are decided on the stream.
-int enqueue_decisions(v3dm_context* h, unsigned const* bits, float minScore, float minRatio)
+// Its decisions and the exact re-check of the listed features.
+void launch_sieve_decisions(v3dm_context* h, unsigned const* bits, bool bounded, float minScore, float minRatio)
+{
+    launch_sieve_finish(h->dL, h->dR, h->nL, h->nR, sieve_best(h, SievePlan{}, bounded), h->flagList, h->capL, h->capR,
+                        h->results, minScore, minRatio, h->colMax, h->rowMax, h->rpart, h->rtickets, bits, h->capL,
+                        h->stream);
+}
+
+void enqueue_mutual(v3dm_context* h, bool work)
+{
+    launch_mutual_compact(h->colMax, h->rowMax, work ? h->nL : 0, h->nR, h->mstatus, next_mutual_epoch(h), h->stripes,
+                          reinterpret_cast<int2*>(h->results + kNumCounters), h->results, h->hostStage, h->stream,
+                          {}, h->mutualWait);
+}
+
+// The full pass's scores, decisions, the exact re-check of open queries and the mutual check.
+// gated: the first three only where the call's sieve gave it to the full pass (the split rows have
+// room).
+int enqueue_full(v3dm_context* h, unsigned const* bits, float epsRel, float minScore, float minRatio, bool gated)
 {
     hipStream_t const st = h->stream;
     int const nL = h->nL, nR = h->nR;
+    int* const gate = gated ? h->results + kCntGate : nullptr;
+    int rc;
+    FusedPlan const p = score_plan(h);
+    if (gated) launch_split_rows(h, h->results);
+    else if (split_fits(h) && (rc = ensure_split_rows(h))) return rc;
+    if (!gated && (rc = prof_begin(h))) return rc;
+    launch_score_pass(h, p, bits, minScore, gate);
+    rc = gated ? V3DM_OK : prof_end(h);  // after an error too: what follows clears what the next call needs clear
+    launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL, h->normR,
+                        h->maxNormBits, score_eps(h, bits, epsRel), minScore, minRatio, h->colMax, h->rowMax,
+                        h->flagList, h->capL, h->results, st, gate);
+    launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore, minRatio,
+                         h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st, bits, h->capL, gate);
+    enqueue_mutual(h, true);
+    return rc;
+}
+
+// Scores, decisions, the exact re-check of open queries and the mutual check of the current
+// features (bits: the guided bitmap or null).  A call that its sieve gives to
+// the full pass is run again when the host reads the result (finish_result), which spares
+// every other call the launches; where the caller has the device pointers of the results, the
+// full pass is enqueued behind the sieve and leaves at once unless it is needed (about 10 us).
+int enqueue_decisions(v3dm_context* h, unsigned const* bits, float minScore, float minRatio)
+{
     int rc;
     float T = 0.0f;
-    if (sieve_fits(h, minScore, minRatio, &T)) {
-        if ((rc = prof_begin(h))) return rc;
-        launch_sieve_pass(h, T, bits);
-        rc = prof_end(h);
-        // also after an error: the decisions leave the sieve's entries at zero for the next call
-        launch_sieve_finish(h->dL, h->dR, nL, nR, sieve_best(h), h->flagList, h->capL, h->capR, h->results, minScore,
-                            minRatio, h->colMax, h->rowMax, h->rpart, h->rtickets, bits, h->capL, st);
-        if (rc) return rc;
-    } else {
-        FusedPlan const p = score_plan(h);
-        if (split_fits(h) && (rc = ensure_split_rows(h))) return rc;
-        if ((rc = prof_begin(h))) return rc;
-        launch_score_pass(h, p, bits, minScore);
-        if ((rc = prof_end(h))) return rc;
-        launch_merge_decide(h->colPart, p.splits, h->capL, h->rowPart, p.leftBlocks, h->capR, nL, nR, h->normL,
-                            h->normR, h->maxNormBits, score_eps(h, bits), minScore, minRatio, h->colMax, h->rowMax,
-                            h->flagList, h->capL, h->results, st);
-        launch_recheck_exact(h->dL, h->dR, nL, nR, h->flagList, h->capL, h->capR, h->results, minScore, minRatio,
-                             h->colMax, h->rowMax, h->rpart, h->rtickets, kRecheckGrid, st, bits, h->capL);
+    h->sieveDeferred = false;
+    if (!sieve_fits(h, minScore, minRatio, &T)) return enqueue_full(h, bits, h->epsRel, minScore, minRatio, false);
+    // (without room for the full pass's rows: no bound, every listed feature is re-checked exactly)
+    bool const chained = h->deviceReaders && have_split_room(h);
+    bool const bounded = chained || !h->deviceReaders;
+    if ((rc = prof_begin(h))) return rc;
+    launch_sieve_pass(h, T, bits, bounded);
+    rc = prof_end(h);
+    launch_sieve_decisions(h, bits, bounded, minScore, minRatio);
+    if (chained) {
+        (void)enqueue_full(h, bits, h->epsRel, minScore, minRatio, true);
+        return rc;
     }
-    return V3DM_OK;
+    enqueue_mutual(h, true);
+    h->sieveDeferred = bounded;
+    h->deferredEps = h->epsRel;
+    h->deferredBits = bits;
+    return rc;
 }
 
 // Enqueue the plain FP32 exact path for the current features; leaves colMax/rowMax
 // decided and the compacted pairs + counters in h->results.
 int enqueue_plain(v3dm_context* h, float minScore, float minRatio)
 {
-    hipStream_t const st = h->stream;
-    int const nL = h->nL, nR = h->nR;
-    bool const work = nL > 0 && nR > 0;
-    if (work) {
-        int const rc = enqueue_decisions(h, nullptr, minScore, minRatio);
-        if (rc) return rc;
-    }
-    launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
-                          reinterpret_cast<int2*>(h->results + kNumCounters), h->results, h->hostStage, st,
-                          {}, h->mutualWait);
+    bool const work = h->nL > 0 && h->nR > 0;
+    h->sieveDeferred = false;
+    if (!work) enqueue_mutual(h, false);
+    else if (int const rc = enqueue_decisions(h, nullptr, minScore, minRatio)) return rc;
     HIPCHECK(h, hipGetLastError());
+    return V3DM_OK;
+}
+
+// Before the host reads a result: waits for it, with a pending sampled check evaluated
+// (ext_finish), and with the full pass run where the sieve gave the call to it.
+int finish_result(v3dm_context* h)
+{
+    int rc = ext_finish(h);
+    if (rc) return rc;
+    HIPCHECK(h, hipStreamSynchronize(h->stream));
+    if (!h->sieveDeferred || !h->hostStage[kCntGate]) {
+        h->sieveDeferred = false;
+        return V3DM_OK;
+    }
+    unsigned const* const bits = h->deferredBits;
+    if (have_split_room(h)) {
+        if ((rc = enqueue_full(h, bits, h->deferredEps, h->lastMinScore, h->lastMinRatio, false))) return rc;
+    } else {  // no room for its rows: the sieve again, without the bound
+        float T = 0.0f;
+        (void)sieve_bound(h->lastMinScore, h->lastMinRatio, &T);
+        launch_sieve_pass(h, T, bits, false);
+        launch_sieve_decisions(h, bits, false, h->lastMinScore, h->lastMinRatio);
+        enqueue_mutual(h, true);
+    }
+    HIPCHECK(h, hipGetLastError());
+    HIPCHECK(h, hipStreamSynchronize(h->stream));
+    h->sieveDeferred = false;
     return V3DM_OK;
 }
 
@@ -428,6 +524,10 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
     if (n > 0 && !src) return fail(h, V3DM_ERR_INVALID, "null descriptor pointer");
     HIPCHECK(h, hipSetDevice(h->device));
     ext_quiesce(h);  // the sampled check's side stream reads the features
+    if (h->haveResult && h->sieveDeferred) {  // readable still should this call fail
+        int const rc = finish_result(h);
+        if (rc) return rc;
+    }
     float* dst = left ? h->dL : h->dR;
     size_t const bytes = (size_t)n * kDim * sizeof(float);
     RowSource from = kRowsInPlace;
@@ -480,7 +580,7 @@ int setFeatures(v3dm_context* h, bool left, int n, const void* src, Source kind)
     HIPCHECK(h, hipStreamSynchronize(h->stream));
     if (left) h->nL = n;
     else h->nR = n;
-    h->haveResult = false;
+    h->haveResult = h->sieveDeferred = false;
     h->masks.clear();
     ext_features_changed(h, left);
     return V3DM_OK;
@@ -490,9 +590,8 @@ int copyResults(v3dm_context* h, int32_t* pairs, int cap, int* nPairs)
 {
     if (!h->haveResult) return fail(h, V3DM_ERR_STATE, "no result: call findPutativeMatches first");
     // the mutual check wrote the counts and the pairs to the pinned block
-    int const rcf = ext_finish(h);
+    int const rcf = finish_result(h);
     if (rcf) return rcf;
-    HIPCHECK(h, hipStreamSynchronize(h->stream));
     if (h->hostStage[kCntMutualError] == (int)h->mutualEpoch)
         return fail(h, V3DM_ERR_HIP, "mutual check: ordering wait between work-groups ran out");
     int const n = h->hostStage[kCntPairs];
@@ -545,13 +644,9 @@ int runGuided(v3dm_context* h, int kind, const double M[9], float distanceThresh
     for (int t = 0; t < 9; ++t) gm.m[t] = m[t];
     gm.sqrThreshold = sqrThreshold;
     h->masks.push_back(gm);
-    if (work) {
-        int const rc = enqueue_decisions(h, h->guidedBits, minScore, minRatio);
-        if (rc) return rc;
-    }
-    launch_mutual_compact(h->colMax, h->rowMax, work ? nL : 0, nR, h->mstatus, next_mutual_epoch(h), h->stripes,
-                          reinterpret_cast<int2*>(h->results + kNumCounters), h->results, h->hostStage, st,
-                          {}, h->mutualWait);
+    h->sieveDeferred = false;
+    if (!work) enqueue_mutual(h, false);
+    else if (int const rc = enqueue_decisions(h, h->guidedBits, minScore, minRatio)) return rc;
     HIPCHECK(h, hipGetLastError());
     h->lastMinScore = minScore;
     h->lastMinRatio = minRatio;
@@ -714,6 +809,7 @@ int v3dm_find_putative_matches_async(v3dm_handle h, float minScore, float minRat
         ext_features_changed(h, false);
     }
     int rc;
+    h->sieveDeferred = false;  // (of the call that this one replaces)
     if (h->precision == V3DM_PREC_FP32) rc = enqueue_plain(h, minScore, minRatio);
     else rc = ext_enqueue(h, h->precision, minScore, minRatio);
     if (rc) return rc;
@@ -744,6 +840,12 @@ int v3dm_device_results(v3dm_handle h, const int32_t** d_pairs, const int32_t** 
 {
     if (!h) return fail(nullptr, V3DM_ERR_INVALID, "null handle");
     if (!h->allocated) return fail(h, V3DM_ERR_STATE, "not allocated");
+    HIPCHECK(h, hipSetDevice(h->device));
+    if (h->haveResult && h->sieveDeferred) {
+        int const rc = finish_result(h);
+        if (rc) return rc;
+    }
+    h->deviceReaders = true;  // from here on results are whole on the stream, whether the host reads them or not
     if (d_pairs) *d_pairs = h->results + kNumCounters;
     if (d_counters) *d_counters = h->results;
     return V3DM_OK;
@@ -754,7 +856,7 @@ int v3dm_get_maxima(v3dm_handle h, int32_t* colMax, int32_t* rowMax)
     if (!h) return fail(nullptr, V3DM_ERR_INVALID, "null handle");
     if (!h->haveResult) return fail(h, V3DM_ERR_STATE, "no result: call findPutativeMatches first");
     HIPCHECK(h, hipSetDevice(h->device));
-    int const rcf = ext_finish(h);
+    int const rcf = finish_result(h);
     if (rcf) return rcf;
     if (colMax && h->lastNL > 0)
         HIPCHECK(h, hipMemcpyAsync(colMax, h->colMax, (size_t)h->lastNL * sizeof(int), hipMemcpyDeviceToHost,
@@ -832,7 +934,7 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
     if (!h || !msPerLaunch || reps < 1) return fail(h, V3DM_ERR_INVALID, "bad argument");
     if (!h->haveResult) return fail(h, V3DM_ERR_STATE, "no result: call findPutativeMatches first");
     HIPCHECK(h, hipSetDevice(h->device));
-    int const rcf = ext_finish(h);
+    int const rcf = finish_result(h);
     if (rcf) return rcf;
     hipEvent_t a = nullptr, b = nullptr;
     HIPCHECK(h, hipEventCreate(&a));
@@ -851,7 +953,7 @@ int v3dm_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
             if (rc) e = hipErrorOutOfMemory;
             if (e == hipSuccess) e = hipEventRecord(a, h->stream);
             for (int r = 0; r < reps && e == hipSuccess; ++r) {
-                if (sieve) launch_sieve_pass(h, T, nullptr);
+                if (sieve) launch_sieve_pass(h, T, nullptr, false);
                 else launch_score_pass(h, p, nullptr, h->lastMinScore);
             }
             if (e == hipSuccess) e = hipEventRecord(b, h->stream);
@@ -900,7 +1002,7 @@ int v3dm_get_stats(v3dm_handle h, v3dm_stats* out)
         if (rc) return rc;
     }
     if (h->haveResult) {
-        int const rcf = ext_finish(h);
+        int const rcf = finish_result(h);
         if (rcf) return rcf;
         int cnt[kNumCounters];
         HIPCHECK(h, hipMemcpyAsync(cnt, h->results, sizeof(cnt), hipMemcpyDeviceToHost, h->stream));

@@ -50,6 +50,10 @@ struct v3dm_context {
     float *resL = nullptr, *resR = nullptr;
     unsigned long long* sieveBest = nullptr;      // of capL left, then capR right features
     unsigned* sieveSecond = nullptr;
+    bool sieveDeferred = false;       // the last result is run again by the full pass if its sieve gave it up ...
+    float deferredEps = 0.0f;         // ... with this error bound and these removed pairs (finish_result)
+    unsigned const* deferredBits = nullptr;
+    bool deviceReaders = false;       // the caller has the results' device pointers
     int* splitFitHost = nullptr;      // mapped: [0] left, [1] right set in the split pass's range
     int* splitFitDev = nullptr;       // the same memory as the kernels address it
     unsigned int* maxNormBits = nullptr;  // [0] = left, [kMaxNormR] = right, with epochs above

@@ -11,9 +11,11 @@ constexpr int kMaxSplits = 64;    // right-feature splits of the fused kernel
 constexpr int kCntPairs = 0;      // counters[0]: number of matches
 constexpr int kCntFlag = 1;       // counters[1]: open left queries of the running call (cleared at its end)
 constexpr int kCntFlagDone = 2;   // counters[2]: queries re-checked exactly by the last call
+constexpr int kCntGate = 3;       // counters[3]: the running call's sieve gave it to the full pass (cleared at its end)
 constexpr int kCntRescoredDone = 4;  // counters[4]: ... by the last call
 constexpr int kCntFlagR = 5;      // counters[5]: open right queries of the running call
 constexpr int kCntMutualError = 6;  // counters[6]: epoch of a mutual check whose ordering wait ran out
+constexpr int kCntScored = 7;     // counters[7]: candidates of the running call's fuller waves (cleared at its end)
 constexpr int kNumCounters = 8;
 // Counts summed by many work-groups go to kStripes slots one cache line apart (atomics on a
 // single address serialise in L2); the gather kernel sums and clears them.
@@ -47,14 +49,15 @@ void launch_norms(float const* X, int n, float* norm, unsigned int* maxNormBits,
 void launch_merge_decide(Top2 const* colPart, int nColParts, int ldc, Top2 const* rowPart, int nRowParts, int ldr,
                          int nL, int nR, float const* normL, float const* normR, unsigned int const* maxNormBits,
                          float epsRel, float minScore, float minRatio, int* colMax, int* rowMax, int* flagList,
-                         int flagOffR, int* counters, hipStream_t st);
+                         int flagOffR, int* counters, hipStream_t st, int const* gate = nullptr);
 // flagList: open left queries at [0, ...) (at most rowsL), open right queries at [rowsL, ...)
 // (at most rowsR); part: (rowsL + rowsR) * kRecheckMaxChunks partials; tickets: rowsL + rowsR
 // ints, zero before the first call and left zero.  gbits: guided-matching bitmap (pairs scored
 // -1e20), or null.
 void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int const* flagList, int rowsL, int rowsR,
                           int const* counters, float minScore, float minRatio, int* colMax, int* rowMax, Top2* part,
-                          int* tickets, int grid, hipStream_t st, unsigned const* gbits = nullptr, int ldi = 0);
+                          int* tickets, int grid, hipStream_t st, unsigned const* gbits = nullptr, int ldi = 0,
+                          int* gate = nullptr);
 // The learned decisions of the S sampled left features of the sampled exact check:
 // out[k] = colMax[sample_row(k, nL, S)], k < S.  out may be mapped host memory.  S = 0:
 // nothing to write.

@@ -194,8 +194,13 @@ void launch_prep_rows(RowSource from, void const* src, float* X, int n, float* n
 // needs them: with the sieve few calls do.
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-__global__ __launch_bounds__(256) void k_split_sets(SplitRowsOf a, SplitRowsOf b)
+__global__ __launch_bounds__(256) void k_split_sets(SplitRowsOf a, SplitRowsOf b, int* __restrict__ gated)
 {
+    if (gated) {
+        if (!gated[kCntGate]) return;
+        // the sieve's list is void, the full pass makes its own
+        if (blockIdx.x == 0 && threadIdx.x == 0) gated[kCntFlag] = gated[kCntFlagR] = 0;
+    }
     int const t = blockIdx.x * 256 + threadIdx.x;
     bool const first = (t >> 4) < a.n;
     SplitRowsOf const& s = first ? a : b;
@@ -223,11 +228,11 @@ __global__ __launch_bounds__(256) void k_split_sets(SplitRowsOf a, SplitRowsOf b
     *reinterpret_cast<v8h*>(s.ints + (size_t)row * kIntRowBytes + c * 16) = q;
 }
 
-void launch_split_sets(SplitRowsOf const& a, SplitRowsOf const& b, hipStream_t st)
+void launch_split_sets(SplitRowsOf const& a, SplitRowsOf const& b, int* gated, hipStream_t st)
 {
     int const rows = a.n + b.n;
     if (rows <= 0) return;
-    hipLaunchKernelGGL(k_split_sets, dim3((rows + 15) / 16), dim3(256), 0, st, a, b);
+    hipLaunchKernelGGL(k_split_sets, dim3((rows + 15) / 16), dim3(256), 0, st, a, b, gated);
 }
 
 // ------------------------------------------------------------------------------ merge + decide
@@ -241,8 +246,10 @@ __global__ __launch_bounds__(256) void k_merge_decide(Top2 const* __restrict__ c
                                                       unsigned int const* __restrict__ maxNormBits, float epsRel,
                                                       float minScore, float minRatio, int* __restrict__ colMax,
                                                       int* __restrict__ rowMax, int* __restrict__ flagList,
-                                                      int flagOffR, int* __restrict__ counters)
+                                                      int flagOffR, int* __restrict__ counters,
+                                                      int const* __restrict__ gate)
 {
+    if (gate && !*gate) return;
     int const sub = threadIdx.x & 7;
     int const g = (int)((blockIdx.x * 256u + threadIdx.x) >> 3);
     bool const valid = g < nL + nR;
@@ -273,13 +280,14 @@ __global__ __launch_bounds__(256) void k_merge_decide(Top2 const* __restrict__ c
 void launch_merge_decide(Top2 const* colPart, int nColParts, int ldc, Top2 const* rowPart, int nRowParts,
                          int ldr, int nL, int nR, float const* normL, float const* normR,
                          unsigned int const* maxNormBits, float epsRel, float minScore, float minRatio,
-                         int* colMax, int* rowMax, int* flagList, int flagOffR, int* counters, hipStream_t st)
+                         int* colMax, int* rowMax, int* flagList, int flagOffR, int* counters, hipStream_t st,
+                         int const* gate)
 {
     int const n = nL + nR;
     if (n <= 0) return;
     hipLaunchKernelGGL(k_merge_decide, dim3((n + 31) / 32), dim3(256), 0, st, colPart, nColParts, ldc, rowPart,
                        nRowParts, ldr, nL, nR, normL, normR, maxNormBits, epsRel, minScore, minRatio, colMax,
-                       rowMax, flagList, flagOffR, counters);
+                       rowMax, flagList, flagOffR, counters, gate);
 }
 
 // ------------------------------------------------------------------------------ exact re-check
@@ -390,7 +398,9 @@ __global__ __launch_bounds__(256, 3) void k_recheck(float const* __restrict__ L,
 {
     __shared__ __attribute__((aligned(16))) float stage[4][kExactLds];
     __shared__ __attribute__((aligned(16))) double qd[4][kRecheckGroup * kDim];
+    bool given = false;  // the call is the full pass's
     if constexpr (kSieve) {
+        given = sieve.gate && *sieve.gate;
         // the other queries' decisions; the listed ones' follow below
         for (int g = blockIdx.x * 256 + threadIdx.x; g < nL + nR; g += gridDim.x * 256) {
             int const q = g < nL ? g : g - nL;
@@ -399,6 +409,7 @@ __global__ __launch_bounds__(256, 3) void k_recheck(float const* __restrict__ L,
             if (d != kFlag) (g < nL ? colMax : rowMax)[q] = d;
         }
     }
+    if (given || (!kSieve && sieve.gate && !*sieve.gate)) return;
     int const cntL = __builtin_amdgcn_readfirstlane(counters[kCntFlag]);
     int const cntR = __builtin_amdgcn_readfirstlane(counters[kCntFlagR]);
     // with many queries open no more chunks than give every wave four wide units
@@ -421,23 +432,22 @@ __global__ __launch_bounds__(256, 3) void k_recheck(float const* __restrict__ L,
 
 void launch_recheck_exact(float const* L, float const* R, int nL, int nR, int const* flagList, int rowsL, int rowsR,
                           int const* counters, float minScore, float minRatio, int* colMax, int* rowMax, Top2* part,
-                          int* tickets, int grid, hipStream_t st, unsigned const* gbits, int ldi)
+                          int* tickets, int grid, hipStream_t st, unsigned const* gbits, int ldi, int* gate)
 {
     if (nL <= 0 || nR <= 0) return;
+    SieveBest none{};
+    none.gate = gate;
     hipLaunchKernelGGL(k_recheck<false>, dim3(grid), dim3(256), 0, st, L, R, nL, nR, flagList, rowsL, rowsR, counters,
-                       part, tickets, gbits, ldi, minScore, minRatio, colMax, rowMax, SieveBest{});
+                       part, tickets, gbits, ldi, minScore, minRatio, colMax, rowMax, none);
 }
 
-// A thread per query; hardly ever is a query listed.  The grid is one generation of work-groups
-// (three per CU beside the re-check's LDS) for the case that many are: with only the decisions'
-// 128 work-groups 8192 x 8192 sets of nearly equal rows took 12.8 ms, 4.5 ms so.
+// A thread per query; hardly ever is a query listed, and then a bounded number (SieveBest).
 void launch_sieve_finish(float const* L, float const* R, int nL, int nR, SieveBest const& b, int const* flagList,
                          int rowsL, int rowsR, int const* counters, float minScore, float minRatio, int* colMax,
                          int* rowMax, Top2* part, int* tickets, unsigned const* gbits, int ldi, hipStream_t st)
 {
     if (nL <= 0 || nR <= 0) return;
-    int const grid = 768;
-    hipLaunchKernelGGL(k_recheck<true>, dim3(grid), dim3(256), 0, st, L, R, nL, nR, flagList, rowsL, rowsR, counters,
+    hipLaunchKernelGGL(k_recheck<true>, dim3(kRecheckGrid), dim3(256), 0, st, L, R, nL, nR, flagList, rowsL, rowsR, counters,
                        part, tickets, gbits, ldi, minScore, minRatio, colMax, rowMax, b);
 }
 
@@ -586,8 +596,11 @@ __global__ __launch_bounds__(256) void k_mutual(int const* __restrict__ colMax, 
             if (host) {
                 host[kCntPairs] = sBase + total;
                 host[kCntFlagDone] = open;
+                host[kCntGate] = counters[kCntGate];
                 host[kCntRescoredDone] = rescored;
             }
+            counters[kCntGate] = 0;
+            counters[kCntScored] = 0;
         }
     }
 }

@@ -39,19 +39,50 @@ struct SieveSet {
 
 // Per query (left, then right at offR): the candidates' best as score bits << 32 | ~index, and
 // the second best's bits.  Zero before a pass; the decisions leave them zero.  Features of a
-// block whose list overflowed hold kSieveFlood and are listed for the exact re-check (flags:
+// wave whose list overflowed hold kSieveFlood and are listed for the exact re-check (flags:
 // left ones from 0, right ones from offR, counted at cntL and cntR; null: the decisions list
 // them).
+//
+// Sets with many nearly equal rows, or rows that int8 holds badly, can have any number of
+// candidates, and the full pass serves any sets at the same speed.  So a wave scores at most
+// `limit` of them, the features of the waves that have more are re-checked exactly, and both have
+// a bound: where the candidates of the waves with more than one round of them (64), summed in
+// *scored, pass `mostScored`, or a side's listed features times the other side's count pass
+// `mostListed`, the call is given to the full pass: *gate is set (for the kernels and the host that
+// follow), its decisions are void, and the remaining waves neither score nor list.  gate null:
+// no bound.
 constexpr unsigned long long kSieveFlood = ~0ull;
+constexpr int kSieveList = 512;  // the largest limit
 
 struct SieveBest {
     unsigned long long* best;
     unsigned* second;
     int offR;
+    int limit;
     int* flags;
     int* cntL;
     int* cntR;
+    unsigned* scored;
+    unsigned mostScored;
+    long long mostListed;
+    int* gate;
 };
+
+// The bounds of `pairs` scores: about the full pass's time each (45 us of launches and a second
+// wait, and 1.3 * 10^6 scores per us).  The card scores 3000 listed candidates per us and re-checks
+// 60000 pairs per us.  A wave's candidates are a chain of rounds of 64, 10 us each: one round for
+// the short runs of small sets, whose full pass is short too, eight for long ones, which may hold a
+// small cluster by themselves (SIFT sets have about ten candidates a wave).  Calls in us with a
+// share of both sides in one cluster of nearly equal rows, 0 / 2 / 10 / 50%: 16384 x 16384 60 / 104 /
+// 334 / 335, 8192 x 8192 40 / 47 / 139 / 153, 2048 x 2048 30 / 30 / 87 / 75; with lists of 2048 and
+// no bounds 60 / 91 / 827 / 15528, 40 / 46 / 263 / 5895 and 29 / 30 / 55 / 457; with the FP32
+// instruction 735, 248 and 81 at any share.
+inline unsigned sieve_most_scored(double pairs) { return (unsigned)(135000.0 + pairs / 430); }
+inline long long sieve_most_listed(double pairs) { return (1LL << 20) + (long long)(pairs / 32); }
+inline int sieve_limit(long long pairs)  // of a wave of `pairs` scores
+{
+    return pairs < 64 * 128 ? 64 : pairs < kSieveList * 128LL ? (int)(pairs / 128) : kSieveList;
+}
 
 struct SievePlan {
     int groups = 1, splits = 1, tiles = 1;

@@ -37,10 +37,8 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // scores its list exactly, a pair per lane, and enters each score for both features: an atomic
 // maximum of (score, ~index) returns the smaller of two keys, which goes to the second best's
 // maximum; so every key but the largest reaches it, and equal scores keep the smallest index.
-// A wave whose list overflows marks all its features for the exact re-check instead.
-// With 512 entries a tenth of 8192 x 8192 rows in one cluster of nearly equal ones overflowed some
-// lists; with 2048 (32 KiB a group, no group fewer per CU) the call takes 0.25 ms there, as the
-// FP32 instruction did, and the lists overflow from about a sixth of both sets on.
+// A wave with more candidates than its limit stops and marks all its features for the exact re-check
+// instead, within the call's bound (SieveBest).
 //
 // What bounds it: the int8 matrix instructions (16384 x 16384: 2^20 of them, 20 us of the 37),
 // then the tail, where each wave waits for the rows and the atomics of its few candidates
@@ -48,7 +46,6 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // against 182 + 6 + 14 of the FP16 split pass, its merge and its re-check (605 of the FP32
 // instruction); 4096 x 4096: 12 + 3 against 24 + 5 + 4; 480 x 512: 9 + 2 against 8 + 5 + 4.
 constexpr int kSieveBlocks = 4;
-constexpr int kSieveList = 2048;
 
 __device__ __forceinline__ int max3i(int a, int b, int c) { return max(max(a, b), c); }
 
@@ -98,13 +95,36 @@ __device__ __forceinline__ void sieve_enter(unsigned long long* best, unsigned* 
     if (loser) atomicMax(second, loser);
 }
 
+// Features [at, end) marked as flooded and, the first time, listed (one count a step of the wave);
+// nOther: the other side's count.
+__device__ __forceinline__ void sieve_mark(unsigned long long* __restrict__ best, int at, int end, int* flags,
+                                           int* count, int nOther, SieveBest const& out, int lane)
+{
+    for (; at < end; at += 64) {
+        int const i = at + lane;
+        bool const fresh = i < end && atomicMax(best + i, kSieveFlood) != kSieveFlood;
+        unsigned long long const m = __builtin_amdgcn_ballot_w64(fresh);
+        if (!flags || m == 0) continue;
+        int const n = __builtin_popcountll(m);
+        int slot = 0;
+        if (lane == 0) {
+            slot = atomicAdd(count, n);
+            if (out.gate && (long long)(slot + n) * nOther > out.mostListed)
+                __hip_atomic_store(out.gate, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        slot = __builtin_amdgcn_readfirstlane(slot);
+        if (fresh)
+            flags[slot + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] = i;
+    }
+}
+
 // One wave: left features [i0, i0 + 128) against right tiles [t0, t1).  ML, MR: the sets' largest
 // norms; bestL / secondL, bestR / secondR: the features' entries.
 __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R, int i0, int t0, int t1, float ML,
                                            float MR, float T, unsigned long long* __restrict__ bestL,
                                            unsigned* __restrict__ secondL, unsigned long long* __restrict__ bestR,
                                            unsigned* __restrict__ secondR, unsigned const* __restrict__ bits, int ldi,
-                                           SieveBest const& flood, int* list, int lane)
+                                           SieveBest const& out, int* list, int lane)
 {
     int const h = lane >> 5;
     int const c32 = lane & 31;
@@ -161,19 +181,27 @@ __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R,
         sieve_tile(a0, R.q, t0, lane);
         sieve_tile(a1, R.q, min(t0 + 1, t1 - 1), lane);
         int t = t0;
-        for (; t + 1 < t1; t += 2) {
+        for (; t + 1 < t1 && cnt <= out.limit; t += 2) {
             tile(a0, t);
             tile(a1, t + 1);
         }
-        if (t < t1) tile(a0, t);
+        if (t < t1 && cnt <= out.limit) tile(a0, t);
     }
-    if (cnt > kSieveList) {
-        for (int i = i0 + lane; i < min(i0 + 32 * kSieveBlocks, L.n); i += 64)
-            if (atomicMax(bestL + i, kSieveFlood) != kSieveFlood && flood.flags)
-                flood.flags[atomicAdd(flood.cntL, 1)] = i;
-        for (int j = t0 * kSieveTile + lane; j < t1 * kSieveTile; j += 64)
-            if (atomicMax(bestR + j, kSieveFlood) != kSieveFlood && flood.flags)
-                flood.flags[flood.offR + atomicAdd(flood.cntR, 1)] = j;
+    if (cnt > 64 && out.gate) {
+        if (__hip_atomic_load(out.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;  // the full pass's call
+        if (cnt <= out.limit) {
+            unsigned sum = 0;
+            if (lane == 0) {
+                sum = atomicAdd(out.scored, (unsigned)cnt) + (unsigned)cnt;
+                if (sum > out.mostScored) __hip_atomic_store(out.gate, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if ((unsigned)__builtin_amdgcn_readfirstlane((int)sum) > out.mostScored) return;
+        }
+    }
+    if (cnt > out.limit) {
+        sieve_mark(bestL, i0, min(i0 + 32 * kSieveBlocks, L.n), out.flags, out.cntL, R.n, out, lane);
+        sieve_mark(bestR, t0 * kSieveTile, t1 * kSieveTile, out.flags ? out.flags + out.offR : nullptr, out.cntR, L.n,
+                   out, lane);
         return;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // LDS operations of one wave are in order
@@ -251,8 +279,10 @@ __device__ __forceinline__ void sieve_item(BatchDev const& b, int4 w, int t0, in
     size_t const l0 = b.imgBase[sl.img], r0 = b.imgBase[sr.img];
     SieveSet const L{b.q8 + l0 * kDim, b.res + l0 / kSieveGroup, b.img + l0 * kDim, sl.n};
     SieveSet const R{b.q8 + r0 * kDim, b.res + r0 / kSieveGroup, b.img + r0 * kDim, sr.n};
+    SieveBest flood{};  // marked features are listed by the decisions
+    flood.limit = kSieveList;
     sieve_wave(L, R, i0, t0, t1, __uint_as_float(b.maxNorm[sl.img]), __uint_as_float(b.maxNorm[sr.img]), T,
-               best + sl.qOff, second + sl.qOff, best + sr.qOff, second + sr.qOff, nullptr, 0, SieveBest{}, list,
+               best + sl.qOff, second + sl.qOff, best + sr.qOff, second + sr.qOff, nullptr, 0, flood, list,
                threadIdx.x & 63);
 }
 

@@ -58,7 +58,9 @@ struct SplitRowsOf {
     unsigned char* ints;
     int n;
 };
-void launch_split_sets(SplitRowsOf const& a, SplitRowsOf const& b, hipStream_t st);
+// gated: the call's counters, for a launch that does nothing unless its sieve gave the call to the
+// full pass (counters[kCntGate]); null: always.  The same for `gate` below.
+void launch_split_sets(SplitRowsOf const& a, SplitRowsOf const& b, int* gated, hipStream_t st);
 
 // One side of a score pass: n split rows, and for sets uploaded as uint8 their components as
 // FP16 integers with the rows' scales (else null).  All padded to kSplitRowPad rows.
@@ -75,7 +77,8 @@ struct SplitSet {
 // null.  A partial's index is -1 where its best does not exceed minScore.
 FusedPlan plan_split(int nL, int nR);
 void launch_split_pass(SplitSet const& L, SplitSet const& R, FusedPlan const& p, Top2* colPart, int ldc,
-                       Top2* rowPart, int ldr, unsigned const* bits, int ldi, float minScore, hipStream_t st);
+                       Top2* rowPart, int ldr, unsigned const* bits, int ldi, float minScore, hipStream_t st,
+                       int const* gate = nullptr);
 
 // Measurement: the scores of the split pass, out[i * nCols + j] (as launch_score_block).
 void launch_score_block_split(unsigned char const* L, unsigned char const* R, int nRows, int nCols, float* out,

@@ -461,8 +461,10 @@ __global__ __launch_bounds__(256, 2) void k_split_pass(unsigned char const* __re
                                                        int nL, int nR, int leftBlocks, int tilesPerSplit,
                                                        Top2* __restrict__ colPart, int ldc,
                                                        Top2* __restrict__ rowPart, int ldr,
-                                                       unsigned const* __restrict__ bits, int ldi, float thr)
+                                                       unsigned const* __restrict__ bits, int ldi, float thr,
+                                                       int const* __restrict__ gate)
 {
+    if (gate && !*gate) return;
     __shared__ SplitLds<kInt, 4> lds;
     // neighbouring work-groups of one XCD share a split's right tiles in its L2
     int const b = xcd_block(blockIdx.x, gridDim.x);
@@ -578,7 +580,8 @@ FusedPlan plan_split(int nL, int nR)
 }
 
 void launch_split_pass(SplitSet const& L, SplitSet const& R, FusedPlan const& p, Top2* colPart, int ldc,
-                       Top2* rowPart, int ldr, unsigned const* bits, int ldi, float minScore, hipStream_t st)
+                       Top2* rowPart, int ldr, unsigned const* bits, int ldi, float minScore, hipStream_t st,
+                       int const* gate)
 {
     if (L.n <= 0 || R.n <= 0) return;
     dim3 const grid(p.leftBlocks * p.splits);
@@ -586,13 +589,13 @@ void launch_split_pass(SplitSet const& L, SplitSet const& R, FusedPlan const& p,
     float const thr = ints ? minScore : minScore / kSplitBack;  // exact: a power of two
     if (ints)
         hipLaunchKernelGGL((k_split_pass<false, true>), grid, dim3(256), 0, st, L.ints, R.ints, L.scale, R.scale, L.n,
-                           R.n, p.leftBlocks, p.tilesPerSplit, colPart, ldc, rowPart, ldr, bits, ldi, thr);
+                           R.n, p.leftBlocks, p.tilesPerSplit, colPart, ldc, rowPart, ldr, bits, ldi, thr, gate);
     else if (bits)
         hipLaunchKernelGGL((k_split_pass<true, false>), grid, dim3(256), 0, st, L.split, R.split, nullptr, nullptr,
-                           L.n, R.n, p.leftBlocks, p.tilesPerSplit, colPart, ldc, rowPart, ldr, bits, ldi, thr);
+                           L.n, R.n, p.leftBlocks, p.tilesPerSplit, colPart, ldc, rowPart, ldr, bits, ldi, thr, gate);
     else
         hipLaunchKernelGGL((k_split_pass<false, false>), grid, dim3(256), 0, st, L.split, R.split, nullptr, nullptr,
-                           L.n, R.n, p.leftBlocks, p.tilesPerSplit, colPart, ldc, rowPart, ldr, bits, ldi, thr);
+                           L.n, R.n, p.leftBlocks, p.tilesPerSplit, colPart, ldc, rowPart, ldr, bits, ldi, thr, gate);
 }
 
 }  // namespace v3dm

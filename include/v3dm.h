@@ -204,7 +204,10 @@ int v3dm_set_right_u8(v3dm_handle h, int n, const uint8_t* q);
 int v3dm_find_putative_matches_async(v3dm_handle h, float minScore, float minRatio);
 /* Waits for the last _async call and copies its matches (as v3dm_find_putative_matches). */
 int v3dm_get_matches(v3dm_handle h, int32_t* pairs, int cap, int* nPairs);
-/* Device pointers of the last result: int2 pairs[], int counters[] (counters[0] = count). */
+/* Device pointers of the last result: int2 pairs[], int counters[] (counters[0] = count).  From the
+ * first call on (until allocate / deallocate) a plain or guided result is whole on the stream when its
+ * kernels have run; before it, the host finishes a result that needs the full pass after its
+ * sieve when it is read (this call too, for a result pending then). */
 int v3dm_device_results(v3dm_handle h, const int32_t** d_pairs, const int32_t** d_counters);
 /* Per-query decisions of the last call (colMax: nLeft ints, rowMax: nRight ints, -1 = none),
  * the arrays of cu:532-533 after the selection kernels. */

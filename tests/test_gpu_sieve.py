@@ -3,6 +3,8 @@ oracle: matches of pairs at block and tile edges, uneven sizes, minimum scores a
 both sides of the rule that takes the path, rows the int8 form holds badly (large components,
 negative components, norms other than one), equal scores, and sets that overflow the candidate
 lists.  Matches are whole numbers: they equal the oracle's."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -214,4 +216,101 @@ def test_batch_tunes_the_pass_it_takes(dtype, cache):
             want = oracle.find_putative_matches(L, R, ms, mr) if len(L) and len(R) else np.zeros((0, 2), np.int32)
             assert np.array_equal(np.asarray(got[p]).reshape(-1, 2), want.reshape(-1, 2)), (p, ms, mr)
     assert m.batch_time_dominant_kernel(2) > 0
+    m.close()
+
+
+def _many_candidates(kind, n):
+    """Sets that the sieve gives to the full pass: clusters of nearly equal rows (spread over the
+    sets, or in one run on each side), rows with two large components among SIFT rows, and rows of
+    few large components throughout."""
+    rng = np.random.default_rng(21)
+    a, b, _ = synth.make_pair(n, n - 64, 0.4, config=7, pair=5)
+    L, R = synth.dequantise(a).copy(), synth.dequantise(b).copy()
+    if kind in ("spread", "runs", "whole"):
+        k = n - 64 if kind == "whole" else n // 3
+        c = _unit(np.abs(rng.standard_normal((1, 128))))
+        i = rng.permutation(n)[:k] if kind == "spread" else np.arange(k)
+        j = rng.permutation(n - 64)[:k] if kind == "spread" else np.arange(n - 64 - k, n - 64)
+        L[i], R[j] = (_unit(c + 0.03 * rng.standard_normal((k, 128))) for _ in range(2))
+    elif kind == "spikes":
+        for X in (L, R):
+            X[::32] = 0
+            X[::32, 3], X[::32, 9] = 0.8, 0.6
+    else:
+        L, R = (_unit(np.maximum(rng.standard_normal((m, 128)) - 1.3, 0) + 1e-6) for m in (n, n - 64))
+        R[:n // 4] = _unit(L[:n // 4] + 0.02 * np.abs(rng.standard_normal((n // 4, 128))))
+    return L, R
+
+
+KINDS = ["spread", "runs", "whole", "spikes", "large"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("n", [512, 2080, 4064])
+def test_many_candidates(kind, n):
+    """Matches, decisions, the guided call behind them and the next ordinary call."""
+    print(f"case sieve given up {kind} {n}", flush=True)
+    L, R = _many_candidates(kind, n)
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(n, n, True)
+    S = oracle.scores(L, R)
+    for ms, mr in ((0.9, 0.8), (0.9, -1.0)):
+        _same(m, L, R, ms, mr)
+        cm, rm = m.get_maxima()
+        assert np.array_equal(cm, oracle.column_maxima(S, ms, mr))
+        assert np.array_equal(rm, oracle.row_maxima(S, ms, mr))
+    rng = np.random.default_rng(22)
+    lxy, rxy = (rng.uniform(0, 1000, (len(X), 2)).astype(np.float32) for X in (L, R))
+    H = np.eye(3)
+    for t in (900.0, 400.0):  # the second call's mask adds to the first's
+        got = m.run_guided_array(True, H, t, lxy, rxy, 0.9, 0.95)
+    assert np.array_equal(got, oracle.guided(S, 1, H, np.float32(400.0), lxy, rxy, 0.9, 0.95))
+    a, b, _ = synth.make_pair(n, n, 0.4, config=7, pair=6)
+    _same(m, synth.dequantise(a), synth.dequantise(b), 0.9, 0.8)
+    m.close()
+
+
+@pytest.mark.parametrize("kind", KINDS + ["sift"])
+@pytest.mark.parametrize("when", ["before", "after"])
+def test_many_candidates_on_the_device(kind, when):
+    """The same with the result read on the device: whole on the stream after an asynchronous call
+    when the caller has the pointers (before), and when it asks for them (after); sets of settings
+    that change between the call and the reading do not reach it."""
+    print(f"case sieve given up, device results {kind} {when}", flush=True)
+    n = 2080
+    if kind == "sift":
+        a, b, _ = synth.make_pair(n, n, 0.4, config=7, pair=5)
+        L, R = synth.dequantise(a), synth.dequantise(b)
+    else:
+        L, R = _many_candidates(kind, n)
+    rt = C.CDLL("libamdhip64.so")
+    rt.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    m = v3dmatch.SIFT_Matching(0)
+    m.enableRoundingWarning(False)
+    m.allocate(n, n)
+    pairs, counts = C.c_void_p(), C.c_void_p()
+
+    def pointers():
+        assert m._lib.v3dm_device_results(m._h, C.byref(pairs), C.byref(counts)) == 0
+
+    if when == "before":
+        pointers()
+    for ms, mr in ((0.9, 0.8), (0.9, -1.0), (0.9, 0.8)):
+        m.setLeftFeatures(len(L), L)
+        m.setRightFeatures(len(R), R)
+        m.find_async(ms, mr)
+        m.set_certification(0.25)
+        if when == "after":
+            pointers()
+        m.synchronize()
+        m.set_certification(2.0 ** -15)
+        cnt = np.zeros(1, np.int32)
+        assert rt.hipMemcpy(cnt.ctypes.data, counts, 4, 2) == 0
+        got = np.zeros((int(cnt[0]), 2), np.int32)
+        if len(got):
+            assert rt.hipMemcpy(got.ctypes.data, pairs, got.nbytes, 2) == 0
+        want = oracle.find_putative_matches(L, R, ms, mr)
+        assert np.array_equal(got, want.reshape(-1, 2))
+        assert np.array_equal(np.asarray(m.get_matches()).reshape(-1, 2), want.reshape(-1, 2))
     m.close()
