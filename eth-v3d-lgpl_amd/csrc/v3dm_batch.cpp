@@ -84,10 +84,12 @@ struct BatchState {
     unsigned* sieveSecond = nullptr;
     int sieveCap = 0;
     int4* sieveItems = nullptr;
-    int nSieveItems = 0, sieveItemCap = 0;
+    int nSieveItems = 0, sieveItemCap = 0, sieveTiles = 1;
     bool sieveValid = false;  // sieveItems hold the current pairs
-    bool lastSieve = false;   // the last run took the sieve, with this bound
+    bool lastSieve = false;   // the last plain run took the sieve, with this bound
     float lastT = 0.0f;
+    bool sieveBounded = false;  // the last run's plain decisions came from a sieve that may have given them up
+    float lastEps = 0.0f;       // its error bound
     bool codesValid = false;
     float codesScale = 0.0f;
     int* imgBase = nullptr;
@@ -115,7 +117,7 @@ struct BatchState {
     // so that a few pairs still spread over the whole GPU)
     Plan plan[4];
     bool planValid[4] = {false, false, false, false};
-    bool planPass[4] = {false, false, false, false};  // ... and is ready for its pass (else the layout alone)
+    int planUse[4] = {0, 0, 0, 0};  // ... and what it is ready for (PlanUse)
     int4* items[4] = {nullptr, nullptr, nullptr, nullptr};
     int itemCap[4] = {0, 0, 0, 0};
     BatchSeg* segD[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -417,7 +419,11 @@ Plan plan_short_batch(BatchState* b, int tiles, int grid, int maxSplits, bool wh
     return pl;
 }
 
-// pass: with room for the partials of the plan's pass (else the layout of the queries alone).
+// What a run needs of the plan of its form: the layout of the queries alone (it takes the sieve), its
+// pass with room for the partials in the default setting, or in the tuned one.
+enum PlanUse { kPlanLayout, kPlanPass, kPlanTuned };
+
+// pass: with room for the partials of the plan's pass.
 int upload_plan(v3dm_context* h, BatchState* b, int form, Plan const& pl, bool pass = true)
 {
     int rc;
@@ -706,15 +712,16 @@ int ensure_sieve(v3dm_context* h, BatchState* b)
                                  h->stream));
     BCHECK(h, hipStreamSynchronize(h->stream));
     b->nSieveItems = (int)items.size();
+    b->sieveTiles = tiles;
     b->sieveValid = true;
     b->version += 1;
     return V3DM_OK;
 }
 
 // The certified decisions' error bound for the scores of launch_plain_pass.
-float plain_eps(v3dm_context const* h, BatchState const* b)
+float plain_eps(BatchState const* b, float epsRel)
 {
-    return b->splitFit ? h->epsRel * (b->haveU8 ? kIntEps : kSplitEps) : h->epsRel;
+    return b->splitFit ? epsRel * (b->haveU8 ? kIntEps : kSplitEps) : epsRel;
 }
 
 // The plain pass of plan `form` (0, or 3: the pairs a learned run hands over) on the images'
@@ -728,6 +735,62 @@ void launch_plain_pass(BatchState* b, int form, int4 const* items, int nItems, i
         launch_batch_split(d, b->haveU8, items, nItems, queue, b->partF, pl.grid, pl.qRows, minScore, st, nItemsDev);
     else
         launch_batch_fused_fp32(d, items, nItems, queue, b->partF, pl.grid, pl.qRows, st, nItemsDev);
+}
+
+int cu_count()
+{
+    int dev = 0, cus = 256;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    return cus;
+}
+
+// The plain decisions of a run by the full pass: of every pair (form 0), or of the pairs that a
+// learned run hands over (form 2: their items, merge masked to their segments; kernels with
+// nothing to do when no pair is flagged).
+void enqueue_full(v3dm_context* h, BatchState* b, int form, float epsRel, float minScore, float minRatio)
+{
+    hipStream_t const st = h->stream;
+    BatchDev const d = dev_view(b, form == 0 ? 0 : 3);
+    if (form == 0) {
+        launch_plain_pass(b, 0, b->items[0], (int)b->plan[0].items.size(), b->counters + 0, minScore, st);
+        launch_batch_merge_decide(d, b->partF, plain_eps(b, epsRel), minScore, minRatio, b->sel, b->flagList,
+                                  b->counters, st);
+    } else {
+        int const np = (int)b->plan[3].items.size(), cus = cu_count();
+        launch_batch_fb_filter(b->items[3], np, b->pairFlag, b->nPairs, b->fbItems, b->counters + kBCntFbItems,
+                               b->segMask, st);
+        // (the rows of a plain run may be there already, of the same images)
+        if (b->splitFit && !(h->cacheDerived && b->splitValid))
+            launch_batch_split_masked(d, b->segMask, b->split, 2 * cus, st);
+        launch_plain_pass(b, 3, b->fbItems, np, b->counters + 0, minScore, st, b->counters + kBCntFbItems);
+        launch_batch_merge_masked(d, b->partF, plain_eps(b, epsRel), minScore, minRatio, b->sel, b->flagList,
+                                  b->counters, b->segMask, 2 * cus, st);
+    }
+    launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio, b->sel,
+                         1024, st);
+}
+
+// The same by the sieve (the rows of form 0 are made).  bounded: with many candidates the decisions
+// are void and counters[kBCntGate] is set; the run's reader then has them made by the full pass.
+void enqueue_sieved(v3dm_context* h, BatchState* b, int form, float T, float minScore, float minRatio, bool bounded)
+{
+    hipStream_t const st = h->stream;
+    BatchDev const d = dev_view(b, form == 0 ? 0 : 3);
+    BatchSieve s{b->sieveItems, b->nSieveItems, nullptr, b->sieveTiles, T, b->sieveBest, b->sieveSecond,
+                 bounded ? b->counters : nullptr};
+    if (form != 0) {
+        s.items = b->fbItems;
+        s.nItemsDev = b->counters + kBCntFbItems;
+        launch_batch_fb_filter(b->sieveItems, b->nSieveItems, b->pairFlag, b->nPairs, b->fbItems,
+                               b->counters + kBCntFbItems, b->segMask, st);
+        if (!(h->cacheDerived && b->q8Valid)) launch_batch_sieve_masked(d, b->segMask, b->q8, b->res, st);
+    }
+    launch_batch_sieve(d, s, st);
+    launch_batch_sieve_decide(d, s, minScore, minRatio, b->sel, b->flagList, b->counters,
+                              form == 0 ? nullptr : b->segMask, st);
+    launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio, b->sel,
+                         1024, st, bounded ? b->counters + kBCntGate : nullptr);
 }
 
 // Enqueue one batch run of `mode` with the current plan of its form.
@@ -745,16 +808,9 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
         else enqueue_derived(h, b, form);
     }
     if (form == 0 && sieve) {
-        launch_batch_sieve(d, b->sieveItems, b->nSieveItems, T, b->sieveBest, b->sieveSecond, st);
-        launch_batch_sieve_decide(d, b->sieveBest, b->sieveSecond, minScore, minRatio, b->sel, b->flagList,
-                                  b->counters, nullptr, st);
-        launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio,
-                             b->sel, 1024, st);
+        enqueue_sieved(h, b, 0, T, minScore, minRatio, true);
     } else if (form == 0) {
-        launch_plain_pass(b, 0, b->items[0], (int)pl.items.size(), b->counters + 0, minScore, st);
-        launch_batch_merge_decide(d, b->partF, plain_eps(h, b), minScore, minRatio, b->sel, b->flagList, b->counters, st);
-        launch_batch_recheck(d, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore, minRatio,
-                             b->sel, 1024, st);
+        enqueue_full(h, b, 0, h->epsRel, minScore, minRatio);
     } else if (form == 1) {
         launch_batch_pass_bf16(d, b->items[1], (int)pl.items.size(), b->counters + 1, b->partB, pl.grid, pl.qRows,
                                st);
@@ -766,9 +822,7 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
         launch_batch_rescore(d, b->partB, 0.0f, h->learnedTopK, learned_margin(h), minScore, minRatio,
                              h->epsRel > 0.0f, b->sel, b->openList, b->counters + kBCntOpenRescore, b->stripes, st);
         if (h->fallbackSamples > 0) {
-            int dev = 0, cus = 256;
-            (void)hipGetDevice(&dev);
-            (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+            int const cus = cu_count();
             MissLimits const lim = miss_limits(h);
             if (b->haveU8) {
                 // exact mutual matches among the samples against the learned result
@@ -788,30 +842,9 @@ int enqueue_run(v3dm_context* h, BatchState* b, int mode, float minScore, float 
                                            h->epsRel, minScore, minRatio, lim, b->sel, b->pairFlag,
                                            b->pairFlag + b->nPairs, st);
             }
-            // pairs whose sampled recall fell short get the plain form's decisions, on the
-            // device: their plain items, merge masked to their segments, exact re-check
-            // (kernels with nothing to do when no pair is flagged)
-            Plan const& pp = b->plan[3];
-            int const np = (int)pp.items.size();
-            BatchDev const d0 = dev_view(b, 3);
-            launch_batch_fb_filter(sieve ? b->sieveItems : b->items[3], sieve ? b->nSieveItems : np, b->pairFlag,
-                                   b->nPairs, b->fbItems, b->counters + kBCntFbItems, b->segMask, st);
-            // (the rows of a plain run may be there already, of the same images)
-            if (sieve) {
-                if (!(h->cacheDerived && b->q8Valid)) launch_batch_sieve_masked(d0, b->segMask, b->q8, b->res, st);
-                launch_batch_sieve_listed(d0, b->fbItems, b->counters + kBCntFbItems, T, b->sieveBest, b->sieveSecond,
-                                          st);
-                launch_batch_sieve_decide(d0, b->sieveBest, b->sieveSecond, minScore, minRatio, b->sel, b->flagList,
-                                          b->counters, b->segMask, st);
-            } else {
-                if (b->splitFit && !(h->cacheDerived && b->splitValid))
-                    launch_batch_split_masked(d0, b->segMask, b->split, 2 * cus, st);
-                launch_plain_pass(b, 3, b->fbItems, np, b->counters + 0, minScore, st, b->counters + kBCntFbItems);
-                launch_batch_merge_masked(d0, b->partF, plain_eps(h, b), minScore, minRatio, b->sel, b->flagList,
-                                          b->counters, b->segMask, 2 * cus, st);
-            }
-            launch_batch_recheck(d0, b->flagList, b->counters, b->partF, b->partFCap, b->tickets, minScore,
-                                 minRatio, b->sel, 1024, st);
+            // pairs whose sampled recall fell short get the plain form's decisions, on the device
+            if (sieve) enqueue_sieved(h, b, 2, T, minScore, minRatio, true);
+            else enqueue_full(h, b, 2, h->epsRel, minScore, minRatio);
         }
     }
     launch_batch_mutual(d, b->sel, b->leftRows, b->tmp, b->blockCount, b->out, b->pairCount, b->stripes,
@@ -854,13 +887,12 @@ int time_pass(v3dm_context* h, BatchState* b, int form, Plan const& pl, float& m
 // rows against 64-candidate tiles, i.e. 2 or 4 waves (FP32 rows: 4 or 8) for the plain form's
 // full pass, 2 or 4 waves for
 // the BF16 and code passes) for a form: the given override, or the fastest candidate
-// measured on this batch, or the default when tuning is off.  pass = false: for a run that takes
-// the sieve and of this plan needs the query layout alone; nothing is timed (the 16 candidates
-// of the plain form took 0.23 s on the 256-pair batch, whose run takes 0.9 ms) and no partials
-// are allocated, until a run takes the pass.
-int ensure_plan(v3dm_context* h, BatchState* b, int form, bool pass)
+// measured on this batch, or the default when tuning is off.  A run that takes the sieve asks for
+// kPlanLayout: nothing is timed (the 16 candidates of the plain form took 0.23 s on the 256-pair
+// batch, whose run takes 0.9 ms) and no partials are allocated, until a run takes the pass.
+int ensure_plan(v3dm_context* h, BatchState* b, int form, PlanUse use)
 {
-    if (b->planValid[form] && (b->planPass[form] || !pass)) return V3DM_OK;
+    if (b->planValid[form] && b->planUse[form] >= use) return V3DM_OK;
     b->planValid[form] = false;  // (should this fail, the next run plans again)
     drop_graphs(b);              // captured runs hold the old buffers
     int dev = 0;
@@ -891,7 +923,14 @@ int ensure_plan(v3dm_context* h, BatchState* b, int form, bool pass)
         bestT = b->forceTiles[form] > 0 ? b->forceTiles[form] : bestT;
         bestQ = b->forceQRows[form] > 0 ? b->forceQRows[form] : bestQ;
         bestG = b->forceGrid[form] > 0 ? b->forceGrid[form] : gridCands(bestQ)[0];
-    } else if (b->autotune && pass) {
+        if (use == kPlanPass) use = kPlanTuned;
+    } else if (!b->autotune) {
+        if (use == kPlanPass) use = kPlanTuned;
+    } else if (use == kPlanPass && form == 0 && b->splitFit) {
+        // the split pass's usual choice: 2.0 ms on the 256-pair uint8 batch, 4 with the default
+        bestT = 32;
+        bestQ = 256;
+    } else if (use == kPlanTuned) {
         for (int q : shapeCands)
             for (int t : tileCands)
                 for (int g : gridCands(q)) {
@@ -908,11 +947,11 @@ int ensure_plan(v3dm_context* h, BatchState* b, int form, bool pass)
     }
     Plan pl = make(bestT, bestG, bestQ);
     pl.passMs = bestMs;
-    int const rc = upload_plan(h, b, form, pl, pass);
+    int const rc = upload_plan(h, b, form, pl, use != kPlanLayout);
     if (rc) return rc;
     b->plan[form] = std::move(pl);
     b->planValid[form] = true;
-    b->planPass[form] = pass;
+    b->planUse[form] = use;
     b->version += 1;
     return V3DM_OK;
 }
@@ -944,6 +983,52 @@ int ensure_fallback_plan(v3dm_context* h, BatchState* b)
         if ((rc = growi(h, b->fbItems, b->fbItemCap, need))) return rc;
         b->version += 1;
     }
+    return V3DM_OK;
+}
+
+// The end of a run: its event, and its counts to the host.
+int enqueue_counts(v3dm_context* h, BatchState* b)
+{
+    hipStream_t const st = h->stream;
+    BCHECK(h, hipEventRecord(b->evB, st));
+    BCHECK(h, hipMemcpyAsync(b->hostRes, b->counters, kBatchCounters * sizeof(int), hipMemcpyDeviceToHost, st));
+    BCHECK(h, hipMemcpyAsync(b->hostRes + kBatchCounters, b->pairCount, b->nPairs * sizeof(int),
+                             hipMemcpyDeviceToHost, st));
+    return V3DM_OK;
+}
+
+// The last run, whose sieve gave its plain decisions up: those by the full pass (in its default
+// setting where none is tuned yet), then the mutual check and the counts again.  Where the pass's
+// buffers do not fit, by the sieve without a bound.
+int redo_plain(v3dm_context* h, BatchState* b)
+{
+    int const form = form_of(b->lastMode);
+    hipStream_t const st = h->stream;
+    int const rescored = b->hostRes[kBCntRescoredDone];
+    bool const room = ensure_split(h, b) == V3DM_OK && (form != 0 || ensure_plan(h, b, 0, kPlanPass) == V3DM_OK);
+    if (!room) {
+        (void)hipGetLastError();
+        int rc;
+        if (form == 0 && (rc = ensure_plan(h, b, 0, kPlanLayout))) return rc;
+        if (form != 0 && (rc = ensure_fallback_plan(h, b))) return rc;
+    }
+    launch_batch_reset(b->counters, b->pairCount, b->nPairs, st);
+    if (!room) {
+        enqueue_sieved(h, b, form, b->lastT, b->lastMinScore, b->lastMinRatio, false);
+    } else {
+        if (form == 0 && !(h->cacheDerived && b->splitValid)) {
+            enqueue_derived(h, b, 0);
+            b->splitValid = h->cacheDerived;
+        }
+        enqueue_full(h, b, form, b->lastEps, b->lastMinScore, b->lastMinRatio);
+    }
+    launch_batch_mutual(dev_view(b, form), b->sel, b->leftRows, b->tmp, b->blockCount, b->out, b->pairCount, b->stripes,
+                        b->counters, st);
+    BCHECK(h, hipGetLastError());
+    int const rc = enqueue_counts(h, b);
+    if (rc) return rc;
+    BCHECK(h, hipStreamSynchronize(st));
+    b->hostRes[kBCntRescoredDone] = rescored;  // (counted by the learned run itself)
     return V3DM_OK;
 }
 
@@ -1248,7 +1333,7 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
     float T = 0.0f;
     bool const sieve = plain && sieve_run(h, b, minScore, minRatio, &T);
     bool const split = plain && !sieve;
-    bool const pass = !(form == 0 && sieve);  // the run takes the pass of its form's plan
+    PlanUse const use = form == 0 && sieve ? kPlanLayout : kPlanTuned;
     if (sieve && (rc = ensure_sieve(h, b))) return rc;
     if (split && (rc = ensure_split(h, b))) return rc;
     // derived copies outside the run when they are cached (else every run derives them)
@@ -1268,10 +1353,10 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
         enqueue_derived(h, b, 2);
         b->codesValid = true;
     }
-    if (!h->cacheDerived && pass && !(b->planValid[form] && b->planPass[form]))
+    if (!h->cacheDerived && use == kPlanTuned && !(b->planValid[form] && b->planUse[form] == kPlanTuned))
         enqueue_derived(h, b, form);  // for the tuner
     if (!h->cacheDerived) b->splitValid = b->q8Valid = false;  // a learned run rewrites rows of its failing pairs
-    if ((rc = ensure_plan(h, b, form, pass))) return rc;
+    if ((rc = ensure_plan(h, b, form, use))) return rc;
     if (form == 2 && h->fallbackSamples > 0 && (rc = ensure_fallback_plan(h, b))) return rc;
     BCHECK(h, hipEventRecord(b->evA, st));
     if (b->useGraph) {
@@ -1300,10 +1385,7 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
     } else if ((rc = enqueue_run(h, b, mode, minScore, minRatio))) {
         return rc;
     }
-    BCHECK(h, hipEventRecord(b->evB, st));
-    BCHECK(h, hipMemcpyAsync(b->hostRes, b->counters, kBatchCounters * sizeof(int), hipMemcpyDeviceToHost, st));
-    BCHECK(h, hipMemcpyAsync(b->hostRes + kBatchCounters, b->pairCount, b->nPairs * sizeof(int),
-                             hipMemcpyDeviceToHost, st));
+    if ((rc = enqueue_counts(h, b))) return rc;
     b->checkPending = form == 2 && h->fallbackSamples > 0;
     if (b->checkPending)
         BCHECK(h, hipMemcpyAsync(b->hostChk, b->pairFlag, 5 * b->nPairs * sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1313,6 +1395,8 @@ int v3dm_batch_match_async(v3dm_handle h, float minScore, float minRatio)
     b->lastMode = mode;
     b->lastSieve = form == 0 && sieve;
     b->lastT = T;
+    b->sieveBounded = sieve;
+    b->lastEps = h->epsRel;
     return V3DM_OK;
 }
 
@@ -1324,6 +1408,10 @@ int v3dm_batch_get_matches(v3dm_handle h, int32_t* offsets, int32_t* pairs, int 
     if (!b->pending) return ctx_fail(h, V3DM_ERR_STATE, "no batch run pending");
     if (!nTotal || cap < 0 || (cap > 0 && !pairs)) return ctx_fail(h, V3DM_ERR_INVALID, "invalid output");
     BCHECK(h, hipStreamSynchronize(h->stream));
+    if (b->sieveBounded && b->hostRes[kBCntGate]) {
+        if ((rc = redo_plain(h, b))) return rc;
+        b->sieveBounded = false;
+    }
     float ms = 0.0f;
     if (hipEventElapsedTime(&ms, b->evA, b->evB) == hipSuccess) b->lastMs = ms;
     h->stats.nFallback = h->stats.nSampled = h->stats.nSampleMissed = 0;
@@ -1387,7 +1475,10 @@ int v3dm_batch_time_dominant_kernel(v3dm_handle h, int reps, float* msPerLaunch)
     for (int r = 0; r < reps && e == hipSuccess; ++r) {
         int const n = (int)pl.items.size();
         if (form == 0 && b->lastSieve)
-            launch_batch_sieve(d, b->sieveItems, b->nSieveItems, b->lastT, b->sieveBest, b->sieveSecond, st);
+            launch_batch_sieve(d,
+                               BatchSieve{b->sieveItems, b->nSieveItems, nullptr, b->sieveTiles, b->lastT, b->sieveBest,
+                                          b->sieveSecond, nullptr},
+                               st);
         else if (form == 0) launch_plain_pass(b, 0, b->items[0], n, q + r, b->lastMinScore, st);
         else if (form == 1) launch_batch_pass_bf16(d, b->items[1], n, q + r, b->partB, pl.grid, pl.qRows, st);
         else launch_batch_pass_code(d, b->items[2], n, q + r, b->partB, pl.grid, pl.qRows, st);

@@ -31,6 +31,9 @@ constexpr int kBCntRescoredDone = 8;
 constexpr int kBCntFbItems = 10;  // plain items of the pairs a learned run hands to the plain form
 constexpr int kBQueueCheck0 = 3;  // work counter of the sampled check of FP32 batches
 constexpr int kBCntOpenRescore = 12;  // open decisions of the shortlist rescoring
+constexpr int kBCntGate = 13;    // the run's sieve gave its plain decisions to the full pass (v3dm_sieve.h)
+constexpr int kBCntScored = 14;  // candidates of its fuller waves
+constexpr int kBCntListed = 15;  // listed features, each with the blocks of 64 features of the other image
 constexpr int kBatchCounters = 16;
 
 struct BatchSeg {
@@ -168,8 +171,10 @@ void launch_batch_check_decide(BatchDev const& b, CheckDev const& c, int phase, 
                                MissLimits const& lim, int const* sel, int* pairFlag, int* counts, hipStream_t st);
 // part: scratch for at least qRows partials (room of them); tickets: qRows ints, zero before the
 // first call and left zero
+// (gate, or null: nothing is done where *gate is set)
 void launch_batch_recheck(BatchDev const& b, int const* flagList, int* counters, Top2* part, size_t room,
-                          int* tickets, float minScore, float minRatio, int* sel, int grid, hipStream_t st);
+                          int* tickets, float minScore, float minRatio, int* sel, int grid, hipStream_t st,
+                          int const* gate = nullptr);
 // the plain items of the pairs with pairFlag set -> fbItems (count in *fbCount, which must
 // be zero), segMask[s] = flag of segment s's pair (2 * nPairs segments)
 void launch_batch_fb_filter(int4 const* items, int nItems, int const* pairFlag, int nPairs, int4* fbItems,
@@ -181,12 +186,19 @@ void launch_batch_mutual(BatchDev const& b, int const* sel, int leftRows, int2* 
 // entry per query row, zero before a pass and after the decisions.
 void launch_batch_sieve_rows(BatchDev const& b, int rows, signed char* q8, float* res, hipStream_t st);
 void launch_batch_sieve_masked(BatchDev const& b, int const* segMask, signed char* q8, float* res, hipStream_t st);
-void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
-                        unsigned* second, hipStream_t st);
-void launch_batch_sieve_listed(BatchDev const& b, int4 const* items, int const* nItems, float T,
-                               unsigned long long* best, unsigned* second, hipStream_t st);
-void launch_batch_sieve_decide(BatchDev const& b, unsigned long long* best, unsigned* second, float minScore,
-                               float minRatio, int* sel, int* flagList, int* counters, int const* segMask,
-                               hipStream_t st);
+// nItems items, or the *nItemsDev first ones (an earlier kernel's count) of at most nItems.
+struct BatchSieve {
+    int4 const* items;
+    int nItems;
+    int const* nItemsDev;
+    int tiles;  // of every item
+    float T;
+    unsigned long long* best;
+    unsigned* second;
+    int* counters;  // null: no bound (v3dm_sieve.h)
+};
+void launch_batch_sieve(BatchDev const& b, BatchSieve const& s, hipStream_t st);
+void launch_batch_sieve_decide(BatchDev const& b, BatchSieve const& s, float minScore, float minRatio, int* sel,
+                               int* flagList, int* counters, int const* segMask, hipStream_t st);
 
 }  // namespace v3dm

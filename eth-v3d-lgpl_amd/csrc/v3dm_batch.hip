@@ -188,8 +188,10 @@ void launch_batch_merge_masked(BatchDev const& b, Top2 const* part, float epsRel
 __global__ __launch_bounds__(256) void k_batch_recheck(BatchDev b, int const* __restrict__ flagList,
                                                        int const* __restrict__ counters, Top2* __restrict__ part,
                                                        long long room, int* __restrict__ tickets, float minScore,
-                                                       float minRatio, int* __restrict__ sel)
+                                                       float minRatio, int* __restrict__ sel,
+                                                       int const* __restrict__ gate)
 {
+    if (gate && *gate) return;
     __shared__ __attribute__((aligned(16))) float stage[4][kExactLds];
     __shared__ __attribute__((aligned(16))) double qd[4][kDim];
     int const lane = threadIdx.x & 63;
@@ -227,10 +229,11 @@ __global__ __launch_bounds__(256) void k_batch_recheck(BatchDev b, int const* __
 }
 
 void launch_batch_recheck(BatchDev const& b, int const* flagList, int* counters, Top2* part, size_t room,
-                          int* tickets, float minScore, float minRatio, int* sel, int grid, hipStream_t st)
+                          int* tickets, float minScore, float minRatio, int* sel, int grid, hipStream_t st,
+                          int const* gate)
 {
     hipLaunchKernelGGL(k_batch_recheck, dim3(grid), dim3(256), 0, st, b, flagList, counters, part, (long long)room,
-                       tickets, minScore, minRatio, sel);
+                       tickets, minScore, minRatio, sel, gate);
 }
 
 // Mutual check over the left-query rows [0, leftRows) of the query space (segments 0 ..

@@ -52,7 +52,7 @@ struct SieveSet {
 // follow), its decisions are void, and the remaining waves neither score nor list.  gate null:
 // no bound.
 constexpr unsigned long long kSieveFlood = ~0ull;
-constexpr int kSieveList = 512;  // the largest limit
+constexpr int kSieveList = 512;  // a pair's largest limit
 
 struct SieveBest {
     unsigned long long* best;
@@ -77,7 +77,7 @@ struct SieveBest {
 // 334 / 335, 8192 x 8192 40 / 47 / 139 / 153, 2048 x 2048 30 / 30 / 87 / 75; with lists of 2048 and
 // no bounds 60 / 91 / 827 / 15528, 40 / 46 / 263 / 5895 and 29 / 30 / 55 / 457; with the FP32
 // instruction 735, 248 and 81 at any share.
-inline unsigned sieve_most_scored(double pairs) { return (unsigned)(135000.0 + pairs / 430); }
+__host__ __device__ inline unsigned sieve_most_scored(double pairs) { return (unsigned)(135000.0 + pairs / 430); }
 inline long long sieve_most_listed(double pairs) { return (1LL << 20) + (long long)(pairs / 32); }
 inline int sieve_limit(long long pairs)  // of a wave of `pairs` scores
 {

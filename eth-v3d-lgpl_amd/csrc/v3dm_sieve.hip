@@ -33,7 +33,7 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // L2 (the four waves of a group take the same tiles), two tiles ahead; there is no LDS staging
 // and no barrier.  Per block the 16 scores of a lane are reduced by 8 max3 and compared with
 // the lane's bound; only a block with a score above it looks at single scores and lists them
-// (LDS, kSieveList per wave; sets hold less than 2^24 rows).  After its last tile the wave
+// (LDS, at most the limit per wave; sets hold less than 2^24 rows).  After its last tile the wave
 // scores its list exactly, a pair per lane, and enters each score for both features: an atomic
 // maximum of (score, ~index) returns the smaller of two keys, which goes to the second best's
 // maximum; so every key but the largest reaches it, and equal scores keep the smallest index.
@@ -118,7 +118,7 @@ __device__ __forceinline__ void sieve_mark(unsigned long long* __restrict__ best
     }
 }
 
-// One wave: left features [i0, i0 + 128) against right tiles [t0, t1).  ML, MR: the sets' largest
+// One wave: left features [i0, i0 + 128) against right tiles [t0, t1); list: out.limit entries.  ML, MR: the sets' largest
 // norms; bestL / secondL, bestR / secondR: the features' entries.
 __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R, int i0, int t0, int t1, float ML,
                                            float MR, float T, unsigned long long* __restrict__ bestL,
@@ -142,7 +142,8 @@ __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R,
         arm = fmaxf(arm, ML + r);
     }
     arm *= 65536.0f;
-    int cnt = 0;  // uniform
+    int cnt = 0;    // uniform
+    int stop = t1;  // ... 0 past the limit
     auto tile = [&](v4i(&a)[4], int t) {
         float const* const rt = R.res + t * (kSieveTile / kSieveGroup);
         float const r = fmaxf(fmaxf(rt[0], rt[1]), fmaxf(rt[2], rt[3]));
@@ -169,9 +170,10 @@ __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R,
                     if (m == 0) continue;
                     int const at = cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
                                                                    __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-                    if (hit && at < kSieveList) list[at] = entry | e;
+                    if (hit && at < out.limit) list[at] = entry | e;
                     cnt += __builtin_popcountll(m);
                 }
+                if (cnt > out.limit) stop = 0;
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -181,11 +183,11 @@ __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R,
         sieve_tile(a0, R.q, t0, lane);
         sieve_tile(a1, R.q, min(t0 + 1, t1 - 1), lane);
         int t = t0;
-        for (; t + 1 < t1 && cnt <= out.limit; t += 2) {
+        for (; t + 1 < stop; t += 2) {
             tile(a0, t);
             tile(a1, t + 1);
         }
-        if (t < t1 && cnt <= out.limit) tile(a0, t);
+        if (t < stop) tile(a0, t);
     }
     if (cnt > 64 && out.gate) {
         if (__hip_atomic_load(out.gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;  // the full pass's call
@@ -267,9 +269,8 @@ void launch_sieve(SieveSet const& L, SieveSet const& R, SievePlan const& p, unsi
 // work-group each.
 // 256 uneven uint8 pairs: 531 us (2.9 TB/s would read the rows, 3.4 POPS of int8 products) + 13 for
 // the decisions, against 2358 + 167 + 23 of the integer-row pass, its merge and its re-check.
-__device__ __forceinline__ void sieve_item(BatchDev const& b, int4 w, int t0, int t1, float T,
-                                           unsigned long long* __restrict__ best, unsigned* __restrict__ second,
-                                           int* list, int wv)
+__device__ __forceinline__ void sieve_item(BatchDev const& b, BatchSieve const& s, int4 w, int t0, int t1, int n,
+                                           int limit, int* list, int wv)
 {
     BatchSeg const sl = b.seg[w.x];
     BatchSeg const sr = b.seg[b.nPairs + w.x];
@@ -279,21 +280,29 @@ __device__ __forceinline__ void sieve_item(BatchDev const& b, int4 w, int t0, in
     size_t const l0 = b.imgBase[sl.img], r0 = b.imgBase[sr.img];
     SieveSet const L{b.q8 + l0 * kDim, b.res + l0 / kSieveGroup, b.img + l0 * kDim, sl.n};
     SieveSet const R{b.q8 + r0 * kDim, b.res + r0 / kSieveGroup, b.img + r0 * kDim, sr.n};
-    SieveBest flood{};  // marked features are listed by the decisions
-    flood.limit = kSieveList;
-    sieve_wave(L, R, i0, t0, t1, __uint_as_float(b.maxNorm[sl.img]), __uint_as_float(b.maxNorm[sr.img]), T,
-               best + sl.qOff, second + sl.qOff, best + sr.qOff, second + sr.qOff, nullptr, 0, flood, list,
+    SieveBest out{};  // (marked features are listed by the decisions)
+    out.limit = limit;
+    if (s.counters) {
+        out.gate = s.counters + kBCntGate;
+        out.scored = reinterpret_cast<unsigned*>(s.counters + kBCntScored);
+        out.mostScored = sieve_most_scored((double)n * s.tiles * (128.0 * kSieveBlocks * kSieveTile));
+    }
+    sieve_wave(L, R, i0, t0, t1, __uint_as_float(b.maxNorm[sl.img]), __uint_as_float(b.maxNorm[sr.img]), s.T,
+               s.best + sl.qOff, s.second + sl.qOff, s.best + sr.qOff, s.second + sr.qOff, nullptr, 0, out, list,
                threadIdx.x & 63);
 }
 
-__global__ __launch_bounds__(256, 3) void k_batch_sieve(BatchDev b, int4 const* __restrict__ items, float T,
-                                                        unsigned long long* __restrict__ best,
-                                                        unsigned* __restrict__ second)
+constexpr int kBatchSieveList = 2048;
+
+__global__ __launch_bounds__(256, 3) void k_batch_sieve(BatchDev b, BatchSieve s)
 {
-    __shared__ int lists[4][kSieveList];
+    // a wave's run of 64 tiles holds 2^18 scores: longer lists than a pair's, since listing its
+    // features for the exact re-check costs far more than scoring some thousand candidates
+    __shared__ int lists[4][kBatchSieveList];
     int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    int4 const w = items[blockIdx.x];
-    sieve_item(b, w, w.z * w.w, (w.z + 1) * w.w, T, best, second, lists[wv], wv);
+    int4 const w = s.items[blockIdx.x];
+    int const limit = min(max(s.tiles * kSieveTile, kSieveList), kBatchSieveList);
+    sieve_item(b, s, w, w.z * w.w, (w.z + 1) * w.w, s.nItems, limit, lists[wv], wv);
 }
 
 // The items of the pairs that a learned run hands over (counted by an earlier kernel): few, so
@@ -302,60 +311,66 @@ __global__ __launch_bounds__(256, 3) void k_batch_sieve(BatchDev b, int4 const* 
 // 256-pair batch, 31 so.
 constexpr int kSieveRun = 8;
 
-__global__ __launch_bounds__(256, 3) void k_batch_sieve_listed(BatchDev b, int4 const* __restrict__ items,
-                                                               int const* __restrict__ nItems, float T,
-                                                               unsigned long long* __restrict__ best,
-                                                               unsigned* __restrict__ second)
+__global__ __launch_bounds__(256, 3) void k_batch_sieve_listed(BatchDev b, BatchSieve s)
 {
     __shared__ int lists[4][kSieveList];
     int const wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    int const n = __builtin_amdgcn_readfirstlane(*nItems);
-    if (n == 0) return;
-    int const runs = (items[0].w + kSieveRun - 1) / kSieveRun;  // every item has the same tiles per split
+    int const n = __builtin_amdgcn_readfirstlane(*s.nItemsDev);
+    int const runs = (s.tiles + kSieveRun - 1) / kSieveRun;
     for (int u = blockIdx.x; u < n * runs; u += gridDim.x) {
-        int4 const w = items[u / runs];
+        int4 const w = s.items[u / runs];
         int const t0 = w.z * w.w + (u % runs) * kSieveRun;
-        sieve_item(b, w, t0, min(t0 + kSieveRun, (w.z + 1) * w.w), T, best, second, lists[wv], wv);
+        sieve_item(b, s, w, t0, min(t0 + kSieveRun, (w.z + 1) * w.w), n, kSieveList, lists[wv], wv);
     }
 }
 
-void launch_batch_sieve(BatchDev const& b, int4 const* items, int nItems, float T, unsigned long long* best,
-                        unsigned* second, hipStream_t st)
+void launch_batch_sieve(BatchDev const& b, BatchSieve const& s, hipStream_t st)
 {
-    if (nItems <= 0) return;
-    hipLaunchKernelGGL(k_batch_sieve, dim3(nItems), dim3(256), 0, st, b, items, T, best, second);
-}
-
-void launch_batch_sieve_listed(BatchDev const& b, int4 const* items, int const* nItems, float T,
-                               unsigned long long* best, unsigned* second, hipStream_t st)
-{
-    if (b.nPairs <= 0) return;
-    hipLaunchKernelGGL(k_batch_sieve_listed, dim3(768), dim3(256), 0, st, b, items, nItems, T, best, second);
+    if (s.nItems <= 0) return;
+    if (s.nItemsDev) hipLaunchKernelGGL(k_batch_sieve_listed, dim3(768), dim3(256), 0, st, b, s);
+    else hipLaunchKernelGGL(k_batch_sieve, dim3(s.nItems), dim3(256), 0, st, b, s);
 }
 
 // ------------------------------------------------------------------------------ decisions
-__global__ __launch_bounds__(256) void k_batch_sieve_decide(BatchDev b, unsigned long long* __restrict__ best,
-                                                            unsigned* __restrict__ second, float minScore,
-                                                            float minRatio, int* __restrict__ sel,
-                                                            int* __restrict__ flagList, int* __restrict__ counters,
+// The bound of the listed features (v3dm_sieve.h): blocks of 64 candidates each, 128 of the run's
+// scores for one; the batch's exact re-check takes 28 pairs per ns.
+__global__ __launch_bounds__(256) void k_batch_sieve_decide(BatchDev b, BatchSieve s, float minScore, float minRatio,
+                                                            int* __restrict__ sel, int* __restrict__ flagList,
+                                                            int* __restrict__ counters,
                                                             int const* __restrict__ segMask)
 {
     int const si = b.segOfBlock[blockIdx.x];  // 256 queries of one segment
     if (segMask && !segMask[si]) return;
     int const g = blockIdx.x * kBatchRowAlign + threadIdx.x;
-    int const d = sieve_decision(best + g, second + g, minScore, minRatio);
-    if (d == kFlag) flagList[atomicAdd(&counters[kBCntFlag], 1)] = g;
+    int const lane = threadIdx.x & 63;
+    int const d = sieve_decision(s.best + g, s.second + g, minScore, minRatio);
     sel[g] = d;
+    unsigned long long const m = __builtin_amdgcn_ballot_w64(d == kFlag);
+    if (m == 0) return;
+    int const n = __builtin_popcountll(m);
+    int slot = 0;
+    if (lane == 0) {
+        slot = atomicAdd(&counters[kBCntFlag], n);
+        if (s.counters && !__hip_atomic_load(&counters[kBCntGate], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+            unsigned const blocks = (unsigned)n * ((b.seg[si].nO + 63) / 64);
+            unsigned const sum = atomicAdd(reinterpret_cast<unsigned*>(&counters[kBCntListed]), blocks) + blocks;
+            double const items = s.nItemsDev ? *s.nItemsDev : s.nItems;
+            if (sum > 16384.0 + items * s.tiles * (128.0 * kSieveBlocks * kSieveTile / 64 / 128))
+                __hip_atomic_store(&counters[kBCntGate], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    slot = __builtin_amdgcn_readfirstlane(slot);
+    if (d == kFlag)
+        flagList[slot + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] = g;
 }
 
-void launch_batch_sieve_decide(BatchDev const& b, unsigned long long* best, unsigned* second, float minScore,
-                               float minRatio, int* sel, int* flagList, int* counters, int const* segMask,
-                               hipStream_t st)
+void launch_batch_sieve_decide(BatchDev const& b, BatchSieve const& s, float minScore, float minRatio, int* sel,
+                               int* flagList, int* counters, int const* segMask, hipStream_t st)
 {
     static_assert(kBatchRowAlign == 256, "a work-group per query block");
     if (b.qRows <= 0) return;
-    hipLaunchKernelGGL(k_batch_sieve_decide, dim3(b.qRows / kBatchRowAlign), dim3(256), 0, st, b, best, second,
-                       minScore, minRatio, sel, flagList, counters, segMask);
+    hipLaunchKernelGGL(k_batch_sieve_decide, dim3(b.qRows / kBatchRowAlign), dim3(256), 0, st, b, s, minScore, minRatio,
+                       sel, flagList, counters, segMask);
 }
 
 // ------------------------------------------------------------------------------ rows of a batch

@@ -314,3 +314,113 @@ def test_many_candidates_on_the_device(kind, when):
         assert np.array_equal(got, want.reshape(-1, 2))
         assert np.array_equal(np.asarray(m.get_matches()).reshape(-1, 2), want.reshape(-1, 2))
     m.close()
+
+
+def _flooded_images(large, seed):
+    """uint8 images of uneven pairs, some of nearly equal rows on both sides: a small pair, whose
+    features are listed and re-checked within the bound, and with `large` pairs past it."""
+    rng = np.random.default_rng(seed)
+    images, shares = [], []
+    sizes = [(300, 700), (512, 480), (640, 513), (32, 32)] + ([(2080, 2048), (1504, 1700)] if large else [])
+    for p, (nL, nR) in enumerate(sizes):
+        a, b, _ = synth.make_pair(nL, nR, 0.5, config=3, pair=seed + p)
+        share = {1: 1.0, 4: 0.4, 5: 1.0}.get(p, 0.0)
+        c = synth.dequantise(a[:1])
+        out = []
+        for q in (a.copy(), b.copy()):
+            k = int(share * len(q))
+            at = rng.permutation(len(q))[:k]
+            q[at] = np.rint(512 * _unit(np.abs(c + 0.02 * rng.standard_normal((k, 128))))).clip(0, 255)
+            out.append(q)
+        images += out
+        shares.append(share)
+    return images, shares
+
+
+def _oracle_batch(images, min_score, min_ratio):
+    want = []
+    for p in range(len(images) // 2):
+        L, R = (synth.dequantise(q[:len(q) // 32 * 32]) for q in images[2 * p:2 * p + 2])
+        want.append(oracle.find_putative_matches(L, R, min_score, min_ratio).reshape(-1, 2))
+    return want
+
+
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("dtype", ["u8", "f32"])
+@pytest.mark.parametrize("cache", [False, True])
+@pytest.mark.parametrize("mode", ["fp32", "learned"])
+def test_batch_many_candidates(large, dtype, cache, mode):
+    """Batches with flooded pairs, in the plain form and as the pairs that a learned run hands over
+    (a constant code): the oracle's matches from the first run, from graph replays, without graphs,
+    with thresholds that take the full pass in between, and with settings changed between a run
+    and its reading."""
+    from v3dmatch import learned
+    print(f"case batch flooded large {large} {dtype} cache {cache} {mode}", flush=True)
+    images, shares = _flooded_images(large, 900)
+    left = np.arange(0, len(images), 2, dtype=np.int32)
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([len(q) for q in images],
+                       np.concatenate(images if dtype == "u8" else [synth.dequantise(q) for q in images]))
+    m.batch_set_pairs(left, left + 1)
+    m.set_derived_cache(cache)
+    if mode == "learned":
+        net = learned.Network(m)
+        params = learned.init_params(3)
+        params["W2"][:] = 0.0
+        params["b2"][:] = 1.0
+        net.set_params(params)
+        net.set_code_scale(60.0)
+        m.set_learned_topk(1)
+        m.set_fallback(128, 1.0)
+        m.set_precision(v3dmatch.PREC_LEARNED)
+    handed = 0
+    for ms, mr, graph in ((0.9, -1.0, True), (0.9, 0.8, True), (0.9, -1.0, True), (0.2, -1.0, True),
+                          (0.9, -1.0, False), (0.9, -1.0, True)):
+        m.batch_use_graph(graph)
+        m.batch_match_async(ms, mr)
+        m.set_certification(0.25)
+        offs, pairs = m.batch_get_matches()
+        again = m.batch_get_matches()
+        m.set_certification(2.0 ** -15)
+        assert np.array_equal(offs, again[0]) and np.array_equal(pairs, again[1])
+        flags = m.batch_get_fallback() if mode == "learned" else np.ones(len(left), int)
+        handed += int(flags.sum())
+        for p, w in enumerate(_oracle_batch(images, ms, mr)):
+            if flags[p]:
+                assert np.array_equal(pairs[offs[p]:offs[p + 1]], w), (p, ms, mr, graph)
+    assert handed >= 6 * len(left) // 2
+    if mode == "fp32":
+        assert m.batch_time_dominant_kernel(2) > 0
+        got = m.batch_match(0.9, -1.0)
+        assert all(np.array_equal(g, w) for g, w in zip(got, _oracle_batch(images, 0.9, -1.0)))
+    m.close()
+
+
+def test_batch_long_lists():
+    """Pairs large enough that a wave's run of right tiles holds more candidates than a single pair's
+    lists do (a small cluster on both sides), against the exact decisions of one pair."""
+    n, share = 12288, 0.045
+    print(f"case batch long lists {n} share {share}", flush=True)
+    rng = np.random.default_rng(31)
+    a, b, _ = synth.make_pair(n, n, 0.4, config=3, pair=950)
+    c = synth.dequantise(a[:1])
+    images = []
+    for q in (a.copy(), b.copy()):
+        k = int(share * n)
+        q[rng.permutation(n)[:k]] = np.rint(512 * _unit(np.abs(c + 0.02 * rng.standard_normal((k, 128))))).clip(0, 255)
+        images.append(q)
+    one = v3dmatch.SIFT_Matching(0)
+    one.allocate(n, n)
+    one.set_left_u8(images[0])
+    one.set_right_u8(images[1])
+    one.set_certification(0.0)
+    want = one.find_putative_matches_array(0.9, 0.8)
+    assert one.stats()["nRechecked"] == 2 * n
+    one.close()
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([n, n], np.concatenate(images))
+    m.batch_set_pairs([0] * 16, [1] * 16)
+    for _ in range(2):
+        for got in m.batch_match(0.9, 0.8):
+            assert np.array_equal(got, want)
+    m.close()
