@@ -129,9 +129,8 @@ def test_every_query_rechecked_exactly(matcher, nL, nR, seed):
 
 
 def test_result_larger_than_previous(matcher):
-    """The match list is copied in one piece sized from the previous result; a result much
-    larger than the previous one (here: 32 features, then 4096 features matched against
-    copies of themselves) is completed by a second copy."""
+    """A result much larger than the previous one (32 features, then 4096 features matched against
+    copies of themselves) arrives whole in the handle's pinned block."""
     m = matcher
     L, R, _ = _pair(32, 32, pair=21)
     _check(m, L, R, 32, 32)
@@ -141,4 +140,4 @@ def test_result_larger_than_previous(matcher):
     X = synth.dequantise(q)
     got = _check(m, X, X.copy(), 4096, 4096)
     say(f"  previous result {small} matches, this one {len(got)}")
-    assert len(got) > 1024 + small + small // 4  # larger than the first copy
+    assert len(got) > 1024 + small + small // 4

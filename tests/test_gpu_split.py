@@ -196,8 +196,8 @@ def test_batch_split(dtype, rows):
 @pytest.mark.parametrize("plain_first", [False, True])
 def test_batch_fallback_split(dtype, cache, plain_first):
     """The pairs that a learned run hands to the plain form (a constant code with one
-    candidate per query) get the exact matches, with the split rows made for them alone or left
-    by a plain run of the same images."""
+    candidate per query) get the exact matches, with the sieve's rows made for them alone or left
+    by a plain run of the same images (the full pass: test_batch_fallback_full_pass)."""
     from v3dmatch import learned
     qs, left, right = _batch(SIZES, 2)
     images = [synth.dequantise(q) for q in qs]
@@ -291,4 +291,82 @@ def test_many_open_queries(n, copies, guided):
     m.set_certification(0.0)
     assert np.array_equal(m.find_putative_matches_array(0.9, 0.8), oracle.find_putative_matches(L, R, 0.9, 0.8))
     assert m.stats()["nRechecked"] == 2 * n
+    m.close()
+
+
+# Thresholds that the sieve refuses (v3dm_sieve.h): these tests run the full pass.
+FULL = [(0.4, 0.99), (0.2, 0.8)]
+
+
+@pytest.mark.parametrize("nL,nR", [(32, 32), (64, 288), (288, 64), (256, 256), (544, 1056), (2272, 2080)])
+@pytest.mark.parametrize("min_score,min_ratio", FULL + [(-2.0, -1.0)])
+@pytest.mark.parametrize("sides", ["both", "left"])
+def test_u8_full_pass(matcher, nL, nR, min_score, min_ratio, sides):
+    """uint8 sets in the full pass: integer rows where both sides are uint8, split rows made from
+    dequantised rows where one is."""
+    print(f"case full pass u8 {sides} {nL} x {nR} min {min_score} ratio {min_ratio}", flush=True)
+    qL, qR, _ = synth.make_pair(nL, nR, 0.5, config=1, pair=nL + 3 * nR)
+    L, R = synth.dequantise(qL), synth.dequantise(qR)
+    matcher.set_left_u8(qL)
+    if sides == "both":
+        matcher.set_right_u8(qR)
+    else:
+        matcher.setRightFeatures(nR, R)
+    _check(matcher, L, R, min_score, min_ratio)
+
+
+@pytest.mark.parametrize("dtype", ["u8", "f32"])
+@pytest.mark.parametrize("cache", [False, True])
+@pytest.mark.parametrize("plain_first", [False, True])
+def test_batch_fallback_full_pass(dtype, cache, plain_first):
+    """test_batch_fallback_split at thresholds that refuse the sieve: the handed-over pairs' rows,
+    the pass over their listed items, the masked merge and the re-check, with the split rows made
+    for them alone or left by a plain run of the same images, and in turn with the sieve."""
+    from v3dmatch import learned
+    qs, left, right = _batch(SIZES, 2)
+    images = [synth.dequantise(q) for q in qs]
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([len(q) for q in qs], np.concatenate(qs if dtype == "u8" else images))
+    m.batch_set_pairs(left, right)
+    m.set_derived_cache(cache)
+    net = learned.Network(m)
+    params = learned.init_params(3)
+    params["W2"][:] = 0.0  # the same code for every descriptor: its candidates are arbitrary
+    params["b2"][:] = 1.0
+    net.set_params(params)
+    net.set_code_scale(60.0)
+    m.set_learned_topk(1)
+    m.set_fallback(128, 1.0)
+    for score, ratio in FULL + [(0.9, 0.8)] + FULL:
+        print(f"case fallback full pass {dtype} cache {cache} first {plain_first} min {score} ratio {ratio}", flush=True)
+        want = _want(images, left, right, score, ratio)
+        for mode in ([v3dmatch.PREC_FP32] if plain_first else []) + [v3dmatch.PREC_LEARNED] * 2:
+            m.set_precision(mode)
+            res = m.batch_match(score, ratio)
+            flags = m.batch_get_fallback() if mode == v3dmatch.PREC_LEARNED else np.ones(len(want), int)
+            for p, w in enumerate(want):
+                if flags[p]:
+                    assert np.array_equal(res[p], w), (p, score, ratio, mode)
+        assert flags.sum() >= 1
+    m.close()
+
+
+@pytest.mark.parametrize("dtype", ["u8", "f32"])
+@pytest.mark.parametrize("rows", [128, 256])
+def test_batch_shapes_full_pass(dtype, rows):
+    """Work-group shapes, items and grids of the full pass, at thresholds where a run takes it."""
+    qs, left, right = _batch(SIZES, 4)
+    images = [synth.dequantise(q) for q in qs]
+    m = v3dmatch.SIFT_Matching(0)
+    m.batch_set_images([len(q) for q in qs], np.concatenate(qs if dtype == "u8" else images))
+    m.batch_set_pairs(left, right)
+    m.batch_set_tile_shape(v3dmatch.PREC_FP32, rows)
+    for score, ratio in FULL:
+        want = _want(images, left, right, score, ratio)
+        for tiles, grid in ((0, 0), (1, 7), (5, 300), (64, 1024)):
+            print(f"case full pass {dtype} rows {rows} tiles {tiles} grid {grid} min {score}", flush=True)
+            m.batch_set_tuning(False, v3dmatch.PREC_FP32, tiles, grid)
+            for got, w in zip(m.batch_match(score, ratio), want):
+                assert np.array_equal(got, w)
+            assert m.batch_get_tile_shape(v3dmatch.PREC_FP32)["query_rows"] == rows
     m.close()
