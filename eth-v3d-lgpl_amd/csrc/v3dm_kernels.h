@@ -17,12 +17,12 @@ constexpr int kCntFlagR = 5;      // counters[5]: open right queries of the runn
 constexpr int kCntMutualError = 6;  // counters[6]: epoch of a mutual check whose ordering wait ran out
 constexpr int kCntScored = 7;     // counters[7]: candidates of the running call's fuller waves (cleared at its end)
 constexpr int kNumCounters = 8;
+constexpr int kSampleRows = 128;  // sampled check of a shortlist result: at most one left block
+constexpr int kSampleMaxSplits = 256;  // ... its right features split into up to 256 work-groups
+constexpr double kFallbackAlpha = 0.05;  // level of the sampled check's one-sided test
+constexpr int kFallbackMaxAccepted = 1 << 24;  // largest count v3dm_fallback_allowed_misses takes
 // Counts summed by many work-groups go to kStripes slots one cache line apart (atomics on a
 // single address serialise in L2); the gather kernel sums and clears them.
-constexpr int kSampleRows = 128;  // sampled check of a shortlist result: at most one left block
-constexpr int kSampleMaxSplits = 256;
-constexpr double kFallbackAlpha = 0.05;  // level of the sampled check's one-sided test
-constexpr int kFallbackMaxAccepted = 1 << 24;  // largest count v3dm_fallback_allowed_misses takes  // ... its right features split into up to 256 work-groups
 constexpr int kStripes = 64;
 constexpr int kStripeStride = 32;  // ints (128 bytes)
 constexpr int kRecheckMaxChunks = 64;  // re-check partials per row of either side

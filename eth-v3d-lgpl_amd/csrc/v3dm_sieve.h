@@ -18,7 +18,11 @@ namespace v3dm {
 //
 // Rule: sets in the range of the split pass (finite rows, v3dm_split.h), certification on, and
 // T >= kSieveMin.  Unrelated SIFT descriptors score below that, so a query has a handful of
-// candidates; with a lower T most pairs would be candidates and the full score pass is faster.
+// candidates; with a low T most pairs would be candidates and the full score pass is faster.
+// Finds in us by T, sieve / full pass (FP32 uploads; uint8 ones): 4096 x 4096 0.6: 103 / 54 (42),
+// 0.65: 34 / 52 (41), 0.75: 33 / 47 (41); 16384 x 16384 0.6: 415 / 292 (181), 0.65: 72 / 233 (143),
+// 0.75: 56 / 206 (134).  The line lies above the crossing of synthetic SIFT sets, for sets whose
+// unrelated descriptors score higher.
 constexpr float kSieveMin = 0.75f;
 constexpr float kSieveScale = 256.0f;
 constexpr int kSieveTile = 32;

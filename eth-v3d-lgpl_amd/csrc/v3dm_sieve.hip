@@ -267,7 +267,7 @@ void launch_sieve(SieveSet const& L, SieveSet const& R, SievePlan const& p, unsi
 
 // Over a batch: item = (pair, group of 512 left features, split, tiles per split), one
 // work-group each.
-// 256 uneven uint8 pairs: 531 us (2.9 TB/s would read the rows, 3.4 POPS of int8 products) + 13 for
+// 256 uneven uint8 pairs: 537 us (2.9 TB/s would read the rows, 3.4 POPS of int8 products) + 13 for
 // the decisions, against 2358 + 167 + 23 of the integer-row pass, its merge and its re-check.
 __device__ __forceinline__ void sieve_item(BatchDev const& b, BatchSieve const& s, int4 w, int t0, int t1, int n,
                                            int limit, int* list, int wv)
