@@ -73,19 +73,20 @@ struct SieveBest {
 };
 
 // The bounds of `pairs` scores: about the full pass's time each (45 us of launches and a second
-// wait, and 1.3 * 10^6 scores per us).  The card scores 3000 listed candidates per us and re-checks
-// 60000 pairs per us.  A wave's candidates are a chain of rounds of 64, 10 us each: one round for
-// the short runs of small sets, whose full pass is short too, eight for long ones, which may hold a
-// small cluster by themselves (SIFT sets have about ten candidates a wave).  Calls in us with a
-// share of both sides in one cluster of nearly equal rows, 0 / 2 / 10 / 50%: 16384 x 16384 60 / 104 /
-// 334 / 335, 8192 x 8192 40 / 47 / 139 / 153, 2048 x 2048 30 / 30 / 87 / 75; with lists of 2048 and
-// no bounds 60 / 91 / 827 / 15528, 40 / 46 / 263 / 5895 and 29 / 30 / 55 / 457; with the FP32
-// instruction 735, 248 and 81 at any share.
-__host__ __device__ inline unsigned sieve_most_scored(double pairs) { return (unsigned)(135000.0 + pairs / 430); }
+// wait, and 1.3 * 10^6 scores per us).  The card takes 3000 candidates per us, with their listing
+// and entering, and re-checks 60000 pairs per us.  A wave's candidates are a chain of rounds of 64
+// of about 10 us: one and a half for the short runs of small sets, whose full pass is short too,
+// eight for long ones, which may hold a small cluster by themselves (SIFT sets have about ten
+// candidates a wave).  Calls in us with a share of both sides in one cluster of nearly equal rows,
+// 0 / 2 / 5 / 10 / 50%: 16384 x 16384 60 / 99 / 465 / 334 / 332, 8192 x 8192 41 / 48 / 106 / 281 / 154,
+// 2048 x 2048 30 / 30 / 36 / 86 / 76; with lists of 2048 and no bounds 61 / 93 / 257 / 857 / 15555,
+// 40 / 46 / 94 / 252 / 5885 and 29 / 29 / 35 / 54 / 435; with the FP32 instruction 740, 245 and 80 at
+// any share.  Lower limits move the two lower figures of the middle up, higher ones the third.
+__host__ __device__ inline unsigned sieve_most_scored(double pairs) { return (unsigned)(120000.0 + pairs / 700); }
 inline long long sieve_most_listed(double pairs) { return (1LL << 20) + (long long)(pairs / 32); }
 inline int sieve_limit(long long pairs)  // of a wave of `pairs` scores
 {
-    return pairs < 64 * 128 ? 64 : pairs < kSieveList * 128LL ? (int)(pairs / 128) : kSieveList;
+    return pairs < 96 * 64 ? 96 : pairs < kSieveList * 64 ? (int)(pairs / 64) : kSieveList;
 }
 
 struct SievePlan {

@@ -46,6 +46,7 @@ bool sieve_bound(float minScore, float minRatio, float* T)
 // against 182 + 6 + 14 of the FP16 split pass, its merge and its re-check (605 of the FP32
 // instruction); 4096 x 4096: 12 + 3 against 24 + 5 + 4; 480 x 512: 9 + 2 against 8 + 5 + 4.
 constexpr int kSieveBlocks = 4;
+constexpr int kSieveLook = 32;  // candidates of a wave above which entries are read before the atomics
 
 __device__ __forceinline__ int max3i(int a, int b, int c) { return max(max(a, b), c); }
 
@@ -88,8 +89,16 @@ __device__ __forceinline__ float sieve_exact(float const* __restrict__ x, float 
     return (float)acc;
 }
 
-__device__ __forceinline__ void sieve_enter(unsigned long long* best, unsigned* second, unsigned long long key)
+// look: the entries are read first (they only grow, so an older value is as good), and a key that
+// changes neither is dropped: with many candidates a feature, most are.
+__device__ __forceinline__ void sieve_enter(unsigned long long* best, unsigned* second, unsigned long long key,
+                                            bool look)
 {
+    if (look) {
+        unsigned const s2 = __hip_atomic_load(second, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((unsigned)(key >> 32) <= s2 && key < __hip_atomic_load(best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            return;
+    }
     unsigned long long const old = atomicMax(best, key);
     unsigned const loser = (unsigned)((old < key ? old : key) >> 32);
     if (loser) atomicMax(second, loser);
@@ -215,8 +224,8 @@ __device__ __forceinline__ void sieve_wave(SieveSet const& L, SieveSet const& R,
         float const s = sieve_exact(L.X + (size_t)i * kDim, R.X + (size_t)j * kDim);
         if (!(s > 0.0f)) continue;  // T > 0: cannot matter
         unsigned long long const v = (unsigned long long)__float_as_uint(s) << 32;
-        sieve_enter(bestL + i, secondL + i, v | (0xffffffffu - (unsigned)j));
-        sieve_enter(bestR + j, secondR + j, v | (0xffffffffu - (unsigned)i));
+        sieve_enter(bestL + i, secondL + i, v | (0xffffffffu - (unsigned)j), cnt > kSieveLook);
+        sieve_enter(bestR + j, secondR + j, v | (0xffffffffu - (unsigned)i), cnt > kSieveLook);
     }
 }
 
